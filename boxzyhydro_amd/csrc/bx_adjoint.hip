@@ -1016,12 +1016,8 @@ extern "C" int bx_adjoint_forward(bx_ctx *c, int32_t nsteps, int32_t every, cons
             j->dlog_cap = nsteps;
         }
         DevScalars *h = c->hsc;  // rate_bits[0]: the Courant rate of the regular check above
-        h->time = 0.0;
-        h->dtold = 0.0;
-        h->step = 0;
-        h->endtime = std::numeric_limits<double>::infinity();
+        h->slot[0] = StepSlot{0.0, 0.0, 0.0, std::numeric_limits<double>::infinity(), 0, 0};
         h->flags = 0;
-        h->logk = 0;
         BX_HIP(hipMemcpyAsync(c->dsc, h, sizeof(DevScalars), hipMemcpyHostToDevice, c->stream));
     }
     // Once the steps have started, the context's state, its u/p/cons_old planes
@@ -1062,7 +1058,7 @@ extern "C" int bx_adjoint_forward(bx_ctx *c, int32_t nsteps, int32_t every, cons
                 return rc;
             }
             j->dts[k] = dts_in[k];
-        } else if ((rc = fused_step_device_dt(c, u0, us, ps, un, j->dlog, nsteps))) {
+        } else if ((rc = fused_step_device_dt(c, k, u0, us, ps, un, j->dlog, nsteps))) {
             invalidate(false);
             return rc;
         }
@@ -1078,6 +1074,7 @@ extern "C" int bx_adjoint_forward(bx_ctx *c, int32_t nsteps, int32_t every, cons
         invalidate(false);
         return rc;
     }
+    if (!frozen && (nsteps & 1)) c->hsc->rate_bits[0] = c->hsc->rate_bits[1];  // the last step's, [nsteps & 1]
     if (flags & (FLAG_IRREGULAR | FLAG_FLOOR)) return refuse(flags);
     if (dts_out)
         for (int k = 0; k < nsteps; k++) dts_out[k] = j->dts[k];

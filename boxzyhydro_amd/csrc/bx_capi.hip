@@ -6,9 +6,11 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <memory>
 #include <new>
 
 #include "bx_internal.h"
+#include "bx_stage.h"
 
 namespace {
 thread_local std::string g_last_error;
@@ -103,16 +105,39 @@ static int build_ghost_table(const bx_params *prm, std::vector<int32_t> &dst, st
         return ineigh;
     };
 
-    // ghost list in cell order (init_grid.f90:166-206)
+    // ghost list in cell order (init_grid.f90:166-206); of a row that is no
+    // ghost row only the two cells at either end can be ghosts
     std::vector<int32_t> ghosts;
     for (int iz = 1; iz <= nz; iz++)
-        for (int iy = 1; iy <= ny; iy++)
-            for (int ix = 1; ix <= nx; ix++)
+        for (int iy = 1; iy <= ny; iy++) {
+            const bool row = iy < 3 || iy > ny - 2 || (nz >= 6 && (iz < 3 || iz > nz - 2));
+            for (int ix = 1; ix <= nx; ix++) {
+                if (!row && ix == 3) ix = std::max(3, nx - 1);
                 if (bnd(ix, iy, iz) > 0) ghosts.push_back(id(ix, iy, iz));
+            }
+        }
 
-    std::vector<int32_t> vsrc(n);
-    std::vector<uint8_t> vsg(n, 0);
-    for (int64_t k = 0; k < n; k++) vsrc[k] = (int32_t)k;
+    // symbolic values, set here for the ghosts only: an interior cell is itself
+    std::unique_ptr<int32_t[]> gsrc(new int32_t[n]);
+    std::unique_ptr<uint8_t[]> gsgn(new uint8_t[n]);
+    for (int32_t g : ghosts) {
+        gsrc[g] = g;
+        gsgn[g] = 0;
+    }
+    auto inside = [&](int32_t c) {
+        const int ix = c % nx + 1, iy = (c / nx) % ny + 1, iz = c / (nx * ny) + 1;
+        return bnd(ix, iy, iz) == 0;
+    };
+    auto take = [&](int32_t g, int32_t from, unsigned flip) {
+        if (inside(from)) {
+            gsrc[g] = from;
+            gsgn[g] = (uint8_t)flip;
+        } else {
+            const int32_t v = gsrc[from];
+            gsgn[g] = (uint8_t)(gsgn[from] ^ flip);
+            gsrc[g] = v;
+        }
+    };
     const int32_t *nof = prm->no_outflow;
     const bool zwall = nz >= 6;  // init_grid.f90:76-79
     auto pass = [&]() {
@@ -137,12 +162,8 @@ static int build_ghost_table(const bx_params *prm, std::vector<int32_t> &dst, st
                 else if (iz == nz - 1) ineigh = nz < 6 ? g : g - pl;
             }
             ineigh = check_corner(ix, iy, iz, ineigh);
-            vsrc[g] = vsrc[ineigh];
-            vsg[g] = vsg[ineigh];
-            auto mirror = [&](int32_t ip, int bit) {
-                vsrc[g] = vsrc[ip];
-                vsg[g] = (uint8_t)(vsg[ip] ^ (1u << bit));
-            };
+            take(g, ineigh, 0u);
+            auto mirror = [&](int32_t ip, int bit) { take(g, ip, 1u << bit); };
             if (nof[0]) {
                 if (ix == 1) mirror(id(ix + 3, iy, iz), 0);
                 else if (ix == 2) mirror(id(ix + 1, iy, iz), 0);
@@ -177,11 +198,11 @@ static int build_ghost_table(const bx_params *prm, std::vector<int32_t> &dst, st
     src.clear();
     sgn.clear();
     scratch_src.clear();
-    std::vector<int32_t> slot(n, -1);
+    std::vector<int32_t> slot;
     for (int32_t g : ghosts) {
-        int32_t s = vsrc[g];
-        int sx = s % nx + 1, sy = (s / nx) % ny + 1, sz = s / (nx * ny) + 1;
-        if (bnd(sx, sy, sz) != 0) {
+        int32_t s = gsrc[g];
+        if (!inside(s)) {
+            if (slot.empty()) slot.assign(n, -1);
             if (slot[s] < 0) {
                 slot[s] = (int32_t)scratch_src.size();
                 scratch_src.push_back(s);
@@ -190,7 +211,7 @@ static int build_ghost_table(const bx_params *prm, std::vector<int32_t> &dst, st
         }
         dst.push_back(g);
         src.push_back(s);
-        sgn.push_back(vsg[g]);
+        sgn.push_back(gsgn[g]);
     }
     return BX_OK;
 }
@@ -263,6 +284,7 @@ int bx_create(const bx_params *prm, int32_t device, bx_ctx **out)
     // step as +-(v's corrector result before source(1)) and is fixed up after
     // the ghost fill.  Deeper chains take the exact sequence.
     std::vector<int32_t> fs(gs), fg(gg), d2dst, d2src, d2sign;
+    std::vector<size_t> d2at;  // their entries in the tables
     c->fghost_ok = true;
     if (!gx.empty()) {
         std::vector<int64_t> entry((size_t)n, -1);
@@ -300,14 +322,53 @@ int bx_create(const bx_params *prm, int32_t device, bx_ctx **out)
             }
             fs[k] = cell2;
             fg[k] = sgn ^ sgn2;
+            d2at.push_back(k);
             d2dst.push_back(gd[k]);
             d2src.push_back(cell2);
             d2sign.push_back(sgn ^ sgn2);
         }
         if ((int)d2dst.size() > kMaxD2) c->fghost_ok = false;
-        if (!c->fghost_ok) d2dst.clear();
+        if (!c->fghost_ok) {
+            d2dst.clear();
+            d2at.clear();
+        }
     }
     c->nd2 = (int)d2dst.size();
+    // whether every ghost's composed donor is the per-axis one (the ghosts are
+    // in cell order: one row after another)
+    c->axis_ghosts = c->fghost_ok;
+    {
+        std::vector<int32_t> to[3];
+        std::vector<uint8_t> flip[3];
+        const int dim[3] = {c->nx, c->ny, c->nz};
+        for (int d = 0; d < 3; d++)
+            for (int i = 0; i < dim[d]; i++) {
+                const int lo = c->prm.no_outflow[2 * d], hi = c->prm.no_outflow[2 * d + 1];
+                const bool axis = d < 2 || !c->flatz;
+                const int t = axis ? axis_donor(i, dim[d], lo, hi) : i;
+                to[d].push_back(t);
+                flip[d].push_back(axis && axis_flip(i, dim[d], lo, hi));
+                if (axis && (t < 2 || t > dim[d] - 3)) c->axis_ghosts = false;
+            }
+        int64_t row = 0;
+        int iy = 0, iz = 0;
+        for (size_t k = 0; k < gd.size() && c->axis_ghosts; k++) {
+            while (gd[k] - row >= c->nx) {
+                row += c->nx;
+                if (++iy == c->ny) iy = 0, iz++;
+            }
+            const int ix = (int)(gd[k] - row);
+            c->axis_ghosts = fg[k] == (flip[0][ix] | flip[1][iy] << 1 | flip[2][iz] << 2) &&
+                             fs[k] == to[0][ix] + c->nx * (to[1][iy] + c->ny * to[2][iz]);
+        }
+    }
+    // the corner ghosts last in the tables, so that a fill can leave them out
+    for (auto *t : {&gd, &gs, &gg, &fs, &fg}) {
+        std::vector<int32_t> last;
+        for (size_t k : d2at) last.push_back((*t)[k]);
+        for (size_t q = d2at.size(); q-- > 0;) t->erase(t->begin() + (int64_t)d2at[q]);
+        t->insert(t->end(), last.begin(), last.end());
+    }
 
     auto fail = [&](hipError_t e, const char *what) {
         int r = hip_check(e, what);
@@ -810,52 +871,60 @@ static int chunk_steps(double time, double dtold, double endtime, int32_t step, 
     return k & ~1;
 }
 
-// K steps replayed from the captured pair (BX_STEP_GRAPH).  The state at the
-// chunk's start is kept; if any step met an irregular branch the chunk is
-// undone (*taken = 0) and the caller takes those steps one at a time.
-static int graph_chunk(bx_ctx *c, int K, double endtime, double *time, double *dtold, int32_t *step, double *dts,
-                       int32_t *taken)
+// A run of K steps with dt formed on the device: replayed from the captured
+// pair (BX_STEP_GRAPH) or enqueued.  The state at the run's start is kept; if
+// any step met an irregular branch the run is undone (*taken = 0) and the
+// caller takes those steps one at a time.
+static int step_run(bx_ctx *c, int K, double endtime, double *time, double *dtold, int32_t *step, double *dts,
+                    int32_t *taken, bool graph)
 {
     *taken = 0;
     const size_t bytes = (c->state_in_32 ? sizeof(float) : sizeof(double)) * 5 * (size_t)c->n;
     void *cur = c->state_in_32 ? (void *)c->cons32 : (void *)c->cons;
-    if (!c->chunk0) BX_HIP(hipMalloc(&c->chunk0, sizeof(double) * 5 * (size_t)c->n));
+    if (!c->chunk0) {
+        const hipError_t e = hipMalloc(&c->chunk0, sizeof(double) * 5 * (size_t)c->n);
+        if (e != hipSuccess) {
+            c->chunk0 = nullptr;
+            if (graph) return hip_check(e, "hipMalloc run start");
+            (void)hipGetLastError();
+            return BX_OK;  // no room for the copy: one step at a time
+        }
+    }
     BX_HIP(hipMemcpyAsync(c->chunk0, cur, bytes, hipMemcpyDeviceToDevice, c->stream));
     const unsigned long long rate0 = c->hsc->rate_bits[0];  // Courant rate of the current state
     DevScalars *h = c->hsc;
-    h->time = *time;
-    h->dtold = *dtold;
-    h->step = *step;
-    h->endtime = endtime;
+    h->slot[0] = StepSlot{0.0, *dtold, *time, endtime, *step, 0};
     h->flags = 0;
-    h->logk = 0;
     BX_HIP(hipMemcpyAsync(c->dsc, h, sizeof(DevScalars), hipMemcpyHostToDevice, c->stream));
-    if (int rc = replay_step_pairs(c, K / 2)) return rc;
+    if (int rc = run_step_pairs(c, K / 2, graph)) return rc;
     double log[kChunkSteps];
     BX_HIP(hipMemcpyAsync(log, c->chunk_dts, sizeof(double) * K, hipMemcpyDeviceToHost, c->stream));
     if (int rc = read_scalars(c)) return rc;
-    if ((h->flags & FLAG_IRREGULAR) || h->step != *step + K) {
+    const StepSlot &s = h->slot[0];  // after an even number of steps
+    if ((h->flags & FLAG_IRREGULAR) || s.step != *step + K) {
         BX_HIP(hipMemcpyAsync(cur, c->chunk0, bytes, hipMemcpyDeviceToDevice, c->stream));
         h->rate_bits[0] = rate0;
         return BX_OK;
     }
-    *time = h->time + h->dt;  // the last step's main.f90:545 (the device advanced time for the others)
-    *dtold = h->dtold;
-    *step = h->step;
+    *time = s.time + s.dt;  // the last step's main.f90:545 (the device advanced time for the others)
+    *dtold = s.dtold;
+    *step = s.step;
     if (dts)
         for (int i = 0; i < K; i++) dts[i] = log[i];
     c->aux_stale = true;
     c->old_stale = true;
     c->p_fused = c->grav_flags != 0;
-    c->graph_steps += K;
+    if (graph) c->graph_steps += K;
     c->nfused += K;
     *taken = K;
     return BX_OK;
 }
 
 // Fused stepping (see include/boxzy.h): returns after `nsteps` steps or
-// endtime.  With `graph`, runs of steps that cannot reach endtime are replayed
-// from a captured pair of steps, with dt formed on the device.
+// endtime.  Runs of steps that cannot reach endtime are enqueued with dt formed
+// on the device and one read-back per run (with `graph`, replayed from a
+// captured pair of steps); the others are taken one at a time.  A read-back
+// per step left the chip idle for 15 of 96 us per step at 32^3.
 static int fused_loop(bx_ctx *c, int32_t nsteps, double endtime, double *time, double *dtold, int32_t *step,
                       double *dts, int32_t *taken, bool graph)
 {
@@ -895,11 +964,12 @@ static int fused_loop(bx_ctx *c, int32_t nsteps, double endtime, double *time, d
                 c->state_in_32 = true;
             }
         }
-        if (graph && single == 0 && !c->prof_on) {
+        if (single == 0 && !c->prof_on) {
             const int K = chunk_steps(*time, *dtold, endtime, *step, nsteps - k);
             if (K >= 2) {
                 int32_t got = 0;
-                if ((rc = graph_chunk(c, K, endtime, time, dtold, step, dts ? dts + k : nullptr, &got))) return rc;
+                if ((rc = step_run(c, K, endtime, time, dtold, step, dts ? dts + k : nullptr, &got, graph)))
+                    return rc;
                 if (got) {
                     k += got;
                     continue;
@@ -919,7 +989,7 @@ static int fused_loop(bx_ctx *c, int32_t nsteps, double endtime, double *time, d
             // an irregular branch: redo this step with the exact sequence from U^n
             // (replays resume after a full chunk's worth of regular steps)
             c->fallbacks++;
-            if (graph) single = kChunkSteps;
+            single = kChunkSteps;
             *time = time0;
             *dtold = dtold0;
             *step = step0;

@@ -41,7 +41,8 @@ namespace bx {
 // LDS, marching in z (bx_tile.h: tile_stage).  P2: every spacing and the
 // cell volume are powers of two (their divisions are multiplications), known
 // at compile time, which keeps the spacings themselves out of the registers.
-template <int STAGE, typename S, int TY, bool P2, bool G = false>
+// G: gravity; W: walls whose ghosts are read from their donors (bx_tile.h).
+template <int STAGE, typename S, int TY, bool P2, bool G, bool W>
 __global__ __launch_bounds__(64 * (TY + 4)) void k_stage(StageArgs a0)
 {
     __shared__ TileLds<S, TY> lds;
@@ -59,7 +60,7 @@ __global__ __launch_bounds__(64 * (TY + 4)) void k_stage(StageArgs a0)
     const unsigned L = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);
     const unsigned xcd = L & 7u, slot = L >> 3, q = T >> 3, rem = T & 7u;
     const unsigned t = xcd * q + (xcd < rem ? xcd : rem) + slot;
-    tile_stage<STAGE, S, TY, G>(a, lds, t % gx, (t / gx) % gy, t / (gx * gy));
+    tile_stage<STAGE, S, TY, G, W>(a, lds, t % gx, (t / gx) % gy, t / (gx * gy));
 }
 
 
@@ -170,8 +171,8 @@ StageArgs base_args(bx_ctx *c, double dt)
     return a;
 }
 
-template <int STAGE, typename S, int TY>
-static int launch_tile(bx_ctx *c, const StageArgs &a)
+template <int STAGE, typename S, int TY, bool W>
+static int launch_tile_w(bx_ctx *c, const StageArgs &a)
 {
     const bool p2 = a.ds_pow2[0] && a.ds_pow2[1] && a.ds_pow2[2] && a.vol_pow2;
     const int nzi = a.zhi - a.zlo;
@@ -183,19 +184,29 @@ static int launch_tile(bx_ctx *c, const StageArgs &a)
         if (a.gf) {
             // the corrector's power-of-two form spills 5 VGPRs at 168; its
             // general form (161, no spill) gives the same bits and is ~1 % faster
-            if (p2 && STAGE == 1) hipLaunchKernelGGL((k_stage<STAGE, S, TY, true, true>), grid, block, 0, c->stream, a);
-            else hipLaunchKernelGGL((k_stage<STAGE, S, TY, false, true>), grid, block, 0, c->stream, a);
+            if (p2 && STAGE == 1)
+                hipLaunchKernelGGL((k_stage<STAGE, S, TY, true, true, W>), grid, block, 0, c->stream, a);
+            else
+                hipLaunchKernelGGL((k_stage<STAGE, S, TY, false, true, W>), grid, block, 0, c->stream, a);
             BX_HIP(hipGetLastError());
             return BX_OK;
         }
     }
     if (a.gf) return set_error(BX_ERR_UNSUPPORTED, "fused step with gravity: FP64 64 x 8 tiles only");
     if (p2)
-        hipLaunchKernelGGL((k_stage<STAGE, S, TY, true>), grid, block, 0, c->stream, a);
+        hipLaunchKernelGGL((k_stage<STAGE, S, TY, true, false, W>), grid, block, 0, c->stream, a);
     else
-        hipLaunchKernelGGL((k_stage<STAGE, S, TY, false>), grid, block, 0, c->stream, a);
+        hipLaunchKernelGGL((k_stage<STAGE, S, TY, false, false, W>), grid, block, 0, c->stream, a);
     BX_HIP(hipGetLastError());
     return BX_OK;
+}
+
+template <int STAGE, typename S, int TY>
+static int launch_tile(bx_ctx *c, const StageArgs &a)
+{
+    bool w = false;
+    for (int i = 0; i < 6; i++) w = w || (a.gmap && a.wall[i]);
+    return w ? launch_tile_w<STAGE, S, TY, true>(c, a) : launch_tile_w<STAGE, S, TY, false>(c, a);
 }
 
 template <int STAGE, typename S>
@@ -274,12 +285,26 @@ int fused_supported(const bx_ctx *c)
     return BX_OK;
 }
 
-// Default work split of the stage kernels: one kernel per stage, FP64 on
-// 64 x 8 tiles (variant 11) with z-chunks of 64 planes, the mixed form on
-// 64 x 4 tiles (variant 10, its FP32 tiles being small enough for several
-// workgroups per CU) with chunks of 32; the chunks are shortened until the
-// grid has two workgroups per CU.  The y chunk (fused_ly) only serves the
-// two-kernel variants.  Allocates nothing.
+// Default work split of the stage kernels: one kernel per stage, marching in z
+// chunks of the interior planes (any length: the chunk is nzi/m rounded up for
+// m chunks).  A workgroup's time is (planes it marches) x (time per plane) + a
+// start that does not depend on the chunk (launch, the first planes of the z
+// queue), so the chunk minimises that over the rounds of workgroups each CU
+// takes; ties go to the longer chunk.  Constants in us for both stages
+// together, from sweeps of the chunk at 16^3..256^3 (MI355X):
+//   FP64, 64 x 8 tiles (variant 11): one workgroup per CU (LDS), 13 per plane
+//     + 33.  96^3: chunk 10 (240 workgroups) 172 us, 16 (144) 247 us.
+//   FP64, 64 x 4 tiles (variant 10): one workgroup per CU, 8.5 per plane + 30:
+//     half the rows per CU, so faster where the 8-row tiles leave CUs idle
+//     (32^3 with one plane each: 50 us against 55; 85 us with chunks of 4
+//     planes on 8-row tiles), and slower where they fill the chip (256^3: 2.5
+//     against 1.95 ms).
+//   Mixed, 64 x 4 tiles: several workgroups share a CU and its issue slots, so
+//     the time is (workgroups per CU) x (chunk + 2 planes), with one alone on
+//     its CU, which waits for its own latencies, counted as 1.6.  192^3: chunk
+//     28 489 us, 32 545 us; 64^3: chunk 2 56 us, 4 64 us.
+// The y chunk (fused_ly) only serves the two-kernel variants.  Allocates
+// nothing.
 void fused_defaults(bx_ctx *c)
 {
     const int64_t want = 2 * 1024;
@@ -290,33 +315,25 @@ void fused_defaults(bx_ctx *c)
         c->fused_ly = ly;
     }
     if (c->fused_lz == 0) {
-        if (c->prm.precision == BX_PREC_MIXED) {
-            int lz = 32;
-            const int64_t tiles = (int64_t)((c->nx - 4 + 63) / 64) * ((c->ny - 4 + 3) / 4);
-            while (lz > 4 && tiles * ((nzi + lz - 1) / lz) < 512) lz /= 2;
-            c->fused_lz = lz;
-            c->fused_occ = 10;
-        } else {
-            // One workgroup per CU at a time (LDS): the chunk that minimises
-            // the rounds of workgroups times the planes each one marches
-            // (its chunk and the 4 halo planes); ties go to the smaller chunk
-            int ncu = 0;
-            if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess ||
-                ncu < 1)
-                ncu = 256;
-            const int64_t tiles = (int64_t)((c->nx - 4 + 63) / 64) * ((c->ny - 4 + 7) / 8);
-            int lz = 4;
-            int64_t best = INT64_MAX;
-            for (int cand = 4; cand <= 256; cand *= 2) {
-                const int64_t chunks = (nzi + cand - 1) / cand;
-                const int64_t cost = (tiles * chunks + ncu - 1) / ncu * ((cand < nzi ? cand : nzi) + 4);
+        int ncu = 0;
+        if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess || ncu < 1)
+            ncu = 256;
+        const bool mixed = c->prm.precision == BX_PREC_MIXED;
+        double best = HUGE_VAL;
+        for (int ty = 8; ty >= 4; ty -= 4) {
+            if (mixed ? ty == 8 : (ty == 4 && c->grav_flags)) continue;  // gravity has the 64 x 8 tiles only
+            const int64_t tiles = (int64_t)((c->nx - 4 + 63) / 64) * ((c->ny - 4 + ty - 1) / ty);
+            for (int m = 1; m <= nzi && m <= 4 * ncu; m++) {
+                const int lz = (nzi + m - 1) / m;
+                const double rounds = (double)((tiles * ((nzi + lz - 1) / lz) + ncu - 1) / ncu);
+                const double cost = mixed ? std::fmax(rounds, 1.6) * (lz + 2)
+                                          : rounds * (ty == 8 ? 13.0 * lz + 33.0 : 8.5 * lz + 30.0);
                 if (cost < best) {
                     best = cost;
-                    lz = cand;
+                    c->fused_lz = lz;
+                    c->fused_occ = ty == 8 ? 11 : 10;
                 }
             }
-            c->fused_lz = lz;
-            c->fused_occ = 11;
         }
     }
 }
@@ -354,11 +371,14 @@ int launch_regular_check(bx_ctx *c)
     return BX_OK;
 }
 
+// corners: whether to fill the two-level corner ghosts too (the last nd2
+// entries of the table) or leave what the fix-up wrote
 template <typename S>
-static int ghosts6(bx_ctx *c, S *planes, S *pstar)
+static int ghosts6(bx_ctx *c, S *planes, S *pstar, bool corners = true)
 {
-    if (c->nghost == 0) return BX_OK;
-    hipLaunchKernelGGL(k_ghosts6<S>, dim3(blocks_for(c->nghost, 256)), dim3(256), 0, c->stream, c->n, c->nghost,
+    const int64_t ng = c->nghost - (corners ? 0 : c->nd2);
+    if (ng <= 0) return BX_OK;
+    hipLaunchKernelGGL(k_ghosts6<S>, dim3(blocks_for(ng, 256)), dim3(256), 0, c->stream, c->n, ng,
                        c->ghost_dst, c->nscratch ? c->fghost_src : c->ghost_src,
                        c->nscratch ? c->fghost_sign : c->ghost_sign, planes, pstar);
     BX_HIP(hipGetLastError());
@@ -369,49 +389,58 @@ static int ghosts6(bx_ctx *c, S *planes, S *pstar)
 // sequence leaves such a ghost holding +-(its interior cell v's corrector
 // result before source(1)); that value reaches the results only through the
 // next step's Courant rate (courant.f90:11-15 runs over every cell) and the
-// stored state.  One lane per ghost evaluates v's corrector update again
-// from the corrector's inputs with the tiled kernel's operations (its six
-// faces, flux.f90:121-190, and the update of flux.f90:213-228), parks the
+// stored state.  One workgroup per ghost evaluates v's corrector update
+// again from the corrector's inputs with the tiled kernel's operations (its
+// six faces, flux.f90:121-190, and the update of flux.f90:213-228), parks the
 // result before source(1), writes the ghost and adds its Courant rate (the
 // state and velocity of main.f90:232 and of the step's last velocity call,
-// state.f90:30-57, velocity.f90:18-21).
-__global__ __launch_bounds__(64) void k_corner_ghosts(StageArgs a0, const int32_t *__restrict__ dst,
+// state.f90:30-57, velocity.f90:18-21).  The kernel is a serial chain of
+// divisions and roots on a step's critical path: one wave takes each
+// direction and one lane each of its two faces, so that a sixth of the faces
+// lies on the chain (with one lane per ghost taking all six: 18.0 us).
+__global__ __launch_bounds__(192) void k_corner_ghosts(StageArgs a0, const int32_t *__restrict__ dst,
                                                       const int32_t *__restrict__ sign)
 {
     const StageArgs a = with_dt(a0);
-    const int j = threadIdx.x;
+    __shared__ double F[3][2][5];
+    const int j = blockIdx.x, d = wave_id(), h = threadIdx.x & 63;
     double rt = 0.0;
     unsigned int flg = 0;
-    if (j < a.nd2) {
-        const int64_t v = a.d2cell[j];
-        const int64_t plane = (int64_t)a.nx * a.ny;
-        const int ix = (int)(v % a.nx), iy = (int)((v / a.nx) % a.ny), iz = (int)(v / plane);
-        auto ghost = [&](int x, int y, int z) {
-            return x < 2 || x > a.nx - 3 || y < 2 || y > a.ny - 3 || (!a.flatz && (z < 2 || z > a.nz - 3));
-        };
-        double F[3][2][5];
-        for (int d = 0; d < 3; d++)
-            for (int h = 0; h < 2; h++)
-                for (int i = 0; i < 5; i++) F[d][h][i] = 0.0;
-        W6<double> q0{};
-        auto faces = [&](auto dirc) {
-            constexpr int d = decltype(dirc)::value;
-            const int64_t e = d == 0 ? 1 : (d == 1 ? a.nx : plane);
-            W6<double> w[5];
-            for (int i = 0; i < 5; i++) w[i] = load_prims<2, double>(a, v + (i - 2) * e, 0u, flg);
-            if (d == 0) q0 = w[2];
-            Side<double> mi[3], pl[3];
-            for (int i = 1; i <= 3; i++) {
-                const int o = i - 2;
-                const bool gh = ghost(ix + (d == 0 ? o : 0), iy + (d == 1 ? o : 0), iz + (d == 2 ? o : 0));
-                dir_states<d>(w[i - 1], w[i], w[i + 1], sound_of(w[i], a.gam), gh, a, mi[i - 1], pl[i - 1]);
+    const int64_t v = a.d2cell[j];
+    const int64_t plane = (int64_t)a.nx * a.ny;
+    const int ix = (int)(v % a.nx), iy = (int)((v / a.nx) % a.ny), iz = (int)(v / plane);
+    // the primitives of the cell o cells from v along axis dir (ghosts from their donors, as the tiles read them)
+    auto prim_at = [&](int dir, int o) -> W6<double> {
+        const int x = ix + (dir == 0 ? o : 0), y = iy + (dir == 1 ? o : 0), z = iz + (dir == 2 ? o : 0);
+        const Donor<double, true> me(a, x, y);
+        W6<double> w = load_prims<2, double>(a, Donor<double, true>::plane(a, plane, z), me.off, flg);
+        me.signs(a, z, w);
+        return w;
+    };
+    if (h < 2) {
+        double f[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+        // face h of this wave's direction: between the cells h-1 and h from v
+        auto face = [&](auto dirc) {
+            constexpr int dir = decltype(dirc)::value;
+            W6<double> w[4];
+            for (int i = 0; i < 4; i++) w[i] = prim_at(dir, h - 2 + i);
+            Side<double> mi[2], pl[2];
+            for (int i = 0; i < 2; i++) {
+                const int o = h - 1 + i;
+                const int x = ix + (dir == 0 ? o : 0), y = iy + (dir == 1 ? o : 0), z = iz + (dir == 2 ? o : 0);
+                const bool gh = x < 2 || x > a.nx - 3 || y < 2 || y > a.ny - 3 || (!a.flatz && (z < 2 || z > a.nz - 3));
+                dir_states<dir>(w[i], w[i + 1], w[i + 2], sound_of(w[i + 1], a.gam), gh, a, mi[i], pl[i]);
             }
-            face_flux<double, d>(pl[0], mi[1], F[d][0]);
-            face_flux<double, d>(pl[1], mi[2], F[d][1]);
+            face_flux<double, dir>(pl[0], mi[1], f);
         };
-        faces(std::integral_constant<int, 0>{});
-        faces(std::integral_constant<int, 1>{});
-        if (!a.flatz) faces(std::integral_constant<int, 2>{});
+        if (d == 0) face(std::integral_constant<int, 0>{});
+        else if (d == 1) face(std::integral_constant<int, 1>{});
+        else if (!a.flatz) face(std::integral_constant<int, 2>{});
+        for (int i = 0; i < 5; i++) F[d][h][i] = f[i];
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const W6<double> q0 = prim_at(0, 0);
         double ui[5], uo[5], ft[5];
         for (int i = 0; i < 5; i++) {
             ui[i] = elem<double>(a.uin, (int64_t)i * a.n + v, 0u);
@@ -465,14 +494,14 @@ __global__ __launch_bounds__(64) void k_corner_ghosts(StageArgs a0, const int32_
              div_by(snd + fabs(v2), a.ds[2], a.inv_ds[2], a.ds_pow2[2]);
     }
     if (flg) atomicOr(a.flags, flg);
-    wave_max_to(rt, a.rate);
+    if (d == 0) wave_max_to(rt, a.rate);
 }
 
-// after the corrector's ghost fill of un (b: the corrector's arguments)
+// after the corrector, and after any ghost fill of un that writes these ghosts (b: the corrector's arguments)
 static int corner_ghosts(bx_ctx *c, const StageArgs &b)
 {
     if (c->nd2 == 0) return BX_OK;
-    hipLaunchKernelGGL(k_corner_ghosts, dim3(1), dim3(64), 0, c->stream, b, c->d2_dst, c->d2_sign);
+    hipLaunchKernelGGL(k_corner_ghosts, dim3((unsigned)c->nd2), dim3(192), 0, c->stream, b, c->d2_dst, c->d2_sign);
     BX_HIP(hipGetLastError());
     return BX_OK;
 }
@@ -508,108 +537,85 @@ static S *grav_pressure(bx_ctx *c, StageArgs &b)
     return nullptr;
 }
 
-// One fused step from U^n (c->cons, or c->cons32 in the mixed form; regular)
-// with full dt; result in c->unext / c->unext32.  The Courant rate of U^{n+1}
-// accumulates into rate_bits[0] and irregular branches into flags (both
-// zeroed here).
+// Whether the stage kernels read donors in place of ghost cells.
+static bool reads_donors(const bx_ctx *c) { return c->axis_ghosts && c->fused_occ >= 10; }
+
+static void read_donors(const bx_ctx *c, StageArgs &a)
+{
+    a.gmap = 1;
+    for (int i = 0; i < 6; i++) a.wall[i] = c->prm.no_outflow[i] ? 1 : 0;
+}
+
+// One fused step u0 -> us, ps -> un from a regular state, with full dt `dt`
+// or, for par = 0 or 1, with dt formed on the device from slot[par] and
+// rate_bits[par] (left in slot[par^1], logged in log[cap]).  The Courant rate
+// of U^{n+1} is left in rate_bits[0] or rate_bits[par^1]; irregular branches
+// are added to the flags.  fill: the ghost cells of us, ps and un hold their
+// donors' values afterwards (otherwise those of the stage inputs need not,
+// and those of un do not, but for the corner ghosts).
 template <typename S>
-static int fused_step_t(bx_ctx *c, double dt, S *u0, S *us, S *ps, S *un, bool reset_flags = true,
-                        const double *dtp = nullptr)
+static int enqueue_step(bx_ctx *c, double dt, int par, double *log, int cap, S *u0, S *us, S *ps, S *un,
+                        bool fill_us, bool fill_un)
 {
     int rc;
-    if (reset_flags) BX_HIP(hipMemsetAsync(&c->dsc->flags, 0, sizeof(unsigned int), c->stream));
-    BX_HIP(hipMemsetAsync(&c->dsc->rate_bits[0], 0, sizeof(unsigned long long), c->stream));
+    const bool donors = reads_donors(c);
+    unsigned long long *rate = &c->dsc->rate_bits[par < 0 ? 0 : par ^ 1];
     StageArgs a = base_args(c, dt);
-    a.dtp = dtp;
+    if (donors) read_donors(c, a);
+    StageArgs b = a;
+    if (par >= 0) {
+        a.slot = &c->dsc->slot[par];
+        a.slot_next = &c->dsc->slot[par ^ 1];
+        a.rate_in = &c->dsc->rate_bits[par];
+        a.cfl = c->prm.cfl;
+        a.log = log;
+        a.log_cap = cap;
+        b.dtp = &c->dsc->slot[par ^ 1].dt;
+    }
+    a.rate_next = rate;
     a.uin = u0;
     a.uout = us;
     a.pout = ps;
-    if (c->prof_on) BX_HIP(hipEventRecord(c->ev[0], c->stream));
-    if ((rc = launch_stage<1, S>(c, a, c->prof_on ? c->ev[1] : nullptr, (S *)c->eflux))) return rc;
-    if (c->prof_on) BX_HIP(hipEventRecord(c->ev[2], c->stream));
-    if ((rc = ghosts6<S>(c, us, ps))) return rc;
-    StageArgs b = base_args(c, dt);
-    b.dtp = dtp;
     b.uin = us;
     b.pin = ps;
     b.uold = u0;
     b.uout = un;
-    b.rate = &c->dsc->rate_bits[0];
+    b.rate = rate;
     S *pfin = grav_pressure<S>(c, b);
+    if (c->prof_on) BX_HIP(hipEventRecord(c->ev[0], c->stream));
+    if ((rc = launch_stage<1, S>(c, a, c->prof_on ? c->ev[1] : nullptr, (S *)c->eflux))) return rc;
+    if (c->prof_on) BX_HIP(hipEventRecord(c->ev[2], c->stream));
+    if ((fill_us || !donors) && (rc = ghosts6<S>(c, us, ps))) return rc;
     if (c->prof_on) BX_HIP(hipEventRecord(c->ev[3], c->stream));
     if ((rc = launch_stage<2, S>(c, b, c->prof_on ? c->ev[4] : nullptr, (S *)c->eflux))) return rc;
     if (c->prof_on) BX_HIP(hipEventRecord(c->ev[5], c->stream));
-    if ((rc = ghosts6<S>(c, un, pfin))) return rc;
+    if ((fill_un || !donors) && (rc = ghosts6<S>(c, un, pfin))) return rc;
     if constexpr (sizeof(S) == 8) return corner_ghosts(c, b);
     return BX_OK;
 }
 
-// ------------------------------------------------------ graph replays
-// One step's scalars on the device (graph replays and the adjoint's Courant
-// forward), in the operations of the host driver (step_dt in bx_capi.hip):
-// first the previous step of the run advances time (main.f90:544-545), then
-// the Courant rate of the current state gives dt (main.f90:266-281), which is
-// logged; the rate is cleared for the corrector kernel to accumulate the next
-// one.  The host adds the last step's dt to time after the run.
-__global__ void k_step_dt(DevScalars *s, double cfl, double *log, int cap)
-{
-    double time = s->time;
-    const int k = s->logk;
-    if (k > 0) {
-        time = time + s->dt;
-        s->time = time;
-    }
-    const double rate = __longlong_as_double((long long)s->rate_bits[0]);
-    const int step = s->step + 1;
-    double dt = cfl / rate;  // courant.f90:29
-    dt = dt * 1.0;
-    const double dtold = s->dtold;
-    if (step > 1 && dtold > 0.0) {
-        const double cap_dt = dtold * 1.1;
-        dt = cap_dt < dt ? cap_dt : dt;  // std::min(dt, cap_dt)
-    }
-    s->dtold = dt;
-    if (dt + time > s->endtime) dt = s->endtime - time;
-    dt = dt * 0.5;
-    dt = dt * 2.0;
-    s->dt = dt;
-    s->step = step;
-    s->rate_bits[0] = 0ull;
-    if (k < cap) log[k] = dt;
-    s->logk = k + 1;
-}
-
+// ------------------------------------------------------ runs of steps
 // Two fused steps, u0 -> un -> u0, with dt from the device scalars.
 template <typename S>
 static int enqueue_pair(bx_ctx *c, S *u0, S *us, S *ps, S *un)
 {
     int rc;
-    for (int h = 0; h < 2; h++) {
-        S *src = h == 0 ? u0 : un, *dst = h == 0 ? un : u0;
-        hipLaunchKernelGGL(k_step_dt, dim3(1), dim3(1), 0, c->stream, c->dsc, c->prm.cfl, c->chunk_dts,
-                           kChunkSteps);
-        BX_HIP(hipGetLastError());
-        StageArgs a = base_args(c, 0.0);
-        a.dtp = &c->dsc->dt;
-        a.uin = src;
-        a.uout = us;
-        a.pout = ps;
-        if ((rc = launch_stage<1, S>(c, a, nullptr, (S *)c->eflux))) return rc;
-        if ((rc = ghosts6<S>(c, us, ps))) return rc;
-        StageArgs b = base_args(c, 0.0);
-        b.dtp = &c->dsc->dt;
-        b.uin = us;
-        b.pin = ps;
-        b.uold = src;
-        b.uout = dst;
-        b.rate = &c->dsc->rate_bits[0];
-        S *pfin = grav_pressure<S>(c, b);
-        if ((rc = launch_stage<2, S>(c, b, nullptr, (S *)c->eflux))) return rc;
-        if ((rc = ghosts6<S>(c, dst, pfin))) return rc;
-        if constexpr (sizeof(S) == 8)
-            if ((rc = corner_ghosts(c, b))) return rc;
-    }
-    return BX_OK;
+    if ((rc = enqueue_step<S>(c, 0.0, 0, c->chunk_dts, kChunkSteps, u0, us, ps, un, false, false))) return rc;
+    return enqueue_step<S>(c, 0.0, 1, c->chunk_dts, kChunkSteps, un, us, ps, u0, false, false);
+}
+
+static int enqueue_current_pair(bx_ctx *c)
+{
+    return c->state_in_32 ? enqueue_pair<float>(c, c->cons32, c->ustar32, c->pstar32, c->unext32)
+                          : enqueue_pair<double>(c, c->cons, c->ustar, c->pstar, c->unext);
+}
+
+// The ghost cells of the current state after a run of pairs.
+static int fill_after_run(bx_ctx *c)
+{
+    if (!reads_donors(c)) return BX_OK;
+    if (c->state_in_32) return ghosts6<float>(c, c->cons32, (float *)nullptr);
+    return ghosts6<double>(c, c->cons, c->grav_flags ? c->p : (double *)nullptr, false);
 }
 
 void drop_step_graphs(bx_ctx *c)
@@ -640,11 +646,9 @@ static int pair_exec(bx_ctx *c, hipGraphExec_t *out)
     c->sexec[slot] = nullptr;
     c->sgraph[slot] = nullptr;
     c->skey[slot] = nullptr;
-    if (!c->chunk_dts) BX_HIP(hipMalloc((void **)&c->chunk_dts, sizeof(double) * kChunkSteps));
     BX_HIP(hipStreamSynchronize(c->stream));
     BX_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-    const int rc = f32 ? enqueue_pair<float>(c, c->cons32, c->ustar32, c->pstar32, c->unext32)
-                       : enqueue_pair<double>(c, c->cons, c->ustar, c->pstar, c->unext);
+    const int rc = enqueue_current_pair(c);
     hipGraph_t g = nullptr;
     const hipError_t e = hipStreamEndCapture(c->stream, &g);
     if (rc) {
@@ -665,17 +669,25 @@ static int pair_exec(bx_ctx *c, hipGraphExec_t *out)
     return BX_OK;
 }
 
-int replay_step_pairs(bx_ctx *c, int pairs)
+int run_step_pairs(bx_ctx *c, int pairs, bool graph)
 {
-    hipGraphExec_t x = nullptr;
-    if (int rc = pair_exec(c, &x)) return rc;
-    for (int i = 0; i < pairs; i++) BX_HIP(hipGraphLaunch(x, c->stream));
-    return BX_OK;
+    int rc;
+    if (!c->chunk_dts) BX_HIP(hipMalloc((void **)&c->chunk_dts, sizeof(double) * kChunkSteps));
+    if (graph) {
+        hipGraphExec_t x = nullptr;
+        if ((rc = pair_exec(c, &x))) return rc;
+        for (int i = 0; i < pairs; i++) BX_HIP(hipGraphLaunch(x, c->stream));
+    } else {
+        for (int i = 0; i < pairs; i++)
+            if ((rc = enqueue_current_pair(c))) return rc;
+    }
+    return fill_after_run(c);
 }
 
 int fused_step_into(bx_ctx *c, double dt, double *u0, double *us, double *ps, double *un, bool reset_flags)
 {
-    return fused_step_t<double>(c, dt, u0, us, ps, un, reset_flags);
+    if (reset_flags) BX_HIP(hipMemsetAsync(&c->dsc->flags, 0, sizeof(unsigned int), c->stream));
+    return enqueue_step<double>(c, dt, -1, nullptr, 0, u0, us, ps, un, true, true);
 }
 
 __global__ void k_clear_scalars(unsigned int *flags, unsigned long long *rate)
@@ -715,20 +727,19 @@ int fused_step_words(bx_ctx *c, double dt, const double *u0, double *us, double 
     return corner_ghosts(c, b);
 }
 
-// A step whose dt is formed on the device from the Courant rate of its state
-// (main.f90:266-281, endtime from the device scalars), logged into log[cap].
-int fused_step_device_dt(bx_ctx *c, double *u0, double *us, double *ps, double *un, double *log, int cap)
+// Step k of a run whose dts are formed on the device (scalars of step 0 in
+// slot[0], its rate in rate_bits[0]), logged into log[cap]
+int fused_step_device_dt(bx_ctx *c, int k, double *u0, double *us, double *ps, double *un, double *log, int cap)
 {
-    hipLaunchKernelGGL(k_step_dt, dim3(1), dim3(1), 0, c->stream, c->dsc, c->prm.cfl, log, cap);
-    BX_HIP(hipGetLastError());
-    return fused_step_t<double>(c, 0.0, u0, us, ps, un, false, &c->dsc->dt);
+    return enqueue_step<double>(c, 0.0, k & 1, log, cap, u0, us, ps, un, true, true);
 }
 
 int fused_step(bx_ctx *c, double dt)
 {
+    BX_HIP(hipMemsetAsync(&c->dsc->flags, 0, sizeof(unsigned int), c->stream));
     if (c->prm.precision == BX_PREC_MIXED)
-        return fused_step_t<float>(c, dt, c->cons32, c->ustar32, c->pstar32, c->unext32);
-    return fused_step_t<double>(c, dt, c->cons, c->ustar, c->pstar, c->unext);
+        return enqueue_step<float>(c, dt, -1, nullptr, 0, c->cons32, c->ustar32, c->pstar32, c->unext32, false, true);
+    return enqueue_step<double>(c, dt, -1, nullptr, 0, c->cons, c->ustar, c->pstar, c->unext, false, true);
 }
 
 }  // namespace bx

@@ -13,20 +13,25 @@ namespace bx {
 
 constexpr int kMaxD2 = 64;  // two-level ghost compositions a context may have (one wave)
 
+// The step scalars of main.f90 as a device-dt step leaves them.
+struct StepSlot {
+    double dt;       // full dt of the step (main.f90:342)
+    double dtold;    // main.f90:271
+    double time;     // at the step's start (main.f90:545 advances it)
+    double endtime;
+    int step;        // main.f90:213
+    int logk;        // steps of the current run so far (index into its dt log)
+};
+
 // Scalars that live on the device so whole steps can run without host syncs.
+// Device-dt steps alternate between the two slots and rates (a step reads one
+// and writes the other), so that no workgroup reads what another one writes.
 struct DevScalars {
     unsigned long long rate_bits[2];  // Courant max-rate (non-negative doubles as bits), ping-pong
     unsigned long long maxv_bits;     // velocity.f90 maxv diagnostic
     unsigned int flags;               // irregular-branch flags raised by the fused kernels
     unsigned int pad;
-    double dt;                        // full dt of the current step (main.f90:342)
-    double dtold;                     // main.f90:271
-    double time;                      // main.f90:545
-    double endtime;
-    int step;                         // main.f90:213
-    int active;                       // 1 while the step loop runs (time<endtime)
-    int logk;                         // steps of the current device-dt run (index into its dt log)
-    int pad2;
+    StepSlot slot[2];
 };
 
 // flags bits
@@ -76,6 +81,9 @@ struct bx_ctx {
     int32_t *fghost_src;
     int32_t *fghost_sign;
     bool fghost_ok;
+    // every ghost's composed donor is the per-axis one (axis_donor), an
+    // interior cell: the tiled kernels then read donors in place of ghosts
+    bool axis_ghosts;
     // ghosts whose pair leaves the pre-pair value of another ghost h2 (whose
     // own pair gives an interior cell v): the corner ghosts of a box walled
     // in y and z.  After a step such a ghost holds +-(v's corrector result
@@ -183,10 +191,11 @@ int fused_step(bx_ctx *c, double dt);
 // one FP64 fused step U^n=u0 -> U*=us, p*=ps -> U^{n+1}=un (ghosts filled); the rate is zeroed
 // first, the flags too when reset_flags (else they accumulate over steps)
 int fused_step_into(bx_ctx *c, double dt, double *u0, double *us, double *ps, double *un, bool reset_flags);
-// the same with dt formed on the device from the current Courant rate (the
-// device scalars carry time, dtold, step and endtime); flags accumulate and
-// each dt is logged into log[cap]
-int fused_step_device_dt(bx_ctx *c, double *u0, double *us, double *ps, double *un, double *log, int cap);
+// the same, step k of a run, with dt formed on the device from the current
+// Courant rate (the device scalars carry time, dtold, step and endtime, at the
+// run's start in slot[0] and rate_bits[0]; after k steps in [k & 1]); flags
+// accumulate and each dt is logged into log[cap]
+int fused_step_device_dt(bx_ctx *c, int k, double *u0, double *us, double *ps, double *un, double *log, int cap);
 void adjoint_free(bx_ctx *c);
 void eos_free(bx_ctx *c);
 void gravity_free(bx_ctx *c);
@@ -196,11 +205,12 @@ bool grav_settled(const bx_ctx *c);
 int grav_fused_planes(bx_ctx *c);
 int launch_state_tab(bx_ctx *c);
 int fused_prepare(bx_ctx *c);
-// BX_STEP_GRAPH: replay `pairs` captured pairs of fused steps from the current
-// state (device dt, flags accumulating); the scalars must be on the device
-int replay_step_pairs(bx_ctx *c, int pairs);
+// `pairs` pairs of fused steps from the current state (device dt, flags
+// accumulating), replayed from a captured graph (BX_STEP_GRAPH) or enqueued;
+// the scalars must be on the device
+int run_step_pairs(bx_ctx *c, int pairs, bool graph);
 void drop_step_graphs(bx_ctx *c);
-constexpr int kChunkSteps = 32;  // steps per replayed chunk, at most
+constexpr int kChunkSteps = 32;  // steps per run, at most
 int narrow_cons(bx_ctx *c);
 int widen_cons(bx_ctx *c);
 

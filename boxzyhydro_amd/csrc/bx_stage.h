@@ -44,7 +44,21 @@ struct StageArgs {
     double gam, gm1, seps, srho, vlimit;
     unsigned int *flags;
     unsigned long long *rate;  // stage 2: next step's Courant rate (max)
-    const double *dtp;         // when set, the step's dt is read from here (graph replays), else dt
+    const double *dtp;         // when set, the step's dt is read from here (device dt), else dt
+    // stage 1 of a device-dt step: every workgroup forms dt from the slot the
+    // last step left and the Courant rate; the first one writes the next slot
+    // and log (null: dtp or dt).  rate_next: cleared by stage 1 for the
+    // corrector to accumulate into (null: cleared by the caller)
+    const StepSlot *slot;
+    StepSlot *slot_next;
+    const unsigned long long *rate_in;
+    unsigned long long *rate_next;
+    double cfl, *log;
+    int log_cap;
+    // gmap: the tiled kernels read a ghost cell from its donor (axis_donor;
+    // wall: the six sides, mirrored with the normal velocity negated), so the
+    // ghost cells of their inputs need not be filled; 0: ghosts from memory
+    int gmap, wall[6];
     // the donors of the two-level corner ghosts, whose corrector result
     // before source(1) is parked in d2ubar (6 per entry: that, then the
     // ghost's pressure)
@@ -58,12 +72,69 @@ struct StageArgs {
     const double *gf;
 };
 
+// One step's scalars on the device, in the operations of the host driver
+// (step_dt in bx_capi.hip): first the previous step of the run advances time
+// (main.f90:544-545), then the Courant rate of the current state gives dt
+// (main.f90:266-281).
+__device__ __forceinline__ StepSlot next_slot(const StepSlot &s, unsigned long long rate_bits, double cfl)
+{
+    StepSlot o = s;
+    if (s.logk > 0) o.time = s.time + s.dt;
+    const double rate = __longlong_as_double((long long)rate_bits);
+    o.step = s.step + 1;
+    double dt = cfl / rate;  // courant.f90:29
+    dt = dt * 1.0;
+    if (o.step > 1 && s.dtold > 0.0) {
+        const double cap_dt = s.dtold * 1.1;
+        dt = cap_dt < dt ? cap_dt : dt;  // std::min(dt, cap_dt)
+    }
+    o.dtold = dt;
+    if (dt + o.time > s.endtime) dt = s.endtime - o.time;
+    dt = dt * 0.5;
+    o.dt = dt * 2.0;
+    o.logk = s.logk + 1;
+    return o;
+}
+
+__device__ __forceinline__ bool first_lane_of_grid()
+{
+    return blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0 && threadIdx.x == 0;
+}
+
 // The arguments of a launch with dt resolved: a kernel reads it once at entry.
+// Forming dt here, in every workgroup of stage 1, instead of in a kernel of
+// its own, takes one dispatch (4.5 us on an otherwise idle chip) from each
+// step; the division runs while the first planes load.
 __device__ __forceinline__ StageArgs with_dt(const StageArgs &a0)
 {
     StageArgs a = a0;
-    if (a0.dtp) a.dt = *a0.dtp;
+    if (a0.slot) {
+        const StepSlot o = next_slot(*a0.slot, *a0.rate_in, a0.cfl);
+        a.dt = o.dt;
+        if (first_lane_of_grid()) {
+            *a0.slot_next = o;
+            if (a0.slot->logk < a0.log_cap) a0.log[a0.slot->logk] = o.dt;
+        }
+    } else if (a0.dtp) {
+        a.dt = *a0.dtp;
+    }
+    if (a0.rate_next && first_lane_of_grid()) *a0.rate_next = 0ull;
     return a;
+}
+
+// Along one axis of n cells, the interior cell that cell i takes its values
+// from after the pair of set_ghost_cells calls: itself, the mirror image at a
+// wall, the nearest interior cell at an open side.
+__host__ __device__ __forceinline__ int axis_donor(int i, int n, int wall_lo, int wall_hi)
+{
+    if (i < 2) return wall_lo ? 3 - i : 2;
+    if (i > n - 3) return wall_hi ? 2 * n - 5 - i : n - 3;
+    return i;
+}
+// whether the velocity along that axis changes sign there
+__host__ __device__ __forceinline__ bool axis_flip(int i, int n, int wall_lo, int wall_hi)
+{
+    return (i < 2 && wall_lo) || (i > n - 3 && wall_hi);
 }
 
 // Stage arguments of a context for a step of full dt (bx_fused.hip)

@@ -40,6 +40,12 @@
 // the y-halo costs 4 rows of primitives, 2 rows of states and 1 row of faces
 // per TY rows; the x-edges 7 cells of primitives, states and faces per row
 // (one wave pass).
+// Ghost cells (StageArgs::gmap): a ghost holds its donor's values, so the loads
+// of a ghost take the donor's address instead (per lane in x and y, per plane
+// in z: the tile's cells keep their own coordinates for the slopes and the
+// outputs), and at a wall (W) the normal velocity changes sign.  The ghost
+// cells of the stage's input then need no fill before it: two dispatches less
+// per step (4.6 us each on small grids, 33 us each at 256^3).
 // Every arithmetic operation is the one the exact sequence performs on the
 // same values, so the results are bit-identical to it.
 #pragma once
@@ -123,6 +129,53 @@ __device__ __forceinline__ T from_upper(T v, T edge, int)
     return wave_shift_t<0x130>(v, edge);  // wave_shl:1
 }
 
+// Where a tile's row (or edge lane) at column x and row y reads its cells, and
+// at walls the sign bits of the velocity components there (0 or the sign bit
+// of the high word; the z component per plane).  prims() of a cell with a
+// negated momentum is prims() of the cell with the velocity negated, bit for
+// bit: quotients and products by a sign are exact.
+template <typename S, bool W>
+struct Donor {
+    unsigned off;     // byte offset within a plane
+    unsigned sx, sy;  // W only
+    __device__ __forceinline__ Donor(const StageArgs &a, int x, int y)
+    {
+        int xd = min(max(x, 0), a.nx - 1), yd = min(max(y, 0), a.ny - 1);
+        sx = sy = 0u;
+        if (a.gmap) {
+            if (W) {
+                sx = axis_flip(xd, a.nx, a.wall[0], a.wall[1]) ? 0x80000000u : 0u;
+                sy = axis_flip(yd, a.ny, a.wall[2], a.wall[3]) ? 0x80000000u : 0u;
+            }
+            xd = axis_donor(xd, a.nx, W && a.wall[0], W && a.wall[1]);
+            yd = axis_donor(yd, a.ny, W && a.wall[2], W && a.wall[3]);
+        }
+        off = (unsigned)(yd * a.nx + xd) * (unsigned)sizeof(S);
+    }
+    // plane k's element offset (uniform)
+    static __device__ __forceinline__ int64_t plane(const StageArgs &a, int64_t plane, int k)
+    {
+        if (a.gmap && !a.flatz) k = axis_donor(k, a.nz, W && a.wall[4], W && a.wall[5]);
+        return (int64_t)k * plane;
+    }
+    static __device__ __forceinline__ S flip(S v, unsigned m)
+    {
+        if constexpr (sizeof(S) == 8)
+            return __longlong_as_double(__double_as_longlong(v) ^ (long long)((unsigned long long)m << 32));
+        else
+            return __int_as_float(__float_as_int(v) ^ (int)m);
+    }
+    __device__ __forceinline__ void signs(const StageArgs &a, int k, W6<S> &w) const
+    {
+        if constexpr (W) {
+            w.u0 = flip(w.u0, sx);
+            w.u1 = flip(w.u1, sy);
+            const bool fz = a.gmap && !a.flatz && axis_flip(k, a.nz, a.wall[4], a.wall[5]);
+            w.u2 = flip(w.u2, fz ? 0x80000000u : 0u);
+        }
+    }
+};
+
 // Per-tile constants of one stage.
 struct TileGeom {
     int nx, ny, nz;
@@ -135,7 +188,7 @@ struct TileGeom {
 // primitives of plane k are read back from the tile where needed, and the x
 // and z flux differences are parked in LDS until the update, to keep the
 // registers live across the barriers few.
-template <int STAGE, typename S, int TY, bool G>
+template <int STAGE, typename S, int TY, bool G, bool W>
 __device__ __forceinline__ void tile_owner(const StageArgs &a, TileLds<S, TY> &L, const TileGeom &g,
                                            unsigned int &flg, double &rmax)
 {
@@ -143,12 +196,12 @@ __device__ __forceinline__ void tile_owner(const StageArgs &a, TileLds<S, TY> &L
     const int lane = g.lane, r = g.r, nx = g.nx, ny = g.ny, nz = g.nz;
     const int64_t n = g.n;
     const int x = g.x0 + lane, y = g.j0 + r;
-    const int xc = min(x, nx - 1), yc = min(y, ny - 1);
-    const unsigned coff = (unsigned)(yc * nx + xc) * (unsigned)sizeof(S);
+    const Donor<S, W> me(a, x, y);
+    const unsigned coff = me.off;
     const bool xy_ghost = x < 2 || x > nx - 3 || y < 2 || y > ny - 3;
     const bool is_out = !xy_ghost;
     const S gamS = S(a.gam);
-    auto zplane = [&](int k) -> int64_t { return (int64_t)k * g.plane; };
+    auto zplane = [&](int k) -> int64_t { return Donor<S, W>::plane(a, g.plane, k); };
     auto zghost = [&](int k) -> bool { return !a.flatz && (k < 2 || k > nz - 3); };
     const int c = (r + 2) * RS + lane + 1;  // this cell in the primitive tiles
     const int o = r * 64 + lane;            // this cell's slot in the per-owner buffers
@@ -160,10 +213,12 @@ __device__ __forceinline__ void tile_owner(const StageArgs &a, TileLds<S, TY> &L
     Raw<S> nxt;
     const int kb = g.kb, ke = g.ke;
     if (!a.flatz) {
-        const W6<S> t0 = load_prims<STAGE, S, G>(a, zplane(kb - 2), coff, flg);
-        const W6<S> t1 = load_prims<STAGE, S, G>(a, zplane(kb - 1), coff, flg);
-        const W6<S> t2 = load_prims<STAGE, S, G>(a, zplane(kb), coff, flg);
-        const W6<S> t3 = load_prims<STAGE, S, G>(a, zplane(kb + 1), coff, flg);
+        auto at = [&](int k) -> W6<S> {
+            W6<S> w = load_prims<STAGE, S, G>(a, zplane(k), coff, flg);
+            me.signs(a, k, w);
+            return w;
+        };
+        const W6<S> t0 = at(kb - 2), t1 = at(kb - 1), t2 = at(kb), t3 = at(kb + 1);
         Side<S> zmi, zpl;
         dir_states<2>(t0, t1, t2, sound_of(t1, a.gam), xy_ghost || zghost(kb - 1), a, zmi, zpl);
         zp_prev = zpl;
@@ -175,7 +230,8 @@ __device__ __forceinline__ void tile_owner(const StageArgs &a, TileLds<S, TY> &L
         q2 = t3;
         nxt = load_raw<STAGE, S, G>(a, zplane(kb + 2), coff);
     } else {
-        const W6<S> w = load_prims<STAGE, S, G>(a, zplane(kb), coff, flg);
+        W6<S> w = load_prims<STAGE, S, G>(a, zplane(kb), coff, flg);
+        me.signs(a, kb, w);
         cs1 = sound_of(w, a.gam);
         store_w(L.P[kb & 1], c, w);
         if (kb + 1 < ke) nxt = load_raw<STAGE, S, G>(a, zplane(kb + 1), coff);
@@ -195,6 +251,7 @@ __device__ __forceinline__ void tile_owner(const StageArgs &a, TileLds<S, TY> &L
             // needs no branch)
             nxt = load_raw<STAGE, S, G>(a, zplane(min(k + 3, nz - 1)), coff);
             q2 = prims<STAGE, S, G>(a, cur, flg);
+            me.signs(a, k + 2, q2);
             cs1 = sound_of(q1, a.gam);
             Side<S> zmi1, zpl1;
             dir_states<2>(fetch_w(L.P[t], c), q1, q2, cs1, xy_ghost || zghost(k + 1), a, zmi1, zpl1);
@@ -211,7 +268,8 @@ __device__ __forceinline__ void tile_owner(const StageArgs &a, TileLds<S, TY> &L
             if (k + 1 < ke) {
                 const Raw<S> cur = nxt;
                 nxt = load_raw<STAGE, S, G>(a, zplane(min(k + 2, ke - 1)), coff);
-                const W6<S> w = prims<STAGE, S, G>(a, cur, flg);
+                W6<S> w = prims<STAGE, S, G>(a, cur, flg);
+                me.signs(a, k + 1, w);
                 cs1 = sound_of(w, a.gam);
                 store_w(L.P[t ^ 1], c, w);
             }
@@ -251,7 +309,7 @@ __device__ __forceinline__ void tile_owner(const StageArgs &a, TileLds<S, TY> &L
         __syncthreads();
         // D: face y r+1/2 and the update
         if (is_out) {
-            const int64_t cz = zplane(k);
+            const int64_t cz = (int64_t)k * g.plane;  // an interior plane, and coff an interior cell's
             double ui[5], uo[5], ft[5];
             for (int i = 0; i < 5; i++) {
                 ui[i] = elem<S>(a.uin, (int64_t)i * n + cz, coff);
@@ -272,23 +330,28 @@ __device__ __forceinline__ void tile_owner(const StageArgs &a, TileLds<S, TY> &L
 
 // Halo rows -2, -1 and TY: their primitives, the y-states of rows -1 and TY,
 // and face y TY-1/2.
-template <int STAGE, typename S, int TY, bool G>
+template <int STAGE, typename S, int TY, bool G, bool W>
 __device__ __forceinline__ void tile_halo(const StageArgs &a, TileLds<S, TY> &L, const TileGeom &g,
                                           unsigned int &flg)
 {
     constexpr int RS = TileLds<S, TY>::RS;
     const int lane = g.lane, r = g.r, nx = g.nx, ny = g.ny, nz = g.nz;
     const int x = g.x0 + lane, y = g.j0 + r;
-    const int xc = min(x, nx - 1), yc = min(y, ny - 1);
-    const unsigned coff = (unsigned)(yc * nx + xc) * (unsigned)sizeof(S);
+    const Donor<S, W> me(a, x, y);
+    const unsigned coff = me.off;
     const bool xy_ghost = x < 2 || x > nx - 3 || y < 2 || y > ny - 3;
     const S gamS = S(a.gam);
-    auto zplane = [&](int k) -> int64_t { return (int64_t)k * g.plane; };
+    auto zplane = [&](int k) -> int64_t { return Donor<S, W>::plane(a, g.plane, k); };
     auto zghost = [&](int k) -> bool { return !a.flatz && (k < 2 || k > nz - 3); };
     const int c = (r + 2) * RS + lane + 1;
     const int kb = g.kb, ke = g.ke;
     Raw<S> nxt;
-    store_w(L.P[kb & 1], c, load_prims<STAGE, S, G>(a, zplane(kb), coff, flg));
+    auto put = [&](int k, const Raw<S> &raw) {
+        W6<S> w = prims<STAGE, S, G>(a, raw, flg);
+        me.signs(a, k, w);
+        store_w(L.P[k & 1], c, w);
+    };
+    put(kb, load_raw<STAGE, S, G>(a, zplane(kb), coff));
     if (kb + 1 < ke) nxt = load_raw<STAGE, S, G>(a, zplane(kb + 1), coff);
     __syncthreads();  // as the owners' first barrier
     for (int k = kb; k < ke; k++) {
@@ -297,7 +360,7 @@ __device__ __forceinline__ void tile_halo(const StageArgs &a, TileLds<S, TY> &L,
             // A: primitives of plane k+1 into the other tile
             const Raw<S> cur = nxt;
             nxt = load_raw<STAGE, S, G>(a, zplane(min(k + 2, ke - 1)), coff);
-            store_w(L.P[t ^ 1], c, prims<STAGE, S, G>(a, cur, flg));
+            put(k + 1, cur);
         }
         Side<S> ymi;
         if (r != -2) {
@@ -321,7 +384,7 @@ __device__ __forceinline__ void tile_halo(const StageArgs &a, TileLds<S, TY> &L,
 // Wave r=TY+1: its own halo row, and the x-edges of the owner rows one plane
 // ahead.  Lane 7*row+j holds column {-2,-1,0,62,63,64,65}[j] of owner row
 // `row`.
-template <int STAGE, typename S, int TY, bool G>
+template <int STAGE, typename S, int TY, bool G, bool W>
 __device__ __forceinline__ void tile_edge(const StageArgs &a, TileLds<S, TY> &L, const TileGeom &g,
                                           unsigned int &flg)
 {
@@ -329,10 +392,10 @@ __device__ __forceinline__ void tile_edge(const StageArgs &a, TileLds<S, TY> &L,
     static_assert(7 * TY <= 64, "x-edge lanes of the owner rows must fit one wave");
     const int lane = g.lane, r = g.r, nx = g.nx, ny = g.ny, nz = g.nz;
     const int x = g.x0 + lane, y = g.j0 + r;
-    const int xc = min(x, nx - 1), yc = min(y, ny - 1);
-    const unsigned coff = (unsigned)(yc * nx + xc) * (unsigned)sizeof(S);
+    const Donor<S, W> me(a, x, y);
+    const unsigned coff = me.off;
     const S gamS = S(a.gam);
-    auto zplane = [&](int k) -> int64_t { return (int64_t)k * g.plane; };
+    auto zplane = [&](int k) -> int64_t { return Donor<S, W>::plane(a, g.plane, k); };
     auto zghost = [&](int k) -> bool { return !a.flatz && (k < 2 || k > nz - 3); };
     const int c = (r + 2) * RS + lane + 1;
 
@@ -340,7 +403,8 @@ __device__ __forceinline__ void tile_edge(const StageArgs &a, TileLds<S, TY> &L,
     const int erow = lane / 7, ej = lane - 7 * (lane / 7);
     const int ecol = ej < 3 ? ej - 2 : ej + 59;
     const int ex = g.x0 + ecol, ey = g.j0 + erow;
-    const unsigned eoff = (unsigned)(min(ey, ny - 1) * nx + min(max(ex, 0), nx - 1)) * (unsigned)sizeof(S);
+    const Donor<S, W> em(a, ex, ey);
+    const unsigned eoff = em.off;
     const bool e_xy_ghost = ex < 2 || ex > nx - 3 || ey < 2 || ey > ny - 3;
 
     // the three parts of the x-edge items of plane k
@@ -348,6 +412,7 @@ __device__ __forceinline__ void tile_edge(const StageArgs &a, TileLds<S, TY> &L,
     Side<S> emi{}, epl{};
     auto edge_prims = [&](int k, const Raw<S> &raw) {
         ew = prims<STAGE, S, G>(a, raw, flg);
+        em.signs(a, k, ew);
         if (ej == 1 || ej == 5) store_w(L.P[k & 1], (erow + 2) * RS + ecol + 1, ew);
     };
     // neighbours within a row's seven lanes through whole-wave shifts (the
@@ -375,7 +440,12 @@ __device__ __forceinline__ void tile_edge(const StageArgs &a, TileLds<S, TY> &L,
 
     const int kb = g.kb, ke = g.ke;
     Raw<S> nxt;
-    store_w(L.P[kb & 1], c, load_prims<STAGE, S, G>(a, zplane(kb), coff, flg));
+    auto put = [&](int k, const Raw<S> &raw) {
+        W6<S> w = prims<STAGE, S, G>(a, raw, flg);
+        me.signs(a, k, w);
+        store_w(L.P[k & 1], c, w);
+    };
+    put(kb, load_raw<STAGE, S, G>(a, zplane(kb), coff));
     if (kb + 1 < ke) nxt = load_raw<STAGE, S, G>(a, zplane(kb + 1), coff);
     Raw<S> enxt{};
     if (e_on) {
@@ -391,7 +461,7 @@ __device__ __forceinline__ void tile_edge(const StageArgs &a, TileLds<S, TY> &L,
             // A: primitives of plane k+1, its own row and the x-edges
             const Raw<S> cur = nxt;
             nxt = load_raw<STAGE, S, G>(a, zplane(min(k + 2, ke - 1)), coff);
-            store_w(L.P[(k + 1) & 1], c, prims<STAGE, S, G>(a, cur, flg));
+            put(k + 1, cur);
             if (e_on) {
                 const Raw<S> ecur = enxt;
                 enxt = load_raw<STAGE, S, G>(a, zplane(min(k + 2, ke - 1)), eoff);
@@ -406,8 +476,9 @@ __device__ __forceinline__ void tile_edge(const StageArgs &a, TileLds<S, TY> &L,
 }
 
 // One stage over the tile (bx, by) of 64 x TY outputs and the z planes of chunk bz.
-// G: with gravity (StageArgs::gf, FP64).
-template <int STAGE, typename S, int TY, bool G>
+// G: with gravity (StageArgs::gf, FP64).  W: some side is a wall (read only
+// with gmap).
+template <int STAGE, typename S, int TY, bool G, bool W>
 __device__ __forceinline__ void tile_stage(const StageArgs &a, TileLds<S, TY> &L, unsigned bx, unsigned by,
                                            unsigned bz)
 {
@@ -432,10 +503,10 @@ __device__ __forceinline__ void tile_stage(const StageArgs &a, TileLds<S, TY> &L
         // win the issue arbitration by age: the owners issue first
         // (2.06 -> 2.00 ms per step at 256^3).
         __builtin_amdgcn_s_setprio(1);
-        tile_owner<STAGE, S, TY, G>(a, L, g, flg, rmax);
+        tile_owner<STAGE, S, TY, G, W>(a, L, g, flg, rmax);
     }
-    else if (g.r == TY + 1) tile_edge<STAGE, S, TY, G>(a, L, g, flg);
-    else tile_halo<STAGE, S, TY, G>(a, L, g, flg);
+    else if (g.r == TY + 1) tile_edge<STAGE, S, TY, G, W>(a, L, g, flg);
+    else tile_halo<STAGE, S, TY, G, W>(a, L, g, flg);
     if (flg) atomicOr(a.flags, flg);
     if (STAGE == 2) wave_max_to(rmax, a.rate);
 }
