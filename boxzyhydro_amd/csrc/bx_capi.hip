@@ -237,15 +237,17 @@ int bx_create(const bx_params *prm, int32_t device, bx_ctx **out)
     const int64_t n = (int64_t)prm->nx * prm->ny * prm->nz;
     if (n > (int64_t)INT32_MAX) return set_error(BX_ERR_ARG, "bx_create: grid exceeds 2^31 cells");
 
-    int ndev = 0;
+    int ndev = 0, ncu = 0;
     BX_HIP(hipGetDeviceCount(&ndev));
     if (device < 0 || device >= ndev) return set_error(BX_ERR_ARG, "bx_create: no such device");
     BX_HIP(hipSetDevice(device));
+    BX_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, device));
 
     bx_ctx *c = new (std::nothrow) bx_ctx();
     if (!c) return set_error(BX_ERR_ARG, "bx_create: out of host memory");
     c->prm = *prm;
     c->device = device;
+    c->ncu = ncu > 0 ? ncu : 256;
     c->nx = prm->nx;
     c->ny = prm->ny;
     c->nz = prm->nz;
@@ -591,7 +593,10 @@ int bx_upload(bx_ctx *c, const double *cons, const double *u, const double *p, c
     }
     if (u && (rc = upload_aos(c, u, 3, c->u))) return rc;
     if (p && (rc = upload_aos(c, p, 1, c->p))) return rc;
-    if (adindx && (rc = upload_aos(c, adindx, 1, c->adindx))) return rc;
+    if (adindx) {
+        if ((rc = upload_aos(c, adindx, 1, c->adindx))) return rc;
+        c->ad_uniform = false;
+    }
     BX_HIP(hipStreamSynchronize(c->stream));
     c->fused_valid = false;
     c->aux_stale = false;

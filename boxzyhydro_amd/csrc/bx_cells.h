@@ -4,10 +4,30 @@
 // the same arithmetic.  Arithmetic order follows the cited reference lines.
 #pragma once
 
+#include <type_traits>
+
 #include "bx_internal.h"
 #include "bx_math.h"
 
 namespace bx {
+
+// max-reduce non-negative doubles of a block (at most 1024 threads) into *dst
+// (as IEEE bits)
+__device__ __forceinline__ void block_max_to(double v, unsigned long long *dst)
+{
+    __shared__ double wmax[16];
+    for (int off = 32; off > 0; off >>= 1) v = vmax(v, __shfl_xor(v, off, 64));
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    if (lane == 0) wmax[w] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double m = wmax[0];
+        for (int k = 1; k < (int)(blockDim.x >> 6); k++) m = vmax(m, wmax[k]);
+        // skip the atomic when the stored maximum is already larger
+        const unsigned long long b = (unsigned long long)__double_as_longlong(m);
+        if (b > __hip_atomic_load(dst, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(dst, b);
+    }
+}
 
 // 1-based (ix,iy,iz) of cell c (utils.f90:191-194 inverse)
 __device__ __forceinline__ void coords(int64_t c, int nx, int ny, int &ix, int &iy, int &iz)
@@ -290,6 +310,45 @@ __device__ __forceinline__ void face_update_cell(int64_t n, int64_t c, int nx, i
     U[0] = vmax(U[0], srho);
     if (U[4] < 0.0) U[4] = 0.5 * (U[1] * U[1] + U[2] * U[2] + U[3] * U[3]) / U[0] + seps;
     for (int i = 0; i < 5; i++) cons[(int64_t)i * n + c] = U[i];
+}
+
+// face_update_cell without the face planes: the six faces of an interior cell
+// formed here, from cons, u, p and ad into the out planes
+__device__ __forceinline__ void flux_cell(int64_t n, int64_t c, int nx, int ny, int nz, bool flatz,
+                                          const double *__restrict__ cons, const double *__restrict__ u,
+                                          const double *__restrict__ p, const double *__restrict__ ad,
+                                          const double *__restrict__ cons_old, double *__restrict__ out, int avg,
+                                          double dt, double dx, double dy, double dz, double srho, double seps)
+{
+    int ix, iy, iz;
+    coords(c, nx, ny, ix, iy, iz);
+    double ftmp[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    if (boundary_of(ix, iy, iz, nx, ny, nz) == 0) {
+        const double axy = dy * dx, ayz = dy * dz, axz = dx * dz, vol = dx * dy * dz;
+        const int64_t sz = flatz ? 0 : (int64_t)nx * ny;
+        double f0[5], f1[5], s[5];
+        auto faces = [&](auto dirc, int64_t st, double ds) {
+            constexpr int d = decltype(dirc)::value;
+            auto side = [&](int64_t q, int pm) { return cell_side<d>(q, pm, n, nx, ny, nz, st, cons, u, p, ad, dt, ds, seps); };
+            face_flux<double, d>(side(c - st, 1), side(c, 0), f0);
+            face_flux<double, d>(side(c, 1), side(c + st, 0), f1);
+        };
+        faces(std::integral_constant<int, 0>{}, 1, dx);
+        for (int i = 0; i < 5; i++) s[i] = ayz * (f1[i] - f0[i]);
+        faces(std::integral_constant<int, 1>{}, nx, dy);
+        for (int i = 0; i < 5; i++) s[i] = s[i] + axz * (f1[i] - f0[i]);
+        faces(std::integral_constant<int, 2>{}, sz, dz);
+        for (int i = 0; i < 5; i++) ftmp[i] = -((s[i] + axy * (f1[i] - f0[i])) * dt / vol);
+    }
+    double U[5];
+    for (int i = 0; i < 5; i++) {
+        const double ft = ftmp[i];
+        const double cu = cons[(int64_t)i * n + c];
+        U[i] = avg == 0 ? cu + ft : 0.5 * (cons_old[(int64_t)i * n + c] + cu + ft);
+    }
+    U[0] = vmax(U[0], srho);
+    if (U[4] < 0.0) U[4] = 0.5 * (U[1] * U[1] + U[2] * U[2] + U[3] * U[3]) / U[0] + seps;
+    for (int i = 0; i < 5; i++) out[(int64_t)i * n + c] = U[i];
 }
 
 }  // namespace bx

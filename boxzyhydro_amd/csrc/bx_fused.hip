@@ -33,6 +33,7 @@
 // Both give the same bits.
 #include <cmath>
 
+#include "bx_cells.h"
 #include "bx_tile.h"
 
 namespace bx {
@@ -41,11 +42,11 @@ namespace bx {
 // LDS, marching in z (bx_tile.h: tile_stage).  P2: every spacing and the
 // cell volume are powers of two (their divisions are multiplications), known
 // at compile time, which keeps the spacings themselves out of the registers.
-// G: gravity; W: walls whose ghosts are read from their donors (bx_tile.h).
-template <int STAGE, typename S, int TY, bool P2, bool G, bool W>
+// V: StageKind; W: walls whose ghosts are read from their donors (bx_tile.h).
+template <int STAGE, typename S, int TY, bool P2, int V, bool W>
 __global__ __launch_bounds__(64 * (TY + 4)) void k_stage(StageArgs a0)
 {
-    __shared__ TileLds<S, TY> lds;
+    __shared__ TileLds<S, TY, V> lds;
     StageArgs a = with_dt(a0);
     if constexpr (P2) {
         a.ds_pow2[0] = a.ds_pow2[1] = a.ds_pow2[2] = 1;
@@ -60,7 +61,7 @@ __global__ __launch_bounds__(64 * (TY + 4)) void k_stage(StageArgs a0)
     const unsigned L = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);
     const unsigned xcd = L & 7u, slot = L >> 3, q = T >> 3, rem = T & 7u;
     const unsigned t = xcd * q + (xcd < rem ? xcd : rem) + slot;
-    tile_stage<STAGE, S, TY, G, W>(a, lds, t % gx, (t / gx) % gy, t / (gx * gy));
+    tile_stage<STAGE, S, TY, V, W>(a, lds, t % gx, (t / gx) % gy, t / (gx * gy));
 }
 
 
@@ -95,11 +96,12 @@ __global__ __launch_bounds__(256) void k_regular(int64_t n, const double *__rest
                                                 double dx, double dy, double dz, unsigned int *flags,
                                                 unsigned long long *rate)
 {
-    const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     unsigned int flg = 0;
-    const double rt = c < n ? regular_cell(n, c, cons, u, gam, seps, dx, dy, dz, flg) : 0.0;
+    double rt = 0.0;
+    for (int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; c < n; c += (int64_t)gridDim.x * blockDim.x)
+        rt = vmax(rt, regular_cell(n, c, cons, u, gam, seps, dx, dy, dz, flg));
     if (flg) atomicOr(flags, flg);
-    wave_max_to(rt, rate);
+    block_max_to(rt, rate);
 }
 
 template <typename S>
@@ -180,23 +182,20 @@ static int launch_tile_w(bx_ctx *c, const StageArgs &a)
     const unsigned gy = (unsigned)((c->ny - 4 + TY - 1) / TY);
     const unsigned gz = (unsigned)((nzi + a.lz - 1) / a.lz);
     const dim3 grid(gx, gy, gz), block(64 * (TY + 4));
-    if constexpr (sizeof(S) == 8 && TY == 8) {
+    if constexpr (sizeof(S) == 8 && TY == 8 && !W) {
         if (a.gf) {
-            // the corrector's power-of-two form spills 5 VGPRs at 168; its
-            // general form (161, no spill) gives the same bits and is ~1 % faster
-            if (p2 && STAGE == 1)
-                hipLaunchKernelGGL((k_stage<STAGE, S, TY, true, true, W>), grid, block, 0, c->stream, a);
-            else
-                hipLaunchKernelGGL((k_stage<STAGE, S, TY, false, true, W>), grid, block, 0, c->stream, a);
+            // the power-of-two forms spill 2 and 7 VGPRs at 168; the general
+            // ones (163, no spill) give the same bits and are ~1 % faster
+            hipLaunchKernelGGL((k_stage<STAGE, S, TY, false, kGravity, false>), grid, block, 0, c->stream, a);
             BX_HIP(hipGetLastError());
             return BX_OK;
         }
     }
     if (a.gf) return set_error(BX_ERR_UNSUPPORTED, "fused step with gravity: FP64 64 x 8 tiles only");
     if (p2)
-        hipLaunchKernelGGL((k_stage<STAGE, S, TY, true, false, W>), grid, block, 0, c->stream, a);
+        hipLaunchKernelGGL((k_stage<STAGE, S, TY, true, kPlain, W>), grid, block, 0, c->stream, a);
     else
-        hipLaunchKernelGGL((k_stage<STAGE, S, TY, false, false, W>), grid, block, 0, c->stream, a);
+        hipLaunchKernelGGL((k_stage<STAGE, S, TY, false, kPlain, W>), grid, block, 0, c->stream, a);
     BX_HIP(hipGetLastError());
     return BX_OK;
 }
@@ -248,6 +247,52 @@ static int launch_stage(bx_ctx *c, const StageArgs &a, hipEvent_t mid, S *eflux)
     return BX_OK;
 }
 
+// The flux subroutine on interior cells (bx_tile.h, stages 3 and 4): cons ->
+// out, with cons_old for avg = 1.  slow: the word that records a value outside
+// the tile's range; slow_next: cleared for the next call.
+int launch_tiled_flux(bx_ctx *c, int avg, double dt, double *out, unsigned int *slow, unsigned int *slow_next)
+{
+    StageArgs a = base_args(c, dt);
+    a.uin = c->cons;
+    a.uold = c->cons_old;
+    a.pin = c->p;
+    a.vel = c->u;
+    a.ad = c->adindx;
+    a.uout = out;
+    a.gf = nullptr;
+    a.flags = slow;
+    a.clear = slow_next;
+    // gamma from its plane unless every cell holds gammafix; the seventh field
+    // leaves room in LDS for 64 x 4 tiles only
+    const bool vg = !c->ad_uniform;
+    int ty = 4;
+    tile_split(c, false, !vg, true, &a.lz, &ty);
+    const bool p2 = a.ds_pow2[0] && a.ds_pow2[1] && a.ds_pow2[2] && a.vol_pow2;
+    const int nzi = a.zhi - a.zlo;
+    const dim3 grid((unsigned)((c->nx - 4 + 63) / 64), (unsigned)((c->ny - 4 + ty - 1) / ty),
+                    (unsigned)((nzi + a.lz - 1) / a.lz));
+    const dim3 block(64 * (ty + 4));
+    auto go = [&](auto stage, auto rows, auto pow2, auto kind) {
+        hipLaunchKernelGGL((k_stage<decltype(stage)::value, double, decltype(rows)::value, decltype(pow2)::value,
+                                    decltype(kind)::value, false>),
+                           grid, block, 0, c->stream, a);
+    };
+    auto with_stage = [&](auto rows, auto pow2, auto kind) {
+        if (avg == 0) go(std::integral_constant<int, 3>{}, rows, pow2, kind);
+        else go(std::integral_constant<int, 4>{}, rows, pow2, kind);
+    };
+    auto with_spacing = [&](auto rows, auto kind) {
+        if (p2) with_stage(rows, std::true_type{}, kind);
+        else with_stage(rows, std::false_type{}, kind);
+    };
+    using Plain = std::integral_constant<int, kPlain>;
+    if (vg) with_spacing(std::integral_constant<int, 4>{}, std::integral_constant<int, kGamma>{});
+    else if (ty == 8) with_spacing(std::integral_constant<int, 8>{}, Plain{});
+    else with_spacing(std::integral_constant<int, 4>{}, Plain{});
+    BX_HIP(hipGetLastError());
+    return BX_OK;
+}
+
 // the pressure plane of the materialised state at the corner ghosts (the
 // value the last fused step's fix-up recorded)
 __global__ __launch_bounds__(64) void k_corner_pressure(int nd2, const int32_t *__restrict__ dst,
@@ -262,6 +307,7 @@ int launch_materialize(bx_ctx *c)
     hipLaunchKernelGGL(k_materialize, dim3(blocks_for(c->n, 256)), dim3(256), 0, c->stream, c->n, c->cons, c->u,
                        c->p_fused ? (double *)nullptr : c->p, c->adindx, c->prm.gammafix, c->prm.small_eps);
     BX_HIP(hipGetLastError());
+    c->ad_uniform = true;
     if (c->nd2 > 0 && c->prm.precision == BX_PREC_FP64) {  // the mixed form copies the donors
         hipLaunchKernelGGL(k_corner_pressure, dim3(1), dim3(64), 0, c->stream, c->nd2, c->d2_dst, c->d2_ubar, c->p);
         BX_HIP(hipGetLastError());
@@ -285,25 +331,46 @@ int fused_supported(const bx_ctx *c)
     return BX_OK;
 }
 
-// Default work split of the stage kernels: one kernel per stage, marching in z
-// chunks of the interior planes (any length: the chunk is nzi/m rounded up for
-// m chunks).  A workgroup's time is (planes it marches) x (time per plane) + a
-// start that does not depend on the chunk (launch, the first planes of the z
-// queue), so the chunk minimises that over the rounds of workgroups each CU
-// takes; ties go to the longer chunk.  Constants in us for both stages
-// together, from sweeps of the chunk at 16^3..256^3 (MI355X):
-//   FP64, 64 x 8 tiles (variant 11): one workgroup per CU (LDS), 13 per plane
-//     + 33.  96^3: chunk 10 (240 workgroups) 172 us, 16 (144) 247 us.
-//   FP64, 64 x 4 tiles (variant 10): one workgroup per CU, 8.5 per plane + 30:
-//     half the rows per CU, so faster where the 8-row tiles leave CUs idle
-//     (32^3 with one plane each: 50 us against 55; 85 us with chunks of 4
-//     planes on 8-row tiles), and slower where they fill the chip (256^3: 2.5
-//     against 1.95 ms).
+// The z chunk (and tile rows, 8 or 4) of the tiled kernels: they march in z
+// chunks of the interior planes (any length: nzi/m rounded up for m chunks).
+// A workgroup's time is (planes it marches) x (time per plane) + a start that
+// does not depend on the chunk (launch, the first planes of the z queue), so
+// the chunk minimises that over the rounds of workgroups each CU takes; ties
+// go to the longer chunk.  Constants in us for both stages together, from
+// sweeps of the chunk at 16^3..256^3 (MI355X):
+//   FP64, 64 x 8 tiles: one workgroup per CU (LDS), 13 per plane + 33.  96^3:
+//     chunk 10 (240 workgroups) 172 us, 16 (144) 247 us.
+//   FP64, 64 x 4 tiles: one workgroup per CU, 8.5 per plane + 30: half the
+//     rows per CU, so faster where the 8-row tiles leave CUs idle (32^3 with
+//     one plane each: 50 us against 55; 85 us with chunks of 4 planes on 8-row
+//     tiles), and slower where they fill the chip (256^3: 2.5 against 1.95 ms).
 //   Mixed, 64 x 4 tiles: several workgroups share a CU and its issue slots, so
 //     the time is (workgroups per CU) x (chunk + 2 planes), with one alone on
 //     its CU, which waits for its own latencies, counted as 1.6.  192^3: chunk
 //     28 489 us, 32 545 us; 64^3: chunk 2 56 us, 4 64 us.
-// The y chunk (fused_ly) only serves the two-kernel variants.  Allocates
+void tile_split(const bx_ctx *c, bool mixed, bool rows8, bool rows4, int *lz, int *ty)
+{
+    const int nzi = c->flatz ? c->nz : c->nz - 4;
+    double best = HUGE_VAL;
+    for (int t = 8; t >= 4; t -= 4) {
+        if (t == 8 ? !rows8 : !rows4) continue;
+        const int64_t tiles = (int64_t)((c->nx - 4 + 63) / 64) * ((c->ny - 4 + t - 1) / t);
+        for (int m = 1; m <= nzi && m <= 4 * c->ncu; m++) {
+            const int l = (nzi + m - 1) / m;
+            const double rounds = (double)((tiles * ((nzi + l - 1) / l) + c->ncu - 1) / c->ncu);
+            const double cost = mixed ? std::fmax(rounds, 1.6) * (l + 2)
+                                      : rounds * (t == 8 ? 13.0 * l + 33.0 : 8.5 * l + 30.0);
+            if (cost < best) {
+                best = cost;
+                *lz = l;
+                *ty = t;
+            }
+        }
+    }
+}
+
+// Default work split of the stage kernels.  The y chunk (fused_ly) only serves
+// the two-kernel variants; gravity has the 64 x 8 tiles only.  Allocates
 // nothing.
 void fused_defaults(bx_ctx *c)
 {
@@ -315,26 +382,10 @@ void fused_defaults(bx_ctx *c)
         c->fused_ly = ly;
     }
     if (c->fused_lz == 0) {
-        int ncu = 0;
-        if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess || ncu < 1)
-            ncu = 256;
         const bool mixed = c->prm.precision == BX_PREC_MIXED;
-        double best = HUGE_VAL;
-        for (int ty = 8; ty >= 4; ty -= 4) {
-            if (mixed ? ty == 8 : (ty == 4 && c->grav_flags)) continue;  // gravity has the 64 x 8 tiles only
-            const int64_t tiles = (int64_t)((c->nx - 4 + 63) / 64) * ((c->ny - 4 + ty - 1) / ty);
-            for (int m = 1; m <= nzi && m <= 4 * ncu; m++) {
-                const int lz = (nzi + m - 1) / m;
-                const double rounds = (double)((tiles * ((nzi + lz - 1) / lz) + ncu - 1) / ncu);
-                const double cost = mixed ? std::fmax(rounds, 1.6) * (lz + 2)
-                                          : rounds * (ty == 8 ? 13.0 * lz + 33.0 : 8.5 * lz + 30.0);
-                if (cost < best) {
-                    best = cost;
-                    c->fused_lz = lz;
-                    c->fused_occ = ty == 8 ? 11 : 10;
-                }
-            }
-        }
+        int ty = 8;
+        tile_split(c, mixed, !mixed, mixed || !c->grav_flags, &c->fused_lz, &ty);
+        c->fused_occ = ty == 8 ? 11 : 10;
     }
 }
 
@@ -364,7 +415,7 @@ int launch_regular_check(bx_ctx *c)
 {
     BX_HIP(hipMemsetAsync(&c->dsc->flags, 0, sizeof(unsigned int), c->stream));
     BX_HIP(hipMemsetAsync(&c->dsc->rate_bits[0], 0, sizeof(unsigned long long), c->stream));
-    hipLaunchKernelGGL(k_regular, dim3(blocks_for(c->n, 256)), dim3(256), 0, c->stream, c->n, c->cons, c->u,
+    hipLaunchKernelGGL(k_regular, dim3(reduce_blocks(c->n)), dim3(256), 0, c->stream, c->n, c->cons, c->u,
                        c->prm.gammafix, c->prm.small_eps, c->prm.dx, c->prm.dy, c->prm.dz, &c->dsc->flags,
                        &c->dsc->rate_bits[0]);
     BX_HIP(hipGetLastError());
@@ -537,8 +588,15 @@ static S *grav_pressure(bx_ctx *c, StageArgs &b)
     return nullptr;
 }
 
-// Whether the stage kernels read donors in place of ghost cells.
-static bool reads_donors(const bx_ctx *c) { return c->axis_ghosts && c->fused_occ >= 10; }
+// Whether the stage kernels read donors in place of ghost cells.  Gravity with
+// walls reads its ghosts from memory: the signs take the gravity form over its
+// registers (12 to 19 VGPRs spilled).
+static bool reads_donors(const bx_ctx *c)
+{
+    bool wall = false;
+    for (int i = 0; i < 6; i++) wall = wall || c->prm.no_outflow[i];
+    return c->axis_ghosts && c->fused_occ >= 10 && !(c->grav_flags && wall);
+}
 
 static void read_donors(const bx_ctx *c, StageArgs &a)
 {
@@ -625,7 +683,7 @@ void drop_step_graphs(bx_ctx *c)
         if (c->sgraph[i]) (void)hipGraphDestroy(c->sgraph[i]);
         c->sexec[i] = nullptr;
         c->sgraph[i] = nullptr;
-        c->skey[i] = nullptr;
+        c->skey[i] = c->skey2[i] = nullptr;
     }
 }
 
@@ -635,17 +693,19 @@ static int pair_exec(bx_ctx *c, hipGraphExec_t *out)
 {
     const bool f32 = c->state_in_32;
     const void *key = f32 ? (const void *)c->cons32 : (const void *)c->cons;
+    const void *key2 = f32 ? (const void *)c->unext32 : (const void *)c->unext;
     for (int i = 0; i < 2; i++)
-        if (c->sexec[i] && c->skey[i] == key) {
+        if (c->sexec[i] && c->skey[i] == key && c->skey2[i] == key2) {
             *out = c->sexec[i];
             return BX_OK;
         }
-    const int slot = c->sexec[0] ? (c->sexec[1] ? 0 : 1) : 0;
+    const int slot = c->sexec[0] ? (c->sexec[1] ? c->snext : 1) : 0;
+    c->snext = 1 - slot;
     if (c->sexec[slot]) (void)hipGraphExecDestroy(c->sexec[slot]);
     if (c->sgraph[slot]) (void)hipGraphDestroy(c->sgraph[slot]);
     c->sexec[slot] = nullptr;
     c->sgraph[slot] = nullptr;
-    c->skey[slot] = nullptr;
+    c->skey[slot] = c->skey2[slot] = nullptr;
     BX_HIP(hipStreamSynchronize(c->stream));
     BX_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     const int rc = enqueue_current_pair(c);
@@ -665,6 +725,7 @@ static int pair_exec(bx_ctx *c, hipGraphExec_t *out)
     c->sgraph[slot] = g;
     c->sexec[slot] = x;
     c->skey[slot] = key;
+    c->skey2[slot] = key2;
     *out = x;
     return BX_OK;
 }

@@ -32,6 +32,7 @@ struct DevScalars {
     unsigned int flags;               // irregular-branch flags raised by the fused kernels
     unsigned int pad;
     StepSlot slot[2];
+    unsigned int slow[2];             // FLAG_SLOW of a tiled flux call; calls alternate between the two words
 };
 
 // flags bits
@@ -40,6 +41,7 @@ enum : unsigned int {
     FLAG_CLAMP = 2u,   // a velocity() call met |u_i|>vlimit (velocity.f90:33)
     FLAG_FLOOR = 8u,   // a floor of the stage update acted (flux.f90:225-228, the source re-round
                        // or the p* eps floor); informational: the step is exact either way
+    FLAG_SLOW = 16u,   // the tiled flux met a value outside its range (bx_stage.h prims)
     FLAG_IRREGULAR = FLAG_LOWRHO | FLAG_CLAMP,
 };
 
@@ -63,7 +65,11 @@ struct bx_ctx {
     double *p;
     double *adindx;
     double *qq;        // 3 planes
-    double *states;    // exact-flux intermediate, state_planes(c) planes (face fluxes or interface states)
+    double *states;    // exact-flux output or intermediate, state_planes(c) planes (the flux's result, which
+                       // trades places with cons; with flux_ang the interface states)
+    bool ad_uniform;   // every cell of adindx holds gammafix
+    unsigned nflux;    // tiled flux calls so far (parity: which slow word a call uses)
+    int ncu;           // compute units of the device
 
     // ghost table: ghost cell id, donor (>=0: cell id; <0: -(scratch slot+1)),
     // sign bits (bit k flips momentum k); scratch holds pre-fill values of
@@ -118,10 +124,12 @@ struct bx_ctx {
     int64_t nfused, nexact;  // steps bx_step took with the fused kernels / the exact sequence
 
     // captured pairs of fused steps (BX_STEP_GRAPH), keyed by the state buffer
-    // they start from (the pair returns the state to it)
+    // they start from (the pair returns the state to it) and the other one
+    // (the exact path's flux trades the state buffer for another)
     hipGraph_t sgraph[2];
     hipGraphExec_t sexec[2];
-    const void *skey[2];
+    const void *skey[2], *skey2[2];
+    int snext;             // the slot the next capture replaces
     void *chunk0;          // 5 planes: the state at the start of a replayed chunk (rollback)
     int64_t graph_steps;   // steps taken from replays (kept, not undone)
     double *chunk_dts;     // dt of each step of a chunk
@@ -167,10 +175,16 @@ int hip_check(hipError_t e, const char *what);
         if (_e != hipSuccess) return bx::hip_check(_e, #call);   \
     } while (0)
 
-// planes of the exact flux's intermediate: the face fluxes, 5 per direction;
-// with flux_ang the interface states, per direction 9 minus + 9 plus (rho, u,
+// planes of the exact flux's output (5 conserved planes); with flux_ang of its
+// intermediate, the interface states, per direction 9 minus + 9 plus (rho, u,
 // v, w, p, eps, gamma, r- and angular momentum)
-inline int state_planes(const bx_ctx *c) { return c->prm.fluxangmom ? 54 : 15; }
+inline int state_planes(const bx_ctx *c) { return c->prm.fluxangmom ? 54 : 5; }
+
+// blocks of a reduction over n cells (256 threads, each taking every
+// gridDim-th 256 cells): few enough that the one atomic per block does not
+// bound the kernel (about 9 ns each on one address: 3,906 blocks at 96^3 took
+// 46 us for a Courant pass that streams in 10)
+inline unsigned int reduce_blocks(int64_t n) { return (unsigned int)((n + 255) / 256 < 1024 ? (n + 255) / 256 : 1024); }
 
 inline unsigned int blocks_for(int64_t n, int threads)
 {
@@ -184,6 +198,8 @@ int launch_courant(bx_ctx *c);
 int launch_source(bx_ctx *c, double dt);
 int launch_ghosts(bx_ctx *c, double *planes5);
 int launch_flux(bx_ctx *c, int avg, double dt);
+int launch_tiled_flux(bx_ctx *c, int avg, double dt, double *out, unsigned int *slow, unsigned int *slow_next);
+void tile_split(const bx_ctx *c, bool mixed, bool rows8, bool rows4, int *lz, int *ty);
 int launch_avisc(bx_ctx *c);
 int launch_materialize(bx_ctx *c);
 int launch_regular_check(bx_ctx *c);

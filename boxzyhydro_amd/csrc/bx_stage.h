@@ -70,6 +70,11 @@ struct StageArgs {
     // donor's force with the ghost's momentum sign flips, so that a ghost's
     // source result is its donor's up to those flips; null without gravity
     const double *gf;
+    // stages 3 and 4 (the flux subroutine on the exact path's planes): the
+    // velocity planes and, with kGamma, adindx; uin, uold and pin are cons,
+    // cons_old and p, uout receives the updated interior cells
+    const double *vel, *ad;
+    unsigned int *clear;  // a word the first lane of the grid clears (may be null)
 };
 
 // One step's scalars on the device, in the operations of the host driver
@@ -119,6 +124,7 @@ __device__ __forceinline__ StageArgs with_dt(const StageArgs &a0)
         a.dt = *a0.dtp;
     }
     if (a0.rate_next && first_lane_of_grid()) *a0.rate_next = 0ull;
+    if (a0.clear && first_lane_of_grid()) *a0.clear = 0u;
     return a;
 }
 
@@ -143,6 +149,15 @@ StageArgs base_args(bx_ctx *c, double dt);
 template <typename T>
 struct W6 {
     T d, u0, u1, u2, p, e;
+    T g;  // gamma, where it varies from cell to cell (StageKind kGamma); elsewhere unused
+};
+
+// What a stage kernel carries beside the plain fixed-gamma flux of a regular
+// state.
+enum StageKind : int {
+    kPlain = 0,
+    kGravity = 1,  // stages 1 and 2: the kick of source() with the force planes gf (FP64)
+    kGamma = 2,    // stages 3 and 4: gamma from the plane ad, reconstructed as the other primitives
 };
 
 template <typename T>
@@ -210,6 +225,7 @@ __device__ __forceinline__ W6<T> wave_shift_w(const W6<T> &w)
     o.u2 = wave_shift_t<CTRL>(w.u2, w.u2);
     o.p = wave_shift_t<CTRL>(w.p, w.p);
     o.e = wave_shift_t<CTRL>(w.e, w.e);
+    o.g = wave_shift_t<CTRL>(w.g, w.g);
     return o;
 }
 template <typename T>
@@ -233,7 +249,7 @@ __device__ __forceinline__ T comp(const W6<T> &w, int j)
 // finite slopes of finite data).  lp and lm enter only as 1-lp and -1-lm,
 // where a zero of either sign gives the same value, so the hardware maximum
 // and minimum stand for vmax/vmin against 0.
-template <int d, typename T>
+template <int d, typename T, bool VG = false>
 __device__ __forceinline__ void dir_states(const W6<T> &wm, const W6<T> &wc, const W6<T> &wp, T sound, bool ghost,
                                            const StageArgs &a, Side<T> &mi, Side<T> &pl)
 {
@@ -262,8 +278,15 @@ __device__ __forceinline__ void dir_states(const W6<T> &wm, const W6<T> &wc, con
     pl.p = p0 + cp * sp;
     mi.e = e0 + cm * se;
     pl.e = e0 + cp * se;
-    mi.g = T(a.gam);  // slope(gamma,gamma,gamma)=0: gamma + (+-0) + 0 = gamma
-    pl.g = T(a.gam);
+    if constexpr (VG) {
+        const T sg = slope_fz(wm.g, wc.g, wp.g);
+        const T g0 = wc.g + z;
+        mi.g = g0 + cm * sg;
+        pl.g = g0 + cp * sg;
+    } else {
+        mi.g = T(a.gam);  // slope(gamma,gamma,gamma)=0: gamma + (+-0) + 0 = gamma
+        pl.g = T(a.gam);
+    }
 }
 
 template <typename T>
@@ -284,22 +307,32 @@ __device__ __forceinline__ T sound_of(const W6<T> &w, double gam)
 template <typename S>
 struct Raw {
     S r, m0, m1, m2, E, p;
-    S g0, g1, g2;  // stage 1 with gravity: the cell's force
+    S g0, g1, g2;  // stage 1 with gravity: the cell's force; kGamma: g0 is gamma
 };
 
 // cell = uniform element offset u + per-lane byte offset boff
-template <int STAGE, typename S, bool G = false>
+template <int STAGE, typename S, int V = kPlain>
 __device__ __forceinline__ Raw<S> load_raw(const StageArgs &a, int64_t u, unsigned boff)
 {
     const int64_t n = a.n;
     Raw<S> v;
+    if constexpr (STAGE >= 3) {
+        v.r = elem<S>(a.uin, u, boff);
+        v.E = elem<S>(a.uin, 4 * n + u, boff);
+        v.m0 = elem<S>(a.vel, u, boff);
+        v.m1 = elem<S>(a.vel, n + u, boff);
+        v.m2 = elem<S>(a.vel, 2 * n + u, boff);
+        v.p = elem<S>(a.pin, u, boff);
+        if constexpr (V == kGamma) v.g0 = elem<S>(a.ad, u, boff);
+        return v;
+    }
     v.r = elem<S>(a.uin, u, boff);
     v.m0 = elem<S>(a.uin, n + u, boff);
     v.m1 = elem<S>(a.uin, 2 * n + u, boff);
     v.m2 = elem<S>(a.uin, 3 * n + u, boff);
     v.E = elem<S>(a.uin, 4 * n + u, boff);
     v.p = STAGE == 2 ? elem<S>(a.pin, u, boff) : S(0);
-    if constexpr (G && STAGE == 1) {
+    if constexpr (V == kGravity && STAGE == 1) {
         v.g0 = elem<S>(a.gf, u, boff);
         v.g1 = elem<S>(a.gf, n + u, boff);
         v.g2 = elem<S>(a.gf, 2 * n + u, boff);
@@ -328,11 +361,29 @@ __device__ __forceinline__ double grav_energy_arg(double r, double E, double ek,
 // FP64 storage: the reference's own operations.  FP32 storage (mixed form):
 // the kinetic energy, the energy/pressure subtraction and u are formed in FP64
 // from the stored values, then rounded for the FP32 reconstruction.
-template <int STAGE, typename S, bool G = false>
+// Stages 3 and 4 take the velocity and pressure planes as they are (the last
+// velocity() and state() calls').  The tile's arithmetic stands for the exact
+// path's (slopes by min/max, a ghost's zero coefficients in place of zero
+// slopes, no z difference on a flat axis) for finite numbers whose products
+// do not overflow and where every sound speed is positive; any other value
+// raises the flag and the cell-by-cell kernel takes that call.
+template <int STAGE, typename S, int V = kPlain>
 __device__ __forceinline__ W6<S> prims(const StageArgs &a, const Raw<S> &v, unsigned int &flg)
 {
     W6<S> w;
-    if constexpr (G && STAGE == 1) {
+    w.g = S(0);
+    if constexpr (STAGE >= 3) {
+        static_assert(sizeof(S) == 8, "the exact path is FP64");
+        w.d = v.r;
+        w.u0 = v.m0;
+        w.u1 = v.m1;
+        w.u2 = v.m2;
+        w.p = v.p;
+        w.e = floor_at(v.E - 0.5 * v.r * (v.m0 * v.m0 + v.m1 * v.m1 + v.m2 * v.m2), a.seps);
+        if constexpr (V == kGamma) w.g = v.g0;
+        const double mag = ((fabs(v.r) + fabs(v.E)) + (fabs(v.m0) + fabs(v.m1))) + ((fabs(v.m2) + fabs(v.p)) + fabs(w.g));
+        if (!(mag <= 1e60) || !(v.r > 0.0) || !(v.p > 0.0)) flg |= FLAG_SLOW;
+    } else if constexpr (V == kGravity && STAGE == 1) {
         static_assert(sizeof(S) == 8, "gravity is FP64 only");
         // source(0) (main.f90:289) with the cell's force: u_old = m/rho is the
         // velocity of the last velocity call (the previous step's), the state
@@ -403,10 +454,23 @@ __device__ __forceinline__ W6<S> prims(const StageArgs &a, const Raw<S> &v, unsi
     return w;
 }
 
-template <int STAGE, typename S, bool G = false>
+template <int STAGE, typename S, int V = kPlain>
 __device__ __forceinline__ W6<S> load_prims(const StageArgs &a, int64_t u, unsigned boff, unsigned int &flg)
 {
-    return prims<STAGE, S, G>(a, load_raw<STAGE, S, G>(a, u, boff), flg);
+    return prims<STAGE, S, V>(a, load_raw<STAGE, S, V>(a, u, boff), flg);
+}
+
+template <int V, typename T>
+__device__ __forceinline__ T sound_at(const W6<T> &w, const StageArgs &a)
+{
+    if constexpr (V == kGamma) {
+        const double x = w.p * w.g / w.d;
+        double r;
+        sqrt_n<1>(&x, &r);
+        return r;
+    } else {
+        return sound_of(w, a.gam);
+    }
 }
 
 

@@ -46,6 +46,9 @@
 // outputs), and at a wall (W) the normal velocity changes sign.  The ghost
 // cells of the stage's input then need no fill before it: two dispatches less
 // per step (4.6 us each on small grids, 33 us each at 256^3).
+// Stages 3 and 4 are the flux subroutine of the exact path (flux(0), flux(1)):
+// the same march over the planes cons, u, p (and adindx) as they stand, ghosts
+// from memory, ending with flux.f90:205-228.
 // Every arithmetic operation is the one the exact sequence performs on the
 // same values, so the results are bit-identical to it.
 #pragma once
@@ -55,20 +58,22 @@
 
 namespace bx {
 
-template <typename S, int TY>
+template <typename S, int TY, int V = kPlain>
 struct TileLds {
     static constexpr int RS = 66;  // row stride of the primitive tile: columns -1..64
-    S P[2][6][(TY + 4) * RS];      // rho, u0, u1, u2, p, eps of planes k, k+1 (tile k&1), rows -2..TY+1
-    S Sy[6][(TY + 1) * 64];        // y-plus states of rows -1..TY-1 (index r+1), then y-face r-1/2 (index r)
-    S SxL[6][TY];                  // x-plus state of column -1, per owner row
+    static constexpr int NF = V == kGamma ? 7 : 6;
+    S P[2][NF][(TY + 4) * RS];     // rho, u0, u1, u2, p, eps (, gamma) of planes k, k+1 (tile k&1), rows -2..TY+1
+    S Sy[NF][(TY + 1) * 64];       // y-plus states of rows -1..TY-1 (index r+1), then y-face r-1/2 (index r)
+    S SxL[NF][TY];                 // x-plus state of column -1, per owner row
     S FxR[5][TY];                  // x-face flux 63+1/2, per owner row
     double Dx[5][TY * 64];         // x flux difference of each owner cell (phase B to D)
     double Dz[5][TY * 64];         // z flux difference of each owner cell (phase A to D)
 };
 
-template <typename S, int N>
-__device__ __forceinline__ void store_w(S (&P)[6][N], int idx, const W6<S> &w)
+template <typename S, int F, int N>
+__device__ __forceinline__ void store_w(S (&P)[F][N], int idx, const W6<S> &w)
 {
+    if constexpr (F == 7) P[F - 1][idx] = w.g;
     P[0][idx] = w.d;
     P[1][idx] = w.u0;
     P[2][idx] = w.u1;
@@ -77,10 +82,12 @@ __device__ __forceinline__ void store_w(S (&P)[6][N], int idx, const W6<S> &w)
     P[5][idx] = w.e;
 }
 
-template <typename S, int N>
-__device__ __forceinline__ W6<S> fetch_w(const S (&P)[6][N], int idx)
+template <typename S, int F, int N>
+__device__ __forceinline__ W6<S> fetch_w(const S (&P)[F][N], int idx)
 {
     W6<S> w;
+    w.g = S(0);
+    if constexpr (F == 7) w.g = P[F - 1][idx];
     w.d = P[0][idx];
     w.u0 = P[1][idx];
     w.u1 = P[2][idx];
@@ -90,9 +97,10 @@ __device__ __forceinline__ W6<S> fetch_w(const S (&P)[6][N], int idx)
     return w;
 }
 
-template <typename S, int N>
-__device__ __forceinline__ void store_side(S (&B)[6][N], int idx, const Side<S> &s)
+template <typename S, int F, int N>
+__device__ __forceinline__ void store_side(S (&B)[F][N], int idx, const Side<S> &s)
 {
+    if constexpr (F == 7) B[F - 1][idx] = s.g;
     B[0][idx] = s.d;
     B[1][idx] = s.v[0];
     B[2][idx] = s.v[1];
@@ -101,8 +109,8 @@ __device__ __forceinline__ void store_side(S (&B)[6][N], int idx, const Side<S> 
     B[5][idx] = s.e;
 }
 
-template <typename S, int N>
-__device__ __forceinline__ Side<S> fetch_side(const S (&B)[6][N], int idx, S gam)
+template <typename S, int F, int N>
+__device__ __forceinline__ Side<S> fetch_side(const S (&B)[F][N], int idx, S gam)
 {
     Side<S> s;
     s.d = B[0][idx];
@@ -112,6 +120,7 @@ __device__ __forceinline__ Side<S> fetch_side(const S (&B)[6][N], int idx, S gam
     s.p = B[4][idx];
     s.e = B[5][idx];
     s.g = gam;
+    if constexpr (F == 7) s.g = B[F - 1][idx];
     return s;
 }
 
@@ -184,15 +193,28 @@ struct TileGeom {
     int kb, ke;
 };
 
+// The end of the flux subroutine at an interior cell (flux.f90:205-228): the
+// stage update with fluxtmp ft and the floors.
+template <int STAGE>
+__device__ __forceinline__ void flux_update(const StageArgs &a, const double ui[5], const double uo[5],
+                                            const double ft[5], int64_t c, unsigned coff)
+{
+    double U[5];
+    for (int i = 0; i < 5; i++) U[i] = STAGE == 3 ? ui[i] + ft[i] : 0.5 * (uo[i] + ui[i] + ft[i]);
+    U[0] = floor_at(U[0], a.srho);
+    if (U[4] < 0.0) U[4] = 0.5 * (U[1] * U[1] + U[2] * U[2] + U[3] * U[3]) / U[0] + a.seps;
+    for (int i = 0; i < 5; i++) elem<double>(a.uout, (int64_t)i * a.n + c, coff) = U[i];
+}
+
 // Owner rows 0..TY-1: the register queue in z and the stage update.  The
 // primitives of plane k are read back from the tile where needed, and the x
 // and z flux differences are parked in LDS until the update, to keep the
 // registers live across the barriers few.
-template <int STAGE, typename S, int TY, bool G, bool W>
-__device__ __forceinline__ void tile_owner(const StageArgs &a, TileLds<S, TY> &L, const TileGeom &g,
+template <int STAGE, typename S, int TY, int V, bool W>
+__device__ __forceinline__ void tile_owner(const StageArgs &a, TileLds<S, TY, V> &L, const TileGeom &g,
                                            unsigned int &flg, double &rmax)
 {
-    constexpr int RS = TileLds<S, TY>::RS;
+    constexpr int RS = TileLds<S, TY, V>::RS;
     const int lane = g.lane, r = g.r, nx = g.nx, ny = g.ny, nz = g.nz;
     const int64_t n = g.n;
     const int x = g.x0 + lane, y = g.j0 + r;
@@ -214,27 +236,27 @@ __device__ __forceinline__ void tile_owner(const StageArgs &a, TileLds<S, TY> &L
     const int kb = g.kb, ke = g.ke;
     if (!a.flatz) {
         auto at = [&](int k) -> W6<S> {
-            W6<S> w = load_prims<STAGE, S, G>(a, zplane(k), coff, flg);
+            W6<S> w = load_prims<STAGE, S, V>(a, zplane(k), coff, flg);
             me.signs(a, k, w);
             return w;
         };
         const W6<S> t0 = at(kb - 2), t1 = at(kb - 1), t2 = at(kb), t3 = at(kb + 1);
         Side<S> zmi, zpl;
-        dir_states<2>(t0, t1, t2, sound_of(t1, a.gam), xy_ghost || zghost(kb - 1), a, zmi, zpl);
+        dir_states<2, S, V == kGamma>(t0, t1, t2, sound_at<V>(t1, a), xy_ghost || zghost(kb - 1), a, zmi, zpl);
         zp_prev = zpl;
-        cs1 = sound_of(t2, a.gam);
-        dir_states<2>(t1, t2, t3, cs1, xy_ghost || zghost(kb), a, zmi, zpl);
+        cs1 = sound_at<V>(t2, a);
+        dir_states<2, S, V == kGamma>(t1, t2, t3, cs1, xy_ghost || zghost(kb), a, zmi, zpl);
         face_flux<S, 2>(zp_prev, zmi, Fz_prev);
         zp_prev = zpl;
         store_w(L.P[kb & 1], c, t2);  // plane kb
         q2 = t3;
-        nxt = load_raw<STAGE, S, G>(a, zplane(kb + 2), coff);
+        nxt = load_raw<STAGE, S, V>(a, zplane(kb + 2), coff);
     } else {
-        W6<S> w = load_prims<STAGE, S, G>(a, zplane(kb), coff, flg);
+        W6<S> w = load_prims<STAGE, S, V>(a, zplane(kb), coff, flg);
         me.signs(a, kb, w);
-        cs1 = sound_of(w, a.gam);
+        cs1 = sound_at<V>(w, a);
         store_w(L.P[kb & 1], c, w);
-        if (kb + 1 < ke) nxt = load_raw<STAGE, S, G>(a, zplane(kb + 1), coff);
+        if (kb + 1 < ke) nxt = load_raw<STAGE, S, V>(a, zplane(kb + 1), coff);
     }
     __syncthreads();  // every row's primitives of plane kb are in the tile
 
@@ -249,12 +271,12 @@ __device__ __forceinline__ void tile_owner(const StageArgs &a, TileLds<S, TY> &L
             const Raw<S> cur = nxt;
             // plane k+3 (the last iteration reloads a plane, so that the queue
             // needs no branch)
-            nxt = load_raw<STAGE, S, G>(a, zplane(min(k + 3, nz - 1)), coff);
-            q2 = prims<STAGE, S, G>(a, cur, flg);
+            nxt = load_raw<STAGE, S, V>(a, zplane(min(k + 3, nz - 1)), coff);
+            q2 = prims<STAGE, S, V>(a, cur, flg);
             me.signs(a, k + 2, q2);
-            cs1 = sound_of(q1, a.gam);
+            cs1 = sound_at<V>(q1, a);
             Side<S> zmi1, zpl1;
-            dir_states<2>(fetch_w(L.P[t], c), q1, q2, cs1, xy_ghost || zghost(k + 1), a, zmi1, zpl1);
+            dir_states<2, S, V == kGamma>(fetch_w(L.P[t], c), q1, q2, cs1, xy_ghost || zghost(k + 1), a, zmi1, zpl1);
             S Fz1[5];
             face_flux<S, 2>(zp_prev, zmi1, Fz1);
             for (int i = 0; i < 5; i++) {
@@ -267,10 +289,10 @@ __device__ __forceinline__ void tile_owner(const StageArgs &a, TileLds<S, TY> &L
             cs0 = cs1;
             if (k + 1 < ke) {
                 const Raw<S> cur = nxt;
-                nxt = load_raw<STAGE, S, G>(a, zplane(min(k + 2, ke - 1)), coff);
-                W6<S> w = prims<STAGE, S, G>(a, cur, flg);
+                nxt = load_raw<STAGE, S, V>(a, zplane(min(k + 2, ke - 1)), coff);
+                W6<S> w = prims<STAGE, S, V>(a, cur, flg);
                 me.signs(a, k + 1, w);
-                cs1 = sound_of(w, a.gam);
+                cs1 = sound_at<V>(w, a);
                 store_w(L.P[t ^ 1], c, w);
             }
         }
@@ -278,7 +300,7 @@ __device__ __forceinline__ void tile_owner(const StageArgs &a, TileLds<S, TY> &L
         {
             const W6<S> q0 = fetch_w(L.P[t], c);
             Side<S> xmi, xpl;
-            dir_states<0>(fetch_w(L.P[t], c - 1), q0, fetch_w(L.P[t], c + 1), cs0, ghost_k, a, xmi, xpl);
+            dir_states<0, S, V == kGamma>(fetch_w(L.P[t], c - 1), q0, fetch_w(L.P[t], c + 1), cs0, ghost_k, a, xmi, xpl);
             Side<S> xl;
             xl.d = from_lower(xpl.d, L.SxL[0][r], lane);
             xl.v[0] = from_lower(xpl.v[0], L.SxL[1][r], lane);
@@ -287,6 +309,7 @@ __device__ __forceinline__ void tile_owner(const StageArgs &a, TileLds<S, TY> &L
             xl.p = from_lower(xpl.p, L.SxL[4][r], lane);
             xl.e = from_lower(xpl.e, L.SxL[5][r], lane);
             xl.g = gamS;
+            if constexpr (V == kGamma) xl.g = from_lower(xpl.g, L.SxL[TileLds<S, TY, V>::NF - 1][r], lane);
             S Fx0[5];
             face_flux<S, 0>(xl, xmi, Fx0);  // face l-1/2
             for (int i = 0; i < 5; i++) {
@@ -297,7 +320,7 @@ __device__ __forceinline__ void tile_owner(const StageArgs &a, TileLds<S, TY> &L
         Side<S> ymi;
         {
             Side<S> ypl;
-            dir_states<1>(fetch_w(L.P[t], c - RS), fetch_w(L.P[t], c), fetch_w(L.P[t], c + RS), cs0, ghost_k, a,
+            dir_states<1, S, V == kGamma>(fetch_w(L.P[t], c - RS), fetch_w(L.P[t], c), fetch_w(L.P[t], c + RS), cs0, ghost_k, a,
                           ymi, ypl);
             store_side(L.Sy, (r + 1) * 64 + lane, ypl);
         }
@@ -313,7 +336,7 @@ __device__ __forceinline__ void tile_owner(const StageArgs &a, TileLds<S, TY> &L
             double ui[5], uo[5], ft[5];
             for (int i = 0; i < 5; i++) {
                 ui[i] = elem<S>(a.uin, (int64_t)i * n + cz, coff);
-                uo[i] = STAGE == 2 ? (double)elem<S>(a.uold, (int64_t)i * n + cz, coff) : 0.0;
+                uo[i] = STAGE == 2 || STAGE == 4 ? (double)elem<S>(a.uold, (int64_t)i * n + cz, coff) : 0.0;
             }
             for (int i = 0; i < 5; i++) {
                 // flux.f90:188-190 in the reference's order, accumulated in FP64
@@ -323,18 +346,19 @@ __device__ __forceinline__ void tile_owner(const StageArgs &a, TileLds<S, TY> &L
                 const double s = (a.ayz * L.Dx[i][o] + ey) + a.axy * dz;
                 ft[i] = -div_by(s * a.dt, a.vol, a.inv_vol, a.vol_pow2);
             }
-            stage_update<STAGE, S, G>(a, ui, uo, ft, fetch_w(L.P[t], c), cz, coff, flg, rmax);
+            if constexpr (STAGE >= 3) flux_update<STAGE>(a, ui, uo, ft, cz, coff);
+            else stage_update<STAGE, S, V == kGravity>(a, ui, uo, ft, fetch_w(L.P[t], c), cz, coff, flg, rmax);
         }
     }
 }
 
 // Halo rows -2, -1 and TY: their primitives, the y-states of rows -1 and TY,
 // and face y TY-1/2.
-template <int STAGE, typename S, int TY, bool G, bool W>
-__device__ __forceinline__ void tile_halo(const StageArgs &a, TileLds<S, TY> &L, const TileGeom &g,
+template <int STAGE, typename S, int TY, int V, bool W>
+__device__ __forceinline__ void tile_halo(const StageArgs &a, TileLds<S, TY, V> &L, const TileGeom &g,
                                           unsigned int &flg)
 {
-    constexpr int RS = TileLds<S, TY>::RS;
+    constexpr int RS = TileLds<S, TY, V>::RS;
     const int lane = g.lane, r = g.r, nx = g.nx, ny = g.ny, nz = g.nz;
     const int x = g.x0 + lane, y = g.j0 + r;
     const Donor<S, W> me(a, x, y);
@@ -347,19 +371,19 @@ __device__ __forceinline__ void tile_halo(const StageArgs &a, TileLds<S, TY> &L,
     const int kb = g.kb, ke = g.ke;
     Raw<S> nxt;
     auto put = [&](int k, const Raw<S> &raw) {
-        W6<S> w = prims<STAGE, S, G>(a, raw, flg);
+        W6<S> w = prims<STAGE, S, V>(a, raw, flg);
         me.signs(a, k, w);
         store_w(L.P[k & 1], c, w);
     };
-    put(kb, load_raw<STAGE, S, G>(a, zplane(kb), coff));
-    if (kb + 1 < ke) nxt = load_raw<STAGE, S, G>(a, zplane(kb + 1), coff);
+    put(kb, load_raw<STAGE, S, V>(a, zplane(kb), coff));
+    if (kb + 1 < ke) nxt = load_raw<STAGE, S, V>(a, zplane(kb + 1), coff);
     __syncthreads();  // as the owners' first barrier
     for (int k = kb; k < ke; k++) {
         const int t = k & 1;
         if (k + 1 < ke) {
             // A: primitives of plane k+1 into the other tile
             const Raw<S> cur = nxt;
-            nxt = load_raw<STAGE, S, G>(a, zplane(min(k + 2, ke - 1)), coff);
+            nxt = load_raw<STAGE, S, V>(a, zplane(min(k + 2, ke - 1)), coff);
             put(k + 1, cur);
         }
         Side<S> ymi;
@@ -367,7 +391,7 @@ __device__ __forceinline__ void tile_halo(const StageArgs &a, TileLds<S, TY> &L,
             // B: y-states of plane k
             const W6<S> w = fetch_w(L.P[t], c);
             Side<S> ypl;
-            dir_states<1>(fetch_w(L.P[t], c - RS), w, fetch_w(L.P[t], c + RS), sound_of(w, a.gam),
+            dir_states<1, S, V == kGamma>(fetch_w(L.P[t], c - RS), w, fetch_w(L.P[t], c + RS), sound_at<V>(w, a),
                           xy_ghost || zghost(k), a, ymi, ypl);
             if (r == -1) store_side(L.Sy, lane, ypl);
         }
@@ -384,11 +408,11 @@ __device__ __forceinline__ void tile_halo(const StageArgs &a, TileLds<S, TY> &L,
 // Wave r=TY+1: its own halo row, and the x-edges of the owner rows one plane
 // ahead.  Lane 7*row+j holds column {-2,-1,0,62,63,64,65}[j] of owner row
 // `row`.
-template <int STAGE, typename S, int TY, bool G, bool W>
-__device__ __forceinline__ void tile_edge(const StageArgs &a, TileLds<S, TY> &L, const TileGeom &g,
+template <int STAGE, typename S, int TY, int V, bool W>
+__device__ __forceinline__ void tile_edge(const StageArgs &a, TileLds<S, TY, V> &L, const TileGeom &g,
                                           unsigned int &flg)
 {
-    constexpr int RS = TileLds<S, TY>::RS;
+    constexpr int RS = TileLds<S, TY, V>::RS;
     static_assert(7 * TY <= 64, "x-edge lanes of the owner rows must fit one wave");
     const int lane = g.lane, r = g.r, nx = g.nx, ny = g.ny, nz = g.nz;
     const int x = g.x0 + lane, y = g.j0 + r;
@@ -411,7 +435,7 @@ __device__ __forceinline__ void tile_edge(const StageArgs &a, TileLds<S, TY> &L,
     W6<S> ew{};
     Side<S> emi{}, epl{};
     auto edge_prims = [&](int k, const Raw<S> &raw) {
-        ew = prims<STAGE, S, G>(a, raw, flg);
+        ew = prims<STAGE, S, V>(a, raw, flg);
         em.signs(a, k, ew);
         if (ej == 1 || ej == 5) store_w(L.P[k & 1], (erow + 2) * RS + ecol + 1, ew);
     };
@@ -419,7 +443,7 @@ __device__ __forceinline__ void tile_edge(const StageArgs &a, TileLds<S, TY> &L,
     // lanes whose neighbour lies in another row or outside the wave are not
     // used: columns -1, 63 and 64 take columns -2..0 and 62..65)
     auto edge_states = [&](int k) {
-        dir_states<0>(lane_below_w(ew), ew, lane_above_w(ew), sound_of(ew, a.gam), e_xy_ghost || zghost(k), a, emi, epl);
+        dir_states<0, S, V == kGamma>(lane_below_w(ew), ew, lane_above_w(ew), sound_at<V>(ew, a), e_xy_ghost || zghost(k), a, emi, epl);
     };
     auto edge_publish = [&]() {
         if (ej == 1) store_side(L.SxL, erow, epl);
@@ -431,6 +455,7 @@ __device__ __forceinline__ void tile_edge(const StageArgs &a, TileLds<S, TY> &L,
         xl.p = lane_below(epl.p);
         xl.e = lane_below(epl.e);
         xl.g = gamS;
+        if constexpr (V == kGamma) xl.g = lane_below(epl.g);
         if (ej == 5) {
             S F[5];
             face_flux<S, 0>(xl, emi, F);  // face 63+1/2
@@ -441,18 +466,18 @@ __device__ __forceinline__ void tile_edge(const StageArgs &a, TileLds<S, TY> &L,
     const int kb = g.kb, ke = g.ke;
     Raw<S> nxt;
     auto put = [&](int k, const Raw<S> &raw) {
-        W6<S> w = prims<STAGE, S, G>(a, raw, flg);
+        W6<S> w = prims<STAGE, S, V>(a, raw, flg);
         me.signs(a, k, w);
         store_w(L.P[k & 1], c, w);
     };
-    put(kb, load_raw<STAGE, S, G>(a, zplane(kb), coff));
-    if (kb + 1 < ke) nxt = load_raw<STAGE, S, G>(a, zplane(kb + 1), coff);
+    put(kb, load_raw<STAGE, S, V>(a, zplane(kb), coff));
+    if (kb + 1 < ke) nxt = load_raw<STAGE, S, V>(a, zplane(kb + 1), coff);
     Raw<S> enxt{};
     if (e_on) {
-        edge_prims(kb, load_raw<STAGE, S, G>(a, zplane(kb), eoff));
+        edge_prims(kb, load_raw<STAGE, S, V>(a, zplane(kb), eoff));
         edge_states(kb);
         edge_publish();
-        if (kb + 1 < ke) enxt = load_raw<STAGE, S, G>(a, zplane(kb + 1), eoff);
+        if (kb + 1 < ke) enxt = load_raw<STAGE, S, V>(a, zplane(kb + 1), eoff);
     }
     __syncthreads();  // as the owners' first barrier
     for (int k = kb; k < ke; k++) {
@@ -460,11 +485,11 @@ __device__ __forceinline__ void tile_edge(const StageArgs &a, TileLds<S, TY> &L,
         if (more) {
             // A: primitives of plane k+1, its own row and the x-edges
             const Raw<S> cur = nxt;
-            nxt = load_raw<STAGE, S, G>(a, zplane(min(k + 2, ke - 1)), coff);
+            nxt = load_raw<STAGE, S, V>(a, zplane(min(k + 2, ke - 1)), coff);
             put(k + 1, cur);
             if (e_on) {
                 const Raw<S> ecur = enxt;
-                enxt = load_raw<STAGE, S, G>(a, zplane(min(k + 2, ke - 1)), eoff);
+                enxt = load_raw<STAGE, S, V>(a, zplane(min(k + 2, ke - 1)), eoff);
                 edge_prims(k + 1, ecur);
                 edge_states(k + 1);  // B
             }
@@ -476,10 +501,9 @@ __device__ __forceinline__ void tile_edge(const StageArgs &a, TileLds<S, TY> &L,
 }
 
 // One stage over the tile (bx, by) of 64 x TY outputs and the z planes of chunk bz.
-// G: with gravity (StageArgs::gf, FP64).  W: some side is a wall (read only
-// with gmap).
-template <int STAGE, typename S, int TY, bool G, bool W>
-__device__ __forceinline__ void tile_stage(const StageArgs &a, TileLds<S, TY> &L, unsigned bx, unsigned by,
+// V: StageKind.  W: some side is a wall (read only with gmap).
+template <int STAGE, typename S, int TY, int V, bool W>
+__device__ __forceinline__ void tile_stage(const StageArgs &a, TileLds<S, TY, V> &L, unsigned bx, unsigned by,
                                            unsigned bz)
 {
     TileGeom g;
@@ -503,10 +527,10 @@ __device__ __forceinline__ void tile_stage(const StageArgs &a, TileLds<S, TY> &L
         // win the issue arbitration by age: the owners issue first
         // (2.06 -> 2.00 ms per step at 256^3).
         __builtin_amdgcn_s_setprio(1);
-        tile_owner<STAGE, S, TY, G, W>(a, L, g, flg, rmax);
+        tile_owner<STAGE, S, TY, V, W>(a, L, g, flg, rmax);
     }
-    else if (g.r == TY + 1) tile_edge<STAGE, S, TY, G, W>(a, L, g, flg);
-    else tile_halo<STAGE, S, TY, G, W>(a, L, g, flg);
+    else if (g.r == TY + 1) tile_edge<STAGE, S, TY, V, W>(a, L, g, flg);
+    else tile_halo<STAGE, S, TY, V, W>(a, L, g, flg);
     if (flg) atomicOr(a.flags, flg);
     if (STAGE == 2) wave_max_to(rmax, a.rate);
 }
