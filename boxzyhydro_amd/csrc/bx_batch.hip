@@ -86,8 +86,8 @@ struct BatchArgs {
     int nqueue;                     // tubes in the queue (order[0..nqueue))
     int ngang, gang_p;              // gangs and members per gang (gang_p > 1: gangs on)
     const int *gang_tube;           // the tube of each gang
-    unsigned *gang_ctr;             // ngang arrival counters
-    unsigned long long *gang_rate;  // 3 per gang
+    unsigned long long *gang_slot;  // kGangSlots per gang
+    double *gang_exch;              // gang_p x kExchMember per gang
     unsigned *gang_fail;
 };
 
@@ -126,15 +126,12 @@ __device__ __forceinline__ double eos_state(const Tube &t, double rho, double &E
     return eps * t.gm1;
 }
 
-// velocity.f90:18-53 on one cell: u = m/rho, then the vlimit clamp
-__device__ __forceinline__ void velocity_of(const Tube &t, double U[5], double v[3], unsigned &flg)
+// velocity.f90:33-53: the vlimit clamp of a cell with u = m/rho in v
+__device__ __forceinline__ void clamp_velocity(const Tube &t, double U[5], double v[3], unsigned &flg)
 {
-    const double rho = U[0];
-    v[0] = qdiv(U[1], rho);
-    v[1] = qdiv(U[2], rho);
-    v[2] = qdiv(U[3], rho);
     if (fabs(v[0]) > t.vlimit || fabs(v[1]) > t.vlimit || fabs(v[2]) > t.vlimit) {
         flg |= FLAG_CLAMP;
+        const double rho = U[0];
         double ekin = 0.5 * (U[1] * U[1] + U[2] * U[2] + U[3] * U[3]) / rho;
         double speed = 0.0;
         for (int d = 0; d < 3; d++) speed = speed + v[d] * v[d];
@@ -149,11 +146,24 @@ __device__ __forceinline__ void velocity_of(const Tube &t, double U[5], double v
     }
 }
 
-// source(): the energy re-round with the gravity vector -0 (source.f90:161-182)
-__device__ __forceinline__ double source_E(const Tube &t, const double U[5])
+// velocity.f90:18-53 on one cell: u = m/rho, then the clamp
+__device__ __forceinline__ void velocity_of(const Tube &t, double U[5], double v[3], unsigned &flg)
 {
-    const double ek = 0.5 * (U[1] * U[1] + U[2] * U[2] + U[3] * U[3]) / U[0];
-    return floor_at(U[4] - ek, t.seps) + ek;
+    div_shared<3>(U + 1, U[0], v);
+    clamp_velocity(t, U, v, flg);
+}
+
+// u = m/rho and the kinetic energy |m|^2/(2 rho) of a cell: four quotients by
+// rho with one reciprocal (velocity and source take the same rho and m)
+__device__ __forceinline__ double velocity_and_ekin(const double U[5], double v[3])
+{
+    const double num[4] = {U[1], U[2], U[3], 0.5 * (U[1] * U[1] + U[2] * U[2] + U[3] * U[3])};
+    double quo[4];
+    div_shared<4>(num, U[0], quo);
+    v[0] = quo[0];
+    v[1] = quo[1];
+    v[2] = quo[2];
+    return quo[3];
 }
 
 // courant.f90:20-21 for one cell
@@ -162,19 +172,25 @@ __device__ __forceinline__ double rate_of(const Tube &t, double rho, double p, d
     const double sq = t.gam * p / rho;
     double sound;
     sqrt_n<1>(&sq, &sound);
-    const double r0 = (sound + fabs(u0)) / t.dx;
-    const double r1 = (sound + fabs(u1)) / t.dy;
-    // the same operands give the same quotient: the z term of a cube cell with |u1|==|u2|
-    const double r2 = (t.dz == t.dy && fabs(u2) == fabs(u1)) ? r1 : (sound + fabs(u2)) / t.dz;
-    return r0 + r1 + r2;
+    const double num[3] = {sound + fabs(u0), sound + fabs(u1), sound + fabs(u2)};
+    if (t.dx == t.dy && t.dy == t.dz) {
+        double r[3];
+        div_shared<3>(num, t.dx, r);
+        return r[0] + r[1] + r[2];
+    }
+    return num[0] / t.dx + num[1] / t.dy + num[2] / t.dz;
 }
 
-// fluxtmp of one component of a row cell (flux.f90:187-191): y and z terms are +0
-__device__ __forceinline__ double flux_tmp(const Tube &t, double dFx, double dt)
+// fluxtmp of a row cell (flux.f90:187-191): y and z terms are +0
+__device__ __forceinline__ void flux_tmp(const Tube &t, const double dFx[5], double dt, double ft[5])
 {
-    const double s = (t.ayz * dFx + 0.0) + 0.0;
-    const double q = s * dt;
-    return -(t.vol_pow2 ? q * t.inv_vol : qdiv(q, t.vol));
+    double q[5];
+    for (int k = 0; k < 5; k++) q[k] = ((t.ayz * dFx[k] + 0.0) + 0.0) * dt;
+    if (t.vol_pow2)
+        for (int k = 0; k < 5; k++) ft[k] = q[k] * t.inv_vol;
+    else
+        div_shared<5>(q, t.vol, ft);
+    for (int k = 0; k < 5; k++) ft[k] = -ft[k];
 }
 
 __device__ __forceinline__ double block_max(double v, double *red, int nw)
@@ -206,7 +222,7 @@ __device__ __forceinline__ void x_faces(const StageArgs &sa, const W6<double> &q
     L.p = lane_below(pl.p);
     L.e = lane_below(pl.e);
     L.g = sa.gam;
-    face_flux<double, 0, true>(L, mi, Fx);
+    face_flux<double, 0>(L, mi, Fx);
 }
 
 // ------------------------------------------------------------------ gangs
@@ -214,24 +230,36 @@ __device__ __forceinline__ void x_faces(const StageArgs &sa, const W6<double> &q
 // taking a contiguous range of its segments.  The predictor of a member also
 // covers the two cells past each shared edge (the neighbour computes them too,
 // with the same operations on the same values), so only the end-of-step state
-// of the four cells on either side of an edge crosses between members: those
-// are written and read with device-coherent (agent-scope) accesses, and the
-// members meet at one barrier on a device counter per step, after the
-// corrector, with the Courant maximum.  Every other cell stays with its
-// member.  The arithmetic per cell is the single-workgroup form's, and the
-// maximum is exact, so a gang gives the same bits.  A barrier that waits
-// longer than kGangSpins sleeps (members not resident together) marks the
-// batch failed and the member leaves the tube; the host then runs the batch
-// again without gangs.
-constexpr unsigned kGangSpins = 1u << 24;
+// of the four cells on either side of an edge crosses between members.  Those
+// go through an exchange buffer with device-coherent (agent-scope) accesses,
+// one half for even steps and one for odd ones: a member may be in the
+// corrector of a step, writing its edge cells, while its neighbour still
+// reads the last step's in the predictor.  Every cell of the rows is read and
+// written by its own member only.  The members meet once per step, after the
+// corrector, where each publishes its Courant maximum: a member writes its own
+// slot and one wave polls all P of them, one lane each, so that meeting and
+// maximum are one store and one load apart (a counter, an atomic maximum and
+// its reading were four round trips to memory).  Three rows of slots rotate;
+// a member empties its slot of the row after next once it has passed a
+// meeting, when everyone has read it.  The arithmetic per cell is the
+// single-workgroup form's, and the maximum is exact, so a gang gives the same
+// bits.  A wait longer than kGangSpins polls (members not resident together)
+// marks the batch failed and the member leaves the tube; the host then runs
+// the batch again without gangs.
+constexpr unsigned kGangSpins = 1u << 23;
+constexpr int kGangMax = 64;                            // members of a gang, at most (one wave polls)
+constexpr unsigned long long kGangEmpty = ~0ull;        // a slot not yet written: no maximum has these bits
+constexpr int kGangSlots = 3 * kGangMax;                // per gang
+constexpr int kExchCells = 4, kExchSide = 9 * kExchCells;  // 9 planes of the 4 cells at one edge
+// exchange buffer of a member: [step parity][side][plane][cell]
+constexpr int kExchMember = 2 * 2 * kExchSide;
 
 struct GangCtx {
-    unsigned *ctr;             // arrivals, monotonic within a run
-    unsigned long long *rate;  // three rotating slots for the Courant maximum (bits of a double >= 0)
+    unsigned long long *slot;  // 3 rows of kGangMax: a member's Courant maximum (bits of a double >= 0)
+    double *exch;              // the gang's exchange buffers
     unsigned *fail;
     int member, p;
-    unsigned epoch;            // barriers passed (the same in every thread)
-    int exch;                  // maxima exchanged
+    unsigned epoch;            // meetings so far (the same in every thread)
 };
 
 __device__ __forceinline__ double load_c(const double *p)
@@ -244,94 +272,393 @@ __device__ __forceinline__ void store_c(double *p, double v)
     __hip_atomic_store((long long *)p, __double_as_longlong(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// false: the wait gave up
-__device__ __forceinline__ bool gang_barrier(GangCtx &g, int *s_ok)
+// The gang's meeting: r becomes the maximum of each member's r (every thread
+// holds its member's), and what the members stored before is visible to all.
+// false: the wait gave up.
+__device__ __forceinline__ bool gang_max(GangCtx &g, double &r, int *s_ok, double *s_r)
 {
-    __builtin_amdgcn_s_waitcnt(0);  // this wave's stores and atomics are complete
+    __builtin_amdgcn_s_waitcnt(0);  // this wave's stores are complete
     __syncthreads();
-    g.epoch++;
-    if (threadIdx.x == 0) {
-        __hip_atomic_fetch_add(g.ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const unsigned target = g.epoch * (unsigned)g.p;
+    if (threadIdx.x < 64) {
+        const int lane = threadIdx.x;
+        unsigned long long *row = g.slot + (g.epoch % 3) * kGangMax;
+        if (lane == 0)
+            __hip_atomic_store(&row[g.member], (unsigned long long)__double_as_longlong(r), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+        unsigned long long v = 0ull;
         unsigned spins = 0;
         int ok = 1;
-        while (__hip_atomic_load(g.ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target) {
-            __builtin_amdgcn_s_sleep(4);
+        for (;;) {
+            if (lane < g.p) v = __hip_atomic_load(&row[lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (!__any(v == kGangEmpty)) break;
             if (++spins > kGangSpins) {
                 ok = 0;
-                __hip_atomic_fetch_or(g.fail, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 break;
             }
+            __builtin_amdgcn_s_sleep(1);
         }
-        *s_ok = ok;
+        for (int off = 32; off > 0; off >>= 1) {
+            const unsigned long long o = __shfl_xor(v, off, 64);
+            v = o > v ? o : v;
+        }
+        if (lane == 0) {
+            if (!ok) __hip_atomic_fetch_or(g.fail, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(&g.slot[((g.epoch + 2) % 3) * kGangMax + g.member], kGangEmpty, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+            *s_r = __longlong_as_double((long long)v);
+            *s_ok = ok;
+        }
     }
+    g.epoch++;
     __syncthreads();
+    r = *s_r;
     return *s_ok != 0;
 }
 
-// the gang's maximum of each member's r (every thread holds its member's r)
-__device__ __forceinline__ bool gang_max(GangCtx &g, double &r, int *s_ok, double *s_r)
+// The range of segments and cells a workgroup takes of a tube.
+struct Range {
+    int nseg, s0, s1;      // segments [s0, s1) of nseg
+    int c_lo, c_hi;        // output cells [c_lo, c_hi)
+    bool left, right;      // whether another member holds the segment before / after
+};
+
+template <bool GANG>
+__device__ __forceinline__ Range tube_range(int nx, const GangCtx &g)
 {
-    const int slot = g.exch % 3;
-    if (threadIdx.x == 0)
-        __hip_atomic_fetch_max(&g.rate[slot], (unsigned long long)__double_as_longlong(r), __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
-    if (!gang_barrier(g, s_ok)) return false;
-    if (threadIdx.x == 0) {
-        *s_r = __longlong_as_double(
-            (long long)__hip_atomic_load(&g.rate[slot], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-        // the slot two exchanges on: every member read it before two barriers ago
-        if (g.member == 0)
-            __hip_atomic_store(&g.rate[(slot + 1) % 3], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    Range r;
+    r.nseg = (nx - 4 + kSegOut - 1) / kSegOut;
+    r.s0 = 0;
+    r.s1 = r.nseg;
+    r.c_lo = 0;
+    r.c_hi = nx;
+    if (GANG) {
+        const int per = (r.nseg + g.p - 1) / g.p;
+        r.s0 = min(r.nseg, g.member * per);
+        r.s1 = min(r.nseg, r.s0 + per);
+        r.c_lo = g.member == 0 ? 0 : r.s0 * kSegOut + 2;
+        r.c_hi = g.member == g.p - 1 ? nx : r.s1 * kSegOut + 2;
     }
+    const bool any = r.s0 < r.s1;  // a short tube leaves the last members without segments
+    r.left = GANG && any && g.member > 0;
+    r.right = GANG && any && g.member < g.p - 1;
+    return r;
+}
+
+// Courant maximum of the set-up (main.f90:232-241) over cells [c_lo, c_hi):
+// every row cell with its own values, and the frame tuple at every c
+template <int W>
+__device__ __forceinline__ double setup_rate(const BatchArgs &a, const Tube &t, const Range &r)
+{
+    const int64_t T = a.total;
+    const double *icr = a.ic + t.off;
+    double r0 = 0.0;
+    for (int c = r.c_lo + (int)threadIdx.x; c < r.c_hi; c += 64 * W) {
+        const double u0 = PL(icr + 5 * T, c), u1 = PL(icr + 6 * T, c), u2 = PL(icr + 7 * T, c), pi = PL(icr + 8 * T, c);
+        unsigned fset = 0;
+        if (c > 0 && c < t.nx - 1) {
+            const double rho = PL(icr, c);
+            double E = PL(icr + 4 * T, c);
+            const double p = eos_state(t, rho, E, u0, u1, u2, pi, fset);
+            r0 = vmax(r0, rate_of(t, rho, p, u0, u1, u2));
+        }
+        double Ef = t.seps;
+        const double pf = eos_state(t, t.srho, Ef, u0, u1, u2, pi, fset);
+        r0 = vmax(r0, rate_of(t, t.srho, pf, u0, u1, u2));
+    }
+    return r0;
+}
+
+// main.f90:266-281 for step `step` (counted from 1)
+__device__ __forceinline__ double tube_dt(const Tube &t, double rate, double time, int step, double &dtold)
+{
+    double dt = t.cfl / rate;
+    dt = dt * 1.0;
+    if (step > 1 && dtold > 0.0) dt = vmin(dt, dtold * 1.1);
+    dtold = dt;
+    if (dt + time > t.endtime) dt = t.endtime - time;
+    dt = dt * 0.5;
+    return dt * 2.0;
+}
+
+// What the step keeps of a cell: rho, mx, my, mz, E, u0, u1, u2, p.
+struct Cell {
+    double U[5], v[3], p;
+};
+
+// main.f90:232-318 at a cell (state, source(0), state, velocity) from the
+// end-of-step state x; U, v, p are then cons_old, the velocity and the pressure
+// of the predictor's flux
+__device__ __forceinline__ void predictor_state(const Tube &t, Cell &x, unsigned &pf)
+{
+    double v[3];
+    const double ek = velocity_and_ekin(x.U, v);                                        // of :289 and :318
+    const double p232 = eos_state(t, x.U[0], x.U[4], x.v[0], x.v[1], x.v[2], x.p, pf);  // :232
+    x.U[4] = floor_at(x.U[4] - ek, t.seps) + ek;                                        // :289 (source.f90:161-182)
+    x.p = eos_state(t, x.U[0], x.U[4], x.v[0], x.v[1], x.v[2], p232, pf);               // :314
+    for (int k = 0; k < 3; k++) x.v[k] = v[k];
+    clamp_velocity(t, x.U, x.v, pf);                                                    // :318
+}
+
+// x-flux differences of every lane's cell
+__device__ __forceinline__ void cell_fluxes(const Tube &t, const StageArgs &sa, const Cell &x, bool ghost, double dF[5])
+{
+    W6<double> q;
+    q.d = x.U[0];
+    q.u0 = x.v[0];
+    q.u1 = x.v[1];
+    q.u2 = x.v[2];
+    q.p = x.p;
+    q.e = floor_at(x.U[4] - 0.5 * q.d * (q.u0 * q.u0 + q.u1 * q.u1 + q.u2 * q.u2), t.seps);
+    q.g = 0.0;
+    double Fx[5];
+    x_faces(sa, q, sound_of(q, t.gam), ghost, Fx);
+    for (int k = 0; k < 5; k++) dF[k] = lane_above(Fx[k]) - Fx[k];
+}
+
+// main.f90:346-355: the predictor's update, state and velocity
+__device__ __forceinline__ Cell predictor_update(const Tube &t, const Cell &x, const double dF[5], double dt,
+                                                 unsigned &flg)
+{
+    Cell y;
+    double ft[5];
+    flux_tmp(t, dF, dt, ft);
+    for (int k = 0; k < 5; k++) y.U[k] = x.U[k] + ft[k];                   // flux.f90:205
+    y.U[0] = floor_at(y.U[0], t.srho);                                     // flux.f90:225-228
+    if (y.U[4] < 0.0) y.U[4] = 0.5 * (y.U[1] * y.U[1] + y.U[2] * y.U[2] + y.U[3] * y.U[3]) / y.U[0] + t.seps;
+    y.p = eos_state(t, y.U[0], y.U[4], x.v[0], x.v[1], x.v[2], x.p, flg);  // :353
+    velocity_of(t, y.U, y.v, flg);                                         // :355
+    return y;
+}
+
+// main.f90:368-515: the corrector's update from cons_old and the predictor's
+// result y, state, velocity, source(1), state, velocity; and the next step's
+// state (:232) and Courant rate (:241)
+__device__ __forceinline__ Cell corrector_update(const Tube &t, const double old[5], const Cell &y, const double dF[5],
+                                                 double dt, unsigned &flg, double &rn)
+{
+    Cell x;
+    double ft[5];
+    flux_tmp(t, dF, dt, ft);
+    for (int k = 0; k < 5; k++) x.U[k] = 0.5 * (old[k] + y.U[k] + ft[k]);  // flux.f90:213
+    x.U[0] = floor_at(x.U[0], t.srho);
+    if (x.U[4] < 0.0) x.U[4] = 0.5 * (x.U[1] * x.U[1] + x.U[2] * x.U[2] + x.U[3] * x.U[3]) / x.U[0] + t.seps;
+    double v[3];
+    double ek = velocity_and_ekin(x.U, v);
+    const double p376 = eos_state(t, x.U[0], x.U[4], y.v[0], y.v[1], y.v[2], y.p, flg);  // :376
+    unsigned cf = 0;
+    clamp_velocity(t, x.U, v, cf);                                                      // :378
+    if (cf) {  // the clamp changed m
+        flg |= cf;
+        double vn[3];
+        ek = velocity_and_ekin(x.U, vn);
+    }
+    x.U[4] = floor_at(x.U[4] - ek, t.seps) + ek;                                        // :490 (source.f90:161-182)
+    x.p = eos_state(t, x.U[0], x.U[4], v[0], v[1], v[2], p376, flg);                    // :513
+    if (cf) {
+        velocity_of(t, x.U, x.v, flg);                                                  // :515
+    } else {  // rho and m are those of :378
+        for (int k = 0; k < 3; k++) x.v[k] = v[k];
+    }
+    double E2 = x.U[4];
+    unsigned fn = 0;
+    const double p2 = eos_state(t, x.U[0], E2, x.v[0], x.v[1], x.v[2], x.p, fn);
+    rn = vmax(rn, rate_of(t, x.U[0], p2, x.v[0], x.v[1], x.v[2]));
+    return x;
+}
+
+__device__ __forceinline__ double &cell_value(Cell &x, int k) { return k < 5 ? x.U[k] : (k < 8 ? x.v[k - 5] : x.p); }
+
+// broadcast of lane l's value
+__device__ __forceinline__ double lane_bcast(double v, int l)
+{
+    const long long b = __double_as_longlong(v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, l);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b >> 32), l);
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// One tube (or a gang member's range of it) whose segments are no more than the
+// workgroup's waves: each wave keeps one segment in registers from the set-up
+// to endtime.  Only the two cells at either end of a segment go through LDS,
+// once after the predictor (Y) and once after the corrector (X); the rows in
+// memory are read once and written once.  A step on few segments is a chain of
+// latencies, and the rows cost it three round trips to L2: a gang member of
+// three segments took 10.4 us per step through the rows.
+template <int W, bool GANG>
+__device__ __forceinline__ void run_tube_regs(const BatchArgs &a, const Tube &t, int ti, GangCtx &g, const Range &r,
+                                              double *red, int *s_ok, double *s_r, unsigned *sflag,
+                                              double (*X)[9][4], double (*Y)[9][4])
+{
+    const int lane = threadIdx.x & 63, wv = wave_id();
+    const int64_t T = a.total;
+    const int nx = t.nx;
+    const int sp0 = r.s0 - (r.left ? 1 : 0), sp1 = r.s1 + (r.right ? 1 : 0);
+    const int s = sp0 + wv;
+    const bool work = s < sp1;                    // this wave has a segment in the predictor
+    const bool mine = s >= r.s0 && s < r.s1;      // and in the corrector
+    const int c = s * kSegOut + lane;             // lane 2 is the segment's first output
+    const int d = donor_of(min(c, nx - 1), nx);
+    const bool ghost = c < 2 || c > nx - 3;
+    const bool out = lane >= 2 && lane < 62 && !ghost;
+    // where a lane's cell comes from: its own lane, the lane of the wave that
+    // holds the last interior cell (ghosts), another wave's edge cells, or
+    // another member's
+    const int dseg = (d - 2) / kSegOut;
+    const bool here = dseg == s;
+    const int own_last = nx - 3 - s * kSegOut;    // that lane, if the segment holds the cell
+    const bool foreign = GANG && (d < r.c_lo || d >= r.c_hi);
+    const int eseg = min(max(dseg - sp0, 0), W - 1);
+    const int el = d - dseg * kSegOut, ej = el < 4 ? (el - 2) & 1 : 2 + (el & 1);  // lanes 2, 3, 60, 61 -> 0..3
+    const double *icr = a.ic + t.off;
+    double *str = a.st + t.off;
+
+    StageArgs sa{};
+    sa.ds[0] = t.dx;
+    sa.inv_ds[0] = t.inv_dx;
+    sa.ds_pow2[0] = t.dx_pow2;
+    sa.gam = t.gam;
+    unsigned flg = 0;
+
+    double rate = uniform_d(block_max(setup_rate<W>(a, t, r), red, W));
+    if (GANG && !gang_max(g, rate, s_ok, s_r)) return;
+
+    // the value of a lane's cell: q where the wave holds it, else E (edge cells in LDS)
+    auto gather = [&](Cell &q, double (*E)[9][4]) {
+        const bool edge = !here;
+        const bool last = own_last >= 2 && own_last < 62;  // uniform: the segment ends the tube
+        for (int k = 0; k < 9; k++) {
+            double v = cell_value(q, k);
+            if (s == 0) {
+                const double b = lane_bcast(v, 2);
+                v = lane < 2 ? b : v;
+            }
+            if (last) {
+                const double b = lane_bcast(v, own_last);
+                v = lane > own_last ? b : v;
+            }
+            if (edge) v = E[eseg][k][ej];
+            cell_value(q, k) = v;
+        }
+    };
+    auto put_edges = [&](Cell &q, double (*E)[9][4]) {
+        if (lane == 2 || lane == 3 || lane == 60 || lane == 61)
+            for (int k = 0; k < 9; k++) E[wv][k][lane < 4 ? lane - 2 : lane - 58] = cell_value(q, k);
+    };
+
+    Cell x{};  // end-of-step state
+    double time = 0.0, dtold = 0.0;
+    int step = 0;
+    unsigned status = 0;
+    for (;;) {
+        if (time >= t.endtime || step >= t.maxsteps) break;  // main.f90:212
+        step++;
+        const double dt = tube_dt(t, rate, time, step, dtold);
+        if (!(dt > 0.0) || !__builtin_isfinite(dt)) {
+            status |= FLAG_BADDT;
+            step--;
+            break;
+        }
+        if (a.dtlog && threadIdx.x == 0 && (!GANG || g.member == 0) && step <= a.maxlog)
+            a.dtlog[(int64_t)ti * a.maxlog + step - 1] = dt;
+        sa.dt = dt;
+
+        // ---------------- predictor: main.f90:232-355
+        Cell y{};
+        double old[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+        if (work) {
+            if (step == 1) {
+                for (int k = 0; k < 9; k++) cell_value(x, k) = PL(icr + k * T, d);
+            } else {
+                gather(x, X);
+                if (foreign) {  // the last step's half of the other member's exchange buffer
+                    const bool lo = d < r.c_lo;
+                    const int j = lo ? max(kExchCells - (r.c_lo - d), 0) : min(d - r.c_hi, kExchCells - 1);
+                    const double *xp = g.exch + (g.member + (lo ? -1 : 1)) * kExchMember +
+                                       ((step - 1) & 1) * 2 * kExchSide + (lo ? 1 : 0) * kExchSide + j;
+                    for (int k = 0; k < 9; k++) cell_value(x, k) = load_c(xp + k * kExchCells);
+                }
+            }
+            // of the segments past an edge only the cells the kept outputs read count
+            const bool count = mine || (c >= r.c_lo - 4 && c < r.c_hi + 4);
+            unsigned pf = 0;
+            predictor_state(t, x, pf);
+            if (count) flg |= pf;
+            double dF[5];
+            cell_fluxes(t, sa, x, ghost, dF);
+            for (int k = 0; k < 5; k++) old[k] = x.U[k];  // cons_old, main.f90:327-333
+            unsigned uf = 0;
+            y = predictor_update(t, x, dF, dt, uf);
+            if (out && (mine || (c >= r.c_lo - 2 && c < r.c_hi + 2))) flg |= uf;
+            put_edges(y, Y);
+        }
+        __syncthreads();
+
+        // ---------------- corrector: main.f90:368-515, then :232-241 of the next step
+        double rn = 0.0;
+        if (mine) {
+            gather(y, Y);
+            double dF[5];
+            cell_fluxes(t, sa, y, ghost, dF);
+            double rc = 0.0;
+            unsigned uf = 0;
+            x = corrector_update(t, old, y, dF, dt, uf, rc);
+            if (out) {
+                flg |= uf;
+                rn = rc;
+                if (GANG) {
+                    auto publish = [&](int side, int j) {
+                        double *e = g.exch + g.member * kExchMember + (step & 1) * 2 * kExchSide + side * kExchSide + j;
+                        for (int k = 0; k < 9; k++) store_c(e + k * kExchCells, cell_value(x, k));
+                    };
+                    if (r.left && c < r.c_lo + kExchCells) publish(0, c - r.c_lo);
+                    if (r.right && c >= r.c_hi - kExchCells) publish(1, c - (r.c_hi - kExchCells));
+                }
+            }
+            put_edges(x, X);
+        }
+        rate = uniform_d(block_max(rn, red, W));  // its barriers also order this phase's stores before the next
+        if (GANG && !gang_max(g, rate, s_ok, s_r)) return;
+        time = time + dt;  // main.f90:545
+    }
+    if (step == 0) {  // no step taken: the state is the set-up
+        for (int q = r.c_lo + (int)threadIdx.x; q < r.c_hi; q += 64 * W)
+            for (int k = 0; k < 9; k++) PL(str + k * T, q) = PL(icr + k * T, q);
+    } else if (mine && out) {
+        for (int k = 0; k < 9; k++) PL(str + k * T, c) = cell_value(x, k);
+    }
+    if (flg) atomicOr(sflag, flg);
     __syncthreads();
-    r = *s_r;
-    g.exch++;
-    return true;
+    if (threadIdx.x == 0) {
+        if (!GANG || g.member == 0) {
+            a.t_out[ti] = time;
+            a.steps_out[ti] = step;
+        }
+        atomicOr(&a.status[ti], *sflag | status);
+    }
 }
 
 // One tube ti; GANG: this workgroup is member g.member of g.p, else the whole
 // tube.  Every thread of the workgroup calls it.
 template <int W, bool GANG>
 __device__ __forceinline__ void run_tube(const BatchArgs &a, const Tube &t, int ti, GangCtx &g, double *red, int *s_ok,
-                         double *s_r, unsigned *sflag, double (*ext)[9][2])
+                         double *s_r, unsigned *sflag, double (*ext)[9][2], double (*X)[9][4], double (*Y)[9][4])
 {
+    const Range r = tube_range<GANG>(t.nx, g);
+    const int sp0 = r.s0 - (r.left ? 1 : 0), sp1 = r.s1 + (r.right ? 1 : 0);
+    if (sp1 - sp0 <= W) {  // a wave per segment: the tube stays in registers
+        run_tube_regs<W, GANG>(a, t, ti, g, r, red, s_ok, s_r, sflag, X, Y);
+        return;
+    }
     const int lane = threadIdx.x & 63, wv = wave_id();  // wave-uniform for the compiler
     const int64_t T = a.total;
     const int nx = t.nx;
-    const int nseg = (nx - 4 + kSegOut - 1) / kSegOut;
-    // segments [s0, s1) and output cells [c_lo, c_hi) of this workgroup
-    int s0 = 0, s1 = nseg, c_lo = 0, c_hi = nx;
-    if (GANG) {
-        const int per = (nseg + g.p - 1) / g.p;
-        s0 = min(nseg, g.member * per);
-        s1 = min(nseg, s0 + per);
-        c_lo = g.member == 0 ? 0 : s0 * kSegOut + 2;
-        c_hi = g.member == g.p - 1 ? nx : s1 * kSegOut + 2;
-    }
+    const int s0 = r.s0, s1 = r.s1, c_lo = r.c_lo, c_hi = r.c_hi;
+    const bool left = r.left, right = r.right;
     // The predictor also takes the two cells beyond each shared edge of the
     // range (the segment before and after, results kept to [w_lo, w_hi)), so
-    // that the corrector needs no other member's predictor results: the
-    // members meet once per step, and exchange the four end-of-step cells on
-    // either side of each shared edge that those extra cells read.  The extra
-    // cells' predictor results stay in LDS (ext[side][plane][cell]): the
-    // neighbour writes the same cells' results to the rows, and two workgroups
-    // writing one line through different caches could leave either's older
-    // bytes in memory.
-    const bool left = GANG && g.member > 0, right = GANG && g.member < g.p - 1;
-    const int sp0 = s0 - (left ? 1 : 0), sp1 = s1 + (right ? 1 : 0);
+    // that the corrector needs no other member's predictor results.  The extra
+    // cells' predictor results stay in LDS (ext[side][plane][cell]).
     const int w_lo = c_lo - (left ? 2 : 0), w_hi = c_hi + (right ? 2 : 0);
-    // a cell another member writes, or one of ours another member reads
-    auto foreign = [&](int c) { return GANG && (c < c_lo || c >= c_hi); };
-    auto shared_out = [&](int c) { return (left && c < c_lo + 4) || (right && c >= c_hi - 4); };
-    auto ld = [&](const double *base, int c) -> double {
-        if (GANG && (foreign(c) || shared_out(c))) return load_c(&PL(base, c));
-        return PL(base, c);
-    };
-    auto st = [&](double *base, int c, double v) {
-        if (GANG && shared_out(c)) store_c(&PL(base, c), v);
-        else PL(base, c) = v;
-    };
     const double *icr = a.ic + t.off;
     double *str = a.st + t.off;
     double *ssr = a.ss + t.off;
@@ -344,23 +671,7 @@ __device__ __forceinline__ void run_tube(const BatchArgs &a, const Tube &t, int 
     sa.gam = t.gam;
     unsigned flg = 0;
 
-    // Courant maximum of the set-up (main.f90:232-241): every row cell
-    // with its own values, and the frame tuple at every c
-    double r0 = 0.0;
-    for (int c = c_lo + (int)threadIdx.x; c < c_hi; c += 64 * W) {
-        const double u0 = PL(icr + 5 * T, c), u1 = PL(icr + 6 * T, c), u2 = PL(icr + 7 * T, c), pi = PL(icr + 8 * T, c);
-        unsigned fset = 0;
-        if (c > 0 && c < nx - 1) {
-            const double rho = PL(icr, c);
-            double E = PL(icr + 4 * T, c);
-            const double p = eos_state(t, rho, E, u0, u1, u2, pi, fset);
-            r0 = vmax(r0, rate_of(t, rho, p, u0, u1, u2));
-        }
-        double Ef = t.seps;
-        const double pf = eos_state(t, t.srho, Ef, u0, u1, u2, pi, fset);
-        r0 = vmax(r0, rate_of(t, t.srho, pf, u0, u1, u2));
-    }
-    double rate = uniform_d(block_max(r0, red, W));
+    double rate = uniform_d(block_max(setup_rate<W>(a, t, r), red, W));
     if (GANG && !gang_max(g, rate, s_ok, s_r)) return;
 
     double time = 0.0, dtold = 0.0;
@@ -369,14 +680,7 @@ __device__ __forceinline__ void run_tube(const BatchArgs &a, const Tube &t, int 
     for (;;) {
         if (time >= t.endtime || step >= t.maxsteps) break;  // main.f90:212
         step++;
-        // main.f90:266-281; every thread forms the same dt
-        double dt = t.cfl / rate;
-        dt = dt * 1.0;
-        if (step > 1 && dtold > 0.0) dt = vmin(dt, dtold * 1.1);
-        dtold = dt;
-        if (dt + time > t.endtime) dt = t.endtime - time;
-        dt = dt * 0.5;
-        dt = dt * 2.0;
+        const double dt = tube_dt(t, rate, time, step, dtold);  // every thread forms the same
         if (!(dt > 0.0) || !__builtin_isfinite(dt)) {
             status |= FLAG_BADDT;
             step--;
@@ -392,51 +696,38 @@ __device__ __forceinline__ void run_tube(const BatchArgs &a, const Tube &t, int 
             const int c = s * kSegOut + lane;  // lane 2 is the segment's first output
             const int d = donor_of(min(c, nx - 1), nx);
             const bool ghost = c < 2 || c > nx - 3;
-            double U[5], v[3];
-            for (int k = 0; k < 5; k++) U[k] = ld(src + k * T, d);
-            const double w0 = ld(src + 5 * T, d), w1 = ld(src + 6 * T, d), w2 = ld(src + 7 * T, d);
-            const double p0 = ld(src + 8 * T, d);
+            // another member's cell: the last step's half of its exchange buffer
+            // (of the cells further off than the four it holds, whose results
+            // are not kept, the nearest)
+            const bool xf = GANG && step > 1 && (d < c_lo || d >= c_hi);
+            const double *xp = nullptr;
+            if (xf) {
+                const bool lo = d < c_lo;
+                const int j = lo ? max(kExchCells - (c_lo - d), 0) : min(d - c_hi, kExchCells - 1);
+                xp = g.exch + (g.member + (lo ? -1 : 1)) * kExchMember + ((step - 1) & 1) * 2 * kExchSide +
+                     (lo ? 1 : 0) * kExchSide + j;
+            }
+            Cell x;
+            for (int k = 0; k < 9; k++) cell_value(x, k) = xf ? load_c(xp + k * kExchCells) : PL(src + k * T, d);
             // in the segments past an edge only the cells the kept outputs read
             // count (the rest may hold an older state)
             const bool count = !GANG || (s >= s0 && s < s1) || (c >= c_lo - 4 && c < c_hi + 4);
             unsigned pf = 0;
-            const double p232 = eos_state(t, U[0], U[4], w0, w1, w2, p0, pf);    // :232
-            U[4] = source_E(t, U);                                               // :289
-            const double p314 = eos_state(t, U[0], U[4], w0, w1, w2, p232, pf);  // :314
-            velocity_of(t, U, v, pf);                                            // :318
+            predictor_state(t, x, pf);
             if (count) flg |= pf;
-            W6<double> q;
-            q.d = U[0];
-            q.u0 = v[0];
-            q.u1 = v[1];
-            q.u2 = v[2];
-            q.p = p314;
-            q.e = floor_at(U[4] - 0.5 * U[0] * (v[0] * v[0] + v[1] * v[1] + v[2] * v[2]), t.seps);
-            double Fx[5];
-            x_faces(sa, q, sound_of(q, t.gam), ghost, Fx);
             double dF[5];
-            for (int k = 0; k < 5; k++) dF[k] = lane_above(Fx[k]) - Fx[k];
+            cell_fluxes(t, sa, x, ghost, dF);
             __asm__ volatile("" ::: "memory");  // keep the update's loads after the faces (register pressure)
             if (lane >= 2 && lane < 62 && !ghost && c >= w_lo && c < w_hi) {
-                double Us[5], us[3];
                 const bool mine = !GANG || (c >= c_lo && c < c_hi);
-                for (int k = 0; k < 5; k++) {
-                    if (mine) PL(oldr + k * T, c) = U[k];         // cons_old, main.f90:327-333
-                    Us[k] = U[k] + flux_tmp(t, dF[k], dt);      // flux.f90:205
-                }
-                Us[0] = floor_at(Us[0], t.srho);                // flux.f90:225-228
-                if (Us[4] < 0.0) Us[4] = 0.5 * (Us[1] * Us[1] + Us[2] * Us[2] + Us[3] * Us[3]) / Us[0] + t.seps;
-                const double ps = eos_state(t, Us[0], Us[4], v[0], v[1], v[2], p314, flg);  // :353
-                velocity_of(t, Us, us, flg);                                             // :355
+                if (mine)
+                    for (int k = 0; k < 5; k++) PL(oldr + k * T, c) = x.U[k];  // cons_old, main.f90:327-333
+                Cell y = predictor_update(t, x, dF, dt, flg);
                 if (mine) {
-                    for (int k = 0; k < 5; k++) PL(ssr + k * T, c) = Us[k];
-                    for (int k = 0; k < 3; k++) PL(ssr + (5 + k) * T, c) = us[k];
-                    PL(ssr + 8 * T, c) = ps;
+                    for (int k = 0; k < 9; k++) PL(ssr + k * T, c) = cell_value(y, k);
                 } else {
                     const int side = c < c_lo ? 0 : 1, j = c < c_lo ? c - w_lo : c - c_hi;
-                    for (int k = 0; k < 5; k++) ext[side][k][j] = Us[k];
-                    for (int k = 0; k < 3; k++) ext[side][5 + k][j] = us[k];
-                    ext[side][8][j] = ps;
+                    for (int k = 0; k < 9; k++) ext[side][k][j] = cell_value(y, k);
                 }
             }
         }
@@ -448,42 +739,30 @@ __device__ __forceinline__ void run_tube(const BatchArgs &a, const Tube &t, int 
             const int c = s * kSegOut + lane;
             const int d = donor_of(min(c, nx - 1), nx);
             const bool ghost = c < 2 || c > nx - 3;
-            W6<double> q;
+            Cell y;
             // the predictor results: the rows, or LDS past a shared edge
             const bool xe = GANG && (d < c_lo || d >= c_hi);
             const int xs = d < c_lo ? 0 : 1, xj = min(max(d < c_lo ? d - w_lo : d - c_hi, 0), 1);
-            auto sv = [&](int k) { return xe ? ext[xs][k][xj] : PL(ssr + k * T, d); };
-            q.d = sv(0);
-            const double E = sv(4);
-            q.u0 = sv(5);
-            q.u1 = sv(6);
-            q.u2 = sv(7);
-            q.p = sv(8);
-            q.e = floor_at(E - 0.5 * q.d * (q.u0 * q.u0 + q.u1 * q.u1 + q.u2 * q.u2), t.seps);
-            double Fx[5];
-            x_faces(sa, q, sound_of(q, t.gam), ghost, Fx);
+            for (int k = 0; k < 9; k++) cell_value(y, k) = xe ? ext[xs][k][xj] : PL(ssr + k * T, d);
             double dF[5];
-            for (int k = 0; k < 5; k++) dF[k] = lane_above(Fx[k]) - Fx[k];
+            cell_fluxes(t, sa, y, ghost, dF);
             __asm__ volatile("" ::: "memory");  // keep the update's loads after the faces (register pressure)
             if (lane >= 2 && lane < 62 && !ghost) {
-                double U[5], v[3], v2[3];
-                for (int k = 0; k < 5; k++)
-                    U[k] = 0.5 * (PL(oldr + k * T, c) + PL(ssr + k * T, c) + flux_tmp(t, dF[k], dt));  // flux.f90:213
-                U[0] = floor_at(U[0], t.srho);
-                if (U[4] < 0.0) U[4] = 0.5 * (U[1] * U[1] + U[2] * U[2] + U[3] * U[3]) / U[0] + t.seps;
-                const double p376 = eos_state(t, U[0], U[4], q.u0, q.u1, q.u2, q.p, flg);    // :376
-                velocity_of(t, U, v, flg);                                                  // :378
-                U[4] = source_E(t, U);                                                      // :490
-                const double p513 = eos_state(t, U[0], U[4], v[0], v[1], v[2], p376, flg);  // :513
-                velocity_of(t, U, v2, flg);                                                 // :515
-                for (int k = 0; k < 5; k++) st(str + k * T, c, U[k]);
-                for (int k = 0; k < 3; k++) st(str + (5 + k) * T, c, v2[k]);
-                st(str + 8 * T, c, p513);
-                // the next step's state (:232) and Courant rate (:241)
-                double E2 = U[4];
-                unsigned fn = 0;
-                const double p2 = eos_state(t, U[0], E2, v2[0], v2[1], v2[2], p513, fn);
-                rn = vmax(rn, rate_of(t, U[0], p2, v2[0], v2[1], v2[2]));
+                double old[5];
+                for (int k = 0; k < 5; k++) {
+                    old[k] = PL(oldr + k * T, c);
+                    y.U[k] = PL(ssr + k * T, c);
+                }
+                Cell x = corrector_update(t, old, y, dF, dt, flg, rn);
+                for (int k = 0; k < 9; k++) PL(str + k * T, c) = cell_value(x, k);
+                if (GANG) {
+                    auto publish = [&](int side, int j) {
+                        double *e = g.exch + g.member * kExchMember + (step & 1) * 2 * kExchSide + side * kExchSide + j;
+                        for (int k = 0; k < 9; k++) store_c(e + k * kExchCells, cell_value(x, k));
+                    };
+                    if (left && c < c_lo + kExchCells) publish(0, c - c_lo);
+                    if (right && c >= c_hi - kExchCells && c < c_hi) publish(1, c - (c_hi - kExchCells));
+                }
             }
         }
         rate = uniform_d(block_max(rn, red, W));  // its barriers also order this phase's stores before the next
@@ -493,7 +772,7 @@ __device__ __forceinline__ void run_tube(const BatchArgs &a, const Tube &t, int 
     if (step == 0) {
         // no step taken: the state is the set-up
         for (int c = c_lo + (int)threadIdx.x; c < c_hi; c += 64 * W)
-            for (int k = 0; k < 9; k++) st(str + k * T, c, PL(icr + k * T, c));
+            for (int k = 0; k < 9; k++) PL(str + k * T, c) = PL(icr + k * T, c);
     }
     if (flg) atomicOr(sflag, flg);
     __syncthreads();
@@ -515,22 +794,22 @@ __global__ __launch_bounds__(64 * W) void k_tubes(BatchArgs a, const Tube *__res
     __shared__ int s_ok;
     __shared__ double s_r;
     __shared__ double ext[2][9][2];
+    __shared__ double X[W][9][4], Y[W][9][4];  // edge cells of each wave's segment
     // the gangs first: workgroups [0, ngang * gang_p), gang blockIdx / gang_p
     if (a.gang_p > 1 && (int)blockIdx.x < a.ngang * a.gang_p) {
         if (threadIdx.x == 0) sflag = 0;
         __syncthreads();
         GangCtx g;
         const int gi = (int)blockIdx.x / a.gang_p;
-        g.ctr = a.gang_ctr + gi;
-        g.rate = a.gang_rate + 3 * gi;
+        g.slot = a.gang_slot + (int64_t)gi * kGangSlots;
+        g.exch = a.gang_exch + (int64_t)gi * a.gang_p * kExchMember;
         g.fail = a.gang_fail;
         g.member = (int)blockIdx.x - gi * a.gang_p;
         g.p = a.gang_p;
         g.epoch = 0;
-        g.exch = 0;
         const int ti = __builtin_amdgcn_readfirstlane(a.gang_tube[gi]);
         const Tube t = tubes[ti];
-        run_tube<W, true>(a, t, ti, g, red, &s_ok, &s_r, &sflag, ext);
+        run_tube<W, true>(a, t, ti, g, red, &s_ok, &s_r, &sflag, ext, X, Y);
     }
     GangCtx none{};
     for (;;) {
@@ -544,22 +823,21 @@ __global__ __launch_bounds__(64 * W) void k_tubes(BatchArgs a, const Tube *__res
         if (qi >= a.nqueue) break;  // the whole workgroup leaves together
         const int ti = __builtin_amdgcn_readfirstlane(order[qi]);
         const Tube t = tubes[ti];
-        run_tube<W, false>(a, t, ti, none, red, &s_ok, &s_r, &sflag, ext);
+        run_tube<W, false>(a, t, ti, none, red, &s_ok, &s_r, &sflag, ext, X, Y);
     }
 }
 
-// Clears the queue counter and the gangs' counters, maxima and failure word
-// (a kernel, not memsets, so that the launch can be captured).
-__global__ void k_tubes_reset(int *queue, int ngang, unsigned *ctr, unsigned long long *rate, unsigned *fail,
-                              unsigned *status, int ntube)
+// Clears the queue counter, the gangs' slots and failure word and the status
+// words (a kernel, not memsets, so that the launch can be captured).
+__global__ void k_tubes_reset(int *queue, int nslot, unsigned long long *slot, unsigned *fail, unsigned *status,
+                              int ntube)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i == 0) {
         *queue = 0;
         if (fail) *fail = 0u;
     }
-    if (i < ngang) ctr[i] = 0u;
-    if (i < 3 * ngang) rate[i] = 0ull;
+    if (i < nslot) slot[i] = kGangEmpty;
     if (i < ntube) status[i] = 0u;
 }
 
@@ -583,13 +861,13 @@ struct bx_batch {
     unsigned *status = nullptr;
     double *dtlog = nullptr;
     int maxlog = 0;
-    int waves = 16, blocks_per_cu = 1, ncu = 0;
+    int waves = 0, blocks_per_cu = 1, ncu = 0;  // waves 0: chosen at the launch (default_waves)
     // gangs: the ngang costliest tubes, gang_p workgroups each (gang_p < 2: off)
     int gang_p = 0, ngang = 0;
     std::vector<int> hsteps;  // steps of each tube in the last finished run (empty: none yet)
     int *gang_tube = nullptr;
-    unsigned *gang_ctr = nullptr;
-    unsigned long long *gang_rate = nullptr;
+    unsigned long long *gang_slot = nullptr;
+    double *gang_exch = nullptr;
     unsigned *gang_fail = nullptr;
     int *qorder = nullptr;  // the queue order without the gang tubes
     int nqueue = 0;
@@ -673,6 +951,19 @@ int ensure_table(bx_batch *b, int maxsteps)
     return 0;
 }
 
+// Waves per workgroup when none were chosen (bx_batch_tune).  The 8-wave build
+// holds a segment per wave in 163 registers, the 16-wave one in 128 with
+// spills: a step of 8 segments takes 8.0 us against 9.1, a gang member's of 3
+// to 5 segments 8.6 against 10.7, but a tube of 16 segments, which only the
+// larger workgroup can hold, 14.4 against 13.6.  With gangs the longest tubes
+// are split, so the smaller one serves.
+int default_waves(const bx_batch *b, bool gangs)
+{
+    int nx = 0;
+    for (const bx::Tube &t : b->htubes) nx = std::max(nx, t.nx);
+    return gangs || nx - 4 <= 8 * bx::kSegOut ? 8 : 16;
+}
+
 int enqueue(bx_batch *b, bool gangs = true)
 {
     const bool g = gangs && b->gang_p > 1 && b->ngang > 0;
@@ -695,17 +986,18 @@ int enqueue(bx_batch *b, bool gangs = true)
     a.ngang = g ? b->ngang : 0;
     a.gang_p = g ? b->gang_p : 0;
     a.gang_tube = b->gang_tube;
-    a.gang_ctr = b->gang_ctr;
-    a.gang_rate = b->gang_rate;
+    a.gang_slot = b->gang_slot;
+    a.gang_exch = b->gang_exch;
     a.gang_fail = b->gang_fail;
     const int *order = g ? b->qorder : b->order;
     const int gwg = a.ngang * a.gang_p;
     const unsigned grid = (unsigned)std::max(std::max(1, gwg), std::min(a.nqueue + gwg, b->ncu * b->blocks_per_cu));
     // the counters are reset by a kernel (not memsets), so the pair can be captured
-    const int nreset = std::max(std::max(b->ntube, 3 * a.ngang), 1);
-    hipLaunchKernelGGL(bx::k_tubes_reset, dim3((nreset + 255) / 256), dim3(256), 0, b->stream, b->queue, a.ngang,
-                       b->gang_ctr, b->gang_rate, b->gang_fail, b->status, b->ntube);
-    switch (b->waves) {
+    const int nslot = a.ngang * bx::kGangSlots;
+    const int nreset = std::max(std::max(b->ntube, nslot), 1);
+    hipLaunchKernelGGL(bx::k_tubes_reset, dim3((nreset + 255) / 256), dim3(256), 0, b->stream, b->queue, nslot,
+                       b->gang_slot, b->gang_fail, b->status, b->ntube);
+    switch (b->waves ? b->waves : default_waves(b, g)) {
     case 4:
         hipLaunchKernelGGL(bx::k_tubes<4>, dim3(grid), dim3(256), 0, b->stream, a, b->tubes, order);
         break;
@@ -754,7 +1046,7 @@ void batch_free(bx_batch *b)
     for (auto &e : b->ev)
         if (e) (void)hipEventDestroy(e);
     void *ptrs[] = {b->tubes, b->order, b->queue, b->ic, b->st, b->ss, b->old, b->t_out, b->steps_out, b->status,
-                    b->dtlog, b->gang_tube, b->gang_ctr, b->gang_rate, b->gang_fail, b->qorder};
+                    b->dtlog, b->gang_tube, b->gang_slot, b->gang_exch, b->gang_fail, b->qorder};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     if (b->stream) (void)hipStreamDestroy(b->stream);
@@ -1008,16 +1300,17 @@ int bx_batch_gang(bx_batch *b, int32_t members, int32_t ntubes)
         std::stable_sort(ord.begin(), ord.end(), [&](int x, int y) { return cost[x] > cost[y]; });
     }
     std::vector<int> gt(ord.begin(), ord.begin() + ntubes), q(ord.begin() + ntubes, ord.end());
-    for (void *p : {(void *)b->gang_tube, (void *)b->gang_ctr, (void *)b->gang_rate, (void *)b->gang_fail,
+    for (void *p : {(void *)b->gang_tube, (void *)b->gang_slot, (void *)b->gang_exch, (void *)b->gang_fail,
                     (void *)b->qorder})
         if (p) (void)hipFree(p);
     b->gang_tube = b->qorder = nullptr;
-    b->gang_ctr = b->gang_fail = nullptr;
-    b->gang_rate = nullptr;
+    b->gang_fail = nullptr;
+    b->gang_slot = nullptr;
+    b->gang_exch = nullptr;
     b->gang_p = b->ngang = 0;
     BX_HIP(hipMalloc((void **)&b->gang_tube, sizeof(int) * ntubes));
-    BX_HIP(hipMalloc((void **)&b->gang_ctr, sizeof(unsigned) * ntubes));
-    BX_HIP(hipMalloc((void **)&b->gang_rate, sizeof(unsigned long long) * 3 * ntubes));
+    BX_HIP(hipMalloc((void **)&b->gang_slot, sizeof(unsigned long long) * bx::kGangSlots * ntubes));
+    BX_HIP(hipMalloc((void **)&b->gang_exch, sizeof(double) * bx::kExchMember * members * ntubes));
     BX_HIP(hipMalloc((void **)&b->gang_fail, sizeof(unsigned)));
     BX_HIP(hipMalloc((void **)&b->qorder, sizeof(int) * std::max<size_t>(q.size(), 1)));
     BX_HIP(hipMemcpy(b->gang_tube, gt.data(), sizeof(int) * ntubes, hipMemcpyHostToDevice));

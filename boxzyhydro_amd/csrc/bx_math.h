@@ -182,21 +182,9 @@ __device__ __forceinline__ void div_shared(const double *a, double b, double *q)
         for (int i = 0; i < N; i++) q[i] = a[i] / b;
 }
 
-// a/b for double, where a zero numerator is answered without the division:
-// for finite nonzero b, IEEE gives the signed zero of sign(a) xor sign(b),
-// which is exactly a*b.  Used where most numerators are exactly +-0 (the
-// transverse components of a one-dimensional flow), so whole waves skip the
-// correctly rounded division sequence.
-__device__ __forceinline__ double qdiv(double a, double b)
-{
-    if (a == 0.0 && b != 0.0 && __builtin_isfinite(b)) return a * b;
-    return a / b;
-}
-
 // flux.f90:512-590 for one face: L = plus state of the cell below the face,
-// R = minus state of the cell above it, direction dir (0,1,2).  ZSKIP: the
-// final quotients go through qdiv (same values).
-template <typename T, int dir, bool ZSKIP = false>
+// R = minus state of the cell above it, direction dir (0,1,2).
+template <typename T, int dir>
 __device__ __forceinline__ void face_flux(const Side<T> &L, const Side<T> &R, T F[5])
 {
     const T h = T(0.5);
@@ -240,7 +228,7 @@ __device__ __forceinline__ void face_flux(const Side<T> &L, const Side<T> &R, T 
     const T am = vmax(vmax(zero, -(vr - cr)), -(vl - cl));
     const T apam = ap * am;
     const T den = ap + am;
-    if constexpr (sizeof(T) == 8 && !ZSKIP) {
+    if constexpr (sizeof(T) == 8) {
         double num[5];
 #pragma unroll
         for (int i = 0; i < 5; i++) num[i] = ap * fl[i] + am * fr[i] - apam * (sr[i] - sl[i]);
@@ -249,10 +237,7 @@ __device__ __forceinline__ void face_flux(const Side<T> &L, const Side<T> &R, T 
 #pragma unroll
         for (int i = 0; i < 5; i++) {
             const T num = ap * fl[i] + am * fr[i] - apam * (sr[i] - sl[i]);
-            if constexpr (ZSKIP && sizeof(T) == 8)
-                F[i] = qdiv(num, den);
-            else
-                F[i] = Arith<T>::div(num, den);
+            F[i] = Arith<T>::div(num, den);
         }
     }
 }
