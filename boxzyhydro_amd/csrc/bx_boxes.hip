@@ -9,8 +9,8 @@
 //   - the exact call sequence, subroutine by subroutine, with the per-cell
 //     bodies of the one-kernel-per-subroutine path (bx_cells.h), for the first
 //     step and for any step from a state that is not regular;
-//   - on a regular state whose ghost donors are all interior cells, fused
-//     steps: the wave bodies of the fused stage kernels (bx_waves.h) over the
+//   - on a regular state, and where the ghosts' donors over a pair of
+//     set_ghost_cells calls are interior cells (any walls), fused steps: the wave bodies of the fused stage kernels (bx_waves.h) over the
 //     grid, the workgroup's waves taking the virtual waves of those kernels'
 //     grids; a step that meets an irregular branch is redone with the exact
 //     sequence from U^n.
@@ -34,6 +34,7 @@
 #include <vector>
 
 #include "bx_cells.h"
+#include "bx_tile.h"
 #include "bx_waves.h"
 
 namespace bx {
@@ -46,13 +47,14 @@ enum : unsigned int {
 // | face fluxes 15, then the ghost-donor snapshot (5 planes of nscratch).  The
 // first 9 planes are the result (cons, u, p).
 constexpr int kRegionPlanes = 30;
-constexpr int kResultPlanes = 9;
 // Set-up, planes of n doubles: cons 5 | u 3 | p
 constexpr int kSetupPlanes = 9;
 
 struct Box {
     int64_t n, ic_off, reg_off, g_off, x_off;
     int64_t ng, ns;
+    int64_t d2_off, d2_scratch;  // corner ghosts: first entry in the tables, scratch (6 doubles each) in the region
+    int nd2;
     int nx, ny, nz, flatz;
     int maxsteps;
     double dx, dy, dz, gam, cfl, endtime, srho, seps, vlimit, muc, rgas;
@@ -74,6 +76,8 @@ struct BoxArgs {
     const double *ic;
     double *reg;
     const int32_t *gdst, *gsrc, *gsign, *gxsrc;
+    const int32_t *fsrc, *fsign;           // the table composed over a pair of calls (fused steps)
+    const int32_t *d2dst, *d2src, *d2sign; // two-level corner ghosts
     double *t_out;
     int *steps_out;
     unsigned *status;
@@ -133,13 +137,84 @@ __device__ __forceinline__ void box_ghosts(const Box &b, double *cons, double *s
     _Pragma("unroll 1") for (int64_t n = opaque_uniform(b.n), c##0 = tid; c##0 < n; c##0 += nt) \
         for (int64_t c = opaque(c##0), c##1 = 0; c##1 < 1; c##1++)
 
+// the stage constants of a grid for a step of full dt
+__device__ __forceinline__ StageArgs box_args(const Box &b, double dt)
+{
+    StageArgs sa = {};
+    sa.n = b.n;
+    sa.nx = b.nx;
+    sa.ny = b.ny;
+    sa.nz = b.nz;
+    sa.flatz = b.flatz;
+    sa.zlo = b.zlo;
+    sa.zhi = b.zhi;
+    sa.lz = b.lz;
+    sa.dt = dt;
+    sa.ds[0] = b.dx;
+    sa.ds[1] = b.dy;
+    sa.ds[2] = b.dz;
+    for (int d = 0; d < 3; d++) {
+        sa.inv_ds[d] = b.inv_ds[d];
+        sa.ds_pow2[d] = b.ds_pow2[d];
+    }
+    sa.ayz = b.ayz;
+    sa.axz = b.axz;
+    sa.axy = b.axy;
+    sa.vol = b.vol;
+    sa.inv_vol = b.inv_vol;
+    sa.vol_pow2 = b.vol_pow2;
+    sa.gam = b.gam;
+    sa.gm1 = b.gm1;
+    sa.seps = b.seps;
+    sa.srho = b.srho;
+    sa.vlimit = b.vlimit;
+    return sa;
+}
+
+// The corner ghosts of a grid after a corrector us, ps, u0 -> un, a trio of
+// waves each (corner_faces, corner_update in bx_tile.h).
 template <int W>
+__device__ __forceinline__ void box_corners(const Box *bp, double dt, double *cons, double *us, double *ps, double *un,
+                                            const int32_t *d2dst, const int32_t *d2src, const int32_t *d2sign,
+                                            double (*F)[3][2][5], unsigned int *sflags, unsigned long long *srate)
+{
+    constexpr int kTrios = W / 3;
+    const int lane = threadIdx.x & 63, wv = wave_id();
+    const Box b = *bp;
+    StageArgs sa = box_args(b, dt);
+    sa.uin = us;
+    sa.pin = ps;
+    sa.uold = cons;
+    sa.uout = un;
+    sa.nd2 = b.nd2;
+    sa.d2cell = d2src;
+    sa.d2ubar = cons + b.d2_scratch;
+    const int trio = wv / 3, d = wv - 3 * trio;
+    for (int j0 = 0; j0 < b.nd2; j0 += kTrios) {
+        const int j = j0 + trio;
+        const bool on = trio < kTrios && j < b.nd2;
+        unsigned flg = 0;
+        double rt = 0.0;
+        if (on) corner_faces(sa, j, d, lane, F[trio], flg);
+        __syncthreads();
+        if (on && d == 0 && lane == 0) rt = corner_update(sa, j, F[trio], d2dst[j], d2sign[j], flg);
+        if (flg) atomicOr(sflags, flg);
+        if (on && d == 0) wave_max_to(rt, srate);
+        __syncthreads();
+    }
+}
+
+// CH: fused steps also of grids whose ghosts chain (walls), with their corner
+// ghosts.  A build of its own: its registers cost outflow batches 13 % (17.1
+// against 15.1 ms for 192 grids).
+template <int W, bool CH>
 __global__ __launch_bounds__(64 * W) void k_boxes(BoxArgs a)
 {
     __shared__ double red[W];
     __shared__ int cur;
     __shared__ unsigned int sflags;       // irregular branches met by a fused step or the regularity check
     __shared__ unsigned long long srate;  // Courant rate (IEEE bits) from the corrector or the check
+    __shared__ double corner[CH ? W / 3 : 1][3][2][5];  // face fluxes of the corner ghosts, three waves each
     const int tid = threadIdx.x, nt = 64 * W;
     const int lane = tid & 63, wv = wave_id();  // wave-uniform for the compiler
     for (;;) {
@@ -161,6 +236,19 @@ __global__ __launch_bounds__(64 * W) void k_boxes(BoxArgs a)
         const double *ic = a.ic + b.ic_off;
         const int32_t *gd = a.gdst + b.g_off, *gs = a.gsrc + b.g_off, *gg = a.gsign + b.g_off;
         const int32_t *gx = a.gxsrc + b.x_off;
+        const bool fusable = b.fusable && (CH || b.ns == 0);
+        const int32_t *fs = (CH ? a.fsrc : a.gsrc) + b.g_off, *fg = (CH ? a.fsign : a.gsign) + b.g_off;
+        const int32_t *d2d = a.d2dst + b.d2_off, *d2g = a.d2sign + b.d2_off;
+        // u, p, adindx of the last fused step's state (main.f90:513-515)
+        auto materialize = [&]() {
+            for (int64_t n = opaque_uniform(b.n), c0 = tid; c0 < n; c0 += nt)
+                materialize_cell(n, opaque(c0), cons, u, p, ad, b.gam, b.seps);
+            __syncthreads();
+            if (CH && b.nd2 > 0) {
+                if (tid < b.nd2) p[d2d[tid]] = cons[b.d2_scratch + 6 * tid + 5];
+                __syncthreads();
+            }
+        };
         const bool flatz = b.flatz != 0;
 
         // the set-up: cons, u, p as uploaded (adindx is set by the first state call)
@@ -187,7 +275,7 @@ __global__ __launch_bounds__(64 * W) void k_boxes(BoxArgs a)
         while (step < b.maxsteps && time < b.endtime) {  // main.f90:212
             double dt_step = 0.0;
             bool fused_done = false;
-            if (b.fusable && regular) {
+            if (fusable && regular) {
                 // main.f90:266-281 on the rate of the current state
                 double dt = b.cfl / rate_f;
                 dt = dt * 1.0;
@@ -203,34 +291,7 @@ __global__ __launch_bounds__(64 * W) void k_boxes(BoxArgs a)
                 }
                 dt = dt * 0.5;
                 dt = dt * 2.0;
-                StageArgs sa = {};
-                sa.n = n;
-                sa.nx = b.nx;
-                sa.ny = b.ny;
-                sa.nz = b.nz;
-                sa.flatz = b.flatz;
-                sa.zlo = b.zlo;
-                sa.zhi = b.zhi;
-                sa.lz = b.lz;
-                sa.dt = dt;
-                sa.ds[0] = b.dx;
-                sa.ds[1] = b.dy;
-                sa.ds[2] = b.dz;
-                for (int d = 0; d < 3; d++) {
-                    sa.inv_ds[d] = b.inv_ds[d];
-                    sa.ds_pow2[d] = b.ds_pow2[d];
-                }
-                sa.ayz = b.ayz;
-                sa.axz = b.axz;
-                sa.axy = b.axy;
-                sa.vol = b.vol;
-                sa.inv_vol = b.inv_vol;
-                sa.vol_pow2 = b.vol_pow2;
-                sa.gam = b.gam;
-                sa.gm1 = b.gm1;
-                sa.seps = b.seps;
-                sa.srho = b.srho;
-                sa.vlimit = b.vlimit;
+                StageArgs sa = box_args(b, dt);
                 sa.flags = &sflags;
                 if (tid == 0) {
                     sflags = 0u;
@@ -270,9 +331,12 @@ __global__ __launch_bounds__(64 * W) void k_boxes(BoxArgs a)
                     }
                     __syncthreads();
                     for (int64_t k0 = tid; k0 < b.ng; k0 += nt)
-                        ghost6_one<double>(n, opaque(k0), gd, gs, gg, stage == 1 ? us : un, stage == 1 ? ps : nullptr);
+                        ghost6_one<double>(n, opaque(k0), gd, fs, fg, stage == 1 ? us : un, stage == 1 ? ps : nullptr);
                     __syncthreads();
                 }
+                if (CH && b.nd2 > 0)
+                    box_corners<W>(a.boxes + bi, dt, cons, us, ps, un, d2d, a.d2src + b.d2_off, d2g, corner, &sflags,
+                                   &srate);
                 if ((__builtin_amdgcn_readfirstlane(sflags) & FLAG_IRREGULAR) == 0u) {
                     BOX_CELLS(c)
                     for (int f = 0; f < 5; f++) cons[f * n + c] = un[f * n + c];
@@ -288,9 +352,8 @@ __global__ __launch_bounds__(64 * W) void k_boxes(BoxArgs a)
                 }
             }
             if (!fused_done) {
-            if (aux_stale) {  // u, p, adindx of the last fused step's state (main.f90:513-515)
-                BOX_CELLS(c) materialize_cell(n, c, cons, u, p, ad, b.gam, b.seps);
-                __syncthreads();
+            if (aux_stale) {
+                materialize();
                 aux_stale = false;
             }
             // state (main.f90:232) and the Courant maximum (main.f90:241)
@@ -368,7 +431,7 @@ __global__ __launch_bounds__(64 * W) void k_boxes(BoxArgs a)
             dt = dt * 2.0;
             dt_step = dt;
             regular = false;
-            if (b.fusable) {
+            if (fusable) {
                 // regularity and Courant rate of the new state (k_regular of the single-grid step)
                 if (tid == 0) {
                     sflags = 0u;
@@ -388,10 +451,7 @@ __global__ __launch_bounds__(64 * W) void k_boxes(BoxArgs a)
             time = time + dt_step;  // main.f90:545
             if (tid == 0 && step - 1 < a.maxlog) a.dtlog[(int64_t)bi * a.maxlog + step - 1] = dt_step;
         }
-        if (aux_stale) {
-            BOX_CELLS(c) materialize_cell(n, c, cons, u, p, ad, b.gam, b.seps);
-            __syncthreads();
-        }
+        if (aux_stale) materialize();
         if (tid == 0) {
             a.t_out[bi] = time;
             a.steps_out[bi] = step;
@@ -404,6 +464,26 @@ __global__ __launch_bounds__(64 * W) void k_boxes(BoxArgs a)
 
 __global__ void k_boxes_reset(int *queue) { *queue = 0; }
 
+// Result planes [first, first+k) of every grid's region as rows of k values,
+// the grids concatenated: elements [e0, e0+cnt) of that array.
+__global__ __launch_bounds__(256) void k_boxes_rows(int nbox, const int64_t *__restrict__ cell0,
+                                                   const int64_t *__restrict__ reg0, const double *__restrict__ reg,
+                                                   int first, int k, int64_t e0, int64_t cnt, double *__restrict__ rows)
+{
+    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= cnt) return;
+    const int64_t cell = (e0 + e) / k;
+    const int f = first + (int)(e0 + e - cell * k);
+    int lo = 0, hi = nbox;  // cell0[lo] <= cell < cell0[hi]
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) / 2;
+        if (cell0[mid] <= cell) lo = mid;
+        else hi = mid;
+    }
+    const int64_t n = cell0[lo + 1] - cell0[lo];
+    rows[e] = reg[reg0[lo] + f * n + (cell - cell0[lo])];
+}
+
 }  // namespace bx
 
 // ===================================================================== C-ABI
@@ -412,6 +492,7 @@ struct bx_boxes {
     hipStream_t stream = nullptr;
     int nbox = 0;
     int64_t cells = 0, interior = 0, reg_total = 0, ic_total = 0;
+    bool chained = false;  // some grid's ghosts chain and its pair of calls composes
     std::vector<bx::Box> hbox;
     std::vector<int> horder;
     bx::Box *boxes = nullptr;
@@ -419,6 +500,10 @@ struct bx_boxes {
     int *queue = nullptr;
     double *ic = nullptr, *reg = nullptr;
     int32_t *gdst = nullptr, *gsrc = nullptr, *gsign = nullptr, *gxsrc = nullptr;
+    int32_t *fsrc = nullptr, *fsign = nullptr, *d2dst = nullptr, *d2src = nullptr, *d2sign = nullptr;
+    int64_t *cell0 = nullptr, *reg0 = nullptr;  // first cell of each grid (nbox+1), first double of its region
+    double *stage = nullptr;                    // device staging of bx_boxes_result
+    bx::HostPipe *pipe = nullptr;
     double *t_out = nullptr;
     int *steps_out = nullptr;
     unsigned *status = nullptr;
@@ -502,6 +587,11 @@ int enqueue(bx_boxes *b)
     a.gsrc = b->gsrc;
     a.gsign = b->gsign;
     a.gxsrc = b->gxsrc;
+    a.fsrc = b->fsrc;
+    a.fsign = b->fsign;
+    a.d2dst = b->d2dst;
+    a.d2src = b->d2src;
+    a.d2sign = b->d2sign;
     a.t_out = b->t_out;
     a.steps_out = b->steps_out;
     a.status = b->status;
@@ -509,9 +599,14 @@ int enqueue(bx_boxes *b)
     const unsigned grid = (unsigned)std::max(1, std::min(b->nbox, b->ncu * b->blocks_per_cu));
     // the queue counter is reset by a kernel (not a memset), so the pair can be captured
     hipLaunchKernelGGL(bx::k_boxes_reset, dim3(1), dim3(1), 0, b->stream, b->queue);
-    if (b->waves == 4) hipLaunchKernelGGL(bx::k_boxes<4>, dim3(grid), dim3(256), 0, b->stream, a);
-    else if (b->waves == 16) hipLaunchKernelGGL(bx::k_boxes<16>, dim3(grid), dim3(1024), 0, b->stream, a);
-    else hipLaunchKernelGGL(bx::k_boxes<8>, dim3(grid), dim3(512), 0, b->stream, a);
+    // Chained grids take fused steps in the 8-wave build only.  A 16-wave one
+    // (128 VGPRs, hundreds spilled) ended with a memory aperture violation,
+    // cause not found; it and the 4-wave one run such grids with the exact
+    // sequence.
+    if (b->waves == 4) hipLaunchKernelGGL((bx::k_boxes<4, false>), dim3(grid), dim3(256), 0, b->stream, a);
+    else if (b->waves == 16) hipLaunchKernelGGL((bx::k_boxes<16, false>), dim3(grid), dim3(1024), 0, b->stream, a);
+    else if (b->chained) hipLaunchKernelGGL((bx::k_boxes<8, true>), dim3(grid), dim3(512), 0, b->stream, a);
+    else hipLaunchKernelGGL((bx::k_boxes<8, false>), dim3(grid), dim3(512), 0, b->stream, a);
     BX_HIP(hipGetLastError());
     return 0;
 }
@@ -549,12 +644,31 @@ void boxes_free(bx_boxes *b)
     drop_graph(b);
     for (auto &e : b->ev)
         if (e) (void)hipEventDestroy(e);
+    bx::pipe_free(b->pipe);
     void *ptrs[] = {b->boxes, b->order, b->queue, b->ic, b->reg, b->gdst, b->gsrc, b->gsign, b->gxsrc,
+                    b->fsrc, b->fsign, b->d2dst, b->d2src, b->d2sign, b->cell0, b->reg0, b->stage,
                     b->t_out, b->steps_out, b->status, b->dtlog};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     if (b->stream) (void)hipStreamDestroy(b->stream);
     delete b;
+}
+
+// the rows of planes [first, first+k) for a chunk of a result array
+struct BoxRows {
+    bx_boxes *b;
+    int first, k;
+};
+
+hipError_t box_rows_get(void *self, size_t off, size_t len, int w, const void **src)
+{
+    const BoxRows &r = *(const BoxRows *)self;
+    const int64_t e0 = (int64_t)(off / sizeof(double)), cnt = (int64_t)(len / sizeof(double));
+    double *to = r.b->stage + (size_t)w * (bx::pipe_slot_bytes() / sizeof(double));
+    hipLaunchKernelGGL(bx::k_boxes_rows, dim3(bx::blocks_for(cnt, 256)), dim3(256), 0, r.b->stream, r.b->nbox,
+                       r.b->cell0, r.b->reg0, r.b->reg, r.first, r.k, e0, cnt, to);
+    *src = to;
+    return hipGetLastError();
 }
 
 }  // namespace
@@ -569,7 +683,8 @@ int bx_boxes_create(int32_t nbox, const bx_params *prm, const double *endtime, c
     if (nbox < 1 || !prm || !endtime || !cons || !u || !p)
         return set_error(BX_ERR_ARG, "bx_boxes_create: null argument or no grids");
     std::vector<bx::Box> hb((size_t)nbox);
-    std::vector<int32_t> gd, gs, gg, gx;
+    std::vector<int32_t> gd, gs, gg, gx, fs, fg, dd, ds2, dg;
+    std::vector<int64_t> cell0, reg0;
     std::vector<double> cost((size_t)nbox);
     int64_t cells = 0, interior = 0, reg = 0, icn = 0;
     const double rgas = rgas_units();
@@ -589,6 +704,22 @@ int bx_boxes_create(int32_t nbox, const bx_params *prm, const double *endtime, c
             return rc;
         bx::Box &b = hb[i];
         b.n = (int64_t)q.nx * q.ny * q.nz;
+        // the tables of the fused steps: a pair of calls composed
+        bx::GhostPair gp;
+        bx::compose_ghosts(b.n, std::vector<int32_t>(gd.begin() + g0, gd.end()),
+                           std::vector<int32_t>(gs.begin() + g0, gs.end()),
+                           std::vector<int32_t>(gg.begin() + g0, gg.end()),
+                           std::vector<int32_t>(gx.begin() + x0, gx.end()), gp);
+        fs.insert(fs.end(), gp.src.begin(), gp.src.end());
+        fg.insert(fg.end(), gp.sign.begin(), gp.sign.end());
+        b.nd2 = gp.ok ? (int)gp.d2dst.size() : 0;
+        b.d2_off = (int64_t)dd.size();
+        if (gp.ok) {
+            dd.insert(dd.end(), gp.d2dst.begin(), gp.d2dst.end());
+            ds2.insert(ds2.end(), gp.d2src.begin(), gp.d2src.end());
+            dg.insert(dg.end(), gp.d2sign.begin(), gp.d2sign.end());
+        }
+        b.d2_scratch = (int64_t)bx::kRegionPlanes * b.n + 5 * ns;
         b.ic_off = icn;
         b.reg_off = reg;
         b.g_off = (int64_t)g0;
@@ -620,8 +751,7 @@ int bx_boxes_create(int32_t nbox, const bx_params *prm, const double *endtime, c
         b.ayz = q.dy * q.dz;
         b.axz = q.dx * q.dz;
         b.vol = q.dx * q.dy * q.dz;
-        // fused steps need every ghost donor to be an interior cell (one fill pass)
-        b.fusable = ns == 0 ? 1 : 0;
+        b.fusable = gp.ok ? 1 : 0;
         b.zlo = b.flatz ? 0 : 2;
         b.zhi = b.flatz ? q.nz : q.nz - 2;
         b.ly = 32;  // rows and planes per virtual wave (32x32 measured fastest of 8..32)
@@ -636,10 +766,12 @@ int bx_boxes_create(int32_t nbox, const bx_params *prm, const double *endtime, c
         b.gm1 = q.gammafix - 1.0;
         const int64_t in_x = q.nx - 4, in_y = q.ny - 4, in_z = q.nz < 6 ? q.nz : q.nz - 4;
         const int64_t off = cells;  // first cell of this grid in the concatenated host arrays
+        cell0.push_back(cells);
+        reg0.push_back(reg);
         cells += b.n;
         interior += std::max<int64_t>(0, in_x) * std::max<int64_t>(0, in_y) * std::max<int64_t>(0, in_z);
         icn += (int64_t)bx::kSetupPlanes * b.n;
-        reg += (int64_t)bx::kRegionPlanes * b.n + 5 * ns;
+        reg += (int64_t)bx::kRegionPlanes * b.n + 5 * ns + 6 * b.nd2;
         // cost estimate for the queue order: cells x steps, steps from the set-up's signal speeds
         double rate = 0.0;
         for (int64_t c = 0; c < b.n; c++) {
@@ -654,6 +786,8 @@ int bx_boxes_create(int32_t nbox, const bx_params *prm, const double *endtime, c
         cost[i] = (double)b.n * std::min(steps, 1e6);
     }
 
+    cell0.push_back(cells);
+
     int ndev = 0;
     BX_HIP(hipGetDeviceCount(&ndev));
     if (device < 0 || device >= ndev) return set_error(BX_ERR_ARG, "bx_boxes_create: no such device");
@@ -667,6 +801,7 @@ int bx_boxes_create(int32_t nbox, const bx_params *prm, const double *endtime, c
     b->reg_total = reg;
     b->ic_total = icn;
     b->hbox = hb;
+    for (const bx::Box &x : hb) b->chained = b->chained || (x.fusable && x.ns > 0);
     b->horder.resize(nbox);
     std::iota(b->horder.begin(), b->horder.end(), 0);
     std::stable_sort(b->horder.begin(), b->horder.end(), [&](int x, int y) { return cost[x] > cost[y]; });
@@ -692,6 +827,13 @@ int bx_boxes_create(int32_t nbox, const bx_params *prm, const double *endtime, c
                   {(void **)&b->gsrc, sizeof(int32_t) * std::max<size_t>(1, gs.size())},
                   {(void **)&b->gsign, sizeof(int32_t) * std::max<size_t>(1, gg.size())},
                   {(void **)&b->gxsrc, sizeof(int32_t) * std::max<size_t>(1, gx.size())},
+                  {(void **)&b->fsrc, sizeof(int32_t) * std::max<size_t>(1, fs.size())},
+                  {(void **)&b->fsign, sizeof(int32_t) * std::max<size_t>(1, fg.size())},
+                  {(void **)&b->d2dst, sizeof(int32_t) * std::max<size_t>(1, dd.size())},
+                  {(void **)&b->d2src, sizeof(int32_t) * std::max<size_t>(1, ds2.size())},
+                  {(void **)&b->d2sign, sizeof(int32_t) * std::max<size_t>(1, dg.size())},
+                  {(void **)&b->cell0, sizeof(int64_t) * ((size_t)nbox + 1)},
+                  {(void **)&b->reg0, sizeof(int64_t) * (size_t)nbox},
                   {(void **)&b->t_out, sizeof(double) * nbox},
                   {(void **)&b->steps_out, sizeof(int) * nbox},
                   {(void **)&b->status, sizeof(unsigned) * nbox},
@@ -723,6 +865,13 @@ int bx_boxes_create(int32_t nbox, const bx_params *prm, const double *endtime, c
         (e = put(b->gsrc, gs.data(), sizeof(int32_t) * gs.size())) != hipSuccess ||
         (e = put(b->gsign, gg.data(), sizeof(int32_t) * gg.size())) != hipSuccess ||
         (e = put(b->gxsrc, gx.data(), sizeof(int32_t) * gx.size())) != hipSuccess ||
+        (e = put(b->fsrc, fs.data(), sizeof(int32_t) * fs.size())) != hipSuccess ||
+        (e = put(b->fsign, fg.data(), sizeof(int32_t) * fg.size())) != hipSuccess ||
+        (e = put(b->d2dst, dd.data(), sizeof(int32_t) * dd.size())) != hipSuccess ||
+        (e = put(b->d2src, ds2.data(), sizeof(int32_t) * ds2.size())) != hipSuccess ||
+        (e = put(b->d2sign, dg.data(), sizeof(int32_t) * dg.size())) != hipSuccess ||
+        (e = put(b->cell0, cell0.data(), sizeof(int64_t) * cell0.size())) != hipSuccess ||
+        (e = put(b->reg0, reg0.data(), sizeof(int64_t) * reg0.size())) != hipSuccess ||
         (e = put(b->order, b->horder.data(), sizeof(int) * nbox)) != hipSuccess)
         return fail(e, "hipMemcpy tables");
     if (int rc = ensure_table(b, 1000000)) {
@@ -834,28 +983,23 @@ int bx_boxes_result(bx_boxes *b, double *cons, double *u, double *p, double *tim
     BX_HIP(hipStreamSynchronize(b->stream));
     const int nb = b->nbox;
     if (cons || u || p) {
-        // the result planes of each grid (cons, u, p), gathered into one host buffer
-        std::vector<double> res((size_t)(b->cells * bx::kResultPlanes));
-        int64_t cell0 = 0;
-        for (int i = 0; i < nb; i++) {
-            const int64_t n = b->hbox[i].n;
-            BX_HIP(hipMemcpyAsync(res.data() + cell0 * bx::kResultPlanes, b->reg + b->hbox[i].reg_off,
-                                  sizeof(double) * bx::kResultPlanes * n, hipMemcpyDeviceToHost, b->stream));
-            cell0 += n;
+        const int64_t most = 5 * b->cells;  // the largest array
+        if (!b->stage) {
+            const size_t bytes = sizeof(double) * (size_t)most;
+            BX_HIP(hipMalloc((void **)&b->stage, bytes < bx::kPipeMin ? bytes : bx::pipe_stage_bytes()));
         }
-        BX_HIP(hipStreamSynchronize(b->stream));
-        cell0 = 0;
-        for (int i = 0; i < nb; i++) {
-            const int64_t n = b->hbox[i].n;
-            const double *r = res.data() + cell0 * bx::kResultPlanes;
-            for (int64_t c = 0; c < n; c++) {
-                if (cons)
-                    for (int f = 0; f < 5; f++) cons[(cell0 + c) * 5 + f] = r[f * n + c];
-                if (u)
-                    for (int f = 0; f < 3; f++) u[(cell0 + c) * 3 + f] = r[(5 + f) * n + c];
-                if (p) p[cell0 + c] = r[8 * n + c];
-            }
-            cell0 += n;
+        struct {
+            double *out;
+            int first, k;
+        } want[] = {{cons, 0, 5}, {u, 5, 3}, {p, 8, 1}};
+        for (auto &w : want) {
+            if (!w.out) continue;
+            BoxRows r{b, w.first, w.k};
+            const bx::PipeChunk ch{box_rows_get, nullptr, nullptr, 0};
+            if (int rc = bx::pipe_download(&b->pipe, b->device, b->stream, (char *)w.out,
+                                           sizeof(double) * (size_t)(w.k * b->cells), sizeof(double) * (size_t)w.k, ch,
+                                           &r))
+                return rc;
         }
     }
     if (time) BX_HIP(hipMemcpy(time, b->t_out, sizeof(double) * nb, hipMemcpyDeviceToHost));

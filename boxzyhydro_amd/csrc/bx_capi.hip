@@ -119,15 +119,12 @@ static int build_ghost_table(const bx_params *prm, std::vector<int32_t> &dst, st
 
     // symbolic values, set here for the ghosts only: an interior cell is itself
     std::unique_ptr<int32_t[]> gsrc(new int32_t[n]);
-    std::unique_ptr<uint8_t[]> gsgn(new uint8_t[n]);
+    std::vector<uint8_t> gsgn(n, 0xff);  // sign bits of a ghost; 0xff marks an interior cell
     for (int32_t g : ghosts) {
         gsrc[g] = g;
         gsgn[g] = 0;
     }
-    auto inside = [&](int32_t c) {
-        const int ix = c % nx + 1, iy = (c / nx) % ny + 1, iz = c / (nx * ny) + 1;
-        return bnd(ix, iy, iz) == 0;
-    };
+    auto inside = [&](int32_t c) { return gsgn[c] == 0xff; };
     auto take = [&](int32_t g, int32_t from, unsigned flip) {
         if (inside(from)) {
             gsrc[g] = from;
@@ -216,6 +213,75 @@ static int build_ghost_table(const bx_params *prm, std::vector<int32_t> &dst, st
     return BX_OK;
 }
 
+// See GhostPair (bx_internal.h).
+void compose_ghosts(int64_t n, const std::vector<int32_t> &gd, const std::vector<int32_t> &gs,
+                    const std::vector<int32_t> &gg, const std::vector<int32_t> &gx, GhostPair &out)
+{
+    // The pair of calls composed: a ghost whose donor is the pre-call value of
+    // ghost h gets h's value after the first call, which is h's donor when
+    // that is an interior cell (sign flips compose).  When h's donor is the
+    // pre-call value of ghost h2 the pair leaves h2's value from before it;
+    // the fused step supports that when h2's own pair gives an interior cell
+    // v (the corner ghosts of a box walled in y and z): such a ghost ends a
+    // step as +-(v's corrector result before source(1)) and is fixed up after
+    // the ghost fill.  Deeper chains take the exact sequence.
+    std::vector<int32_t> &fs = out.src, &fg = out.sign;
+    fs = gs;
+    fg = gg;
+    out.ok = true;
+    out.d2at.clear();
+    out.d2dst.clear();
+    out.d2src.clear();
+    out.d2sign.clear();
+    if (!gx.empty()) {
+        std::vector<int64_t> entry((size_t)n, -1);
+        for (size_t k = 0; k < gd.size(); k++) entry[(size_t)gd[k]] = (int64_t)k;
+        // the pair's value of entry k: -1 with the interior cell and sign, or
+        // the entry of the ghost whose pre-pair value it is (sign: its sign)
+        auto pair_of = [&](size_t k, int32_t &cell, int32_t &sgn) -> int64_t {
+            if (gs[k] >= 0) {
+                cell = gs[k];
+                sgn = gg[k];
+                return -1;
+            }
+            const int64_t h = entry[(size_t)gx[(size_t)(-gs[k] - 1)]];
+            if (h < 0) return -2;
+            sgn = gg[k] ^ gg[(size_t)h];
+            if (gs[(size_t)h] >= 0) {
+                cell = gs[(size_t)h];
+                return -1;
+            }
+            const int64_t h2 = entry[(size_t)gx[(size_t)(-gs[(size_t)h] - 1)]];
+            return h2 < 0 ? -2 : h2;
+        };
+        for (size_t k = 0; k < gd.size() && out.ok; k++) {
+            int32_t cell = 0, sgn = 0;
+            const int64_t r = pair_of(k, cell, sgn);
+            if (r == -1) {
+                fs[k] = cell;
+                fg[k] = sgn;
+                continue;
+            }
+            int32_t cell2 = 0, sgn2 = 0;
+            if (r < 0 || pair_of((size_t)r, cell2, sgn2) != -1) {
+                out.ok = false;
+                break;
+            }
+            fs[k] = cell2;
+            fg[k] = sgn ^ sgn2;
+            out.d2at.push_back(k);
+            out.d2dst.push_back(gd[k]);
+            out.d2src.push_back(cell2);
+            out.d2sign.push_back(sgn ^ sgn2);
+        }
+        if ((int)out.d2dst.size() > kMaxD2) out.ok = false;
+        if (!out.ok) {
+            out.d2dst.clear();
+            out.d2at.clear();
+        }
+    }
+}
+
 }  // namespace bx
 
 using namespace bx;
@@ -277,64 +343,10 @@ int bx_create(const bx_params *prm, int32_t device, bx_ctx **out)
     }
     c->nghost = (int64_t)gd.size();
     c->nscratch = (int64_t)gx.size();
-    // The pair of calls composed: a ghost whose donor is the pre-call value of
-    // ghost h gets h's value after the first call, which is h's donor when
-    // that is an interior cell (sign flips compose).  When h's donor is the
-    // pre-call value of ghost h2 the pair leaves h2's value from before it;
-    // the fused step supports that when h2's own pair gives an interior cell
-    // v (the corner ghosts of a box walled in y and z): such a ghost ends a
-    // step as +-(v's corrector result before source(1)) and is fixed up after
-    // the ghost fill.  Deeper chains take the exact sequence.
-    std::vector<int32_t> fs(gs), fg(gg), d2dst, d2src, d2sign;
-    std::vector<size_t> d2at;  // their entries in the tables
-    c->fghost_ok = true;
-    if (!gx.empty()) {
-        std::vector<int64_t> entry((size_t)n, -1);
-        for (size_t k = 0; k < gd.size(); k++) entry[(size_t)gd[k]] = (int64_t)k;
-        // the pair's value of entry k: -1 with the interior cell and sign, or
-        // the entry of the ghost whose pre-pair value it is (sign: its sign)
-        auto pair_of = [&](size_t k, int32_t &cell, int32_t &sgn) -> int64_t {
-            if (gs[k] >= 0) {
-                cell = gs[k];
-                sgn = gg[k];
-                return -1;
-            }
-            const int64_t h = entry[(size_t)gx[(size_t)(-gs[k] - 1)]];
-            if (h < 0) return -2;
-            sgn = gg[k] ^ gg[(size_t)h];
-            if (gs[(size_t)h] >= 0) {
-                cell = gs[(size_t)h];
-                return -1;
-            }
-            const int64_t h2 = entry[(size_t)gx[(size_t)(-gs[(size_t)h] - 1)]];
-            return h2 < 0 ? -2 : h2;
-        };
-        for (size_t k = 0; k < gd.size() && c->fghost_ok; k++) {
-            int32_t cell = 0, sgn = 0;
-            const int64_t r = pair_of(k, cell, sgn);
-            if (r == -1) {
-                fs[k] = cell;
-                fg[k] = sgn;
-                continue;
-            }
-            int32_t cell2 = 0, sgn2 = 0;
-            if (r < 0 || pair_of((size_t)r, cell2, sgn2) != -1) {
-                c->fghost_ok = false;
-                break;
-            }
-            fs[k] = cell2;
-            fg[k] = sgn ^ sgn2;
-            d2at.push_back(k);
-            d2dst.push_back(gd[k]);
-            d2src.push_back(cell2);
-            d2sign.push_back(sgn ^ sgn2);
-        }
-        if ((int)d2dst.size() > kMaxD2) c->fghost_ok = false;
-        if (!c->fghost_ok) {
-            d2dst.clear();
-            d2at.clear();
-        }
-    }
+    GhostPair gp;
+    compose_ghosts(n, gd, gs, gg, gx, gp);
+    std::vector<int32_t> &fs = gp.src, &fg = gp.sign, &d2dst = gp.d2dst, &d2src = gp.d2src, &d2sign = gp.d2sign;
+    c->fghost_ok = gp.ok;
     c->nd2 = (int)d2dst.size();
     // whether every ghost's composed donor is the per-axis one (the ghosts are
     // in cell order: one row after another)
@@ -367,8 +379,8 @@ int bx_create(const bx_params *prm, int32_t device, bx_ctx **out)
     // the corner ghosts last in the tables, so that a fill can leave them out
     for (auto *t : {&gd, &gs, &gg, &fs, &fg}) {
         std::vector<int32_t> last;
-        for (size_t k : d2at) last.push_back((*t)[k]);
-        for (size_t q = d2at.size(); q-- > 0;) t->erase(t->begin() + (int64_t)d2at[q]);
+        for (size_t k : gp.d2at) last.push_back((*t)[k]);
+        for (size_t q = gp.d2at.size(); q-- > 0;) t->erase(t->begin() + (int64_t)gp.d2at[q]);
         t->insert(t->end(), last.begin(), last.end());
     }
 
@@ -461,6 +473,7 @@ int bx_destroy(bx_ctx *c)
                    c->cons32, c->ustar32, c->unext32, c->pstar32, c->eflux, c->chunk0, c->chunk_dts, c->stage};
     for (void *p : dev)
         if (p) (void)hipFree(p);
+    pipe_free(c->pipe);
     if (c->hsc) (void)hipHostFree(c->hsc);
     for (int i = 0; i < 6; i++)
         if (c->ev[i]) (void)hipEventDestroy(c->ev[i]);
@@ -506,8 +519,8 @@ int bx_sync(bx_ctx *c)
 
 // Host arrays in the reference's layout, cons(5,n) etc. (field fastest), and
 // the context's planes (one field after another): the transfer moves the
-// caller's bytes as they are through a device staging buffer, and a kernel
-// reorders them on the device.  Element e of a chunk of cells [n0, n0+cnt/k)
+// caller's bytes as they are through a device staging buffer (bx_transfer.hip),
+// and a kernel reorders them on the device.  Element e of a chunk of cells [n0, n0+cnt/k)
 // is field e%k of cell n0+e/k.
 __global__ __launch_bounds__(256) void k_rows_to_planes(int64_t n0, int64_t cnt, int k, int64_t n,
                                                         const double *__restrict__ rows, double *__restrict__ planes)
@@ -527,59 +540,77 @@ __global__ __launch_bounds__(256) void k_planes_to_rows(int64_t n0, int64_t cnt,
     rows[e] = planes[(int64_t)(e - cell * k) * n + n0 + cell];
 }
 
-constexpr int64_t kStageDoubles = int64_t(1) << 23;  // 64 MiB
-
+// The device staging buffer: a slot for each worker of a large transfer, or
+// the whole array of a small one.
 static int ensure_stage(bx_ctx *c)
 {
     if (c->stage) return BX_OK;
-    const int64_t len = std::min<int64_t>(kStageDoubles, 5 * c->n);  // at least one cell of any k <= 5
+    const int64_t all = 5 * c->n;  // the largest array
+    const int64_t len = sizeof(double) * (size_t)all < kPipeMin ? all : (int64_t)(pipe_stage_bytes() / sizeof(double));
     BX_HIP(hipMalloc((void **)&c->stage, sizeof(double) * (size_t)len));
     c->stage_len = len;
     return BX_OK;
 }
 
+// One transfer of k planes (d) in the host layout (k, n).
+struct Rows {
+    bx_ctx *c;
+    int k;
+    double *d;
+    double *slot(int w) const { return c->stage + (size_t)w * (pipe_slot_bytes() / sizeof(double)); }
+};
+
+static hipError_t rows_get(void *self, size_t off, size_t len, int w, const void **src)
+{
+    const Rows &r = *(const Rows *)self;
+    const int64_t e0 = (int64_t)(off / sizeof(double)), cnt = (int64_t)(len / sizeof(double));
+    if (r.k == 1) {
+        *src = r.d + e0;
+        return hipSuccess;
+    }
+    hipLaunchKernelGGL(k_planes_to_rows, dim3(blocks_for(cnt, 256)), dim3(256), 0, r.c->stream, e0 / r.k, cnt, r.k,
+                       r.c->n, r.d, r.slot(w));
+    *src = r.slot(w);
+    return hipGetLastError();
+}
+
+static hipError_t rows_room(void *self, size_t off, size_t, int w, void **to)
+{
+    const Rows &r = *(const Rows *)self;
+    *to = r.k == 1 ? r.d + off / sizeof(double) : r.slot(w);
+    return hipSuccess;
+}
+
+static hipError_t rows_put(void *self, size_t off, size_t len, int w)
+{
+    const Rows &r = *(const Rows *)self;
+    if (r.k == 1) return hipSuccess;
+    const int64_t e0 = (int64_t)(off / sizeof(double)), cnt = (int64_t)(len / sizeof(double));
+    hipLaunchKernelGGL(k_rows_to_planes, dim3(blocks_for(cnt, 256)), dim3(256), 0, r.c->stream, e0 / r.k, cnt, r.k,
+                       r.c->n, r.slot(w), r.d);
+    return hipGetLastError();
+}
+
 // host array (k, n) -> k device planes
 static int upload_aos(bx_ctx *c, const double *h, int k, double *d)
 {
-    const int64_t n = c->n;
-    if (k == 1) {
-        BX_HIP(hipMemcpyAsync(d, h, sizeof(double) * (size_t)n, hipMemcpyHostToDevice, c->stream));
-        BX_HIP(hipStreamSynchronize(c->stream));
-        return BX_OK;
-    }
-    if (int rc = ensure_stage(c)) return rc;
-    for (int64_t n0 = 0; n0 < n;) {
-        const int64_t m = std::min<int64_t>(n - n0, c->stage_len / k), cnt = m * k;
-        BX_HIP(hipMemcpyAsync(c->stage, h + n0 * k, sizeof(double) * (size_t)cnt, hipMemcpyHostToDevice, c->stream));
-        hipLaunchKernelGGL(k_rows_to_planes, dim3(blocks_for(cnt, 256)), dim3(256), 0, c->stream, n0, cnt, k, n,
-                           c->stage, d);
-        BX_HIP(hipGetLastError());
-        n0 += m;
-    }
-    BX_HIP(hipStreamSynchronize(c->stream));
-    return BX_OK;
+    if (k > 1)
+        if (int rc = ensure_stage(c)) return rc;
+    Rows r{c, k, d};
+    const PipeChunk ch{rows_get, rows_room, rows_put, k > 1 ? (size_t)c->stage_len * sizeof(double) : 0};
+    return pipe_upload(&c->pipe, c->device, c->stream, (const char *)h, sizeof(double) * (size_t)(k * c->n),
+                       sizeof(double) * (size_t)k, ch, &r);
 }
 
 // k device planes -> host array (k, n)
 static int download_aos(bx_ctx *c, const double *d, int k, double *h)
 {
-    const int64_t n = c->n;
-    if (k == 1) {
-        BX_HIP(hipMemcpyAsync(h, d, sizeof(double) * (size_t)n, hipMemcpyDeviceToHost, c->stream));
-        BX_HIP(hipStreamSynchronize(c->stream));
-        return BX_OK;
-    }
-    if (int rc = ensure_stage(c)) return rc;
-    for (int64_t n0 = 0; n0 < n;) {
-        const int64_t m = std::min<int64_t>(n - n0, c->stage_len / k), cnt = m * k;
-        hipLaunchKernelGGL(k_planes_to_rows, dim3(blocks_for(cnt, 256)), dim3(256), 0, c->stream, n0, cnt, k, n, d,
-                           c->stage);
-        BX_HIP(hipGetLastError());
-        BX_HIP(hipMemcpyAsync(h + n0 * k, c->stage, sizeof(double) * (size_t)cnt, hipMemcpyDeviceToHost, c->stream));
-        n0 += m;
-    }
-    BX_HIP(hipStreamSynchronize(c->stream));
-    return BX_OK;
+    if (k > 1)
+        if (int rc = ensure_stage(c)) return rc;
+    Rows r{c, k, const_cast<double *>(d)};
+    const PipeChunk ch{rows_get, rows_room, rows_put, k > 1 ? (size_t)c->stage_len * sizeof(double) : 0};
+    return pipe_download(&c->pipe, c->device, c->stream, (char *)h, sizeof(double) * (size_t)(k * c->n),
+                         sizeof(double) * (size_t)k, ch, &r);
 }
 
 int bx_upload(bx_ctx *c, const double *cons, const double *u, const double *p, const double *adindx)

@@ -436,114 +436,17 @@ static int ghosts6(bx_ctx *c, S *planes, S *pstar, bool corners = true)
     return BX_OK;
 }
 
-// The two-level corner ghosts after the corrector's ghost fill.  The exact
-// sequence leaves such a ghost holding +-(its interior cell v's corrector
-// result before source(1)); that value reaches the results only through the
-// next step's Courant rate (courant.f90:11-15 runs over every cell) and the
-// stored state.  One workgroup per ghost evaluates v's corrector update
-// again from the corrector's inputs with the tiled kernel's operations (its
-// six faces, flux.f90:121-190, and the update of flux.f90:213-228), parks the
-// result before source(1), writes the ghost and adds its Courant rate (the
-// state and velocity of main.f90:232 and of the step's last velocity call,
-// state.f90:30-57, velocity.f90:18-21).  The kernel is a serial chain of
-// divisions and roots on a step's critical path: one wave takes each
-// direction and one lane each of its two faces, so that a sixth of the faces
-// lies on the chain (with one lane per ghost taking all six: 18.0 us).
 __global__ __launch_bounds__(192) void k_corner_ghosts(StageArgs a0, const int32_t *__restrict__ dst,
-                                                      const int32_t *__restrict__ sign)
+                                                       const int32_t *__restrict__ sign)
 {
-    const StageArgs a = with_dt(a0);
     __shared__ double F[3][2][5];
-    const int j = blockIdx.x, d = wave_id(), h = threadIdx.x & 63;
+    const StageArgs a = with_dt(a0);
+    const int j = blockIdx.x, d = wave_id();
     double rt = 0.0;
     unsigned int flg = 0;
-    const int64_t v = a.d2cell[j];
-    const int64_t plane = (int64_t)a.nx * a.ny;
-    const int ix = (int)(v % a.nx), iy = (int)((v / a.nx) % a.ny), iz = (int)(v / plane);
-    // the primitives of the cell o cells from v along axis dir (ghosts from their donors, as the tiles read them)
-    auto prim_at = [&](int dir, int o) -> W6<double> {
-        const int x = ix + (dir == 0 ? o : 0), y = iy + (dir == 1 ? o : 0), z = iz + (dir == 2 ? o : 0);
-        const Donor<double, true> me(a, x, y);
-        W6<double> w = load_prims<2, double>(a, Donor<double, true>::plane(a, plane, z), me.off, flg);
-        me.signs(a, z, w);
-        return w;
-    };
-    if (h < 2) {
-        double f[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-        // face h of this wave's direction: between the cells h-1 and h from v
-        auto face = [&](auto dirc) {
-            constexpr int dir = decltype(dirc)::value;
-            W6<double> w[4];
-            for (int i = 0; i < 4; i++) w[i] = prim_at(dir, h - 2 + i);
-            Side<double> mi[2], pl[2];
-            for (int i = 0; i < 2; i++) {
-                const int o = h - 1 + i;
-                const int x = ix + (dir == 0 ? o : 0), y = iy + (dir == 1 ? o : 0), z = iz + (dir == 2 ? o : 0);
-                const bool gh = x < 2 || x > a.nx - 3 || y < 2 || y > a.ny - 3 || (!a.flatz && (z < 2 || z > a.nz - 3));
-                dir_states<dir>(w[i], w[i + 1], w[i + 2], sound_of(w[i + 1], a.gam), gh, a, mi[i], pl[i]);
-            }
-            face_flux<double, dir>(pl[0], mi[1], f);
-        };
-        if (d == 0) face(std::integral_constant<int, 0>{});
-        else if (d == 1) face(std::integral_constant<int, 1>{});
-        else if (!a.flatz) face(std::integral_constant<int, 2>{});
-        for (int i = 0; i < 5; i++) F[d][h][i] = f[i];
-    }
+    corner_faces(a, j, d, threadIdx.x & 63, F, flg);
     __syncthreads();
-    if (threadIdx.x == 0) {
-        const W6<double> q0 = prim_at(0, 0);
-        double ui[5], uo[5], ft[5];
-        for (int i = 0; i < 5; i++) {
-            ui[i] = elem<double>(a.uin, (int64_t)i * a.n + v, 0u);
-            uo[i] = elem<double>(a.uold, (int64_t)i * a.n + v, 0u);
-            const double dx = F[0][1][i] - F[0][0][i];
-            const double ey = a.axz * (F[1][1][i] - F[1][0][i]);
-            const double dz = a.flatz ? 0.0 : F[2][1][i] - F[2][0][i];
-            const double sm = (a.ayz * dx + ey) + a.axy * dz;
-            ft[i] = -div_by(sm * a.dt, a.vol, a.inv_vol, a.vol_pow2);
-        }
-        double rv = 0.0;
-        // rewrites U^{n+1} of v with the bits the tiled kernel wrote and parks
-        // the result before source(1) in d2ubar (with gravity also p of v)
-        if (a.gf) stage_update<2, double, true>(a, ui, uo, ft, q0, v, 0u, flg, rv, true);
-        else stage_update<2, double>(a, ui, uo, ft, q0, v, 0u, flg, rv, true);
-        double U[5];
-        for (int i = 0; i < 5; i++) U[i] = a.d2ubar[6 * j + i];
-        // the pressure the exact sequence leaves in the ghost: the state call
-        // after the last ghost pair (main.f90:511-513) takes the velocity of
-        // the previous velocity call, when the ghost held h2's value from
-        // before the third pair, 0.5*(cons_old + U* + 0) of v up to signs
-        // (flux.f90:213, cons_old = U^n after source(0), which leaves rho as
-        // it is and, without gravity, m too; with gravity m is kicked by v's
-        // force); the signs drop out of |u|^2
-        {
-            double rc = 0.5 * ((uo[0] + ui[0]) + 0.0);
-            rc = vmax(rc, a.srho);
-            double mo[3] = {uo[1], uo[2], uo[3]};
-            if (a.gf) {
-                const double g[3] = {a.gf[v], a.gf[a.n + v], a.gf[2 * a.n + v]};
-                const double m[3] = {uo[1], uo[2], uo[3]};
-                grav_momenta(uo[0], m, g, a.dt * 0.5, mo);
-            }
-            double uc[3];
-            for (int d = 0; d < 3; d++) uc[d] = (0.5 * ((mo[d] + ui[1 + d]) + 0.0)) / rc;
-            const double ek = U[0] * 0.5 * (uc[0] * uc[0] + uc[1] * uc[1] + uc[2] * uc[2]);
-            a.d2ubar[6 * j + 5] = vmax(U[4] - ek, a.seps) * a.gm1;
-        }
-        const int sg = sign[j];
-        for (int f = 1; f <= 3; f++)
-            if ((sg >> (f - 1)) & 1) U[f] = -U[f];
-        const int64_t gcell = dst[j];
-        double *un = (double *)a.uout;
-        for (int i = 0; i < 5; i++) un[(int64_t)i * a.n + gcell] = U[i];
-        const double v0 = U[1] / U[0], v1 = U[2] / U[0], v2 = U[3] / U[0];
-        const double ekin = U[0] * 0.5 * (v0 * v0 + v1 * v1 + v2 * v2);
-        const double p = vmax(U[4] - ekin, a.seps) * a.gm1;
-        const double snd = sqrt(a.gam * p / U[0]);
-        rt = div_by(snd + fabs(v0), a.ds[0], a.inv_ds[0], a.ds_pow2[0]) +
-             div_by(snd + fabs(v1), a.ds[1], a.inv_ds[1], a.ds_pow2[1]) +
-             div_by(snd + fabs(v2), a.ds[2], a.inv_ds[2], a.ds_pow2[2]);
-    }
+    if (threadIdx.x == 0) rt = corner_update(a, j, F, dst[j], sign[j], flg);
     if (flg) atomicOr(a.flags, flg);
     if (d == 0) wave_max_to(rt, a.rate);
 }

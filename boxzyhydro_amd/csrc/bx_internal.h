@@ -11,6 +11,8 @@
 
 namespace bx {
 
+struct HostPipe;
+
 constexpr int kMaxD2 = 64;  // two-level ghost compositions a context may have (one wave)
 
 // The step scalars of main.f90 as a device-dt step leaves them.
@@ -135,6 +137,7 @@ struct bx_ctx {
     double *chunk_dts;     // dt of each step of a chunk
     double *stage;         // device staging of host transfers (Fortran layout), stage_len doubles
     int64_t stage_len;
+    struct bx::HostPipe *pipe;  // pinned slots of large host transfers (bx_transfer.hip), or null
 
     bx::DevScalars *dsc;   // device scalars
     bx::DevScalars *hsc;   // pinned host mirror
@@ -229,5 +232,41 @@ void drop_step_graphs(bx_ctx *c);
 constexpr int kChunkSteps = 32;  // steps per run, at most
 int narrow_cons(bx_ctx *c);
 int widen_cons(bx_ctx *c);
+
+// The ghost table of a grid (bx_ghost_table's gd, gs, gg, gx) composed over a
+// pair of set_ghost_cells calls: ghost gd[k] <- +-(interior cell src[k]); ok
+// when every entry resolves, the two-level corner ghosts (entries d2at, see
+// bx_ctx) among them.
+struct GhostPair {
+    std::vector<int32_t> src, sign;
+    std::vector<size_t> d2at;
+    std::vector<int32_t> d2dst, d2src, d2sign;
+    bool ok;
+};
+void compose_ghosts(int64_t n, const std::vector<int32_t> &gd, const std::vector<int32_t> &gs,
+                    const std::vector<int32_t> &gg, const std::vector<int32_t> &gx, GhostPair &out);
+
+// Large host transfers (bx_transfer.hip).  A transfer is cut into chunks of
+// whole units (bytes); worker w of kWorkers calls, with `self`, for the bytes
+// [off, off+len) of the host array: get (download) enqueues whatever forms
+// them on the device and returns where they are; room (upload) says where they
+// go and put enqueues what follows the copy.  Device memory a callback hands
+// out must be w's own.  Without a pipe (small transfers, no pinned memory)
+// chunks of at most stage_bytes (0: any size) go one after another with w = 0.
+// Calls return after the transfer.
+struct PipeChunk {
+    hipError_t (*get)(void *self, size_t off, size_t len, int w, const void **src);
+    hipError_t (*room)(void *self, size_t off, size_t len, int w, void **to);
+    hipError_t (*put)(void *self, size_t off, size_t len, int w);
+    size_t stage_bytes;
+};
+constexpr size_t kPipeMin = size_t(8) << 20;  // smaller transfers are copied directly
+size_t pipe_stage_bytes();                    // device staging that gives every worker a slot of its own
+size_t pipe_slot_bytes();
+int pipe_download(HostPipe **slot, int device, hipStream_t stream, char *dst, size_t bytes, size_t unit,
+                  const PipeChunk &chunk, void *self);
+int pipe_upload(HostPipe **slot, int device, hipStream_t stream, const char *src, size_t bytes, size_t unit,
+                const PipeChunk &chunk, void *self);
+void pipe_free(HostPipe *p);
 
 }  // namespace bx
