@@ -453,6 +453,9 @@ int bx_create(const bx_params *prm, int32_t device, bx_ctx **out)
     if ((e = hipHostMalloc((void **)&c->hsc, sizeof(DevScalars), hipHostMallocDefault)) != hipSuccess)
         return fail(e, "hipHostMalloc");
     std::memset(c->hsc, 0, sizeof(DevScalars));
+    const size_t mb = sizeof(unsigned long long) * kMaxSlots * kMaxStride;
+    if ((e = hipMalloc((void **)&c->dmax, mb)) != hipSuccess) return fail(e, "hipMalloc maxima");
+    if ((e = hipHostMalloc((void **)&c->hmax, mb, hipHostMallocDefault)) != hipSuccess) return fail(e, "hipHostMalloc");
     if ((e = hipStreamSynchronize(c->stream)) != hipSuccess) return fail(e, "hipStreamSynchronize");
     *out = c;
     return BX_OK;
@@ -474,6 +477,8 @@ int bx_destroy(bx_ctx *c)
     for (void *p : dev)
         if (p) (void)hipFree(p);
     pipe_free(c->pipe);
+    if (c->dmax) (void)hipFree(c->dmax);
+    if (c->hmax) (void)hipHostFree(c->hmax);
     if (c->hsc) (void)hipHostFree(c->hsc);
     for (int i = 0; i < 6; i++)
         if (c->ev[i]) (void)hipEventDestroy(c->ev[i]);
@@ -700,14 +705,7 @@ int bx_velocity(bx_ctx *c, double *maxv)
     if (!c) return set_error(BX_ERR_ARG, "bx_velocity: null context");
     int rc = ensure_aux(c);
     if (rc || (rc = launch_velocity(c, maxv != nullptr))) return rc;
-    if (maxv) {
-        BX_HIP(hipMemcpyAsync(&c->hsc->maxv_bits, &c->dsc->maxv_bits, sizeof(unsigned long long),
-                              hipMemcpyDeviceToHost, c->stream));
-        BX_HIP(hipStreamSynchronize(c->stream));
-        unsigned long long b = c->hsc->maxv_bits;
-        std::memcpy(maxv, &b, sizeof(double));
-    }
-    return BX_OK;
+    return maxv ? read_max(c, maxv) : BX_OK;
 }
 
 int bx_courant(bx_ctx *c, double *dt)
@@ -715,12 +713,8 @@ int bx_courant(bx_ctx *c, double *dt)
     if (!c || !dt) return set_error(BX_ERR_ARG, "bx_courant: null argument");
     int rc = ensure_aux(c);
     if (rc || (rc = launch_courant(c))) return rc;
-    BX_HIP(hipMemcpyAsync(&c->hsc->rate_bits[0], &c->dsc->rate_bits[0], sizeof(unsigned long long),
-                          hipMemcpyDeviceToHost, c->stream));
-    BX_HIP(hipStreamSynchronize(c->stream));
     double rate;
-    unsigned long long b = c->hsc->rate_bits[0];
-    std::memcpy(&rate, &b, sizeof(double));
+    if ((rc = read_max(c, &rate))) return rc;
     *dt = c->prm.cfl / rate;  // courant.f90:29
     return BX_OK;
 }
@@ -748,7 +742,7 @@ int bx_flux(bx_ctx *c, int32_t avg, double dt)
     int rc = ensure_aux(c);
     if (rc) return rc;
     if (!c->states) BX_HIP(hipMalloc((void **)&c->states, sizeof(double) * state_planes(c) * (size_t)c->n));
-    return launch_flux(c, avg, dt);
+    return launch_flux(c, avg, dt, true);
 }
 
 int bx_copy_old(bx_ctx *c)
@@ -800,53 +794,64 @@ namespace bx {
 // is an interior cell (one call then already gives the fixed point).
 static int ghosts_again(bx_ctx *c) { return c->nscratch > 0 ? launch_ghosts(c, c->cons) : BX_OK; }
 
-// One step of main.f90:211-555 with the reference's kernel sequence.
-// dt logic (main.f90:266-281) runs on the host in the same IEEE operations.
-static int exact_step(bx_ctx *c, double endtime, double *time, double *dtold, int32_t *step, double *dt_out)
+// One step of main.f90:211-555 in the reference's call sequence, the pointwise
+// calls between two ghost fills or fluxes in fused passes (bx_pass.hip).  dt
+// logic (main.f90:266-281) runs on the host in the same IEEE operations.
+// started: the previous step's last pass has made this step's first state call
+// and Courant rate; *next (may be null): on entry whether a further step is
+// wanted, on return whether its start is made.
+static int exact_step(bx_ctx *c, double endtime, double *time, double *dtold, int32_t *step, double *dt_out,
+                      bool started = false, bool *next = nullptr)
 {
     int rc;
     if (!c->states) BX_HIP(hipMalloc((void **)&c->states, sizeof(double) * state_planes(c) * (size_t)c->n));
+    const bool chained = c->nscratch > 0, ang = c->prm.fluxangmom != 0;
     *step += 1;
-    if ((rc = launch_state(c))) return rc;  // :232
-    double dt;
-    {
-        if ((rc = launch_courant(c))) return rc;  // :241
-        BX_HIP(hipMemcpyAsync(&c->hsc->rate_bits[0], &c->dsc->rate_bits[0], sizeof(unsigned long long),
-                              hipMemcpyDeviceToHost, c->stream));
-        BX_HIP(hipStreamSynchronize(c->stream));
-        double rate;
-        unsigned long long b = c->hsc->rate_bits[0];
-        std::memcpy(&rate, &b, sizeof(double));
-        dt = c->prm.cfl / rate;
-    }
+    if (!started && (rc = launch_pass(c, kStateRate, 0.0, true, nullptr))) return rc;  // :232, :241
+    double rate;
+    if ((rc = read_max(c, &rate))) return rc;
+    double dt = c->prm.cfl / rate;
     const double f1 = 1.0;
     dt = dt * f1;
     if (*step > 1 && *dtold > 0.0) dt = std::min(dt, *dtold * 1.1);
     *dtold = dt;
     if (dt + *time > endtime) dt = endtime - *time;
     dt = dt * 0.5;
-    if ((rc = launch_source(c, dt))) return rc;  // :289 (+ ghosts, source.f90:199)
-    if ((rc = ghosts_again(c))) return rc;       // :312
-    if ((rc = launch_state(c))) return rc;       // :314
-    if ((rc = launch_velocity(c, false))) return rc;  // :318
-    BX_HIP(hipMemcpyAsync(c->cons_old, c->cons, sizeof(double) * 5 * c->n, hipMemcpyDeviceToDevice,
-                          c->stream));  // :327-333
+    // :289 (+ ghosts, source.f90:199), :312, :314, :318; cons_old (:327-333) is
+    // written by the pass for flux_ang, which works in place, and is otherwise
+    // the buffer that flux(0) leaves behind
+    if (chained) {
+        if ((rc = launch_source(c, dt)) || (rc = ghosts_again(c))) return rc;
+        if ((rc = launch_pass(c, kAfterFlux, 0.0, true, nullptr))) return rc;
+        if (ang)
+            BX_HIP(hipMemcpyAsync(c->cons_old, c->cons, sizeof(double) * 5 * c->n, hipMemcpyDeviceToDevice, c->stream));
+    } else if ((rc = launch_pass(c, kBeforeFlux, dt, false, ang ? c->cons_old : nullptr))) {
+        return rc;
+    }
     dt = dt * 2.0;
-    if ((rc = launch_flux(c, 0, dt))) return rc;  // :346 (+ ghosts, flux.f90:231)
-    if ((rc = ghosts_again(c))) return rc;        // :351
-    if ((rc = launch_state(c))) return rc;
-    if ((rc = launch_velocity(c, false))) return rc;
-    if ((rc = launch_flux(c, 1, dt))) return rc;  // :368 (+ ghosts, flux.f90:231)
-    if ((rc = ghosts_again(c))) return rc;        // :374
-    if ((rc = launch_state(c))) return rc;
-    if ((rc = launch_velocity(c, false))) return rc;
+    if ((rc = launch_flux(c, 0, dt, chained))) return rc;  // :346 (+ ghosts, flux.f90:231), :351
+    if (!ang) std::swap(c->cons_old, c->states);
+    if (chained && (rc = ghosts_again(c))) return rc;
+    if ((rc = launch_pass(c, kAfterFlux, 0.0, chained, nullptr))) return rc;
+    const bool ext = (c->grav_flags & BX_GRAV_EXTERNAL) != 0;  // its mass moments take the ghosts' density
+    if ((rc = launch_flux(c, 1, dt, chained || ext))) return rc;  // :368 (+ ghosts, flux.f90:231), :374
+    if (chained) {
+        if ((rc = ghosts_again(c))) return rc;
+        if ((rc = launch_pass(c, kAfterFlux, 0.0, true, nullptr))) return rc;
+    }
     dt = 0.5 * dt;
-    if ((c->grav_flags & BX_GRAV_POTENTIAL) && (rc = launch_calc_gforce(c))) return rc;   // :481
-    if ((c->grav_flags & BX_GRAV_EXTERNAL) && (rc = launch_external_grav(c))) return rc;  // :487
-    if ((rc = launch_source(c, dt))) return rc;  // :490 (+ ghosts, source.f90:199)
-    if ((rc = ghosts_again(c))) return rc;       // :511
-    if ((rc = launch_state(c))) return rc;
-    if ((rc = launch_velocity(c, false))) return rc;
+    // the state and velocity of :374 change neither density nor force
+    if ((c->grav_flags & BX_GRAV_POTENTIAL) && (rc = launch_calc_gforce(c))) return rc;  // :481
+    if (ext && (rc = launch_external_grav(c))) return rc;                                // :487
+    const bool more = next && *next && *time + dt * 2.0 < endtime && *step < 1000000;
+    if (chained) {  // :490 (+ ghosts, source.f90:199), :511
+        if ((rc = launch_source(c, dt)) || (rc = ghosts_again(c))) return rc;
+        if ((rc = launch_pass(c, kAfterFlux, 0.0, true, nullptr))) return rc;
+        if (next) *next = false;
+    } else {
+        if ((rc = launch_pass(c, more ? kEndNext : kEnd, dt, false, nullptr))) return rc;
+        if (next) *next = more;
+    }
     dt = dt * 2.0;
     *time = *time + dt;
     *dt_out = dt;
@@ -1092,9 +1097,12 @@ extern "C" int bx_step(bx_ctx *c, int32_t mode, int32_t nsteps, double endtime, 
         rc = fused_loop(c, nsteps, endtime, time, dtold, step, dts, &k, graph);
     } else {
         if ((rc = ensure_aux(c))) return rc;
+        bool started = false;
         while (k < nsteps && *time < endtime && *step < 1000000) {
             double dt;
-            if ((rc = exact_step(c, endtime, time, dtold, step, &dt))) break;
+            bool next = k + 1 < nsteps;
+            if ((rc = exact_step(c, endtime, time, dtold, step, &dt, started, &next))) break;
+            started = next;
             c->ghosts_filled = true;
             if (dts) dts[k] = dt;
             k++;

@@ -29,6 +29,17 @@ __device__ __forceinline__ void block_max_to(double v, unsigned long long *dst)
     }
 }
 
+// A maximum over a whole grid goes into kMaxSlots words, each in a cache line
+// of its own, a block's share into the slot of its index; the host takes the
+// largest.  One word for all cost about 9 ns per block: 46 us at 96^3 for a
+// Courant pass that streams in 10.
+__device__ __forceinline__ unsigned long long *max_slot(unsigned long long *slots)
+{
+    return slots + (blockIdx.x % kMaxSlots) * kMaxStride;
+}
+
+static __global__ void k_clear_max(unsigned long long *slots) { slots[threadIdx.x * kMaxStride] = 0ull; }
+
 // 1-based (ix,iy,iz) of cell c (utils.f90:191-194 inverse)
 __device__ __forceinline__ void coords(int64_t c, int nx, int ny, int &ix, int &iy, int &iz)
 {
@@ -51,45 +62,43 @@ __device__ __forceinline__ int boundary_of(int ix, int iy, int iz, int nx, int n
 // centred coordinate of cell index i (1-based) on an axis of n cells (init_grid.f90:85-93)
 __device__ __forceinline__ double centre(double d, int i, int n) { return d * ((double)i - ((double)n + 1.0) / 2.0); }
 
-// state.f90:30-57, H2STAT=-1 branch
-__device__ __forceinline__ void state_cell(int64_t n, int64_t c, double *__restrict__ cons,
-                                           const double *__restrict__ u, double *__restrict__ p,
-                                           double *__restrict__ ad, double gam, double seps, double muc, double rgas)
+// One cell of the exact path in registers.
+struct CellState {
+    double U[5], v[3], p;
+};
+
+// state.f90:30-57, H2STAT=-1 branch: p, and E of a low-density cell
+__device__ __forceinline__ void state_of(CellState &x, double gam, double seps, double muc, double rgas)
 {
-    const double rho = cons[c], E = cons[4 * n + c];
-    const double u0 = u[c], u1 = u[n + c], u2 = u[2 * n + c];
-    const double ekin = rho * 0.5 * (u0 * u0 + u1 * u1 + u2 * u2);
-    double eps = vmax(E - ekin, seps);
-    ad[c] = gam;
+    const double rho = x.U[0];
+    const double ekin = rho * 0.5 * (x.v[0] * x.v[0] + x.v[1] * x.v[1] + x.v[2] * x.v[2]);
+    double eps = vmax(x.U[4] - ekin, seps);
     if (rho < 1e-4) {
-        const double tk = vmin(5e3, p[c] / (rho * rgas) * muc);
+        const double tk = vmin(5e3, x.p / (rho * rgas) * muc);
         const double pc = rho * tk * rgas / muc;
-        p[c] = pc;
+        x.p = pc;
         eps = pc / (gam - 1.0);
-        cons[4 * n + c] = eps + ekin;
+        x.U[4] = eps + ekin;
     } else {
-        p[c] = eps * (gam - 1.0);
+        x.p = eps * (gam - 1.0);
     }
 }
 
-// velocity.f90:18-53: u = m/rho, vlimit clamp; returns max |u_d| before the clamp
-__device__ __forceinline__ double velocity_cell(int64_t n, int64_t c, double *__restrict__ cons,
-                                                double *__restrict__ u, double vlimit, double seps)
+// velocity.f90:18-53: u = m/rho, vlimit clamp; returns max |u_d| before the
+// clamp and whether it acted
+__device__ __forceinline__ double velocity_of(CellState &x, double vlimit, double seps, bool &clamped)
 {
     double vm = 0.0;
-    const double rho = cons[c];
-    double m[3], v[3];
+    const double rho = x.U[0];
+    div_shared<3>(x.U + 1, rho, x.v);
+    clamped = false;
     for (int d = 0; d < 3; d++) {
-        m[d] = cons[(1 + d) * n + c];
-        v[d] = m[d] / rho;
+        vm = vmax(vm, fabs(x.v[d]));
+        if (fabs(x.v[d]) > vlimit) clamped = true;
     }
-    int flag = 0;
-    for (int d = 0; d < 3; d++) {
-        vm = vmax(vm, fabs(v[d]));
-        if (fabs(v[d]) > vlimit) flag = 1;
-    }
-    if (flag) {
-        double E = cons[4 * n + c];
+    if (clamped) {
+        double *m = x.U + 1, *v = x.v;
+        double E = x.U[4];
         double ekin = 0.5 * (m[0] * m[0] + m[1] * m[1] + m[2] * m[2]) / rho;
         double speed = 0.0;
         for (int d = 0; d < 3; d++) speed = speed + v[d] * v[d];
@@ -97,13 +106,80 @@ __device__ __forceinline__ double velocity_cell(int64_t n, int64_t c, double *__
         for (int d = 0; d < 3; d++) {
             v[d] = v[d] * vlimit / speed;
             m[d] = v[d] * rho;
-            cons[(1 + d) * n + c] = m[d];
         }
         E = E - ekin;
         ekin = 0.5 * (m[0] * m[0] + m[1] * m[1] + m[2] * m[2]) / rho;
-        cons[4 * n + c] = vmax(E, seps) + ekin;
+        x.U[4] = vmax(E, seps) + ekin;
     }
-    for (int d = 0; d < 3; d++) u[d * n + c] = v[d];
+    return vm;
+}
+
+// source.f90:148-182 with the force g; with fluxangmom the terms of
+// source.f90:73-90 come first (the pforce of source.f90:64-66 feeds nothing on
+// the hydro path), x and y being the cell's centre
+__device__ __forceinline__ void source_of(CellState &s, double dt, double g0, double g1, double g2, double seps,
+                                          int ang, double x, double y)
+{
+    const double rho = s.U[0];
+    double m0 = s.U[1], m1 = s.U[2], m2 = s.U[3];
+    const double ux = s.v[0], uy = s.v[1], uz = s.v[2];
+    if (ang) {
+        const double r = sqrt(x * x + y * y);
+        // r**4 as the reference's build evaluates it: a left-to-right product
+        const double w = x * uy - y * ux, r4 = ((r * r) * r) * r;
+        m1 = m1 + rho * (w * w) * y / r4 * dt;
+        m0 = m0 + rho * (w * w) * x / r4 * dt;
+    }
+    m1 = m1 + (rho * g1) * dt;
+    m0 = m0 + (rho * g0) * dt;
+    m2 = m2 + (g2 * rho) * dt;
+    const double ekin = 0.5 * (m0 * m0 + m1 * m1 + m2 * m2) / rho;
+    s.U[1] = m0;
+    s.U[2] = m1;
+    s.U[3] = m2;
+    s.U[4] = vmax(s.U[4] - ekin + dt * rho * (ux * g0 + uy * g1 + uz * g2), seps) + ekin;
+}
+
+// courant.f90:17-21: sum_d (c+|u_d|)/Delta_d
+__device__ __forceinline__ double courant_of(const CellState &x, double ad, double dx, double dy, double dz)
+{
+    const double sound = sqrt(ad * x.p / x.U[0]);
+    return (sound + fabs(x.v[0])) / dx + (sound + fabs(x.v[1])) / dy + (sound + fabs(x.v[2])) / dz;
+}
+
+__device__ __forceinline__ void state_cell(int64_t n, int64_t c, double *__restrict__ cons,
+                                           const double *__restrict__ u, double *__restrict__ p,
+                                           double *__restrict__ ad, double gam, double seps, double muc, double rgas)
+{
+    CellState x;
+    x.U[0] = cons[c];
+    x.U[4] = cons[4 * n + c];
+    for (int d = 0; d < 3; d++) x.v[d] = u[d * n + c];
+    const bool low = x.U[0] < 1e-4;
+    if (low) x.p = p[c];
+    state_of(x, gam, seps, muc, rgas);
+    ad[c] = gam;
+    if (low) cons[4 * n + c] = x.U[4];
+    p[c] = x.p;
+}
+
+__device__ __forceinline__ double velocity_cell(int64_t n, int64_t c, double *__restrict__ cons,
+                                                double *__restrict__ u, double vlimit, double seps)
+{
+    CellState x;
+    for (int d = 0; d < 4; d++) x.U[d] = cons[d * n + c];
+    x.U[4] = 0.0;
+    bool clamped;
+    double vm = 0.0;
+    div_shared<3>(x.U + 1, x.U[0], x.v);
+    for (int d = 0; d < 3; d++) vm = vmax(vm, fabs(x.v[d]));
+    if (vm > vlimit || !(vm == vm) || fabs(x.v[0]) > vlimit || fabs(x.v[1]) > vlimit || fabs(x.v[2]) > vlimit) {
+        x.U[4] = cons[4 * n + c];
+        vm = velocity_of(x, vlimit, seps, clamped);
+        if (clamped)
+            for (int d = 1; d < 5; d++) cons[d * n + c] = x.U[d];
+    }
+    for (int d = 0; d < 3; d++) u[d * n + c] = x.v[d];
     return vm;
 }
 
@@ -112,14 +188,16 @@ __device__ __forceinline__ double courant_cell(int64_t n, int64_t c, const doubl
                                                const double *__restrict__ u, const double *__restrict__ p,
                                                const double *__restrict__ ad, double dx, double dy, double dz)
 {
-    const double sound = sqrt(ad[c] * p[c] / cons[c]);
-    return (sound + fabs(u[c])) / dx + (sound + fabs(u[n + c])) / dy + (sound + fabs(u[2 * n + c])) / dz;
+    CellState x;
+    x.U[0] = cons[c];
+    x.p = p[c];
+    for (int d = 0; d < 3; d++) x.v[d] = u[d * n + c];
+    return courant_of(x, ad[c], dx, dy, dz);
 }
 
-// source.f90:148-182 on an interior cell with the gforce planes gf, or without
-// them a uniform gravity vector g (the reference's g = -(phi(+)-phi(-))/(2d)
-// = -0.0 for phi=0); with fluxangmom the terms of source.f90:73-90 come first
-// (the pforce of source.f90:64-66 feeds nothing on the hydro path)
+// source() on an interior cell with the gforce planes gf, or without them a
+// uniform gravity vector g (the reference's g = -(phi(+)-phi(-))/(2d) = -0.0
+// for phi=0)
 __device__ __forceinline__ void source_cell(int64_t n, int64_t c, int nx, int ny, int nz, double *__restrict__ cons,
                                             const double *__restrict__ u, double dt, double g0, double g1, double g2,
                                             double seps, int ang, double dx, double dy,
@@ -128,31 +206,16 @@ __device__ __forceinline__ void source_cell(int64_t n, int64_t c, int nx, int ny
     int ix, iy, iz;
     coords(c, nx, ny, ix, iy, iz);
     if (boundary_of(ix, iy, iz, nx, ny, nz) > 0) return;
-    const double rho = cons[c];
-    double m0 = cons[n + c], m1 = cons[2 * n + c], m2 = cons[3 * n + c];
-    const double ux = u[c], uy = u[n + c], uz = u[2 * n + c];
-    if (ang) {
-        const double x = centre(dx, ix, nx), y = centre(dy, iy, ny);
-        const double r = sqrt(x * x + y * y);
-        // r**4 as the reference's build evaluates it: a left-to-right product
-        const double w = x * uy - y * ux, r4 = ((r * r) * r) * r;
-        m1 = m1 + rho * (w * w) * y / r4 * dt;
-        m0 = m0 + rho * (w * w) * x / r4 * dt;
-    }
+    CellState x;
+    for (int f = 0; f < 5; f++) x.U[f] = cons[f * n + c];
+    for (int d = 0; d < 3; d++) x.v[d] = u[d * n + c];
     if (gf) {  // gforce(1:3, igrid) of calc_gforce / external_grav
         g0 = gf[c];
         g1 = gf[n + c];
         g2 = gf[2 * n + c];
     }
-    m1 = m1 + (rho * g1) * dt;
-    m0 = m0 + (rho * g0) * dt;
-    m2 = m2 + (g2 * rho) * dt;
-    const double ekin = 0.5 * (m0 * m0 + m1 * m1 + m2 * m2) / rho;
-    const double E = cons[4 * n + c];
-    cons[n + c] = m0;
-    cons[2 * n + c] = m1;
-    cons[3 * n + c] = m2;
-    cons[4 * n + c] = vmax(E - ekin + dt * rho * (ux * g0 + uy * g1 + uz * g2), seps) + ekin;
+    source_of(x, dt, g0, g1, g2, seps, ang, centre(dx, ix, nx), centre(dy, iy, ny));
+    for (int f = 1; f < 5; f++) cons[f * n + c] = x.U[f];
 }
 
 // utils.f90:314-403 as resolved on the host into (ghost, donor, momentum sign

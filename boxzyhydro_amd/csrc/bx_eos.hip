@@ -26,8 +26,7 @@
 #include <thread>
 #include <vector>
 
-#include "bx_internal.h"
-#include "bx_math.h"
+#include "bx_eos_dev.h"
 #include "bx_units.h"
 
 namespace bx {
@@ -35,13 +34,6 @@ namespace bx {
 // parameters.f90:9-10 and eos.f90:16-19
 constexpr double kRgasCGS = 8.254e7, kMp = 1.6726e-24, kKb = 1.38065e-16, kHplanck = 6.626e-27,
                  kMelec = 9.10934e-28, kPi = 3.1415926535897931;
-
-// Fortran INT() of a real(8) as the reference's x86-64 build computes it
-// (cvttsd2si): truncation, and INT_MIN for NaN and out-of-range values.
-__host__ __device__ __forceinline__ int fort_int(double q)
-{
-    return (q > -2147483649.0 && q < 2147483648.0) ? (int)q : INT_MIN;
-}
 
 struct H2Row {  // per temperature row
     double tk, zp, zoprime, ze, dzpdt, dzedt, dzoprimedt;
@@ -291,121 +283,7 @@ static int build_tables(const bx_params *p, const bx_eos_params *e, Tables &t)
     return BX_OK;
 }
 
-// ------------------------------------------------------------------ device
-// One entry of table 2 at (itk, irho): the values and, for itk < NEOS, the
-// slopes (v(itk+1)-v(itk))/(eng2(itk+1)-eng2(itk)) that get_gamma2 forms at
-// run time -- the same IEEE divisions of the same table values, done once.
-struct alignas(64) TabEntry {
-    double eng, gam, muc, tk, sg, sm, st, pad;
-};
-// The entries (itk, irho) and (itk, irho+1) side by side in one 128-byte
-// line: a lookup, which needs both rows at the same itk, reads one line.
-struct alignas(128) TabPair {
-    TabEntry lo, hi;
-};
-// Per density row: rho_table(irho), 1/(rho_table(irho+1)-rho_table(irho))
-// (NaN where the reference does not interpolate in rho), log10 of the first
-// energy, deng_eos_array, and the first and last energies of the row.
-struct alignas(64) RhoRow {
-    double r0, inv_dr, leng1, deng, e_first, e_last, pad0, pad1;
-};
-
-struct EosDev {
-    int neos, nrho;
-    double log_rho_low, drho, density, tk_bgrnd;
-    const TabPair *tab;  // (irho, itk), itk fastest (code units); hi = row irho+1
-    const RhoRow *rows;
-};
-
-// eos.f90:653-699
-__device__ __forceinline__ void get_gamma2(const EosDev &e, double eps, double rho, double &tk, double &m,
-                                           double &gam)
-{
-    int irho = fort_int((log10(rho * e.density) - e.log_rho_low) / e.drho) + 1;
-    irho = irho < e.nrho ? irho : e.nrho;
-    if (irho < 1) irho = 1;
-    const RhoRow R = e.rows[irho - 1];
-    double eng = eps / rho;
-    int ientry = fort_int((log10(eng) - R.leng1) / R.deng) + 1;
-    if (ientry > e.neos - 1) {
-        ientry = e.neos - 1;
-        eng = R.e_last;
-    }
-    if (ientry < 1 || eng < R.e_first) {
-        ientry = 1;
-        eng = R.e_first;
-    }
-    const TabPair *pr = e.tab + (int64_t)(irho - 1) * e.neos + (ientry - 1);
-    const TabEntry a = pr->lo, ap = pr->hi;  // hi: row irho+1 (the row itself on the last row)
-    gam = a.gam + a.sg * (eng - a.eng);
-    m = a.muc + a.sm * (eng - a.eng);
-    tk = a.tk + a.st * (eng - a.eng);
-    // rho_table(irho) /= rho_table(irhop): interpolate in rho; written as
-    // selects so that no branch waits on the table load
-    const double gamp = ap.gam + ap.sg * (eng - ap.eng);
-    const double mp = ap.muc + ap.sm * (eng - ap.eng);
-    const double tkp = ap.tk + ap.st * (eng - ap.eng);
-    const double slope = R.inv_dr * (rho - R.r0);
-    const bool interp = R.inv_dr == R.inv_dr;
-    gam = interp ? gam + (gamp - gam) * slope : gam;
-    m = interp ? m + (mp - m) * slope : m;
-    tk = interp ? tk + (tkp - tk) * slope : tk;
-}
-
-// state.f90:30-79, tabulated branch (H2STAT >= 0).  Each thread takes CPT
-// cells a block apart (coalesced), with indices clamped for the loads, so the
-// table lookups of its cells are in flight together.
-template <int CPT>
-__global__ __launch_bounds__(256) void k_state_tab(int64_t n, double *__restrict__ cons,
-                                                   const double *__restrict__ u, double *__restrict__ p,
-                                                   double *__restrict__ ad, double *__restrict__ mucp,
-                                                   EosDev e, double gamfix, double seps, double muc,
-                                                   double rgas, int disk, int nx, int ny, double dx, double dy)
-{
-    const int64_t base = (int64_t)blockIdx.x * blockDim.x * CPT + threadIdx.x;
-    double rho[CPT], ekin[CPT], tk[CPT], m[CPT], g[CPT];
-#pragma unroll
-    for (int k = 0; k < CPT; k++) {
-        const int64_t c0 = base + (int64_t)k * blockDim.x, c = c0 < n ? c0 : n - 1;
-        rho[k] = cons[c];
-        const double E = cons[4 * n + c];
-        const double u0 = u[c], u1 = u[n + c], u2 = u[2 * n + c];
-        ekin[k] = rho[k] * 0.5 * (u0 * u0 + u1 * u1 + u2 * u2);
-        const double eps = vmax(E - ekin[k], seps);
-        if (disk) {
-            // nz == 1: the column is a disk of scale height hscale (state.f90:61-69)
-            const int ix = (int)(c % nx) + 1, iy = (int)((c / nx) % ny) + 1;
-            const double x = dx * ((double)ix - ((double)nx + 1.0) / 2.0);
-            const double y = dy * ((double)iy - ((double)ny + 1.0) / 2.0);
-            const double hscale = sqrt((ad[c] - 1.0) * eps / (2.0 * ekin[k]) * (x * x + y * y));
-            get_gamma2(e, eps / (2.0 * hscale), rho[k] / (2.0 * hscale), tk[k], m[k], g[k]);
-        } else {
-            get_gamma2(e, eps, rho[k], tk[k], m[k], g[k]);
-        }
-    }
-#pragma unroll
-    for (int k = 0; k < CPT; k++) {
-        const int64_t c = base + (int64_t)k * blockDim.x;
-        if (c >= n) break;
-        ad[c] = g[k];
-        mucp[c] = m[k];
-        double pc = rho[k] * tk[k] * rgas / m[k];
-        if (rho[k] < 1e-4) {
-            pc = rgas * e.tk_bgrnd / muc * rho[k];
-            cons[4 * n + c] = pc / (gamfix - 1.0) + ekin[k];
-        }
-        p[c] = pc;
-    }
-}
-
 }  // namespace bx
-
-struct bx_eos {
-    bx::EosDev dev;
-    bx::TabPair *tab;
-    bx::RhoRow *rows;
-    double *muc_plane;
-};
 
 namespace bx {
 
@@ -422,18 +300,6 @@ void eos_free(bx_ctx *c)
     if (!c) return;
     eos_release(c->eos);
     c->eos = nullptr;
-}
-
-int launch_state_tab(bx_ctx *c)
-{
-    const bx_eos *q = c->eos;
-    constexpr int kCpt = 2;
-    hipLaunchKernelGGL(k_state_tab<kCpt>, dim3(blocks_for(c->n, 256 * kCpt)), dim3(256), 0, c->stream, c->n, c->cons,
-                       c->u, c->p,
-                       c->adindx, q->muc_plane, q->dev, c->prm.gammafix, c->prm.small_eps, c->muc, c->rgas,
-                       c->nz == 1 ? 1 : 0, c->nx, c->ny, c->prm.dx, c->prm.dy);
-    BX_HIP(hipGetLastError());
-    return BX_OK;
 }
 
 }  // namespace bx

@@ -4,6 +4,8 @@
 // bx_source/bx_set_ghost_cells/bx_flux/bx_avisc, and the exact fallback of
 // the fused step.  Arithmetic order follows the cited reference lines so the
 // results are bit-identical to the reference's FP64 step.
+#include <algorithm>
+#include <cstring>
 #include <utility>
 
 #include "bx_cells.h"
@@ -12,25 +14,14 @@ namespace bx {
 
 constexpr int kThreads = 256;
 
-// ------------------------------------------------------------------ state
-__global__ __launch_bounds__(kThreads) void k_state(int64_t n, double *__restrict__ cons,
-                                                   const double *__restrict__ u, double *__restrict__ p,
-                                                   double *__restrict__ ad, double gam, double seps,
-                                                   double muc, double rgas)
-{
-    const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (c < n) state_cell(n, c, cons, u, p, ad, gam, seps, muc, rgas);
-}
-
 // --------------------------------------------------------------- velocity
 __global__ __launch_bounds__(kThreads) void k_velocity(int64_t n, double *__restrict__ cons,
                                                       double *__restrict__ u, double vlimit,
                                                       double seps, unsigned long long *maxv)
 {
-    double vm = 0.0;
-    for (int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; c < n; c += (int64_t)gridDim.x * blockDim.x)
-        vm = vmax(vm, velocity_cell(n, c, cons, u, vlimit, seps));
-    if (maxv) block_max_to(vm, maxv);
+    const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const double vm = c < n ? velocity_cell(n, c, cons, u, vlimit, seps) : 0.0;
+    if (maxv) block_max_to(vm, max_slot(maxv));
 }
 
 // ---------------------------------------------------------------- courant
@@ -41,10 +32,8 @@ __global__ __launch_bounds__(kThreads) void k_courant(int64_t n, const double *_
                                                      const double *__restrict__ ad, double dx,
                                                      double dy, double dz, unsigned long long *rate)
 {
-    double r = 0.0;
-    for (int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; c < n; c += (int64_t)gridDim.x * blockDim.x)
-        r = vmax(r, courant_cell(n, c, cons, u, p, ad, dx, dy, dz));
-    block_max_to(r, rate);
+    const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    block_max_to(c < n ? courant_cell(n, c, cons, u, p, ad, dx, dy, dz) : 0.0, max_slot(rate));
 }
 
 // ----------------------------------------------------------------- source
@@ -417,34 +406,42 @@ __global__ __launch_bounds__(kThreads) void k_avisc(int64_t n, int nx, int ny, i
 }
 
 // ------------------------------------------------------------- launchers
-int launch_state(bx_ctx *c)
+int launch_state(bx_ctx *c) { return launch_pass(c, kState, 0.0, true, nullptr); }
+
+static int clear_max(bx_ctx *c)
 {
-    if (c->eos) {  // H2STAT >= 0 (bx_eos.hip)
-        c->ad_uniform = false;
-        return launch_state_tab(c);
-    }
-    hipLaunchKernelGGL(k_state, dim3(blocks_for(c->n, kThreads)), dim3(kThreads), 0, c->stream, c->n, c->cons,
-                       c->u, c->p, c->adindx, c->prm.gammafix, c->prm.small_eps, c->muc, c->rgas);
+    hipLaunchKernelGGL(k_clear_max, dim3(1), dim3(kMaxSlots), 0, c->stream, c->dmax);
     BX_HIP(hipGetLastError());
-    c->ad_uniform = true;
+    return BX_OK;
+}
+
+// The grid-wide maximum of the last kernel that formed one (waits for it).
+int read_max(bx_ctx *c, double *out)
+{
+    BX_HIP(hipMemcpyAsync(c->hmax, c->dmax, sizeof(unsigned long long) * kMaxSlots * kMaxStride, hipMemcpyDeviceToHost,
+                          c->stream));
+    BX_HIP(hipStreamSynchronize(c->stream));
+    unsigned long long m = 0ull;  // non-negative doubles order as their bits
+    for (int i = 0; i < kMaxSlots; i++) m = std::max(m, c->hmax[i * kMaxStride]);
+    std::memcpy(out, &m, sizeof(double));
     return BX_OK;
 }
 
 int launch_velocity(bx_ctx *c, bool want_maxv)
 {
-    if (want_maxv) BX_HIP(hipMemsetAsync(&c->dsc->maxv_bits, 0, sizeof(unsigned long long), c->stream));
-    hipLaunchKernelGGL(k_velocity, dim3(want_maxv ? reduce_blocks(c->n) : blocks_for(c->n, kThreads)), dim3(kThreads), 0, c->stream, c->n,
-                       c->cons, c->u, c->prm.vlimit, c->prm.small_eps,
-                       want_maxv ? &c->dsc->maxv_bits : (unsigned long long *)nullptr);
+    if (want_maxv)
+        if (int rc = clear_max(c)) return rc;
+    hipLaunchKernelGGL(k_velocity, dim3(blocks_for(c->n, kThreads)), dim3(kThreads), 0, c->stream, c->n, c->cons, c->u,
+                       c->prm.vlimit, c->prm.small_eps, want_maxv ? c->dmax : (unsigned long long *)nullptr);
     BX_HIP(hipGetLastError());
     return BX_OK;
 }
 
 int launch_courant(bx_ctx *c)
 {
-    BX_HIP(hipMemsetAsync(&c->dsc->rate_bits[0], 0, sizeof(unsigned long long), c->stream));
-    hipLaunchKernelGGL(k_courant, dim3(reduce_blocks(c->n)), dim3(kThreads), 0, c->stream, c->n, c->cons,
-                       c->u, c->p, c->adindx, c->prm.dx, c->prm.dy, c->prm.dz, &c->dsc->rate_bits[0]);
+    if (int rc = clear_max(c)) return rc;
+    hipLaunchKernelGGL(k_courant, dim3(blocks_for(c->n, kThreads)), dim3(kThreads), 0, c->stream, c->n, c->cons, c->u,
+                       c->p, c->adindx, c->prm.dx, c->prm.dy, c->prm.dz, c->dmax);
     BX_HIP(hipGetLastError());
     return BX_OK;
 }
@@ -478,13 +475,13 @@ int launch_source(bx_ctx *c, double dt)
 // on the device), into the states planes, which then trade places with cons.
 // One kernel in place of face fluxes to memory and an update: 5.5 -> 2.2 ms
 // for the two calls of a step at 256^3.
-static int launch_flux_plain(bx_ctx *c, int avg, double dt)
+static int launch_flux_plain(bx_ctx *c, int avg, double dt, bool ghosts)
 {
     double *out = c->states;
     unsigned int *slow = &c->dsc->slow[c->nflux & 1], *next = &c->dsc->slow[(c->nflux + 1) & 1];
     c->nflux++;
     if (int rc = launch_tiled_flux(c, avg, dt, out, slow, next)) return rc;
-    hipLaunchKernelGGL(k_flux_slow, dim3(reduce_blocks(c->n)), dim3(kThreads), 0, c->stream, slow, c->n, c->nx, c->ny,
+    hipLaunchKernelGGL(k_flux_slow, dim3(std::min(reduce_blocks(c->n), 256u)), dim3(kThreads), 0, c->stream, slow, c->n, c->nx, c->ny,
                        c->nz, c->flatz, c->cons, c->u, c->p, c->adindx, c->cons_old, out, avg, dt, c->prm.dx,
                        c->prm.dy, c->prm.dz, c->prm.small_rho, c->prm.small_eps);
     BX_HIP(hipGetLastError());
@@ -495,12 +492,12 @@ static int launch_flux_plain(bx_ctx *c, int avg, double dt)
         BX_HIP(hipGetLastError());
     }
     std::swap(c->cons, c->states);
-    return launch_ghosts(c, c->cons);
+    return ghosts ? launch_ghosts(c, c->cons) : BX_OK;
 }
 
-int launch_flux(bx_ctx *c, int avg, double dt)
+int launch_flux(bx_ctx *c, int avg, double dt, bool ghosts)
 {
-    if (!c->prm.fluxangmom) return launch_flux_plain(c, avg, dt);
+    if (!c->prm.fluxangmom) return launch_flux_plain(c, avg, dt, ghosts);
     const double dx = c->prm.dx, dy = c->prm.dy, dz = c->prm.dz;
     const dim3 grid(blocks_for(c->n, kThreads));
     hipLaunchKernelGGL(k_ang_to, grid, dim3(kThreads), 0, c->stream, c->n, c->nx, c->ny, c->cons, c->cons_old, avg, dx,
@@ -515,7 +512,7 @@ int launch_flux(bx_ctx *c, int avg, double dt)
                        c->states, c->cons, c->cons_old, avg, dt, areayz, areaxz, areaxy, vol, c->prm.small_rho,
                        c->prm.small_eps, dx, dy, c->prm.yoffset);
     BX_HIP(hipGetLastError());
-    return launch_ghosts(c, c->cons);
+    return ghosts ? launch_ghosts(c, c->cons) : BX_OK;
 }
 
 int launch_avisc(bx_ctx *c)

@@ -13,6 +13,8 @@ namespace bx {
 
 struct HostPipe;
 
+constexpr int kMaxSlots = 32, kMaxStride = 16;  // slots of a grid-wide maximum, and 8-byte words from one to the next
+
 constexpr int kMaxD2 = 64;  // two-level ghost compositions a context may have (one wave)
 
 // The step scalars of main.f90 as a device-dt step leaves them.
@@ -30,7 +32,6 @@ struct StepSlot {
 // and writes the other), so that no workgroup reads what another one writes.
 struct DevScalars {
     unsigned long long rate_bits[2];  // Courant max-rate (non-negative doubles as bits), ping-pong
-    unsigned long long maxv_bits;     // velocity.f90 maxv diagnostic
     unsigned int flags;               // irregular-branch flags raised by the fused kernels
     unsigned int pad;
     StepSlot slot[2];
@@ -139,6 +140,8 @@ struct bx_ctx {
     int64_t stage_len;
     struct bx::HostPipe *pipe;  // pinned slots of large host transfers (bx_transfer.hip), or null
 
+    unsigned long long *dmax, *hmax;  // slots of a grid-wide maximum (bx_cells.h), and their pinned mirror
+
     bx::DevScalars *dsc;   // device scalars
     bx::DevScalars *hsc;   // pinned host mirror
 
@@ -183,10 +186,8 @@ int hip_check(hipError_t e, const char *what);
 // v, w, p, eps, gamma, r- and angular momentum)
 inline int state_planes(const bx_ctx *c) { return c->prm.fluxangmom ? 54 : 5; }
 
-// blocks of a reduction over n cells (256 threads, each taking every
-// gridDim-th 256 cells): few enough that the one atomic per block does not
-// bound the kernel (about 9 ns each on one address: 3,906 blocks at 96^3 took
-// 46 us for a Courant pass that streams in 10)
+// blocks of a reduction over n cells into one word (256 threads, each taking
+// every gridDim-th 256 cells), or of a kernel that mostly has nothing to do
 inline unsigned int reduce_blocks(int64_t n) { return (unsigned int)((n + 255) / 256 < 1024 ? (n + 255) / 256 : 1024); }
 
 inline unsigned int blocks_for(int64_t n, int threads)
@@ -200,7 +201,8 @@ int launch_velocity(bx_ctx *c, bool want_maxv);
 int launch_courant(bx_ctx *c);
 int launch_source(bx_ctx *c, double dt);
 int launch_ghosts(bx_ctx *c, double *planes5);
-int launch_flux(bx_ctx *c, int avg, double dt);
+// ghosts: whether to fill the ghost cells after it (flux.f90:231)
+int launch_flux(bx_ctx *c, int avg, double dt, bool ghosts);
 int launch_tiled_flux(bx_ctx *c, int avg, double dt, double *out, unsigned int *slow, unsigned int *slow_next);
 void tile_split(const bx_ctx *c, bool mixed, bool rows8, bool rows4, int *lz, int *ty);
 int launch_avisc(bx_ctx *c);
@@ -222,7 +224,17 @@ int launch_calc_gforce(bx_ctx *c);
 int launch_external_grav(bx_ctx *c);
 bool grav_settled(const bx_ctx *c);
 int grav_fused_planes(bx_ctx *c);
-int launch_state_tab(bx_ctx *c);
+// the pointwise calls of the exact step in fused passes (bx_pass.hip)
+enum Pass : int {
+    kState = 0,       // state
+    kStateRate = 1,   // state, Courant rate                           main.f90:232-241
+    kAfterFlux = 2,   // (ghosts,) state, velocity                     :351-355
+    kBeforeFlux = 3,  // source, (ghosts,) state, velocity             :289-318
+    kEnd = 4,         // (ghosts,) state, velocity, source, (ghosts,) state, velocity  :374-515
+    kEndNext = 5,     // kEnd, then the next step's kStateRate
+};
+int launch_pass(bx_ctx *c, int pass, double dt, bool filled, double *old);
+int read_max(bx_ctx *c, double *out);
 int fused_prepare(bx_ctx *c);
 // `pairs` pairs of fused steps from the current state (device dt, flags
 // accumulating), replayed from a captured graph (BX_STEP_GRAPH) or enqueued;
