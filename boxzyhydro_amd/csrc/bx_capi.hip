@@ -741,7 +741,7 @@ int bx_flux(bx_ctx *c, int32_t avg, double dt)
     if (avg != 0 && avg != 1) return set_error(BX_ERR_ARG, "bx_flux: avg must be 0 or 1");
     int rc = ensure_aux(c);
     if (rc) return rc;
-    if (!c->states) BX_HIP(hipMalloc((void **)&c->states, sizeof(double) * state_planes(c) * (size_t)c->n));
+    if (!c->states) BX_HIP(hipMalloc((void **)&c->states, sizeof(double) * 5 * (size_t)c->n));
     return launch_flux(c, avg, dt, true);
 }
 
@@ -804,10 +804,10 @@ static int exact_step(bx_ctx *c, double endtime, double *time, double *dtold, in
                       bool started = false, bool *next = nullptr)
 {
     int rc;
-    if (!c->states) BX_HIP(hipMalloc((void **)&c->states, sizeof(double) * state_planes(c) * (size_t)c->n));
-    const bool chained = c->nscratch > 0, ang = c->prm.fluxangmom != 0;
+    if (!c->states) BX_HIP(hipMalloc((void **)&c->states, sizeof(double) * 5 * (size_t)c->n));
+    const bool chained = c->nscratch > 0;
     *step += 1;
-    if (!started && (rc = launch_pass(c, kStateRate, 0.0, true, nullptr))) return rc;  // :232, :241
+    if (!started && (rc = launch_pass(c, kStateRate, 0.0, true))) return rc;  // :232, :241
     double rate;
     if ((rc = read_max(c, &rate))) return rc;
     double dt = c->prm.cfl / rate;
@@ -818,26 +818,23 @@ static int exact_step(bx_ctx *c, double endtime, double *time, double *dtold, in
     if (dt + *time > endtime) dt = endtime - *time;
     dt = dt * 0.5;
     // :289 (+ ghosts, source.f90:199), :312, :314, :318; cons_old (:327-333) is
-    // written by the pass for flux_ang, which works in place, and is otherwise
     // the buffer that flux(0) leaves behind
     if (chained) {
         if ((rc = launch_source(c, dt)) || (rc = ghosts_again(c))) return rc;
-        if ((rc = launch_pass(c, kAfterFlux, 0.0, true, nullptr))) return rc;
-        if (ang)
-            BX_HIP(hipMemcpyAsync(c->cons_old, c->cons, sizeof(double) * 5 * c->n, hipMemcpyDeviceToDevice, c->stream));
-    } else if ((rc = launch_pass(c, kBeforeFlux, dt, false, ang ? c->cons_old : nullptr))) {
+        if ((rc = launch_pass(c, kAfterFlux, 0.0, true))) return rc;
+    } else if ((rc = launch_pass(c, kBeforeFlux, dt, false))) {
         return rc;
     }
     dt = dt * 2.0;
     if ((rc = launch_flux(c, 0, dt, chained))) return rc;  // :346 (+ ghosts, flux.f90:231), :351
-    if (!ang) std::swap(c->cons_old, c->states);
+    std::swap(c->cons_old, c->states);
     if (chained && (rc = ghosts_again(c))) return rc;
-    if ((rc = launch_pass(c, kAfterFlux, 0.0, chained, nullptr))) return rc;
+    if ((rc = launch_pass(c, kAfterFlux, 0.0, chained))) return rc;
     const bool ext = (c->grav_flags & BX_GRAV_EXTERNAL) != 0;  // its mass moments take the ghosts' density
     if ((rc = launch_flux(c, 1, dt, chained || ext))) return rc;  // :368 (+ ghosts, flux.f90:231), :374
     if (chained) {
         if ((rc = ghosts_again(c))) return rc;
-        if ((rc = launch_pass(c, kAfterFlux, 0.0, true, nullptr))) return rc;
+        if ((rc = launch_pass(c, kAfterFlux, 0.0, true))) return rc;
     }
     dt = 0.5 * dt;
     // the state and velocity of :374 change neither density nor force
@@ -846,10 +843,10 @@ static int exact_step(bx_ctx *c, double endtime, double *time, double *dtold, in
     const bool more = next && *next && *time + dt * 2.0 < endtime && *step < 1000000;
     if (chained) {  // :490 (+ ghosts, source.f90:199), :511
         if ((rc = launch_source(c, dt)) || (rc = ghosts_again(c))) return rc;
-        if ((rc = launch_pass(c, kAfterFlux, 0.0, true, nullptr))) return rc;
+        if ((rc = launch_pass(c, kAfterFlux, 0.0, true))) return rc;
         if (next) *next = false;
     } else {
-        if ((rc = launch_pass(c, more ? kEndNext : kEnd, dt, false, nullptr))) return rc;
+        if ((rc = launch_pass(c, more ? kEndNext : kEnd, dt, false))) return rc;
         if (next) *next = more;
     }
     dt = dt * 2.0;

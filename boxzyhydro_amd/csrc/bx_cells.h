@@ -59,9 +59,6 @@ __device__ __forceinline__ int boundary_of(int ix, int iy, int iz, int nx, int n
     return f2 ? 2 : 0;
 }
 
-// centred coordinate of cell index i (1-based) on an axis of n cells (init_grid.f90:85-93)
-__device__ __forceinline__ double centre(double d, int i, int n) { return d * ((double)i - ((double)n + 1.0) / 2.0); }
-
 // One cell of the exact path in registers.
 struct CellState {
     double U[5], v[3], p;
@@ -256,12 +253,24 @@ __device__ __forceinline__ void ghost_fill_one(int64_t n, int64_t k, const int32
 
 // ------------------------------------------ flux: one HLL flux per face
 // The side of cell q in direction d (minus: pm=0, plus: pm=1) exactly as
-// k_flux_states forms it (flux.f90:253-295 slopes, 312-482 states).
-template <int d>
+// the reference forms it (flux.f90:253-295 slopes, 312-482 states).
+// ANG: flux_ang.f90:301-482, with the r- and angular momenta, which get no
+// transverse term.
+struct AngGrid {
+    double dx, dy, yoffset;
+};
+// the centre that flux_ang's momentum transform takes (with yoffset)
+__device__ __forceinline__ AngCentre ang_centre(const AngGrid &g, int64_t c, int nx, int ny)
+{
+    const double x = centre(g.dx, (int)(c % nx) + 1, nx), y = centre(g.dy, (int)((c / nx) % ny) + 1, ny) + g.yoffset;
+    return {x, y, sqrt(x * x + y * y)};
+}
+template <int d, bool ANG = false>
 __device__ __forceinline__ Side<double> cell_side(int64_t q, int pm, int64_t n, int nx, int ny, int nz,
                                                  int64_t stride, const double *__restrict__ cons,
                                                  const double *__restrict__ u, const double *__restrict__ p,
-                                                 const double *__restrict__ ad, double dt, double ds, double seps)
+                                                 const double *__restrict__ ad, double dt, double ds, double seps,
+                                                 const AngGrid &ang = AngGrid{})
 {
     int ix, iy, iz;
     coords(q, nx, ny, ix, iy, iz);
@@ -309,6 +318,18 @@ __device__ __forceinline__ Side<double> cell_side(int64_t q, int pm, int64_t n, 
     sd7.p = o[4] + zc;
     sd7.e = o[5] + zc;
     sd7.g = o[6] + zc;
+    if constexpr (ANG) {
+        double w[3][2];
+        for (int k = -1; k <= 1; k++) {
+            const int64_t e = ghost ? q : q + k * stride;
+            ang_centre(ang, e, nx, ny).to(cons[n + e], cons[2 * n + e], w[k + 1][0], w[k + 1][1]);
+        }
+        double m[2], pp[2];
+        for (int j = 0; j < 2; j++)
+            muscl(w[1][j], lm, lp, ghost ? 0.0 : slope(w[0][j], w[1][j], w[2][j]), m[j], pp[j]);
+        sd7.s1 = pm ? pp[0] : m[0];
+        sd7.s2 = pm ? pp[1] : m[1];
+    }
     return sd7;
 }
 
@@ -375,13 +396,52 @@ __device__ __forceinline__ void face_update_cell(int64_t n, int64_t c, int nx, i
     for (int i = 0; i < 5; i++) cons[(int64_t)i * n + c] = U[i];
 }
 
+// The end of the flux subroutine on one cell with fluxtmp ft (flux.f90:205-228);
+// ANG: in the transformed momenta, back to linear ones, then the floors
+// (flux_ang.f90:223-281).
+template <bool ANG>
+__device__ __forceinline__ void flux_end(int64_t n, int64_t c, int nx, int ny, const double *__restrict__ cons,
+                                         const double *__restrict__ cons_old, double *__restrict__ out, int avg,
+                                         const double *ft, double srho, double seps, const AngGrid &ang)
+{
+    double cu[5], co[5] = {}, U[5];
+    for (int i = 0; i < 5; i++) cu[i] = cons[i * n + c];
+    if (avg)
+        for (int i = 0; i < 5; i++) co[i] = cons_old[i * n + c];
+    AngCentre tr;
+    if constexpr (ANG) {
+        tr = ang_centre(ang, c, nx, ny);
+        double rm, am;
+        tr.to(cu[1], cu[2], rm, am);
+        cu[1] = rm;
+        cu[2] = am;
+        if (avg) {
+            tr.to(co[1], co[2], rm, am);
+            co[1] = rm;
+            co[2] = am;
+        }
+    }
+    for (int i = 0; i < 5; i++) U[i] = avg == 0 ? cu[i] + ft[i] : 0.5 * (co[i] + cu[i] + ft[i]);
+    if constexpr (ANG) {
+        double m1, m2;
+        tr.back(U[1], U[2], m1, m2);
+        U[1] = m1;
+        U[2] = m2;
+    }
+    U[0] = vmax(U[0], srho);
+    if (U[4] < 0.0) U[4] = 0.5 * (U[1] * U[1] + U[2] * U[2] + U[3] * U[3]) / U[0] + seps;
+    for (int i = 0; i < 5; i++) out[i * n + c] = U[i];
+}
+
 // face_update_cell without the face planes: the six faces of an interior cell
-// formed here, from cons, u, p and ad into the out planes
+// formed here, from cons, u, p and ad into the out planes.  ANG: flux_ang.f90.
+template <bool ANG>
 __device__ __forceinline__ void flux_cell(int64_t n, int64_t c, int nx, int ny, int nz, bool flatz,
                                           const double *__restrict__ cons, const double *__restrict__ u,
                                           const double *__restrict__ p, const double *__restrict__ ad,
                                           const double *__restrict__ cons_old, double *__restrict__ out, int avg,
-                                          double dt, double dx, double dy, double dz, double srho, double seps)
+                                          double dt, double dx, double dy, double dz, double srho, double seps,
+                                          const AngGrid &ang)
 {
     int ix, iy, iz;
     coords(c, nx, ny, ix, iy, iz);
@@ -392,9 +452,18 @@ __device__ __forceinline__ void flux_cell(int64_t n, int64_t c, int nx, int ny, 
         double f0[5], f1[5], s[5];
         auto faces = [&](auto dirc, int64_t st, double ds) {
             constexpr int d = decltype(dirc)::value;
-            auto side = [&](int64_t q, int pm) { return cell_side<d>(q, pm, n, nx, ny, nz, st, cons, u, p, ad, dt, ds, seps); };
-            face_flux<double, d>(side(c - st, 1), side(c, 0), f0);
-            face_flux<double, d>(side(c, 1), side(c + st, 0), f1);
+            auto side = [&](int64_t q, int pm) {
+                return cell_side<d, ANG>(q, pm, n, nx, ny, nz, st, cons, u, p, ad, dt, ds, seps, ang);
+            };
+            if constexpr (ANG) {
+                const AngCentre at = ang_centre({dx, dy, 0.0}, c, nx, ny);
+                double g[2];
+                face_flux_ang<d>(side(c - st, 1), side(c, 0), at, at, f0, g);
+                face_flux_ang<d>(side(c, 1), side(c + st, 0), at, at, f1, g);
+            } else {
+                face_flux<double, d>(side(c - st, 1), side(c, 0), f0);
+                face_flux<double, d>(side(c, 1), side(c + st, 0), f1);
+            }
         };
         faces(std::integral_constant<int, 0>{}, 1, dx);
         for (int i = 0; i < 5; i++) s[i] = ayz * (f1[i] - f0[i]);
@@ -403,15 +472,7 @@ __device__ __forceinline__ void flux_cell(int64_t n, int64_t c, int nx, int ny, 
         faces(std::integral_constant<int, 2>{}, sz, dz);
         for (int i = 0; i < 5; i++) ftmp[i] = -((s[i] + axy * (f1[i] - f0[i])) * dt / vol);
     }
-    double U[5];
-    for (int i = 0; i < 5; i++) {
-        const double ft = ftmp[i];
-        const double cu = cons[(int64_t)i * n + c];
-        U[i] = avg == 0 ? cu + ft : 0.5 * (cons_old[(int64_t)i * n + c] + cu + ft);
-    }
-    U[0] = vmax(U[0], srho);
-    if (U[4] < 0.0) U[4] = 0.5 * (U[1] * U[1] + U[2] * U[2] + U[3] * U[3]) / U[0] + seps;
-    for (int i = 0; i < 5; i++) out[(int64_t)i * n + c] = U[i];
+    flux_end<ANG>(n, c, nx, ny, cons, cons_old, out, avg, ftmp, srho, seps, ang);
 }
 
 }  // namespace bx

@@ -262,11 +262,12 @@ int launch_tiled_flux(bx_ctx *c, int avg, double dt, double *out, unsigned int *
     a.gf = nullptr;
     a.flags = slow;
     a.clear = slow_next;
-    // gamma from its plane unless every cell holds gammafix; the seventh field
-    // leaves room in LDS for 64 x 4 tiles only
-    const bool vg = !c->ad_uniform;
+    a.yoffset = c->prm.yoffset;
+    // gamma from its plane unless every cell holds gammafix; a seventh field
+    // (and the eighth and ninth of flux_ang) leaves room in LDS for 64 x 4 tiles
+    const bool vg = !c->ad_uniform, ang = c->prm.fluxangmom != 0;
     int ty = 4;
-    tile_split(c, false, !vg, true, &a.lz, &ty);
+    tile_split(c, false, !vg && !ang, true, &a.lz, &ty);
     const bool p2 = a.ds_pow2[0] && a.ds_pow2[1] && a.ds_pow2[2] && a.vol_pow2;
     const int nzi = a.zhi - a.zlo;
     const dim3 grid((unsigned)((c->nx - 4 + 63) / 64), (unsigned)((c->ny - 4 + ty - 1) / ty),
@@ -286,7 +287,9 @@ int launch_tiled_flux(bx_ctx *c, int avg, double dt, double *out, unsigned int *
         else with_stage(rows, std::false_type{}, kind);
     };
     using Plain = std::integral_constant<int, kPlain>;
-    if (vg) with_spacing(std::integral_constant<int, 4>{}, std::integral_constant<int, kGamma>{});
+    if (ang && vg) with_spacing(std::integral_constant<int, 4>{}, std::integral_constant<int, kAngGamma>{});
+    else if (ang) with_spacing(std::integral_constant<int, 4>{}, std::integral_constant<int, kAng>{});
+    else if (vg) with_spacing(std::integral_constant<int, 4>{}, std::integral_constant<int, kGamma>{});
     else if (ty == 8) with_spacing(std::integral_constant<int, 8>{}, Plain{});
     else with_spacing(std::integral_constant<int, 4>{}, Plain{});
     BX_HIP(hipGetLastError());

@@ -68,8 +68,7 @@ struct bx_ctx {
     double *p;
     double *adindx;
     double *qq;        // 3 planes
-    double *states;    // exact-flux output or intermediate, state_planes(c) planes (the flux's result, which
-                       // trades places with cons; with flux_ang the interface states)
+    double *states;    // 5 planes: the exact flux's result, which trades places with cons
     bool ad_uniform;   // every cell of adindx holds gammafix
     unsigned nflux;    // tiled flux calls so far (parity: which slow word a call uses)
     int ncu;           // compute units of the device
@@ -181,11 +180,6 @@ int hip_check(hipError_t e, const char *what);
         if (_e != hipSuccess) return bx::hip_check(_e, #call);   \
     } while (0)
 
-// planes of the exact flux's output (5 conserved planes); with flux_ang of its
-// intermediate, the interface states, per direction 9 minus + 9 plus (rho, u,
-// v, w, p, eps, gamma, r- and angular momentum)
-inline int state_planes(const bx_ctx *c) { return c->prm.fluxangmom ? 54 : 5; }
-
 // blocks of a reduction over n cells into one word (256 threads, each taking
 // every gridDim-th 256 cells), or of a kernel that mostly has nothing to do
 inline unsigned int reduce_blocks(int64_t n) { return (unsigned int)((n + 255) / 256 < 1024 ? (n + 255) / 256 : 1024); }
@@ -233,7 +227,7 @@ enum Pass : int {
     kEnd = 4,         // (ghosts,) state, velocity, source, (ghosts,) state, velocity  :374-515
     kEndNext = 5,     // kEnd, then the next step's kStateRate
 };
-int launch_pass(bx_ctx *c, int pass, double dt, bool filled, double *old);
+int launch_pass(bx_ctx *c, int pass, double dt, bool filled);
 int read_max(bx_ctx *c, double *out);
 int fused_prepare(bx_ctx *c);
 // `pairs` pairs of fused steps from the current state (device dt, flags

@@ -134,6 +134,7 @@ struct Prim {
 template <typename T>
 struct Side {
     T d, v[3], p, e, g;
+    T s1, s2;  // flux_ang: r- and angular momentum; elsewhere unused
 };
 
 // flux.f90:299-308 interface_muscl
@@ -240,6 +241,82 @@ __device__ __forceinline__ void face_flux(const Side<T> &L, const Side<T> &R, T 
             F[i] = Arith<T>::div(num, den);
         }
     }
+}
+
+// centred coordinate of cell index i (1-based) on an axis of n cells (init_grid.f90:85-93)
+__device__ __forceinline__ double centre(double d, int i, int n) { return d * ((double)i - ((double)n + 1.0) / 2.0); }
+
+// flux_ang.f90:523-618 (get_fluxes_ang) for one face: the momentum slots carry
+// the reconstructed r- and angular momenta, and the pressure force is projected
+// with the centre (x, y, r) of the cell whose flux it is: the cell above the
+// face (F, all five) and the cell below it (G, the two momentum slots; the
+// others are F's).  Along z there is no projection and G is F's.
+struct AngCentre {
+    double x, y, r;
+    // flux_ang.f90:40-61: linear momenta to r- and angular momentum
+    __device__ __forceinline__ void to(double m1, double m2, double &rm, double &am) const
+    {
+        am = x * m2 - y * m1;
+        rm = (m1 * x + m2 * y) / r;
+    }
+    // flux_ang.f90:245-268: and back
+    __device__ __forceinline__ void back(double rm, double am, double &m1, double &m2) const
+    {
+        m1 = (rm * x - am * y / r) / r;
+        m2 = (rm * y + am * x / r) / r;
+    }
+};
+template <int dir>
+__device__ __forceinline__ void face_flux_ang(const Side<double> &L, const Side<double> &R, const AngCentre &up,
+                                              const AngCentre &below, double F[5], double G[2])
+{
+    const double sl[5] = {L.d, L.s1, L.s2, L.d * L.v[2],
+                          L.e + 0.5 * L.d * (L.v[0] * L.v[0] + L.v[1] * L.v[1] + L.v[2] * L.v[2])};
+    const double sr[5] = {R.d, R.s1, R.s2, R.d * R.v[2],
+                          R.e + 0.5 * R.d * (R.v[0] * R.v[0] + R.v[1] * R.v[1] + R.v[2] * R.v[2])};
+    const double vl = L.v[dir], vr = R.v[dir];
+    // flux_hll, flux.f90:583-589
+    const double sq[2] = {R.g * R.p / R.d, L.g * L.p / L.d};
+    double rt[2];
+    sqrt_n<2>(sq, rt);
+    const double ap = vmax(vmax(0.0, vr + rt[0]), vl + rt[1]);
+    const double am = vmax(vmax(0.0, -(vr - rt[0])), -(vl - rt[1]));
+    const double apam = ap * am;
+    auto numerator = [&](int i, double pl, double pr) {
+        const double fl = pl + sl[i] * vl, fr = pr + sr[i] * vr;
+        return ap * fl + am * fr - apam * (sr[i] - sl[i]);
+    };
+    auto momenta = [&](const AngCentre &c, double num[2]) {
+        double pl1 = 0.0, pl2 = 0.0, pr1 = 0.0, pr2 = 0.0;
+        if (dir < 2) {
+            const double q[2] = {L.p * (dir == 0 ? c.x : c.y), R.p * (dir == 0 ? c.x : c.y)};
+            double o[2];
+            div_shared<2>(q, c.r, o);
+            pl1 = o[0];
+            pr1 = o[1];
+            pl2 = dir == 0 ? -(L.p * c.y) : L.p * c.x;
+            pr2 = dir == 0 ? -(R.p * c.y) : R.p * c.x;
+        }
+        num[0] = numerator(1, pl1, pr1);
+        num[1] = numerator(2, pl2, pr2);
+    };
+    double num[7];
+    num[0] = ap * (sl[0] * vl) + am * (sr[0] * vr) - apam * (sr[0] - sl[0]);
+    momenta(up, num + 1);
+    num[3] = numerator(3, dir == 2 ? L.p : 0.0, dir == 2 ? R.p : 0.0);
+    num[4] = ap * ((sl[4] + L.p) * vl) + am * ((sr[4] + R.p) * vr) - apam * (sr[4] - sl[4]);
+    double q[7];
+    if constexpr (dir < 2) {
+        momenta(below, num + 5);
+        div_shared<7>(num, ap + am, q);
+        G[0] = q[5];
+        G[1] = q[6];
+    } else {
+        div_shared<5>(num, ap + am, q);
+        G[0] = q[1];
+        G[1] = q[2];
+    }
+    for (int i = 0; i < 5; i++) F[i] = q[i];
 }
 
 }  // namespace bx

@@ -31,7 +31,6 @@ struct PassArgs {
     int64_t n;
     int nx, ny, nz;
     double *cons, *u, *p, *ad, *mucp;  // ad: null where every cell already holds gamma; mucp: tabulated EOS
-    double *old;                       // kBeforeFlux: receives cons (main.f90:327-333); may be null
     double gam, seps, muc, rgas, vlimit, dt;
     double g0, g1, g2;
     const double *gf;
@@ -118,8 +117,6 @@ __device__ __forceinline__ void store_cell(const PassArgs &a, int64_t c, const C
     a.p[c] = x.p;
     if (TAB || a.ad) a.ad[c] = ad;
     if constexpr (TAB) a.mucp[c] = mu;
-    if (PASS == kBeforeFlux && a.old)
-        for (int f = 0; f < 5; f++) a.old[f * a.n + c] = x.U[f];
 }
 
 // Each thread takes CPT cells a block apart (coalesced), so that the table
@@ -219,7 +216,7 @@ __global__ __launch_bounds__(kPassThreads) void k_pass_ghosts(PassArgs a, int64_
     if (PASS == kEndNext) block_max_to(rate, max_slot(a.rate));
 }
 
-static PassArgs pass_args(bx_ctx *c, double dt, bool all, double *old)
+static PassArgs pass_args(bx_ctx *c, double dt, bool all)
 {
     PassArgs a{};
     a.n = c->n;
@@ -230,7 +227,6 @@ static PassArgs pass_args(bx_ctx *c, double dt, bool all, double *old)
     a.u = c->u;
     a.p = c->p;
     a.ad = !c->eos && c->ad_uniform ? nullptr : c->adindx;
-    a.old = old;
     a.gam = c->prm.gammafix;
     a.seps = c->prm.small_eps;
     a.muc = c->muc;
@@ -287,13 +283,13 @@ static void go_ghosts(bx_ctx *c, int pass, const PassArgs &a)
 // A pass over every cell.  `filled`: the ghosts hold what the sequence's fill
 // gives them (kState, kStateRate, or kAfterFlux after the fills); otherwise the
 // pass fills them (no chained ghosts).
-int launch_pass(bx_ctx *c, int pass, double dt, bool filled, double *old)
+int launch_pass(bx_ctx *c, int pass, double dt, bool filled)
 {
     if (pass == kEndNext || pass == kStateRate) {
         hipLaunchKernelGGL(k_clear_max, dim3(1), dim3(kMaxSlots), 0, c->stream, c->dmax);
         BX_HIP(hipGetLastError());
     }
-    const PassArgs a = pass_args(c, dt, filled, old);
+    const PassArgs a = pass_args(c, dt, filled);
     if (!filled && c->nghost > 0) {
         if (c->eos) go_ghosts<true>(c, pass, a);
         else go_ghosts<false>(c, pass, a);

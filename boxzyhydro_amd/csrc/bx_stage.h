@@ -75,6 +75,7 @@ struct StageArgs {
     // cons_old and p, uout receives the updated interior cells
     const double *vel, *ad;
     unsigned int *clear;  // a word the first lane of the grid clears (may be null)
+    double yoffset;  // flux_ang: y shift of the momentum transform
 };
 
 // One step's scalars on the device, in the operations of the host driver
@@ -149,7 +150,8 @@ StageArgs base_args(bx_ctx *c, double dt);
 template <typename T>
 struct W6 {
     T d, u0, u1, u2, p, e;
-    T g;  // gamma, where it varies from cell to cell (StageKind kGamma); elsewhere unused
+    T g;       // gamma, where it varies from cell to cell (has_gamma); elsewhere unused
+    T rm, am;  // r- and angular momentum (has_ang); elsewhere unused
 };
 
 // What a stage kernel carries beside the plain fixed-gamma flux of a regular
@@ -158,7 +160,11 @@ enum StageKind : int {
     kPlain = 0,
     kGravity = 1,  // stages 1 and 2: the kick of source() with the force planes gf (FP64)
     kGamma = 2,    // stages 3 and 4: gamma from the plane ad, reconstructed as the other primitives
+    kAng = 3,      // stages 3 and 4: flux_ang, r- and angular momentum reconstructed and fluxed
+    kAngGamma = 4, // both
 };
+constexpr bool has_gamma(int v) { return v == kGamma || v == kAngGamma; }
+constexpr bool has_ang(int v) { return v == kAng || v == kAngGamma; }
 
 template <typename T>
 __device__ __forceinline__ T div_by(T x, double d, double inv, int pow2)
@@ -226,6 +232,8 @@ __device__ __forceinline__ W6<T> wave_shift_w(const W6<T> &w)
     o.p = wave_shift_t<CTRL>(w.p, w.p);
     o.e = wave_shift_t<CTRL>(w.e, w.e);
     o.g = wave_shift_t<CTRL>(w.g, w.g);
+    o.rm = wave_shift_t<CTRL>(w.rm, w.rm);
+    o.am = wave_shift_t<CTRL>(w.am, w.am);
     return o;
 }
 template <typename T>
@@ -249,7 +257,7 @@ __device__ __forceinline__ T comp(const W6<T> &w, int j)
 // finite slopes of finite data).  lp and lm enter only as 1-lp and -1-lm,
 // where a zero of either sign gives the same value, so the hardware maximum
 // and minimum stand for vmax/vmin against 0.
-template <int d, typename T, bool VG = false>
+template <int d, typename T, int V = kPlain>
 __device__ __forceinline__ void dir_states(const W6<T> &wm, const W6<T> &wc, const W6<T> &wp, T sound, bool ghost,
                                            const StageArgs &a, Side<T> &mi, Side<T> &pl)
 {
@@ -278,7 +286,7 @@ __device__ __forceinline__ void dir_states(const W6<T> &wm, const W6<T> &wc, con
     pl.p = p0 + cp * sp;
     mi.e = e0 + cm * se;
     pl.e = e0 + cp * se;
-    if constexpr (VG) {
+    if constexpr (has_gamma(V)) {
         const T sg = slope_fz(wm.g, wc.g, wp.g);
         const T g0 = wc.g + z;
         mi.g = g0 + cm * sg;
@@ -286,6 +294,17 @@ __device__ __forceinline__ void dir_states(const W6<T> &wm, const W6<T> &wc, con
     } else {
         mi.g = T(a.gam);  // slope(gamma,gamma,gamma)=0: gamma + (+-0) + 0 = gamma
         pl.g = T(a.gam);
+    }
+    if constexpr (has_ang(V)) {
+        // flux_ang.f90:319-320, 377-380: no transverse term follows, so a zero
+        // keeps its sign: the slope's zero is +0 and a ghost's slope is it
+        const T s1 = ghost ? T(0) : slope_finite(wm.rm, wc.rm, wp.rm);
+        const T s2 = ghost ? T(0) : slope_finite(wm.am, wc.am, wp.am);
+        const T tm = T(0.5) * (T(-1) - lm), tp = T(0.5) * (T(1) - lp);
+        mi.s1 = wc.rm + tm * s1;
+        pl.s1 = wc.rm + tp * s1;
+        mi.s2 = wc.am + tm * s2;
+        pl.s2 = wc.am + tp * s2;
     }
 }
 
@@ -307,7 +326,7 @@ __device__ __forceinline__ T sound_of(const W6<T> &w, double gam)
 template <typename S>
 struct Raw {
     S r, m0, m1, m2, E, p;
-    S g0, g1, g2;  // stage 1 with gravity: the cell's force; kGamma: g0 is gamma
+    S g0, g1, g2;  // stage 1 with gravity: the cell's force; has_gamma: g0 is gamma; has_ang: g1, g2 the x and y momenta
 };
 
 // cell = uniform element offset u + per-lane byte offset boff
@@ -323,7 +342,11 @@ __device__ __forceinline__ Raw<S> load_raw(const StageArgs &a, int64_t u, unsign
         v.m1 = elem<S>(a.vel, n + u, boff);
         v.m2 = elem<S>(a.vel, 2 * n + u, boff);
         v.p = elem<S>(a.pin, u, boff);
-        if constexpr (V == kGamma) v.g0 = elem<S>(a.ad, u, boff);
+        if constexpr (has_gamma(V)) v.g0 = elem<S>(a.ad, u, boff);
+        if constexpr (has_ang(V)) {
+            v.g1 = elem<S>(a.uin, n + u, boff);
+            v.g2 = elem<S>(a.uin, 2 * n + u, boff);
+        }
         return v;
     }
     v.r = elem<S>(a.uin, u, boff);
@@ -371,7 +394,7 @@ template <int STAGE, typename S, int V = kPlain>
 __device__ __forceinline__ W6<S> prims(const StageArgs &a, const Raw<S> &v, unsigned int &flg)
 {
     W6<S> w;
-    w.g = S(0);
+    w.g = w.rm = w.am = S(0);
     if constexpr (STAGE >= 3) {
         static_assert(sizeof(S) == 8, "the exact path is FP64");
         w.d = v.r;
@@ -380,8 +403,9 @@ __device__ __forceinline__ W6<S> prims(const StageArgs &a, const Raw<S> &v, unsi
         w.u2 = v.m2;
         w.p = v.p;
         w.e = floor_at(v.E - 0.5 * v.r * (v.m0 * v.m0 + v.m1 * v.m1 + v.m2 * v.m2), a.seps);
-        if constexpr (V == kGamma) w.g = v.g0;
-        const double mag = ((fabs(v.r) + fabs(v.E)) + (fabs(v.m0) + fabs(v.m1))) + ((fabs(v.m2) + fabs(v.p)) + fabs(w.g));
+        if constexpr (has_gamma(V)) w.g = v.g0;
+        double mag = ((fabs(v.r) + fabs(v.E)) + (fabs(v.m0) + fabs(v.m1))) + ((fabs(v.m2) + fabs(v.p)) + fabs(w.g));
+        if constexpr (has_ang(V)) mag += fabs(v.g1) + fabs(v.g2);
         if (!(mag <= 1e60) || !(v.r > 0.0) || !(v.p > 0.0)) flg |= FLAG_SLOW;
     } else if constexpr (V == kGravity && STAGE == 1) {
         static_assert(sizeof(S) == 8, "gravity is FP64 only");
@@ -463,7 +487,7 @@ __device__ __forceinline__ W6<S> load_prims(const StageArgs &a, int64_t u, unsig
 template <int V, typename T>
 __device__ __forceinline__ T sound_at(const W6<T> &w, const StageArgs &a)
 {
-    if constexpr (V == kGamma) {
+    if constexpr (has_gamma(V)) {
         const double x = w.p * w.g / w.d;
         double r;
         sqrt_n<1>(&x, &r);

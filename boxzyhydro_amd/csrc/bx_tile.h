@@ -48,7 +48,9 @@
 // per step (4.6 us each on small grids, 33 us each at 256^3).
 // Stages 3 and 4 are the flux subroutine of the exact path (flux(0), flux(1)):
 // the same march over the planes cons, u, p (and adindx) as they stand, ghosts
-// from memory, ending with flux.f90:205-228.
+// from memory, ending with flux.f90:205-228.  With flux_ang (has_ang) two more
+// fields are reconstructed, and each x and y face is projected twice, for the
+// cell above and the cell below it.
 // Every arithmetic operation is the one the exact sequence performs on the
 // same values, so the results are bit-identical to it.
 #pragma once
@@ -63,8 +65,8 @@ namespace bx {
 template <typename S, int TY, int V = kPlain>
 struct TileLds {
     static constexpr int RS = 66;  // row stride of the primitive tile: columns -1..64
-    static constexpr int NF = V == kGamma ? 7 : 6;
-    S P[2][NF][(TY + 4) * RS];     // rho, u0, u1, u2, p, eps (, gamma) of planes k, k+1 (tile k&1), rows -2..TY+1
+    static constexpr int NF = 6 + (has_gamma(V) ? 1 : 0) + (has_ang(V) ? 2 : 0);
+    S P[2][NF][(TY + 4) * RS];     // rho, u0, u1, u2, p, eps (, gamma) (, r- and angular momentum) of planes k, k+1 (tile k&1), rows -2..TY+1
     S Sy[NF][(TY + 1) * 64];       // y-plus states of rows -1..TY-1 (index r+1), then y-face r-1/2 (index r)
     S SxL[NF][TY];                 // x-plus state of column -1, per owner row
     S FxR[5][TY];                  // x-face flux 63+1/2, per owner row
@@ -75,7 +77,11 @@ struct TileLds {
 template <typename S, int F, int N>
 __device__ __forceinline__ void store_w(S (&P)[F][N], int idx, const W6<S> &w)
 {
-    if constexpr (F == 7) P[F - 1][idx] = w.g;
+    if constexpr (F == 7 || F == 9) P[6][idx] = w.g;
+    if constexpr (F >= 8) {
+        P[F - 2][idx] = w.rm;
+        P[F - 1][idx] = w.am;
+    }
     P[0][idx] = w.d;
     P[1][idx] = w.u0;
     P[2][idx] = w.u1;
@@ -88,8 +94,12 @@ template <typename S, int F, int N>
 __device__ __forceinline__ W6<S> fetch_w(const S (&P)[F][N], int idx)
 {
     W6<S> w;
-    w.g = S(0);
-    if constexpr (F == 7) w.g = P[F - 1][idx];
+    w.g = w.rm = w.am = S(0);
+    if constexpr (F == 7 || F == 9) w.g = P[6][idx];
+    if constexpr (F >= 8) {
+        w.rm = P[F - 2][idx];
+        w.am = P[F - 1][idx];
+    }
     w.d = P[0][idx];
     w.u0 = P[1][idx];
     w.u1 = P[2][idx];
@@ -102,7 +112,11 @@ __device__ __forceinline__ W6<S> fetch_w(const S (&P)[F][N], int idx)
 template <typename S, int F, int N>
 __device__ __forceinline__ void store_side(S (&B)[F][N], int idx, const Side<S> &s)
 {
-    if constexpr (F == 7) B[F - 1][idx] = s.g;
+    if constexpr (F == 7 || F == 9) B[6][idx] = s.g;
+    if constexpr (F >= 8) {
+        B[F - 2][idx] = s.s1;
+        B[F - 1][idx] = s.s2;
+    }
     B[0][idx] = s.d;
     B[1][idx] = s.v[0];
     B[2][idx] = s.v[1];
@@ -122,7 +136,11 @@ __device__ __forceinline__ Side<S> fetch_side(const S (&B)[F][N], int idx, S gam
     s.p = B[4][idx];
     s.e = B[5][idx];
     s.g = gam;
-    if constexpr (F == 7) s.g = B[F - 1][idx];
+    if constexpr (F == 7 || F == 9) s.g = B[6][idx];
+    if constexpr (F >= 8) {
+        s.s1 = B[F - 2][idx];
+        s.s2 = B[F - 1][idx];
+    }
     return s;
 }
 
@@ -187,6 +205,45 @@ struct Donor {
     }
 };
 
+// flux_ang: a column's centre as the transform of the momenta takes it (with
+// yoffset) and as the pressure projection does (without), for the column and
+// its lower neighbours in x and y.
+template <int V>
+struct AngColumn {
+    AngCentre at, lowx, lowy;  // projection (get_fluxes_ang: no yoffset)
+    AngCentre tr;              // transform
+    __device__ __forceinline__ AngColumn(const StageArgs &a, int x, int y)
+    {
+        if constexpr (has_ang(V)) {
+            const double cx = centre(a.ds[0], x + 1, a.nx), cy = centre(a.ds[1], y + 1, a.ny);
+            const double lx = centre(a.ds[0], x, a.nx), ly = centre(a.ds[1], y, a.ny), ty = cy + a.yoffset;
+            at = {cx, cy, sqrt(cx * cx + cy * cy)};
+            lowx = {lx, cy, sqrt(lx * lx + cy * cy)};
+            lowy = {cx, ly, sqrt(cx * cx + ly * ly)};
+            tr = {cx, ty, sqrt(cx * cx + ty * ty)};
+        }
+    }
+    // the cell's r- and angular momentum; outside the finite slopes' range the
+    // call goes to the cell-by-cell kernel
+    template <typename S>
+    __device__ __forceinline__ void momenta(const Raw<S> &v, W6<S> &w, unsigned int &flg) const
+    {
+        if constexpr (has_ang(V)) {
+            tr.to(v.g1, v.g2, w.rm, w.am);
+            if (!(fabs(w.rm) + fabs(w.am) <= 1e60)) flg |= FLAG_SLOW;
+        }
+    }
+};
+
+// the flux of a face for the cell above it (F) and, with flux_ang, the two
+// momentum fluxes of the cell below it (G)
+template <typename S, int dir, int V>
+__device__ __forceinline__ void stage_face(const Side<S> &L, const Side<S> &R, const AngColumn<V> &col, S F[5], S G[2])
+{
+    if constexpr (has_ang(V)) face_flux_ang<dir>(L, R, col.at, dir == 0 ? col.lowx : col.lowy, F, G);
+    else face_flux<S, dir>(L, R, F);
+}
+
 // Per-tile constants of one stage.
 struct TileGeom {
     int nx, ny, nz;
@@ -197,12 +254,28 @@ struct TileGeom {
 
 // The end of the flux subroutine at an interior cell (flux.f90:205-228): the
 // stage update with fluxtmp ft and the floors.
-template <int STAGE>
-__device__ __forceinline__ void flux_update(const StageArgs &a, const double ui[5], const double uo[5],
-                                            const double ft[5], int64_t c, unsigned coff)
+template <int STAGE, int V>
+__device__ __forceinline__ void flux_update(const StageArgs &a, double ui[5], double uo[5], const double ft[5],
+                                            const W6<double> &q0, const AngColumn<V> &col, int64_t c, unsigned coff)
 {
     double U[5];
+    if constexpr (has_ang(V)) {
+        ui[1] = q0.rm;
+        ui[2] = q0.am;
+        if (STAGE == 4) {
+            double rm, am;
+            col.tr.to(uo[1], uo[2], rm, am);
+            uo[1] = rm;
+            uo[2] = am;
+        }
+    }
     for (int i = 0; i < 5; i++) U[i] = STAGE == 3 ? ui[i] + ft[i] : 0.5 * (uo[i] + ui[i] + ft[i]);
+    if constexpr (has_ang(V)) {
+        double m1, m2;
+        col.tr.back(U[1], U[2], m1, m2);
+        U[1] = m1;
+        U[2] = m2;
+    }
     U[0] = floor_at(U[0], a.srho);
     if (U[4] < 0.0) U[4] = 0.5 * (U[1] * U[1] + U[2] * U[2] + U[3] * U[3]) / U[0] + a.seps;
     for (int i = 0; i < 5; i++) elem<double>(a.uout, (int64_t)i * a.n + c, coff) = U[i];
@@ -222,6 +295,7 @@ __device__ __forceinline__ void tile_owner(const StageArgs &a, TileLds<S, TY, V>
     const int x = g.x0 + lane, y = g.j0 + r;
     const Donor<S, W> me(a, x, y);
     const unsigned coff = me.off;
+    const AngColumn<V> col(a, min(x, nx - 1), min(y, ny - 1));
     const bool xy_ghost = x < 2 || x > nx - 3 || y < 2 || y > ny - 3;
     const bool is_out = !xy_ghost;
     const S gamS = S(a.gam);
@@ -238,24 +312,29 @@ __device__ __forceinline__ void tile_owner(const StageArgs &a, TileLds<S, TY, V>
     const int kb = g.kb, ke = g.ke;
     if (!a.flatz) {
         auto at = [&](int k) -> W6<S> {
-            W6<S> w = load_prims<STAGE, S, V>(a, zplane(k), coff, flg);
+            const Raw<S> v = load_raw<STAGE, S, V>(a, zplane(k), coff);
+            W6<S> w = prims<STAGE, S, V>(a, v, flg);
             me.signs(a, k, w);
+            col.momenta(v, w, flg);
             return w;
         };
         const W6<S> t0 = at(kb - 2), t1 = at(kb - 1), t2 = at(kb), t3 = at(kb + 1);
         Side<S> zmi, zpl;
-        dir_states<2, S, V == kGamma>(t0, t1, t2, sound_at<V>(t1, a), xy_ghost || zghost(kb - 1), a, zmi, zpl);
+        dir_states<2, S, V>(t0, t1, t2, sound_at<V>(t1, a), xy_ghost || zghost(kb - 1), a, zmi, zpl);
         zp_prev = zpl;
         cs1 = sound_at<V>(t2, a);
-        dir_states<2, S, V == kGamma>(t1, t2, t3, cs1, xy_ghost || zghost(kb), a, zmi, zpl);
-        face_flux<S, 2>(zp_prev, zmi, Fz_prev);
+        dir_states<2, S, V>(t1, t2, t3, cs1, xy_ghost || zghost(kb), a, zmi, zpl);
+        S gz[2];
+        stage_face<S, 2, V>(zp_prev, zmi, col, Fz_prev, gz);
         zp_prev = zpl;
         store_w(L.P[kb & 1], c, t2);  // plane kb
         q2 = t3;
         nxt = load_raw<STAGE, S, V>(a, zplane(kb + 2), coff);
     } else {
-        W6<S> w = load_prims<STAGE, S, V>(a, zplane(kb), coff, flg);
+        const Raw<S> v = load_raw<STAGE, S, V>(a, zplane(kb), coff);
+        W6<S> w = prims<STAGE, S, V>(a, v, flg);
         me.signs(a, kb, w);
+        col.momenta(v, w, flg);
         cs1 = sound_at<V>(w, a);
         store_w(L.P[kb & 1], c, w);
         if (kb + 1 < ke) nxt = load_raw<STAGE, S, V>(a, zplane(kb + 1), coff);
@@ -276,11 +355,12 @@ __device__ __forceinline__ void tile_owner(const StageArgs &a, TileLds<S, TY, V>
             nxt = load_raw<STAGE, S, V>(a, zplane(min(k + 3, nz - 1)), coff);
             q2 = prims<STAGE, S, V>(a, cur, flg);
             me.signs(a, k + 2, q2);
+            col.momenta(cur, q2, flg);
             cs1 = sound_at<V>(q1, a);
             Side<S> zmi1, zpl1;
-            dir_states<2, S, V == kGamma>(fetch_w(L.P[t], c), q1, q2, cs1, xy_ghost || zghost(k + 1), a, zmi1, zpl1);
-            S Fz1[5];
-            face_flux<S, 2>(zp_prev, zmi1, Fz1);
+            dir_states<2, S, V>(fetch_w(L.P[t], c), q1, q2, cs1, xy_ghost || zghost(k + 1), a, zmi1, zpl1);
+            S Fz1[5], gz[2];
+            stage_face<S, 2, V>(zp_prev, zmi1, col, Fz1, gz);
             for (int i = 0; i < 5; i++) {
                 L.Dz[i][o] = (double)Fz1[i] - (double)Fz_prev[i];
                 Fz_prev[i] = Fz1[i];
@@ -294,6 +374,7 @@ __device__ __forceinline__ void tile_owner(const StageArgs &a, TileLds<S, TY, V>
                 nxt = load_raw<STAGE, S, V>(a, zplane(min(k + 2, ke - 1)), coff);
                 W6<S> w = prims<STAGE, S, V>(a, cur, flg);
                 me.signs(a, k + 1, w);
+                col.momenta(cur, w, flg);
                 cs1 = sound_at<V>(w, a);
                 store_w(L.P[t ^ 1], c, w);
             }
@@ -302,7 +383,7 @@ __device__ __forceinline__ void tile_owner(const StageArgs &a, TileLds<S, TY, V>
         {
             const W6<S> q0 = fetch_w(L.P[t], c);
             Side<S> xmi, xpl;
-            dir_states<0, S, V == kGamma>(fetch_w(L.P[t], c - 1), q0, fetch_w(L.P[t], c + 1), cs0, ghost_k, a, xmi, xpl);
+            dir_states<0, S, V>(fetch_w(L.P[t], c - 1), q0, fetch_w(L.P[t], c + 1), cs0, ghost_k, a, xmi, xpl);
             Side<S> xl;
             xl.d = from_lower(xpl.d, L.SxL[0][r], lane);
             xl.v[0] = from_lower(xpl.v[0], L.SxL[1][r], lane);
@@ -311,26 +392,33 @@ __device__ __forceinline__ void tile_owner(const StageArgs &a, TileLds<S, TY, V>
             xl.p = from_lower(xpl.p, L.SxL[4][r], lane);
             xl.e = from_lower(xpl.e, L.SxL[5][r], lane);
             xl.g = gamS;
-            if constexpr (V == kGamma) xl.g = from_lower(xpl.g, L.SxL[TileLds<S, TY, V>::NF - 1][r], lane);
-            S Fx0[5];
-            face_flux<S, 0>(xl, xmi, Fx0);  // face l-1/2
+            constexpr int NF = TileLds<S, TY, V>::NF;
+            if constexpr (has_gamma(V)) xl.g = from_lower(xpl.g, L.SxL[6][r], lane);
+            if constexpr (has_ang(V)) {
+                xl.s1 = from_lower(xpl.s1, L.SxL[NF - 2][r], lane);
+                xl.s2 = from_lower(xpl.s2, L.SxL[NF - 1][r], lane);
+            }
+            S Fx0[5], gx[2];
+            stage_face<S, 0, V>(xl, xmi, col, Fx0, gx);  // face l-1/2
             for (int i = 0; i < 5; i++) {
-                const S fx1 = from_upper(Fx0[i], L.FxR[i][r], lane);  // face l+1/2
+                // face l+1/2, as this cell has it
+                const S fx1 = from_upper(has_ang(V) && (i == 1 || i == 2) ? gx[i - 1] : Fx0[i], L.FxR[i][r], lane);
                 L.Dx[i][o] = (double)fx1 - (double)Fx0[i];
             }
         }
         Side<S> ymi;
         {
             Side<S> ypl;
-            dir_states<1, S, V == kGamma>(fetch_w(L.P[t], c - RS), fetch_w(L.P[t], c), fetch_w(L.P[t], c + RS), cs0, ghost_k, a,
+            dir_states<1, S, V>(fetch_w(L.P[t], c - RS), fetch_w(L.P[t], c), fetch_w(L.P[t], c + RS), cs0, ghost_k, a,
                           ymi, ypl);
             store_side(L.Sy, (r + 1) * 64 + lane, ypl);
         }
         __syncthreads();
         // C: face y r-1/2, published over the y-plus state of row r-1
-        S Fy0[5];
-        face_flux<S, 1>(fetch_side(L.Sy, r * 64 + lane, gamS), ymi, Fy0);
-        for (int i = 0; i < 5; i++) L.Sy[i][r * 64 + lane] = Fy0[i];
+        S Fy0[5], gy[2];
+        stage_face<S, 1, V>(fetch_side(L.Sy, r * 64 + lane, gamS), ymi, col, Fy0, gy);
+        for (int i = 0; i < 5; i++)  // as row r-1 has it
+            L.Sy[i][r * 64 + lane] = has_ang(V) && (i == 1 || i == 2) ? gy[i - 1] : Fy0[i];
         __syncthreads();
         // D: face y r+1/2 and the update
         if (is_out) {
@@ -348,7 +436,7 @@ __device__ __forceinline__ void tile_owner(const StageArgs &a, TileLds<S, TY, V>
                 const double s = (a.ayz * L.Dx[i][o] + ey) + a.axy * dz;
                 ft[i] = -div_by(s * a.dt, a.vol, a.inv_vol, a.vol_pow2);
             }
-            if constexpr (STAGE >= 3) flux_update<STAGE>(a, ui, uo, ft, cz, coff);
+            if constexpr (STAGE >= 3) flux_update<STAGE, V>(a, ui, uo, ft, fetch_w(L.P[t], c), col, cz, coff);
             else stage_update<STAGE, S, V == kGravity>(a, ui, uo, ft, fetch_w(L.P[t], c), cz, coff, flg, rmax);
         }
     }
@@ -365,6 +453,7 @@ __device__ __forceinline__ void tile_halo(const StageArgs &a, TileLds<S, TY, V> 
     const int x = g.x0 + lane, y = g.j0 + r;
     const Donor<S, W> me(a, x, y);
     const unsigned coff = me.off;
+    const AngColumn<V> col(a, min(x, nx - 1), min(y, ny - 1));
     const bool xy_ghost = x < 2 || x > nx - 3 || y < 2 || y > ny - 3;
     const S gamS = S(a.gam);
     auto zplane = [&](int k) -> int64_t { return Donor<S, W>::plane(a, g.plane, k); };
@@ -375,6 +464,7 @@ __device__ __forceinline__ void tile_halo(const StageArgs &a, TileLds<S, TY, V> 
     auto put = [&](int k, const Raw<S> &raw) {
         W6<S> w = prims<STAGE, S, V>(a, raw, flg);
         me.signs(a, k, w);
+        col.momenta(raw, w, flg);
         store_w(L.P[k & 1], c, w);
     };
     put(kb, load_raw<STAGE, S, V>(a, zplane(kb), coff));
@@ -393,15 +483,16 @@ __device__ __forceinline__ void tile_halo(const StageArgs &a, TileLds<S, TY, V> 
             // B: y-states of plane k
             const W6<S> w = fetch_w(L.P[t], c);
             Side<S> ypl;
-            dir_states<1, S, V == kGamma>(fetch_w(L.P[t], c - RS), w, fetch_w(L.P[t], c + RS), sound_at<V>(w, a),
+            dir_states<1, S, V>(fetch_w(L.P[t], c - RS), w, fetch_w(L.P[t], c + RS), sound_at<V>(w, a),
                           xy_ghost || zghost(k), a, ymi, ypl);
             if (r == -1) store_side(L.Sy, lane, ypl);
         }
         __syncthreads();
         if (r == TY) {
-            S F[5];
-            face_flux<S, 1>(fetch_side(L.Sy, TY * 64 + lane, gamS), ymi, F);
-            for (int i = 0; i < 5; i++) L.Sy[i][TY * 64 + lane] = F[i];
+            S F[5], gy[2];
+            stage_face<S, 1, V>(fetch_side(L.Sy, TY * 64 + lane, gamS), ymi, col, F, gy);
+            for (int i = 0; i < 5; i++)
+                L.Sy[i][TY * 64 + lane] = has_ang(V) && (i == 1 || i == 2) ? gy[i - 1] : F[i];
         }
         __syncthreads();
     }
@@ -420,6 +511,7 @@ __device__ __forceinline__ void tile_edge(const StageArgs &a, TileLds<S, TY, V> 
     const int x = g.x0 + lane, y = g.j0 + r;
     const Donor<S, W> me(a, x, y);
     const unsigned coff = me.off;
+    const AngColumn<V> col(a, min(x, nx - 1), min(y, ny - 1));
     const S gamS = S(a.gam);
     auto zplane = [&](int k) -> int64_t { return Donor<S, W>::plane(a, g.plane, k); };
     auto zghost = [&](int k) -> bool { return !a.flatz && (k < 2 || k > nz - 3); };
@@ -430,6 +522,7 @@ __device__ __forceinline__ void tile_edge(const StageArgs &a, TileLds<S, TY, V> 
     const int ecol = ej < 3 ? ej - 2 : ej + 59;
     const int ex = g.x0 + ecol, ey = g.j0 + erow;
     const Donor<S, W> em(a, ex, ey);
+    const AngColumn<V> eang(a, min(max(ex, 0), nx - 1), min(ey, ny - 1));
     const unsigned eoff = em.off;
     const bool e_xy_ghost = ex < 2 || ex > nx - 3 || ey < 2 || ey > ny - 3;
 
@@ -439,13 +532,14 @@ __device__ __forceinline__ void tile_edge(const StageArgs &a, TileLds<S, TY, V> 
     auto edge_prims = [&](int k, const Raw<S> &raw) {
         ew = prims<STAGE, S, V>(a, raw, flg);
         em.signs(a, k, ew);
+        eang.momenta(raw, ew, flg);
         if (ej == 1 || ej == 5) store_w(L.P[k & 1], (erow + 2) * RS + ecol + 1, ew);
     };
     // neighbours within a row's seven lanes through whole-wave shifts (the
     // lanes whose neighbour lies in another row or outside the wave are not
     // used: columns -1, 63 and 64 take columns -2..0 and 62..65)
     auto edge_states = [&](int k) {
-        dir_states<0, S, V == kGamma>(lane_below_w(ew), ew, lane_above_w(ew), sound_at<V>(ew, a), e_xy_ghost || zghost(k), a, emi, epl);
+        dir_states<0, S, V>(lane_below_w(ew), ew, lane_above_w(ew), sound_at<V>(ew, a), e_xy_ghost || zghost(k), a, emi, epl);
     };
     auto edge_publish = [&]() {
         if (ej == 1) store_side(L.SxL, erow, epl);
@@ -457,11 +551,15 @@ __device__ __forceinline__ void tile_edge(const StageArgs &a, TileLds<S, TY, V> 
         xl.p = lane_below(epl.p);
         xl.e = lane_below(epl.e);
         xl.g = gamS;
-        if constexpr (V == kGamma) xl.g = lane_below(epl.g);
+        if constexpr (has_gamma(V)) xl.g = lane_below(epl.g);
+        if constexpr (has_ang(V)) {
+            xl.s1 = lane_below(epl.s1);
+            xl.s2 = lane_below(epl.s2);
+        }
         if (ej == 5) {
-            S F[5];
-            face_flux<S, 0>(xl, emi, F);  // face 63+1/2
-            for (int i = 0; i < 5; i++) L.FxR[i][erow] = F[i];
+            S F[5], gx[2];
+            stage_face<S, 0, V>(xl, emi, eang, F, gx);  // face 63+1/2, as column 63 has it
+            for (int i = 0; i < 5; i++) L.FxR[i][erow] = has_ang(V) && (i == 1 || i == 2) ? gx[i - 1] : F[i];
         }
     };
 
@@ -470,6 +568,7 @@ __device__ __forceinline__ void tile_edge(const StageArgs &a, TileLds<S, TY, V> 
     auto put = [&](int k, const Raw<S> &raw) {
         W6<S> w = prims<STAGE, S, V>(a, raw, flg);
         me.signs(a, k, w);
+        col.momenta(raw, w, flg);
         store_w(L.P[k & 1], c, w);
     };
     put(kb, load_raw<STAGE, S, V>(a, zplane(kb), coff));
