@@ -258,41 +258,36 @@ __device__ __forceinline__ void add_to(double *__restrict__ LW, int64_t n, int64
 }
 
 // ------------------------------------------------- direction kernels (y, z)
-// A wave holds 64 interior x-cells of one interior line along direction d
-// (d=1: y lines of a z-plane, d=2: z lines of a y-row) and marches along it
-// over the cells of chunk [jb, je), emitting the primitive adjoints of those
-// cells: faces j+1/2 for j in [jb-2, je], state reverses for [jb-1, je].
+// A lane holds an interior line along direction d (d=1: a y line, d=2: a z
+// line) and marches along it over the cells of chunk [jb, je), emitting the
+// primitive adjoints of those cells: faces j+1/2 for j in [jb-2, je], state
+// reverses for [jb-1, je].  The lanes take the lines x first, rw to a row:
+// the interior width itself, so that only the last wave has idle lanes (with
+// whole waves per row, 28% of the lanes idled at 96^3), or that width rounded
+// up to whole waves where a wave's lines would lie too far apart for 32-bit
+// offsets.
 // g = gscale * lam is the adjoint of fluxtmp (zero on ghost cells).  The
 // y kernel runs first and assigns its cells' primitive adjoints; the z kernel
 // assigns on z-ghost cells (no y line passes through them) and adds elsewhere.
 template <int STAGE, int d>
 __global__ __launch_bounds__(256) void k_adj_march(StageArgs a, const double *__restrict__ lam, double gscale,
-                                                   double kappa, double *__restrict__ LW, int chunk)
+                                                   double kappa, double *__restrict__ LW, int chunk, unsigned rw)
 {
-    const int lane = threadIdx.x & 63;
-    const int w = wave_id();
     const int nx = a.nx, ny = a.ny;
     const int64_t n = a.n, plane = (int64_t)nx * ny;
-    const int x = 2 + blockIdx.x * 64 + lane;
-    const bool xin = x <= nx - 3;
-    const int xc = xin ? x : nx - 3;
-    const unsigned xoff = (unsigned)xc * 8u;
-    int64_t base, stride;
-    int nd;
-    if (d == 1) {
-        const int z = a.zlo + blockIdx.y * 4 + w;
-        if (z >= a.zhi) return;
-        base = (int64_t)z * plane;
-        stride = nx;
-        nd = ny;
-    } else {
-        const int y = 2 + blockIdx.y * 4 + w;
-        if (y > ny - 3) return;
-        base = (int64_t)y * nx;
-        stride = plane;
-        nd = a.nz;
-    }
-    const int jb = max(1, (int)blockIdx.z * chunk), je = min(nd - 1, (int)blockIdx.z * chunk + chunk);
+    const unsigned t = blockIdx.x * 256u + threadIdx.x;
+    const int lines = d == 1 ? a.zhi - a.zlo : ny - 4;
+    const unsigned row = t / rw;
+    const int x = 2 + (int)(t - row * rw);
+    const bool xin = x <= nx - 3 && (int)row < lines;
+    const int line = min((int)row, lines - 1);
+    if (__builtin_amdgcn_readfirstlane((int)row) >= lines) return;
+    const int line0 = __builtin_amdgcn_readfirstlane(line);  // the wave's first: lines do not decrease with the lane
+    const int64_t pitch = d == 1 ? plane : nx, stride = d == 1 ? nx : plane;
+    const int64_t base = (line0 + (d == 1 ? a.zlo : 2)) * pitch;
+    const unsigned xoff = ((unsigned)((line - line0) * pitch) + (unsigned)min(x, nx - 3)) * 8u;
+    const int nd = d == 1 ? ny : a.nz;
+    const int jb = max(1, (int)blockIdx.y * chunk), je = min(nd - 1, (int)blockIdx.y * chunk + chunk);
     if (jb >= je) return;
     auto U = [&](int j) -> int64_t { return base + (int64_t)j * stride; };
     auto ghost = [&](int j) -> bool { return j < 2 || j > nd - 3; };
@@ -381,13 +376,6 @@ __global__ __launch_bounds__(256) void k_adj_march(StageArgs a, const double *__
 struct GhostInv {
     const int32_t *slot, *start, *gidx, *gsign;
 };
-
-__device__ __forceinline__ void add_signed(double acc[5], const double v[5], int sg)
-{
-    acc[0] += v[0];
-    for (int f = 1; f <= 3; f++) acc[f] += ((sg >> (f - 1)) & 1) ? -v[f] : v[f];
-    acc[4] += v[4];
-}
 
 // stage 2 at one cell: primitive adjoints lw of W* = (rho*, m*/rho*, p*, e*)
 // at U* = (r, m, E) -> adjoint of U* (out[0..4]) and of p* (out[5])
@@ -625,26 +613,52 @@ __global__ __launch_bounds__(256) void k_adj_x(StageArgs a, const double *__rest
 }
 
 // ------------------------------------------------------- pointwise kernels
-// The donors (interior cells some ghost copies), after the stage-2
-// directions: their own W* reverse plus their ghosts', then mid2_tail.
-// Ghost entries of lus and lsum stay zero.
+// The donors (interior cells some ghost copies) and their ghosts: kLanes lanes
+// take a donor, one its own cell and the others a ghost each, round by round,
+// and the contributions are added in the table's order (the same sum as one
+// lane makes in turn).  A corner's donor has 26 ghosts: with a lane for each
+// donor these few chains were the kernels' time: 28 us each at 96^3, now 19.
+constexpr int kLanes = 8;
+
+// value(cell, v) fills NV values of a cell; sum (all lanes of the group): the
+// donor's plus its ghosts', momenta with the ghosts' signs
+template <int NV, typename F>
+__device__ __forceinline__ void gather_ghosts(int kd, int64_t c, const GhostInv &gi, const F &value, double sum[NV])
+{
+    const int sub = threadIdx.x & (kLanes - 1);
+    const int t0 = gi.start[kd], cnt = gi.start[kd + 1] - t0 + 1;
+    for (int e0 = 0; e0 < cnt; e0 += kLanes) {
+        const int e = e0 + sub;
+        double v[NV] = {};
+        if (e < cnt) {
+            value(e == 0 ? c : (int64_t)gi.gidx[t0 + e - 1], v);
+            const int sg = e == 0 ? 0 : gi.gsign[t0 + e - 1];
+            for (int f = 1; f <= 3; f++)
+                if ((sg >> (f - 1)) & 1) v[f] = -v[f];
+        }
+        const int m = min(kLanes, cnt - e0);
+        for (int l = 0; l < m; l++)
+            for (int f = 0; f < NV; f++) {
+                const double w = __shfl(v[f], l, kLanes);
+                sum[f] = e0 + l == 0 ? w : sum[f] + w;
+            }
+    }
+}
+
+// After the stage-2 directions: the W* reverse, then mid2_tail.  Ghost entries
+// of lus and lsum stay zero.
 __global__ __launch_bounds__(256) void k_adj_mid2(int64_t n, int ndonor, const int32_t *__restrict__ donor,
                                                  double gm1, double seps, const double *__restrict__ u0,
                                                  const double *__restrict__ us, const double *__restrict__ lam,
                                                  const double *__restrict__ LW, GhostInv gi,
                                                  double *__restrict__ lus, double *__restrict__ lsum)
 {
-    const int kd = blockIdx.x * blockDim.x + threadIdx.x;
+    const int kd = (blockIdx.x * blockDim.x + threadIdx.x) / kLanes;
     if (kd >= ndonor) return;
     const int64_t c = donor[kd];
     double a[6];
-    fin2_cell(n, c, seps, us, LW, a);
-    for (int t = gi.start[kd]; t < gi.start[kd + 1]; t++) {
-        double b[6];
-        fin2_cell(n, gi.gidx[t], seps, us, LW, b);
-        add_signed(a, b, gi.gsign[t]);
-        a[5] += b[5];
-    }
+    gather_ghosts<6>(kd, c, gi, [&](int64_t q, double *v) { fin2_cell(n, q, seps, us, LW, v); }, a);
+    if ((threadIdx.x & (kLanes - 1)) != 0) return;
     double hl[5], ls[5], lsm[5];
     for (int f = 0; f < 5; f++) hl[f] = 0.5 * lam[f * n + c];
     const double m0[3] = {u0[n + c], u0[2 * n + c], u0[3 * n + c]};
@@ -655,23 +669,19 @@ __global__ __launch_bounds__(256) void k_adj_mid2(int64_t n, int ndonor, const i
     }
 }
 
-// The donors after the stage-1 directions: the adjoint of U^n at the cell
-// plus that of the ghosts it donates to (ghost entries of lout stay zero).
+// After the stage-1 directions: the adjoint of U^n (ghost entries of lout stay
+// zero).
 __global__ __launch_bounds__(256) void k_adj_fin1(int64_t n, int ndonor, const int32_t *__restrict__ donor,
                                                  double gm1, double seps, const double *__restrict__ u0,
                                                  const double *__restrict__ lsum, const double *__restrict__ LW,
                                                  GhostInv gi, double *__restrict__ lout)
 {
-    const int kd = blockIdx.x * blockDim.x + threadIdx.x;
+    const int kd = (blockIdx.x * blockDim.x + threadIdx.x) / kLanes;
     if (kd >= ndonor) return;
     const int64_t c = donor[kd];
     double a[5];
-    fin1_cell(n, c, gm1, seps, u0, lsum, LW, a);
-    for (int t = gi.start[kd]; t < gi.start[kd + 1]; t++) {
-        double b[5];
-        fin1_cell(n, gi.gidx[t], gm1, seps, u0, lsum, LW, b);
-        add_signed(a, b, gi.gsign[t]);
-    }
+    gather_ghosts<5>(kd, c, gi, [&](int64_t q, double *v) { fin1_cell(n, q, gm1, seps, u0, lsum, LW, v); }, a);
+    if ((threadIdx.x & (kLanes - 1)) != 0) return;
     for (int f = 0; f < 5; f++) lout[f * n + c] = a[f];
 }
 
@@ -745,20 +755,45 @@ void adjoint_free(bx_ctx *c)
     c->adj = nullptr;
 }
 
+// lanes per row of the marches' lines (k_adj_march), whose rows lie `pitch` cells apart
+static unsigned march_row(const bx_ctx *c, int64_t pitch)
+{
+    const int64_t width = c->nx - 4, apart = (63 + width - 1) / width + 1;  // rows that a wave's lanes can span
+    const bool far = (apart * pitch + c->nx) * 8 >= ((int64_t)1 << 32);
+    return (unsigned)(far ? (width + 63) / 64 * 64 : width);
+}
+static unsigned march_blocks(unsigned rw, int lines) { return (unsigned)(((int64_t)rw * lines + 255) / 256); }
+
+// Cells per chunk of a march over nd cells.  A wave pays about three cells'
+// work before its first cell; a CU holds two blocks (256 registers), which
+// take 1.25 times as long as one, and more blocks run in turn.  One reverse
+// step, all kernels, in us by chunk length (the rule's choice in brackets):
+// 64^3 163 [4], 198 8, 274 16; 96^3 392 4, [8] 349, 368 16, 442 24;
+// 128^3 745 8, [16] 691, 745 32; 128x60x40 204 4, [5] 178, 222 10.
+static int march_chunk(const bx_ctx *c, unsigned blocks, int nd)
+{
+    double best = 0.0;
+    int at = nd;
+    for (int parts = 1; parts <= (nd + 3) / 4; parts++) {
+        const int len = (nd + parts - 1) / parts;
+        const int64_t deep = ((int64_t)blocks * ((nd + len - 1) / len) + c->ncu - 1) / c->ncu;  // blocks per CU
+        const double cost = (deep <= 1 ? 1.0 : 0.625 * ((deep + 1) / 2 * 2)) * (len + 3);
+        if (parts == 1 || cost < best) {
+            best = cost;
+            at = len;
+        }
+    }
+    return at;
+}
+
 static int adj_init(bx_ctx *c)
 {
     if (c->adj) return BX_OK;
     bx_adj *j = new (std::nothrow) bx_adj();
     if (!j) return set_error(BX_ERR_ARG, "adjoint: out of host memory");
     c->adj = j;
-    // chunk lengths: shortened on small grids until the march kernels have
-    // about 2 waves per SIMD to run
-    {
-        const int64_t want = 2 * 1024, bx = (c->nx - 4 + 63) / 64;
-        const int nzi = c->flatz ? c->nz : c->nz - 4;
-        while (j->chunk_y > 8 && bx * ((nzi + 3) / 4) * 4 * ((c->ny + j->chunk_y - 1) / j->chunk_y) < want) j->chunk_y /= 2;
-        while (j->chunk_z > 8 && bx * (c->ny - 4) * ((c->nz + j->chunk_z - 1) / j->chunk_z) < want) j->chunk_z /= 2;
-    }
+    j->chunk_y = march_chunk(c, march_blocks(march_row(c, (int64_t)c->nx * c->ny), c->flatz ? c->nz : c->nz - 4), c->ny);
+    j->chunk_z = march_chunk(c, march_blocks(march_row(c, c->nx), c->ny - 4), c->nz);
     const size_t pb = sizeof(double) * (size_t)c->n;
     BX_HIP(hipMalloc((void **)&j->lam[0], 5 * pb));
     BX_HIP(hipMalloc((void **)&j->lam[1], 5 * pb));
@@ -838,17 +873,18 @@ static int directions(bx_ctx *c, const StageArgs &a, const double *lam, double g
     bx_adj *j = c->adj;
     const double kx = a.ayz * a.dt / a.vol, ky = a.axz * a.dt / a.vol, kz = a.axy * a.dt / a.vol;
     const int nzi = a.zhi - a.zlo;
-    const unsigned bx = (unsigned)((c->nx - 4 + 63) / 64);
     {
-        dim3 grid(bx, (unsigned)((nzi + 3) / 4), (unsigned)((c->ny + j->chunk_y - 1) / j->chunk_y));
+        const unsigned rw = march_row(c, (int64_t)c->nx * c->ny);
+        dim3 grid(march_blocks(rw, nzi), (unsigned)((c->ny + j->chunk_y - 1) / j->chunk_y));
         hipLaunchKernelGGL((k_adj_march<STAGE, 1>), grid, dim3(256), 0, c->stream, a, lam, gscale, ky, j->lw,
-                           j->chunk_y);
+                           j->chunk_y, rw);
         BX_HIP(hipGetLastError());
     }
     if (!c->flatz) {  // flat z: the z terms are exactly zero
-        dim3 grid(bx, (unsigned)((c->ny - 4 + 3) / 4), (unsigned)((c->nz + j->chunk_z - 1) / j->chunk_z));
+        const unsigned rw = march_row(c, c->nx);
+        dim3 grid(march_blocks(rw, c->ny - 4), (unsigned)((c->nz + j->chunk_z - 1) / j->chunk_z));
         hipLaunchKernelGGL((k_adj_march<STAGE, 2>), grid, dim3(256), 0, c->stream, a, lam, gscale, kz, j->lw,
-                           j->chunk_z);
+                           j->chunk_z, rw);
         BX_HIP(hipGetLastError());
     }
     {
@@ -881,7 +917,7 @@ static int adj_step(bx_ctx *c, double dt, const double *un, const double *us, co
     const int64_t n = c->n;
     const GhostInv gi = ghost_inv(c);
     const int32_t *donor = j->fold;
-    const unsigned nbd = blocks_for(j->ndonor, 256);
+    const unsigned nbd = blocks_for((int64_t)j->ndonor * kLanes, 256);
     StageArgs b = base_args(c, dt);
     b.uin = us;
     b.pin = ps;
