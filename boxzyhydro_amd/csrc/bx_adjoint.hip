@@ -945,7 +945,7 @@ static int read_flags_rate(bx_ctx *c, unsigned *flags, double *rate)
     BX_HIP(hipMemcpyAsync(c->hsc, c->dsc, sizeof(DevScalars), hipMemcpyDeviceToHost, c->stream));
     BX_HIP(hipStreamSynchronize(c->stream));
     *flags = c->hsc->flags;
-    unsigned long long b = c->hsc->rate_bits[0];
+    unsigned long long b = rate_bits(c->hsc, 0);
     std::memcpy(rate, &b, sizeof(double));
     return BX_OK;
 }
@@ -1051,7 +1051,7 @@ extern "C" int bx_adjoint_forward(bx_ctx *c, int32_t nsteps, int32_t every, cons
             BX_HIP(hipMalloc((void **)&j->dlog, sizeof(double) * (size_t)nsteps));
             j->dlog_cap = nsteps;
         }
-        DevScalars *h = c->hsc;  // rate_bits[0]: the Courant rate of the regular check above
+        DevScalars *h = c->hsc;  // rate[0]: the Courant rate of the regular check above
         h->slot[0] = StepSlot{0.0, 0.0, 0.0, std::numeric_limits<double>::infinity(), 0, 0};
         h->flags = 0;
         BX_HIP(hipMemcpyAsync(c->dsc, h, sizeof(DevScalars), hipMemcpyHostToDevice, c->stream));
@@ -1110,7 +1110,7 @@ extern "C" int bx_adjoint_forward(bx_ctx *c, int32_t nsteps, int32_t every, cons
         invalidate(false);
         return rc;
     }
-    if (!frozen && (nsteps & 1)) c->hsc->rate_bits[0] = c->hsc->rate_bits[1];  // the last step's, [nsteps & 1]
+    if (!frozen && (nsteps & 1)) set_rate_bits(c->hsc, 0, rate_bits(c->hsc, 1));  // the last step's, [nsteps & 1]
     if (flags & (FLAG_IRREGULAR | FLAG_FLOOR)) return refuse(flags);
     if (dts_out)
         for (int k = 0; k < nsteps; k++) dts_out[k] = j->dts[k];

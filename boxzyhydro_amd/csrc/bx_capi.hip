@@ -929,7 +929,7 @@ static int step_run(bx_ctx *c, int K, double endtime, double *time, double *dtol
         }
     }
     BX_HIP(hipMemcpyAsync(c->chunk0, cur, bytes, hipMemcpyDeviceToDevice, c->stream));
-    const unsigned long long rate0 = c->hsc->rate_bits[0];  // Courant rate of the current state
+    const unsigned long long rate0 = rate_bits(c->hsc, 0);  // Courant rate of the current state
     DevScalars *h = c->hsc;
     h->slot[0] = StepSlot{0.0, *dtold, *time, endtime, *step, 0};
     h->flags = 0;
@@ -941,7 +941,7 @@ static int step_run(bx_ctx *c, int K, double endtime, double *time, double *dtol
     const StepSlot &s = h->slot[0];  // after an even number of steps
     if ((h->flags & FLAG_IRREGULAR) || s.step != *step + K) {
         BX_HIP(hipMemcpyAsync(cur, c->chunk0, bytes, hipMemcpyDeviceToDevice, c->stream));
-        h->rate_bits[0] = rate0;
+        set_rate_bits(h, 0, rate0);
         return BX_OK;
     }
     *time = s.time + s.dt;  // the last step's main.f90:545 (the device advanced time for the others)
@@ -969,7 +969,7 @@ static int fused_loop(bx_ctx *c, int32_t nsteps, double endtime, double *time, d
     int rc;
     int32_t k = 0;
     int32_t single = 0;  // steps to take one at a time (after an undone chunk or an irregular step)
-    // While fused_valid holds, hsc->rate_bits[0] is the Courant rate of the
+    // While fused_valid holds, hsc->rate[0] is the Courant rate of the
     // current state (from the regularity check or the last fused step).
     while (k < nsteps && *time < endtime && *step < 1000000) {
         if (!c->fused_valid) {
@@ -1016,7 +1016,7 @@ static int fused_loop(bx_ctx *c, int32_t nsteps, double endtime, double *time, d
             }
         }
         if (single > 0) single--;
-        const double rate = rate_from_bits(c->hsc->rate_bits[0]);
+        const double rate = rate_from_bits(rate_bits(c->hsc, 0));
         const double time0 = *time, dtold0 = *dtold;
         const int32_t step0 = *step;
         *step += 1;

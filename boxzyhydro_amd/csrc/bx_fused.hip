@@ -101,7 +101,7 @@ __global__ __launch_bounds__(256) void k_regular(int64_t n, const double *__rest
     for (int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; c < n; c += (int64_t)gridDim.x * blockDim.x)
         rt = vmax(rt, regular_cell(n, c, cons, u, gam, seps, dx, dy, dz, flg));
     if (flg) atomicOr(flags, flg);
-    block_max_to(rt, rate);
+    block_max_to(rt, rate + (blockIdx.x % kRateSlots) * kMaxStride);
 }
 
 template <typename S>
@@ -417,10 +417,10 @@ int fused_prepare(bx_ctx *c)
 int launch_regular_check(bx_ctx *c)
 {
     BX_HIP(hipMemsetAsync(&c->dsc->flags, 0, sizeof(unsigned int), c->stream));
-    BX_HIP(hipMemsetAsync(&c->dsc->rate_bits[0], 0, sizeof(unsigned long long), c->stream));
+    BX_HIP(hipMemsetAsync(c->dsc->rate[0], 0, sizeof(c->dsc->rate[0]), c->stream));
     hipLaunchKernelGGL(k_regular, dim3(reduce_blocks(c->n)), dim3(256), 0, c->stream, c->n, c->cons, c->u,
                        c->prm.gammafix, c->prm.small_eps, c->prm.dx, c->prm.dy, c->prm.dz, &c->dsc->flags,
-                       &c->dsc->rate_bits[0]);
+                       c->dsc->rate[0]);
     BX_HIP(hipGetLastError());
     return BX_OK;
 }
@@ -451,7 +451,7 @@ __global__ __launch_bounds__(192) void k_corner_ghosts(StageArgs a0, const int32
     __syncthreads();
     if (threadIdx.x == 0) rt = corner_update(a, j, F, dst[j], sign[j], flg);
     if (flg) atomicOr(a.flags, flg);
-    if (d == 0) wave_max_to(rt, a.rate);
+    if (d == 0) wave_max_to(rt, rate_slot(a, (unsigned)j));
 }
 
 // after the corrector, and after any ghost fill of un that writes these ghosts (b: the corrector's arguments)
@@ -512,8 +512,8 @@ static void read_donors(const bx_ctx *c, StageArgs &a)
 
 // One fused step u0 -> us, ps -> un from a regular state, with full dt `dt`
 // or, for par = 0 or 1, with dt formed on the device from slot[par] and
-// rate_bits[par] (left in slot[par^1], logged in log[cap]).  The Courant rate
-// of U^{n+1} is left in rate_bits[0] or rate_bits[par^1]; irregular branches
+// rate[par] (left in slot[par^1], logged in log[cap]).  The Courant rate of
+// U^{n+1} is left in rate[0] or rate[par^1]; irregular branches
 // are added to the flags.  fill: the ghost cells of us, ps and un hold their
 // donors' values afterwards (otherwise those of the stage inputs need not,
 // and those of un do not, but for the corner ghosts).
@@ -523,14 +523,14 @@ static int enqueue_step(bx_ctx *c, double dt, int par, double *log, int cap, S *
 {
     int rc;
     const bool donors = reads_donors(c);
-    unsigned long long *rate = &c->dsc->rate_bits[par < 0 ? 0 : par ^ 1];
+    unsigned long long *rate = c->dsc->rate[par < 0 ? 0 : par ^ 1];
     StageArgs a = base_args(c, dt);
     if (donors) read_donors(c, a);
     StageArgs b = a;
     if (par >= 0) {
         a.slot = &c->dsc->slot[par];
         a.slot_next = &c->dsc->slot[par ^ 1];
-        a.rate_in = &c->dsc->rate_bits[par];
+        a.rate_in = c->dsc->rate[par];
         a.cfl = c->prm.cfl;
         a.log = log;
         a.log_cap = cap;
@@ -545,6 +545,7 @@ static int enqueue_step(bx_ctx *c, double dt, int par, double *log, int cap, S *
     b.uold = u0;
     b.uout = un;
     b.rate = rate;
+    b.rate_mask = kRateSlots - 1;
     S *pfin = grav_pressure<S>(c, b);
     if (c->prof_on) BX_HIP(hipEventRecord(c->ev[0], c->stream));
     if ((rc = launch_stage<1, S>(c, a, c->prof_on ? c->ev[1] : nullptr, (S *)c->eflux))) return rc;
@@ -659,21 +660,20 @@ int fused_step_into(bx_ctx *c, double dt, double *u0, double *us, double *ps, do
 
 __global__ void k_clear_scalars(unsigned int *flags, unsigned long long *rate)
 {
-    *flags = 0u;
-    *rate = 0ull;
+    if (threadIdx.x == 0) *flags = 0u;
+    rate[threadIdx.x * kMaxStride] = 0ull;
 }
 
 // One FP64 fused step u0 -> us, ps -> un (ey: the y-term planes) on the
-// context's stream with the flags and the Courant rate accumulated into the
-// given device words, which
-// a kernel clears first (no memset nodes, so the sequence can be captured).
+// context's stream with the flags and the Courant rate (kRateSlots slots)
+// accumulated into the given device words, which a kernel clears first (no memset nodes, so the sequence can be captured).
 // Allocates nothing; the tile defaults must be set (fused_defaults).
 int fused_step_words(bx_ctx *c, double dt, const double *u0, double *us, double *ps, double *un, double *ey,
                      unsigned int *flags, unsigned long long *rate)
 {
     if (c->grav_flags) return set_error(BX_ERR_UNSUPPORTED, "this fused step entry takes no gravity configuration");
     int rc;
-    hipLaunchKernelGGL(k_clear_scalars, dim3(1), dim3(1), 0, c->stream, flags, rate);
+    hipLaunchKernelGGL(k_clear_scalars, dim3(1), dim3(kRateSlots), 0, c->stream, flags, rate);
     BX_HIP(hipGetLastError());
     StageArgs a = base_args(c, dt);
     a.flags = flags;
@@ -689,13 +689,14 @@ int fused_step_words(bx_ctx *c, double dt, const double *u0, double *us, double 
     b.uold = u0;
     b.uout = un;
     b.rate = rate;
+    b.rate_mask = kRateSlots - 1;
     if ((rc = launch_stage<2, double>(c, b, nullptr, ey))) return rc;
     if ((rc = ghosts6<double>(c, un, (double *)nullptr))) return rc;
     return corner_ghosts(c, b);
 }
 
 // Step k of a run whose dts are formed on the device (scalars of step 0 in
-// slot[0], its rate in rate_bits[0]), logged into log[cap]
+// slot[0], its rate in rate[0]), logged into log[cap]
 int fused_step_device_dt(bx_ctx *c, int k, double *u0, double *us, double *ps, double *un, double *log, int cap)
 {
     return enqueue_step<double>(c, 0.0, k & 1, log, cap, u0, us, ps, un, true, true);

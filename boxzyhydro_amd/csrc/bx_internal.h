@@ -17,6 +17,11 @@ constexpr int kMaxSlots = 32, kMaxStride = 16;  // slots of a grid-wide maximum,
 
 constexpr int kMaxD2 = 64;  // two-level ghost compositions a context may have (one wave)
 
+// Slots of the fused step's Courant rate (a power of two, one row of 16 lanes
+// reads them).  Every wave of stage 2 looks at the rate and adds its share:
+// 784 waves on one word took half of a 32^3 stage 2 (22.6 us, with slots 13.3).
+constexpr int kRateSlots = 16;
+
 // The step scalars of main.f90 as a device-dt step leaves them.
 struct StepSlot {
     double dt;       // full dt of the step (main.f90:342)
@@ -31,12 +36,24 @@ struct StepSlot {
 // Device-dt steps alternate between the two slots and rates (a step reads one
 // and writes the other), so that no workgroup reads what another one writes.
 struct DevScalars {
-    unsigned long long rate_bits[2];  // Courant max-rate (non-negative doubles as bits), ping-pong
+    // Courant max-rate (non-negative doubles as bits), ping-pong, each in
+    // kRateSlots words of a cache line each: a rate is their maximum
+    unsigned long long rate[2][kRateSlots * kMaxStride];
     unsigned int flags;               // irregular-branch flags raised by the fused kernels
     unsigned int pad;
     StepSlot slot[2];
     unsigned int slow[2];             // FLAG_SLOW of a tiled flux call; calls alternate between the two words
 };
+inline unsigned long long rate_bits(const DevScalars *s, int par)
+{
+    unsigned long long m = 0ull;
+    for (int i = 0; i < kRateSlots; i++) m = s->rate[par][i * kMaxStride] > m ? s->rate[par][i * kMaxStride] : m;
+    return m;
+}
+inline void set_rate_bits(DevScalars *s, int par, unsigned long long bits)
+{
+    for (int i = 0; i < kRateSlots; i++) s->rate[par][i * kMaxStride] = i == 0 ? bits : 0ull;
+}
 
 // flags bits
 enum : unsigned int {
@@ -208,7 +225,7 @@ int fused_step(bx_ctx *c, double dt);
 int fused_step_into(bx_ctx *c, double dt, double *u0, double *us, double *ps, double *un, bool reset_flags);
 // the same, step k of a run, with dt formed on the device from the current
 // Courant rate (the device scalars carry time, dtold, step and endtime, at the
-// run's start in slot[0] and rate_bits[0]; after k steps in [k & 1]); flags
+// run's start in slot[0] and rate[0]; after k steps in [k & 1]); flags
 // accumulate and each dt is logged into log[cap]
 int fused_step_device_dt(bx_ctx *c, int k, double *u0, double *us, double *ps, double *un, double *log, int cap);
 void adjoint_free(bx_ctx *c);

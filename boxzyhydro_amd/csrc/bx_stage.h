@@ -5,6 +5,8 @@
 // kernels operation for operation.
 #pragma once
 
+#include <type_traits>
+
 #include "bx_internal.h"
 #include "bx_math.h"
 
@@ -44,6 +46,7 @@ struct StageArgs {
     double gam, gm1, seps, srho, vlimit;
     unsigned int *flags;
     unsigned long long *rate;  // stage 2: next step's Courant rate (max)
+    unsigned rate_mask;        // slots of it - 1 (kMaxStride words apart); 0: one word
     const double *dtp;         // when set, the step's dt is read from here (device dt), else dt
     // stage 1 of a device-dt step: every workgroup forms dt from the slot the
     // last step left and the Courant rate; the first one writes the next slot
@@ -102,6 +105,28 @@ __device__ __forceinline__ StepSlot next_slot(const StepSlot &s, unsigned long l
     return o;
 }
 
+// The maximum of kRateSlots slots: a row of 16 lanes loads them, the maximum
+// goes round the row.
+__device__ __forceinline__ unsigned long long slots_max(const unsigned long long *slots)
+{
+    static_assert(kRateSlots == 16, "one row of lanes");
+    unsigned long long v = slots[(threadIdx.x & 15) * kMaxStride];
+    auto turn = [&](auto ctrl) {
+        constexpr int c = decltype(ctrl)::value;
+        const int lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)v, c, 0xf, 0xf, false);
+        const int hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(v >> 32), c, 0xf, 0xf, false);
+        const unsigned long long o = ((unsigned long long)(unsigned)hi << 32) | (unsigned)lo;
+        v = o > v ? o : v;
+    };
+    turn(std::integral_constant<int, 0x128>{});  // row_ror by 8, 4, 2, 1
+    turn(std::integral_constant<int, 0x124>{});
+    turn(std::integral_constant<int, 0x122>{});
+    turn(std::integral_constant<int, 0x121>{});
+    const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)v);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(v >> 32));
+    return ((unsigned long long)hi << 32) | lo;
+}
+
 __device__ __forceinline__ bool first_lane_of_grid()
 {
     return blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0 && threadIdx.x == 0;
@@ -115,7 +140,7 @@ __device__ __forceinline__ StageArgs with_dt(const StageArgs &a0)
 {
     StageArgs a = a0;
     if (a0.slot) {
-        const StepSlot o = next_slot(*a0.slot, *a0.rate_in, a0.cfl);
+        const StepSlot o = next_slot(*a0.slot, slots_max(a0.rate_in), a0.cfl);
         a.dt = o.dt;
         if (first_lane_of_grid()) {
             *a0.slot_next = o;
@@ -124,7 +149,8 @@ __device__ __forceinline__ StageArgs with_dt(const StageArgs &a0)
     } else if (a0.dtp) {
         a.dt = *a0.dtp;
     }
-    if (a0.rate_next && first_lane_of_grid()) *a0.rate_next = 0ull;
+    if (a0.rate_next && blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0 && threadIdx.x < kRateSlots)
+        a0.rate_next[threadIdx.x * kMaxStride] = 0ull;
     if (a0.clear && first_lane_of_grid()) *a0.clear = 0u;
     return a;
 }

@@ -15,7 +15,7 @@ void fused_defaults(bx_ctx *c);
 int fused_step_words(bx_ctx *c, double dt, const double *u0, double *us, double *ps, double *un, double *ey,
                      unsigned int *flags, unsigned long long *rate);
 
-constexpr size_t kStaticHeader = 256;  // flag and rate words, then the planes
+constexpr size_t kStaticHeader = 256 + 8 * kRateSlots * kMaxStride;  // flag word, rate slots, then the planes
 constexpr size_t kStaticBytes = kStaticHeader + (size_t)BX_STATIC_MAX_CELLS * BX_STATIC_BYTES_PER_CELL;
 
 static __device__ __align__(256) unsigned char scratch[kStaticBytes];
@@ -47,7 +47,9 @@ __global__ void k_static_out(const unsigned int *flags, const unsigned long long
                              double *rate_out)
 {
     if (flags_out) *flags_out = *flags;
-    if (rate_out) *rate_out = __longlong_as_double((long long)*rate);
+    unsigned long long m = 0ull;
+    for (int i = 0; i < kRateSlots; i++) m = rate[i * kMaxStride] > m ? rate[i * kMaxStride] : m;
+    if (rate_out) *rate_out = __longlong_as_double((long long)m);
 }
 
 }  // namespace bx
@@ -71,7 +73,7 @@ extern "C" int bx_step_static(bx_ctx *c, const double *cons_in, double *cons_out
     if (int rc = scratch_ptr(c->device, &base)) return rc;
     fused_defaults(c);
     unsigned int *flags = (unsigned int *)base;
-    unsigned long long *rate = (unsigned long long *)(base + 64);
+    unsigned long long *rate = (unsigned long long *)(base + 256);
     double *us = (double *)(base + kStaticHeader);
     double *ps = us + 5 * c->n;
     double *ey = ps + c->n;

@@ -633,7 +633,7 @@ __device__ __forceinline__ void tile_stage(const StageArgs &a, TileLds<S, TY, V>
     else if (g.r == TY + 1) tile_edge<STAGE, S, TY, V, W>(a, L, g, flg);
     else tile_halo<STAGE, S, TY, V, W>(a, L, g, flg);
     if (flg) atomicOr(a.flags, flg);
-    if (STAGE == 2) wave_max_to(rmax, a.rate);
+    if (STAGE == 2) wave_max_to(rmax, rate_slot(a, bx + by + bz + (unsigned)g.r));
 }
 
 // The two-level corner ghosts after the corrector's ghost fill.  The exact

@@ -22,6 +22,12 @@ __device__ __forceinline__ void wave_max_to(double v, unsigned long long *dst)
     }
 }
 
+// the slot of the Courant rate that the k-th share goes to
+__device__ __forceinline__ unsigned long long *rate_slot(const StageArgs &a, unsigned k)
+{
+    return a.rate + (k & a.rate_mask) * kMaxStride;
+}
+
 // ---------------------------------------------------------------------------
 // y-direction kernel: each wave holds 64 consecutive interior x-cells of one
 // z-plane and marches in y, keeping the primitives of rows j..j+2, the y-plus
@@ -381,7 +387,7 @@ __device__ __forceinline__ void xz_wave(const StageArgs &a, const S *__restrict_
     }
 
     if (flg) atomicOr(a.flags, flg);
-    if (STAGE == 2) wave_max_to(rmax, a.rate);
+    if (STAGE == 2) wave_max_to(rmax, rate_slot(a, blockIdx.x + blockIdx.y + blockIdx.z + wave_id()));
 }
 
 // u = m/rho, p = state() of a regular cell, adindx = gamma: the velocity and
