@@ -20,8 +20,8 @@
 // the step with the exact sequence.
 //
 // Work decomposition (gfx950, wave64): by default each stage is one kernel,
-// k_stage, a workgroup holding a 64 x TY tile of outputs with its +-2 halo in
-// LDS and marching in z (bx_tile.h).  The tuning variants 0, 1 and 4
+// k_stage, a workgroup holding a tile of outputs (64 x 8, 64 x 4, 32 x 16 or
+// 32 x 8 columns) with its +-2 halo in LDS and marching in z (bx_tile.h).  The tuning variants 0, 1 and 4
 // (bx_tune) run the earlier form, two kernels per stage with every wave
 // independent (no LDS, no block barriers):
 //   * k_ydir: a wave holds 64 interior x-cells of one z-plane and marches in y
@@ -38,15 +38,15 @@
 
 namespace bx {
 
-// One stage as one kernel: x-y tile of 64 x TY outputs with its +-2 halo in
+// One stage as one kernel: x-y tile of WX x TY outputs with its +-2 halo in
 // LDS, marching in z (bx_tile.h: tile_stage).  P2: every spacing and the
 // cell volume are powers of two (their divisions are multiplications), known
 // at compile time, which keeps the spacings themselves out of the registers.
 // V: StageKind; W: walls whose ghosts are read from their donors (bx_tile.h).
-template <int STAGE, typename S, int TY, bool P2, int V, bool W>
-__global__ __launch_bounds__(64 * (TY + 4)) void k_stage(StageArgs a0)
+template <int STAGE, typename S, int TY, bool P2, int V, bool W, int WX>
+__global__ __launch_bounds__(64 * tile_waves(TY, WX)) void k_stage(StageArgs a0)
 {
-    __shared__ TileLds<S, TY, V> lds;
+    __shared__ TileLds<S, TY, V, WX> lds;
     StageArgs a = with_dt(a0);
     if constexpr (P2) {
         a.ds_pow2[0] = a.ds_pow2[1] = a.ds_pow2[2] = 1;
@@ -61,7 +61,7 @@ __global__ __launch_bounds__(64 * (TY + 4)) void k_stage(StageArgs a0)
     const unsigned L = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);
     const unsigned xcd = L & 7u, slot = L >> 3, q = T >> 3, rem = T & 7u;
     const unsigned t = xcd * q + (xcd < rem ? xcd : rem) + slot;
-    tile_stage<STAGE, S, TY, V, W>(a, lds, t % gx, (t / gx) % gy, t / (gx * gy));
+    tile_stage<STAGE, S, TY, V, W, WX>(a, lds, t % gx, (t / gx) % gy, t / (gx * gy));
 }
 
 
@@ -173,39 +173,42 @@ StageArgs base_args(bx_ctx *c, double dt)
     return a;
 }
 
-template <int STAGE, typename S, int TY, bool W>
+// the grid of the tiled kernels: tiles of wx x ty columns by chunks of lz planes
+static dim3 tile_grid(const bx_ctx *c, const StageArgs &a, int ty, int wx)
+{
+    return dim3((unsigned)((c->nx - 4 + wx - 1) / wx), (unsigned)((c->ny - 4 + ty - 1) / ty),
+                (unsigned)((a.zhi - a.zlo + a.lz - 1) / a.lz));
+}
+
+template <int STAGE, typename S, int TY, int WX, bool W>
 static int launch_tile_w(bx_ctx *c, const StageArgs &a)
 {
     const bool p2 = a.ds_pow2[0] && a.ds_pow2[1] && a.ds_pow2[2] && a.vol_pow2;
-    const int nzi = a.zhi - a.zlo;
-    const unsigned gx = (unsigned)((c->nx - 4 + 63) / 64);
-    const unsigned gy = (unsigned)((c->ny - 4 + TY - 1) / TY);
-    const unsigned gz = (unsigned)((nzi + a.lz - 1) / a.lz);
-    const dim3 grid(gx, gy, gz), block(64 * (TY + 4));
-    if constexpr (sizeof(S) == 8 && TY == 8 && !W) {
+    const dim3 grid = tile_grid(c, a, TY, WX), block(64 * tile_waves(TY, WX));
+    if constexpr (sizeof(S) == 8 && TY * WX == 512 && !W) {
         if (a.gf) {
             // the power-of-two forms spill 2 and 7 VGPRs at 168; the general
             // ones (163, no spill) give the same bits and are ~1 % faster
-            hipLaunchKernelGGL((k_stage<STAGE, S, TY, false, kGravity, false>), grid, block, 0, c->stream, a);
+            hipLaunchKernelGGL((k_stage<STAGE, S, TY, false, kGravity, false, WX>), grid, block, 0, c->stream, a);
             BX_HIP(hipGetLastError());
             return BX_OK;
         }
     }
-    if (a.gf) return set_error(BX_ERR_UNSUPPORTED, "fused step with gravity: FP64 64 x 8 tiles only");
+    if (a.gf) return set_error(BX_ERR_UNSUPPORTED, "fused step with gravity: FP64 64 x 8 or 32 x 16 tiles only");
     if (p2)
-        hipLaunchKernelGGL((k_stage<STAGE, S, TY, true, kPlain, W>), grid, block, 0, c->stream, a);
+        hipLaunchKernelGGL((k_stage<STAGE, S, TY, true, kPlain, W, WX>), grid, block, 0, c->stream, a);
     else
-        hipLaunchKernelGGL((k_stage<STAGE, S, TY, false, kPlain, W>), grid, block, 0, c->stream, a);
+        hipLaunchKernelGGL((k_stage<STAGE, S, TY, false, kPlain, W, WX>), grid, block, 0, c->stream, a);
     BX_HIP(hipGetLastError());
     return BX_OK;
 }
 
-template <int STAGE, typename S, int TY>
+template <int STAGE, typename S, int TY, int WX>
 static int launch_tile(bx_ctx *c, const StageArgs &a)
 {
     bool w = false;
     for (int i = 0; i < 6; i++) w = w || (a.gmap && a.wall[i]);
-    return w ? launch_tile_w<STAGE, S, TY, true>(c, a) : launch_tile_w<STAGE, S, TY, false>(c, a);
+    return w ? launch_tile_w<STAGE, S, TY, WX, true>(c, a) : launch_tile_w<STAGE, S, TY, WX, false>(c, a);
 }
 
 template <int STAGE, typename S>
@@ -215,9 +218,13 @@ static int launch_stage(bx_ctx *c, const StageArgs &a, hipEvent_t mid, S *eflux)
     if (c->fused_occ >= 10) {
         if (mid) BX_HIP(hipEventRecord(mid, c->stream));
         switch (c->fused_occ) {
-        case 10: return launch_tile<STAGE, S, 4>(c, a);
-        default: return launch_tile<STAGE, S, 8>(c, a);
+        case kTile64x4: return launch_tile<STAGE, S, 4, 64>(c, a);
+        case kTile64x8: return launch_tile<STAGE, S, 8, 64>(c, a);
+        case kTile32x8: return launch_tile<STAGE, S, 8, 32>(c, a);
+        default: break;
         }
+        if constexpr (sizeof(S) == 8) return launch_tile<STAGE, S, 16, 32>(c, a);
+        return set_error(BX_ERR_UNSUPPORTED, "mixed form: no 32 x 16 tiles");
     }
     if (a.gf) return set_error(BX_ERR_UNSUPPORTED, "fused step with gravity: the tiled kernel only (variant 11)");
     const int nzi = a.zhi - a.zlo;
@@ -263,35 +270,46 @@ int launch_tiled_flux(bx_ctx *c, int avg, double dt, double *out, unsigned int *
     a.flags = slow;
     a.clear = slow_next;
     a.yoffset = c->prm.yoffset;
-    // gamma from its plane unless every cell holds gammafix; a seventh field
-    // (and the eighth and ninth of flux_ang) leaves room in LDS for 64 x 4 tiles
+    // gamma from its plane unless every cell holds gammafix; with it as a
+    // seventh field the 64 x 8 tile, and with the eighth and ninth of flux_ang
+    // either tile of eight owner waves, is too large for LDS
     const bool vg = !c->ad_uniform, ang = c->prm.fluxangmom != 0;
-    int ty = 4;
-    tile_split(c, false, !vg && !ang, true, &a.lz, &ty);
+    unsigned tiles = tile_bit(kTile64x4) | tile_bit(kTile32x8);
+    if (!ang) tiles |= tile_bit(kTile32x16) | (vg ? 0u : tile_bit(kTile64x8));
+    const int tile = tile_split(c, false, tiles, &a.lz);
     const bool p2 = a.ds_pow2[0] && a.ds_pow2[1] && a.ds_pow2[2] && a.vol_pow2;
-    const int nzi = a.zhi - a.zlo;
-    const dim3 grid((unsigned)((c->nx - 4 + 63) / 64), (unsigned)((c->ny - 4 + ty - 1) / ty),
-                    (unsigned)((nzi + a.lz - 1) / a.lz));
-    const dim3 block(64 * (ty + 4));
-    auto go = [&](auto stage, auto rows, auto pow2, auto kind) {
-        hipLaunchKernelGGL((k_stage<decltype(stage)::value, double, decltype(rows)::value, decltype(pow2)::value,
-                                    decltype(kind)::value, false>),
-                           grid, block, 0, c->stream, a);
+    auto go = [&](auto stage, auto rows, auto cols, auto pow2, auto kind) {
+        constexpr int TY = decltype(rows)::value, WX = decltype(cols)::value;
+        hipLaunchKernelGGL((k_stage<decltype(stage)::value, double, TY, decltype(pow2)::value, decltype(kind)::value,
+                                    false, WX>),
+                           tile_grid(c, a, TY, WX), dim3(64 * tile_waves(TY, WX)), 0, c->stream, a);
     };
-    auto with_stage = [&](auto rows, auto pow2, auto kind) {
-        if (avg == 0) go(std::integral_constant<int, 3>{}, rows, pow2, kind);
-        else go(std::integral_constant<int, 4>{}, rows, pow2, kind);
+    auto with_stage = [&](auto rows, auto cols, auto pow2, auto kind) {
+        if (avg == 0) go(std::integral_constant<int, 3>{}, rows, cols, pow2, kind);
+        else go(std::integral_constant<int, 4>{}, rows, cols, pow2, kind);
     };
-    auto with_spacing = [&](auto rows, auto kind) {
-        if (p2) with_stage(rows, std::true_type{}, kind);
-        else with_stage(rows, std::false_type{}, kind);
+    auto with_spacing = [&](auto rows, auto cols, auto kind) {
+        if (p2) with_stage(rows, cols, std::true_type{}, kind);
+        else with_stage(rows, cols, std::false_type{}, kind);
     };
-    using Plain = std::integral_constant<int, kPlain>;
-    if (ang && vg) with_spacing(std::integral_constant<int, 4>{}, std::integral_constant<int, kAngGamma>{});
-    else if (ang) with_spacing(std::integral_constant<int, 4>{}, std::integral_constant<int, kAng>{});
-    else if (vg) with_spacing(std::integral_constant<int, 4>{}, std::integral_constant<int, kGamma>{});
-    else if (ty == 8) with_spacing(std::integral_constant<int, 8>{}, Plain{});
-    else with_spacing(std::integral_constant<int, 4>{}, Plain{});
+    using R4 = std::integral_constant<int, 4>;
+    using R8 = std::integral_constant<int, 8>;
+    using R16 = std::integral_constant<int, 16>;
+    using C32 = std::integral_constant<int, 32>;
+    using C64 = std::integral_constant<int, 64>;
+    auto with_tile = [&](auto kind) {
+        constexpr int V = decltype(kind)::value;
+        if constexpr (V == kPlain)
+            if (tile == kTile64x8) return with_spacing(R8{}, C64{}, kind);
+        if constexpr (!has_ang(V))
+            if (tile == kTile32x16) return with_spacing(R16{}, C32{}, kind);
+        if (tile == kTile32x8) return with_spacing(R8{}, C32{}, kind);
+        with_spacing(R4{}, C64{}, kind);
+    };
+    if (ang && vg) with_tile(std::integral_constant<int, kAngGamma>{});
+    else if (ang) with_tile(std::integral_constant<int, kAng>{});
+    else if (vg) with_tile(std::integral_constant<int, kGamma>{});
+    else with_tile(std::integral_constant<int, kPlain>{});
     BX_HIP(hipGetLastError());
     return BX_OK;
 }
@@ -334,47 +352,63 @@ int fused_supported(const bx_ctx *c)
     return BX_OK;
 }
 
-// The z chunk (and tile rows, 8 or 4) of the tiled kernels: they march in z
-// chunks of the interior planes (any length: nzi/m rounded up for m chunks).
-// A workgroup's time is (planes it marches) x (time per plane) + a start that
-// does not depend on the chunk (launch, the first planes of the z queue), so
-// the chunk minimises that over the rounds of workgroups each CU takes; ties
-// go to the longer chunk.  Constants in us for both stages together, from
-// sweeps of the chunk at 16^3..256^3 (MI355X):
-//   FP64, 64 x 8 tiles: one workgroup per CU (LDS), 13 per plane + 33.  96^3:
-//     chunk 10 (240 workgroups) 172 us, 16 (144) 247 us.
-//   FP64, 64 x 4 tiles: one workgroup per CU, 8.5 per plane + 30: half the
-//     rows per CU, so faster where the 8-row tiles leave CUs idle (32^3 with
-//     one plane each: 50 us against 55; 85 us with chunks of 4 planes on 8-row
-//     tiles), and slower where they fill the chip (256^3: 2.5 against 1.95 ms).
-//   Mixed, 64 x 4 tiles: several workgroups share a CU and its issue slots, so
-//     the time is (workgroups per CU) x (chunk + 2 planes), with one alone on
-//     its CU, which waits for its own latencies, counted as 1.6.  192^3: chunk
-//     28 489 us, 32 545 us; 64^3: chunk 2 56 us, 4 64 us.
-void tile_split(const bx_ctx *c, bool mixed, bool rows8, bool rows4, int *lz, int *ty)
+// The tile and z chunk of the tiled kernels: they march in z chunks of the
+// interior planes (any length: nzi/m rounded up for m chunks).  A workgroup's
+// time is (planes it marches) x (time per plane) + a start that does not
+// depend on the chunk (launch, the first planes of the z queue), so the choice
+// minimises that over the rounds of workgroups each CU takes; ties go to the
+// longer chunk and the tile listed first.  Constants in us for both stages
+// together, from sweeps of the chunk at 16^3..256^3 (MI355X):
+//   FP64, eight owner waves: one workgroup per CU (LDS), 13 per plane + 33.
+//     Tiles of 32 columns fill the lanes where the interior width is just
+//     above a multiple of 64: 96^3 interior cells 187 us in 64 x 8 tiles, 154
+//     in 32 x 16; where both fill them they take 1 % more (128^3 302, 294).
+//   FP64, four owner waves: one workgroup per CU, 8.5 per plane + 30: half the
+//     rows per CU, so faster where the wide tiles leave CUs idle (32^3 with
+//     one plane each 41 us in 64 x 4 and 38 in 32 x 8 tiles, 46 in wide ones),
+//     and slower where they fill the chip (256^3: 2.5 against 1.95 ms).
+//   Mixed, four owner waves: several workgroups share a CU and its issue
+//     slots, so the time is (workgroups per CU) x (chunk + 2 planes), with one
+//     alone on its CU, which waits for its own latencies, counted as 1.6.
+//     192^3: chunk 28 489 us, 32 545 us; 96^3 interior: 105 us in 64 x 4
+//     tiles, 85 in 32 x 8; 100 x 130 x 90: 131, 132.
+// tiles: the set to choose from (tile_bit).
+int tile_split(const bx_ctx *c, bool mixed, unsigned tiles, int *lz)
 {
     const int nzi = c->flatz ? c->nz : c->nz - 4;
+    struct Shape {
+        int tile, wx, ty;
+        double plane, start, mixed;
+    };
+    static const Shape shapes[] = {
+        {kTile64x8, 64, 8, 13.0, 33.0, 0.0},
+        {kTile32x16, 32, 16, 13.2, 33.3, 0.0},
+        {kTile64x4, 64, 4, 8.5, 30.0, 1.0},
+        {kTile32x8, 32, 8, 9.0, 28.0, 1.02},
+    };
     double best = HUGE_VAL;
-    for (int t = 8; t >= 4; t -= 4) {
-        if (t == 8 ? !rows8 : !rows4) continue;
-        const int64_t tiles = (int64_t)((c->nx - 4 + 63) / 64) * ((c->ny - 4 + t - 1) / t);
+    int at = kTile64x4;
+    *lz = nzi;
+    for (const Shape &t : shapes) {
+        if (!(tiles & tile_bit(t.tile))) continue;
+        const int64_t n = (int64_t)((c->nx - 4 + t.wx - 1) / t.wx) * ((c->ny - 4 + t.ty - 1) / t.ty);
         for (int m = 1; m <= nzi && m <= 4 * c->ncu; m++) {
             const int l = (nzi + m - 1) / m;
-            const double rounds = (double)((tiles * ((nzi + l - 1) / l) + c->ncu - 1) / c->ncu);
-            const double cost = mixed ? std::fmax(rounds, 1.6) * (l + 2)
-                                      : rounds * (t == 8 ? 13.0 * l + 33.0 : 8.5 * l + 30.0);
+            const double rounds = (double)((n * ((nzi + l - 1) / l) + c->ncu - 1) / c->ncu);
+            const double cost = mixed ? t.mixed * std::fmax(rounds, 1.6) * (l + 2) : rounds * (t.plane * l + t.start);
             if (cost < best) {
                 best = cost;
                 *lz = l;
-                *ty = t;
+                at = t.tile;
             }
         }
     }
+    return at;
 }
 
 // Default work split of the stage kernels.  The y chunk (fused_ly) only serves
-// the two-kernel variants; gravity has the 64 x 8 tiles only.  Allocates
-// nothing.
+// the two-kernel variants; gravity has the tiles of eight owner waves
+// only.  Allocates nothing.
 void fused_defaults(bx_ctx *c)
 {
     const int64_t want = 2 * 1024;
@@ -386,9 +420,9 @@ void fused_defaults(bx_ctx *c)
     }
     if (c->fused_lz == 0) {
         const bool mixed = c->prm.precision == BX_PREC_MIXED;
-        int ty = 8;
-        tile_split(c, mixed, !mixed, mixed || !c->grav_flags, &c->fused_lz, &ty);
-        c->fused_occ = ty == 8 ? 11 : 10;
+        const unsigned wide = tile_bit(kTile64x8) | tile_bit(kTile32x16);
+        const unsigned narrow = tile_bit(kTile64x4) | tile_bit(kTile32x8);
+        c->fused_occ = tile_split(c, mixed, mixed ? narrow : (c->grav_flags ? wide : wide | narrow), &c->fused_lz);
     }
 }
 

@@ -131,7 +131,7 @@ struct bx_ctx {
     bool fused_unsupported;
     bool ghosts_filled;  // ghost cells hold their donors' values (after any exact step)
     int fused_ly, fused_lz;  // y rows and z planes per wave of the stage kernels
-    int fused_occ;           // stage kernel variant (bx_tune): 0, 1, 4 two kernels; 10, 11 one tiled kernel
+    int fused_occ;           // stage kernel variant: 0, 1, 4 two kernels; from 10 one tiled kernel (Tile; bx_tune: 10, 11)
     double *eflux;           // 5 planes: y-term of fluxtmp (FP64)
     bool prof_on;
     hipEvent_t ev[6];   // per stage: before the y kernel, between the two kernels, after the x/z kernel
@@ -215,7 +215,11 @@ int launch_ghosts(bx_ctx *c, double *planes5);
 // ghosts: whether to fill the ghost cells after it (flux.f90:231)
 int launch_flux(bx_ctx *c, int avg, double dt, bool ghosts);
 int launch_tiled_flux(bx_ctx *c, int avg, double dt, double *out, unsigned int *slow, unsigned int *slow_next);
-void tile_split(const bx_ctx *c, bool mixed, bool rows8, bool rows4, int *lz, int *ty);
+// tiles of the tiled kernels (fused_occ of the fused step): columns x rows;
+// 64 x 4 and 32 x 8 have four waves of owners, the others eight
+enum Tile : int { kTile64x4 = 10, kTile64x8 = 11, kTile32x8 = 12, kTile32x16 = 13 };
+constexpr unsigned tile_bit(int tile) { return 1u << (tile - kTile64x4); }
+int tile_split(const bx_ctx *c, bool mixed, unsigned tiles, int *lz);
 int launch_avisc(bx_ctx *c);
 int launch_materialize(bx_ctx *c);
 int launch_regular_check(bx_ctx *c);

@@ -1,9 +1,14 @@
 // bx_tile.h -- one RK stage of the fused step as a single kernel: a workgroup
 // holds an x-y tile of the grid with its +-2 halo in LDS and marches in z.
 //
-// Tile: 64 x-cells (one per lane) by TY rows of outputs.  The workgroup has
-// TY+4 waves; wave w holds row r = w-2 of the tile (rows -2..TY+1, the two
-// outer rows on each side being the y-halo).  The primitives of a plane are
+// Tile: WX x-cells by TY rows of outputs.  With WX = 64 the workgroup has TY+4
+// waves, wave w with row r = w-2 of the tile (rows -2..TY+1, the two outer
+// rows on each side being the y-halo), a cell per lane.  With WX = 32 a wave
+// holds two rows, and the x-edges have waves of their own: for 16 rows again
+// 12 waves, 8 of them owners.  Grids whose interior width lies just above a
+// multiple of 64 fill the lanes of narrow tiles (tile_split chooses): at 96^3
+// interior cells the step takes 154 us in place of 187, at 160x144x128 with
+// gravity 498 in place of 572.  The primitives of a plane are
 // kept in a tile in LDS with one column of x-halo on each side; there are two
 // such tiles, for planes k and k+1.  Every row writes its primitives one
 // plane ahead, so that the tile of plane k is complete when plane k starts.
@@ -12,21 +17,22 @@
 //   A  owner rows 0..TY-1 take the z face k+1/2 from their register queue in
 //      z (the primitives of plane k from the tile, k+1 and k+2 in registers)
 //      and park the z flux difference of plane k in LDS; every row writes its
-//      primitives of plane k+1 into the other tile.  Wave r=TY+1 also takes
-//      the x-edges of the owner rows on plane k+1: columns -2,-1,0 and
-//      62..65, seven lanes per row, their primitives (columns -1 and 64 go
-//      into the plane-(k+1) tile) and x-states.
+//      primitives of plane k+1 into the other tile.  The edge wave
+//      (with WX = 64 wave r=TY+1, else one per 8 rows) takes the x-edges of
+//      the owner rows on plane k+1: columns -2,-1,0 and WX-2..WX+1, seven
+//      lanes per row, their primitives (columns -1 and WX go into the
+//      plane-(k+1) tile) and x-states.
 //   B  owner rows form their x-states from the neighbours' primitives
 //      (flux.f90:253-351, 391-479), the x-faces l-1/2 (the left plus state
-//      from the next lower lane, or column -1's for lane 0) and with face
-//      l+1/2 (next higher lane, or face 63+1/2) the x flux difference, parked
+//      from the next lower lane, or column -1's for column 0) and with face
+//      l+1/2 (next higher lane, or face WX-1/2) the x flux difference, parked
 //      in LDS; then their y-states, publishing the y-plus state (row r-1's
 //      is needed by row r's face r-1/2).  Row -1 publishes its y-plus state,
 //      row TY keeps its y-minus state.                            -- barrier
 //   C  owner rows and row TY evaluate their face y r-1/2 and publish it over
-//      the y-plus state they read (no other row reads that slot).  Wave
-//      r=TY+1 publishes the x-plus state of column -1 and evaluates face
-//      x 63+1/2 of plane k+1 (the owners read plane k's in B).    -- barrier
+//      the y-plus state they read (no other row reads that slot).  The
+//      edge wave publishes the x-plus state of column -1 and evaluates face
+//      x WX-1/2 of plane k+1 (the owners read plane k's in B).    -- barrier
 //   D  owner rows read face y r+1/2 and apply the stage update and
 //      everything pointwise up to the next stage (as the two-kernel form
 //      does).
@@ -62,16 +68,26 @@
 
 namespace bx {
 
-template <typename S, int TY, int V = kPlain>
+// A wave of a tile of WX columns holds 64 columns of one row or 32 of two.
+// Its waves: halo rows, owner rows, and the x-edges of the owner rows, 7 lanes
+// to a row, kEdgeRows rows to a wave (with 64 columns the one edge wave has a
+// halo row besides).
+constexpr int kEdgeRows = 8;
+constexpr int tile_waves(int TY, int WX)
+{
+    return WX == 64 ? TY + 4 : TY / 2 + 2 + (TY + kEdgeRows - 1) / kEdgeRows;
+}
+
+template <typename S, int TY, int V = kPlain, int WX = 64>
 struct TileLds {
-    static constexpr int RS = 66;  // row stride of the primitive tile: columns -1..64
+    static constexpr int RS = WX + 2;  // row stride of the primitive tile: columns -1..WX
     static constexpr int NF = 6 + (has_gamma(V) ? 1 : 0) + (has_ang(V) ? 2 : 0);
     S P[2][NF][(TY + 4) * RS];     // rho, u0, u1, u2, p, eps (, gamma) (, r- and angular momentum) of planes k, k+1 (tile k&1), rows -2..TY+1
-    S Sy[NF][(TY + 1) * 64];       // y-plus states of rows -1..TY-1 (index r+1), then y-face r-1/2 (index r)
+    S Sy[NF][(TY + 1) * WX];       // y-plus states of rows -1..TY-1 (index r+1), then y-face r-1/2 (index r)
     S SxL[NF][TY];                 // x-plus state of column -1, per owner row
-    S FxR[5][TY];                  // x-face flux 63+1/2, per owner row
-    double Dx[5][TY * 64];         // x flux difference of each owner cell (phase B to D)
-    double Dz[5][TY * 64];         // z flux difference of each owner cell (phase A to D)
+    S FxR[5][TY];                  // x-face flux WX-1/2, per owner row
+    double Dx[5][TY * WX];         // x flux difference of each owner cell (phase B to D)
+    double Dz[5][TY * WX];         // z flux difference of each owner cell (phase A to D)
 };
 
 template <typename S, int F, int N>
@@ -144,18 +160,20 @@ __device__ __forceinline__ Side<S> fetch_side(const S (&B)[F][N], int idx, S gam
     return s;
 }
 
-// value of the next lower lane; lane 0 takes `edge`
-template <typename T>
-__device__ __forceinline__ T from_lower(T v, T edge, int)
+// value of the next lower column; column 0 takes `edge`
+template <int WX, typename T>
+__device__ __forceinline__ T from_lower(T v, T edge, int col)
 {
-    return wave_shift_t<0x138>(v, edge);  // wave_shr:1
+    const T w = wave_shift_t<0x138>(v, edge);  // wave_shr:1
+    return WX < 64 && col == 0 ? edge : w;
 }
 
-// value of the next higher lane; lane 63 takes `edge`
-template <typename T>
-__device__ __forceinline__ T from_upper(T v, T edge, int)
+// value of the next higher column; the last column takes `edge`
+template <int WX, typename T>
+__device__ __forceinline__ T from_upper(T v, T edge, int col)
 {
-    return wave_shift_t<0x130>(v, edge);  // wave_shl:1
+    const T w = wave_shift_t<0x130>(v, edge);  // wave_shl:1
+    return WX < 64 && col == WX - 1 ? edge : w;
 }
 
 // Where a tile's row (or edge lane) at column x and row y reads its cells, and
@@ -244,11 +262,12 @@ __device__ __forceinline__ void stage_face(const Side<S> &L, const Side<S> &R, c
     else face_flux<S, dir>(L, R, F);
 }
 
-// Per-tile constants of one stage.
+// Per-tile constants of one stage; col, row: the lane's place in the tile.
 struct TileGeom {
     int nx, ny, nz;
     int64_t n, plane;
-    int x0, j0, r, lane;
+    int x0, j0, row, col;
+    int edge;  // first owner row of an edge wave, else -1
     int kb, ke;
 };
 
@@ -285,24 +304,24 @@ __device__ __forceinline__ void flux_update(const StageArgs &a, double ui[5], do
 // primitives of plane k are read back from the tile where needed, and the x
 // and z flux differences are parked in LDS until the update, to keep the
 // registers live across the barriers few.
-template <int STAGE, typename S, int TY, int V, bool W>
-__device__ __forceinline__ void tile_owner(const StageArgs &a, TileLds<S, TY, V> &L, const TileGeom &g,
+template <int STAGE, typename S, int TY, int V, bool W, int WX>
+__device__ __forceinline__ void tile_owner(const StageArgs &a, TileLds<S, TY, V, WX> &L, const TileGeom &g,
                                            unsigned int &flg, double &rmax)
 {
-    constexpr int RS = TileLds<S, TY, V>::RS;
-    const int lane = g.lane, r = g.r, nx = g.nx, ny = g.ny, nz = g.nz;
+    constexpr int RS = TileLds<S, TY, V, WX>::RS;
+    const int col = g.col, row = g.row, nx = g.nx, ny = g.ny, nz = g.nz;
     const int64_t n = g.n;
-    const int x = g.x0 + lane, y = g.j0 + r;
+    const int x = g.x0 + col, y = g.j0 + row;
     const Donor<S, W> me(a, x, y);
     const unsigned coff = me.off;
-    const AngColumn<V> col(a, min(x, nx - 1), min(y, ny - 1));
+    const AngColumn<V> ang(a, min(x, nx - 1), min(y, ny - 1));
     const bool xy_ghost = x < 2 || x > nx - 3 || y < 2 || y > ny - 3;
     const bool is_out = !xy_ghost;
     const S gamS = S(a.gam);
     auto zplane = [&](int k) -> int64_t { return Donor<S, W>::plane(a, g.plane, k); };
     auto zghost = [&](int k) -> bool { return !a.flatz && (k < 2 || k > nz - 3); };
-    const int c = (r + 2) * RS + lane + 1;  // this cell in the primitive tiles
-    const int o = r * 64 + lane;            // this cell's slot in the per-owner buffers
+    const int c = (row + 2) * RS + col + 1;  // this cell in the primitive tiles
+    const int o = row * WX + col;           // this cell's slot in the per-owner buffers
 
     W6<S> q2{};  // primitives of plane k+1 (k+2 after the z face of plane k)
     S cs0 = S(0), cs1 = S(0);
@@ -315,7 +334,7 @@ __device__ __forceinline__ void tile_owner(const StageArgs &a, TileLds<S, TY, V>
             const Raw<S> v = load_raw<STAGE, S, V>(a, zplane(k), coff);
             W6<S> w = prims<STAGE, S, V>(a, v, flg);
             me.signs(a, k, w);
-            col.momenta(v, w, flg);
+            ang.momenta(v, w, flg);
             return w;
         };
         const W6<S> t0 = at(kb - 2), t1 = at(kb - 1), t2 = at(kb), t3 = at(kb + 1);
@@ -325,7 +344,7 @@ __device__ __forceinline__ void tile_owner(const StageArgs &a, TileLds<S, TY, V>
         cs1 = sound_at<V>(t2, a);
         dir_states<2, S, V>(t1, t2, t3, cs1, xy_ghost || zghost(kb), a, zmi, zpl);
         S gz[2];
-        stage_face<S, 2, V>(zp_prev, zmi, col, Fz_prev, gz);
+        stage_face<S, 2, V>(zp_prev, zmi, ang, Fz_prev, gz);
         zp_prev = zpl;
         store_w(L.P[kb & 1], c, t2);  // plane kb
         q2 = t3;
@@ -334,7 +353,7 @@ __device__ __forceinline__ void tile_owner(const StageArgs &a, TileLds<S, TY, V>
         const Raw<S> v = load_raw<STAGE, S, V>(a, zplane(kb), coff);
         W6<S> w = prims<STAGE, S, V>(a, v, flg);
         me.signs(a, kb, w);
-        col.momenta(v, w, flg);
+        ang.momenta(v, w, flg);
         cs1 = sound_at<V>(w, a);
         store_w(L.P[kb & 1], c, w);
         if (kb + 1 < ke) nxt = load_raw<STAGE, S, V>(a, zplane(kb + 1), coff);
@@ -355,12 +374,12 @@ __device__ __forceinline__ void tile_owner(const StageArgs &a, TileLds<S, TY, V>
             nxt = load_raw<STAGE, S, V>(a, zplane(min(k + 3, nz - 1)), coff);
             q2 = prims<STAGE, S, V>(a, cur, flg);
             me.signs(a, k + 2, q2);
-            col.momenta(cur, q2, flg);
+            ang.momenta(cur, q2, flg);
             cs1 = sound_at<V>(q1, a);
             Side<S> zmi1, zpl1;
             dir_states<2, S, V>(fetch_w(L.P[t], c), q1, q2, cs1, xy_ghost || zghost(k + 1), a, zmi1, zpl1);
             S Fz1[5], gz[2];
-            stage_face<S, 2, V>(zp_prev, zmi1, col, Fz1, gz);
+            stage_face<S, 2, V>(zp_prev, zmi1, ang, Fz1, gz);
             for (int i = 0; i < 5; i++) {
                 L.Dz[i][o] = (double)Fz1[i] - (double)Fz_prev[i];
                 Fz_prev[i] = Fz1[i];
@@ -374,7 +393,7 @@ __device__ __forceinline__ void tile_owner(const StageArgs &a, TileLds<S, TY, V>
                 nxt = load_raw<STAGE, S, V>(a, zplane(min(k + 2, ke - 1)), coff);
                 W6<S> w = prims<STAGE, S, V>(a, cur, flg);
                 me.signs(a, k + 1, w);
-                col.momenta(cur, w, flg);
+                ang.momenta(cur, w, flg);
                 cs1 = sound_at<V>(w, a);
                 store_w(L.P[t ^ 1], c, w);
             }
@@ -385,24 +404,24 @@ __device__ __forceinline__ void tile_owner(const StageArgs &a, TileLds<S, TY, V>
             Side<S> xmi, xpl;
             dir_states<0, S, V>(fetch_w(L.P[t], c - 1), q0, fetch_w(L.P[t], c + 1), cs0, ghost_k, a, xmi, xpl);
             Side<S> xl;
-            xl.d = from_lower(xpl.d, L.SxL[0][r], lane);
-            xl.v[0] = from_lower(xpl.v[0], L.SxL[1][r], lane);
-            xl.v[1] = from_lower(xpl.v[1], L.SxL[2][r], lane);
-            xl.v[2] = from_lower(xpl.v[2], L.SxL[3][r], lane);
-            xl.p = from_lower(xpl.p, L.SxL[4][r], lane);
-            xl.e = from_lower(xpl.e, L.SxL[5][r], lane);
+            xl.d = from_lower<WX>(xpl.d, L.SxL[0][row], col);
+            xl.v[0] = from_lower<WX>(xpl.v[0], L.SxL[1][row], col);
+            xl.v[1] = from_lower<WX>(xpl.v[1], L.SxL[2][row], col);
+            xl.v[2] = from_lower<WX>(xpl.v[2], L.SxL[3][row], col);
+            xl.p = from_lower<WX>(xpl.p, L.SxL[4][row], col);
+            xl.e = from_lower<WX>(xpl.e, L.SxL[5][row], col);
             xl.g = gamS;
-            constexpr int NF = TileLds<S, TY, V>::NF;
-            if constexpr (has_gamma(V)) xl.g = from_lower(xpl.g, L.SxL[6][r], lane);
+            constexpr int NF = TileLds<S, TY, V, WX>::NF;
+            if constexpr (has_gamma(V)) xl.g = from_lower<WX>(xpl.g, L.SxL[6][row], col);
             if constexpr (has_ang(V)) {
-                xl.s1 = from_lower(xpl.s1, L.SxL[NF - 2][r], lane);
-                xl.s2 = from_lower(xpl.s2, L.SxL[NF - 1][r], lane);
+                xl.s1 = from_lower<WX>(xpl.s1, L.SxL[NF - 2][row], col);
+                xl.s2 = from_lower<WX>(xpl.s2, L.SxL[NF - 1][row], col);
             }
             S Fx0[5], gx[2];
-            stage_face<S, 0, V>(xl, xmi, col, Fx0, gx);  // face l-1/2
+            stage_face<S, 0, V>(xl, xmi, ang, Fx0, gx);  // face l-1/2
             for (int i = 0; i < 5; i++) {
                 // face l+1/2, as this cell has it
-                const S fx1 = from_upper(has_ang(V) && (i == 1 || i == 2) ? gx[i - 1] : Fx0[i], L.FxR[i][r], lane);
+                const S fx1 = from_upper<WX>(has_ang(V) && (i == 1 || i == 2) ? gx[i - 1] : Fx0[i], L.FxR[i][row], col);
                 L.Dx[i][o] = (double)fx1 - (double)Fx0[i];
             }
         }
@@ -411,14 +430,14 @@ __device__ __forceinline__ void tile_owner(const StageArgs &a, TileLds<S, TY, V>
             Side<S> ypl;
             dir_states<1, S, V>(fetch_w(L.P[t], c - RS), fetch_w(L.P[t], c), fetch_w(L.P[t], c + RS), cs0, ghost_k, a,
                           ymi, ypl);
-            store_side(L.Sy, (r + 1) * 64 + lane, ypl);
+            store_side(L.Sy, (row + 1) * WX + col, ypl);
         }
         __syncthreads();
         // C: face y r-1/2, published over the y-plus state of row r-1
         S Fy0[5], gy[2];
-        stage_face<S, 1, V>(fetch_side(L.Sy, r * 64 + lane, gamS), ymi, col, Fy0, gy);
+        stage_face<S, 1, V>(fetch_side(L.Sy, row * WX + col, gamS), ymi, ang, Fy0, gy);
         for (int i = 0; i < 5; i++)  // as row r-1 has it
-            L.Sy[i][r * 64 + lane] = has_ang(V) && (i == 1 || i == 2) ? gy[i - 1] : Fy0[i];
+            L.Sy[i][row * WX + col] = has_ang(V) && (i == 1 || i == 2) ? gy[i - 1] : Fy0[i];
         __syncthreads();
         // D: face y r+1/2 and the update
         if (is_out) {
@@ -430,13 +449,13 @@ __device__ __forceinline__ void tile_owner(const StageArgs &a, TileLds<S, TY, V>
             }
             for (int i = 0; i < 5; i++) {
                 // flux.f90:188-190 in the reference's order, accumulated in FP64
-                const S fy1 = L.Sy[i][(r + 1) * 64 + lane];
+                const S fy1 = L.Sy[i][(row + 1) * WX + col];
                 const double ey = (double)(S)(a.axz * ((double)fy1 - (double)Fy0[i]));
                 const double dz = a.flatz ? 0.0 : L.Dz[i][o];
                 const double s = (a.ayz * L.Dx[i][o] + ey) + a.axy * dz;
                 ft[i] = -div_by(s * a.dt, a.vol, a.inv_vol, a.vol_pow2);
             }
-            if constexpr (STAGE >= 3) flux_update<STAGE, V>(a, ui, uo, ft, fetch_w(L.P[t], c), col, cz, coff);
+            if constexpr (STAGE >= 3) flux_update<STAGE, V>(a, ui, uo, ft, fetch_w(L.P[t], c), ang, cz, coff);
             else stage_update<STAGE, S, V == kGravity>(a, ui, uo, ft, fetch_w(L.P[t], c), cz, coff, flg, rmax);
         }
     }
@@ -444,27 +463,27 @@ __device__ __forceinline__ void tile_owner(const StageArgs &a, TileLds<S, TY, V>
 
 // Halo rows -2, -1 and TY: their primitives, the y-states of rows -1 and TY,
 // and face y TY-1/2.
-template <int STAGE, typename S, int TY, int V, bool W>
-__device__ __forceinline__ void tile_halo(const StageArgs &a, TileLds<S, TY, V> &L, const TileGeom &g,
+template <int STAGE, typename S, int TY, int V, bool W, int WX>
+__device__ __forceinline__ void tile_halo(const StageArgs &a, TileLds<S, TY, V, WX> &L, const TileGeom &g,
                                           unsigned int &flg)
 {
-    constexpr int RS = TileLds<S, TY, V>::RS;
-    const int lane = g.lane, r = g.r, nx = g.nx, ny = g.ny, nz = g.nz;
-    const int x = g.x0 + lane, y = g.j0 + r;
+    constexpr int RS = TileLds<S, TY, V, WX>::RS;
+    const int col = g.col, row = g.row, nx = g.nx, ny = g.ny, nz = g.nz;
+    const int x = g.x0 + col, y = g.j0 + row;
     const Donor<S, W> me(a, x, y);
     const unsigned coff = me.off;
-    const AngColumn<V> col(a, min(x, nx - 1), min(y, ny - 1));
+    const AngColumn<V> ang(a, min(x, nx - 1), min(y, ny - 1));
     const bool xy_ghost = x < 2 || x > nx - 3 || y < 2 || y > ny - 3;
     const S gamS = S(a.gam);
     auto zplane = [&](int k) -> int64_t { return Donor<S, W>::plane(a, g.plane, k); };
     auto zghost = [&](int k) -> bool { return !a.flatz && (k < 2 || k > nz - 3); };
-    const int c = (r + 2) * RS + lane + 1;
+    const int c = (row + 2) * RS + col + 1;
     const int kb = g.kb, ke = g.ke;
     Raw<S> nxt;
     auto put = [&](int k, const Raw<S> &raw) {
         W6<S> w = prims<STAGE, S, V>(a, raw, flg);
         me.signs(a, k, w);
-        col.momenta(raw, w, flg);
+        ang.momenta(raw, w, flg);
         store_w(L.P[k & 1], c, w);
     };
     put(kb, load_raw<STAGE, S, V>(a, zplane(kb), coff));
@@ -479,47 +498,49 @@ __device__ __forceinline__ void tile_halo(const StageArgs &a, TileLds<S, TY, V> 
             put(k + 1, cur);
         }
         Side<S> ymi;
-        if (r != -2) {
+        if (row == -1 || row == TY) {
             // B: y-states of plane k
             const W6<S> w = fetch_w(L.P[t], c);
             Side<S> ypl;
             dir_states<1, S, V>(fetch_w(L.P[t], c - RS), w, fetch_w(L.P[t], c + RS), sound_at<V>(w, a),
                           xy_ghost || zghost(k), a, ymi, ypl);
-            if (r == -1) store_side(L.Sy, lane, ypl);
+            if (row == -1) store_side(L.Sy, col, ypl);
         }
         __syncthreads();
-        if (r == TY) {
+        if (row == TY) {
             S F[5], gy[2];
-            stage_face<S, 1, V>(fetch_side(L.Sy, TY * 64 + lane, gamS), ymi, col, F, gy);
+            stage_face<S, 1, V>(fetch_side(L.Sy, TY * WX + col, gamS), ymi, ang, F, gy);
             for (int i = 0; i < 5; i++)
-                L.Sy[i][TY * 64 + lane] = has_ang(V) && (i == 1 || i == 2) ? gy[i - 1] : F[i];
+                L.Sy[i][TY * WX + col] = has_ang(V) && (i == 1 || i == 2) ? gy[i - 1] : F[i];
         }
         __syncthreads();
     }
 }
 
-// Wave r=TY+1: its own halo row, and the x-edges of the owner rows one plane
-// ahead.  Lane 7*row+j holds column {-2,-1,0,62,63,64,65}[j] of owner row
-// `row`.
-template <int STAGE, typename S, int TY, int V, bool W>
-__device__ __forceinline__ void tile_edge(const StageArgs &a, TileLds<S, TY, V> &L, const TileGeom &g,
+// An edge wave: the x-edges of kEdgeRows owner rows one plane ahead (and with
+// 64 columns its own halo row TY+1).  Lane 7*i+j holds column
+// {-2,-1,0,WX-2,WX-1,WX,WX+1}[j] of owner row g.edge + i.
+template <int STAGE, typename S, int TY, int V, bool W, int WX>
+__device__ __forceinline__ void tile_edge(const StageArgs &a, TileLds<S, TY, V, WX> &L, const TileGeom &g,
                                           unsigned int &flg)
 {
-    constexpr int RS = TileLds<S, TY, V>::RS;
-    static_assert(7 * TY <= 64, "x-edge lanes of the owner rows must fit one wave");
-    const int lane = g.lane, r = g.r, nx = g.nx, ny = g.ny, nz = g.nz;
-    const int x = g.x0 + lane, y = g.j0 + r;
+    constexpr int RS = TileLds<S, TY, V, WX>::RS;
+    static_assert(7 * kEdgeRows <= 64 && (WX < 64 || TY <= kEdgeRows), "x-edge lanes of the owner rows");
+    constexpr bool kHalo = WX == 64;
+    const int lane = threadIdx.x & 63;
+    const int col = g.col, row = g.row, nx = g.nx, ny = g.ny, nz = g.nz;
+    const int x = g.x0 + col, y = g.j0 + row;
     const Donor<S, W> me(a, x, y);
     const unsigned coff = me.off;
-    const AngColumn<V> col(a, min(x, nx - 1), min(y, ny - 1));
+    const AngColumn<V> ang(a, min(x, nx - 1), min(y, ny - 1));
     const S gamS = S(a.gam);
     auto zplane = [&](int k) -> int64_t { return Donor<S, W>::plane(a, g.plane, k); };
     auto zghost = [&](int k) -> bool { return !a.flatz && (k < 2 || k > nz - 3); };
-    const int c = (r + 2) * RS + lane + 1;
+    const int c = (row + 2) * RS + col + 1;
 
-    const bool e_on = lane < 7 * TY;
-    const int erow = lane / 7, ej = lane - 7 * (lane / 7);
-    const int ecol = ej < 3 ? ej - 2 : ej + 59;
+    const int er = lane / 7, ej = lane - 7 * er, erow = g.edge + er;
+    const bool e_on = er < kEdgeRows && erow < TY;
+    const int ecol = ej < 3 ? ej - 2 : ej + WX - 5;
     const int ex = g.x0 + ecol, ey = g.j0 + erow;
     const Donor<S, W> em(a, ex, ey);
     const AngColumn<V> eang(a, min(max(ex, 0), nx - 1), min(ey, ny - 1));
@@ -537,7 +558,7 @@ __device__ __forceinline__ void tile_edge(const StageArgs &a, TileLds<S, TY, V> 
     };
     // neighbours within a row's seven lanes through whole-wave shifts (the
     // lanes whose neighbour lies in another row or outside the wave are not
-    // used: columns -1, 63 and 64 take columns -2..0 and 62..65)
+    // used: columns -1, WX-1 and WX take columns -2..0 and WX-2..WX+1)
     auto edge_states = [&](int k) {
         dir_states<0, S, V>(lane_below_w(ew), ew, lane_above_w(ew), sound_at<V>(ew, a), e_xy_ghost || zghost(k), a, emi, epl);
     };
@@ -558,21 +579,23 @@ __device__ __forceinline__ void tile_edge(const StageArgs &a, TileLds<S, TY, V> 
         }
         if (ej == 5) {
             S F[5], gx[2];
-            stage_face<S, 0, V>(xl, emi, eang, F, gx);  // face 63+1/2, as column 63 has it
+            stage_face<S, 0, V>(xl, emi, eang, F, gx);  // face WX-1/2, as column WX-1 has it
             for (int i = 0; i < 5; i++) L.FxR[i][erow] = has_ang(V) && (i == 1 || i == 2) ? gx[i - 1] : F[i];
         }
     };
 
     const int kb = g.kb, ke = g.ke;
-    Raw<S> nxt;
+    Raw<S> nxt{};
     auto put = [&](int k, const Raw<S> &raw) {
         W6<S> w = prims<STAGE, S, V>(a, raw, flg);
         me.signs(a, k, w);
-        col.momenta(raw, w, flg);
+        ang.momenta(raw, w, flg);
         store_w(L.P[k & 1], c, w);
     };
-    put(kb, load_raw<STAGE, S, V>(a, zplane(kb), coff));
-    if (kb + 1 < ke) nxt = load_raw<STAGE, S, V>(a, zplane(kb + 1), coff);
+    if (kHalo) {
+        put(kb, load_raw<STAGE, S, V>(a, zplane(kb), coff));
+        if (kb + 1 < ke) nxt = load_raw<STAGE, S, V>(a, zplane(kb + 1), coff);
+    }
     Raw<S> enxt{};
     if (e_on) {
         edge_prims(kb, load_raw<STAGE, S, V>(a, zplane(kb), eoff));
@@ -585,9 +608,11 @@ __device__ __forceinline__ void tile_edge(const StageArgs &a, TileLds<S, TY, V> 
         const bool more = k + 1 < ke;
         if (more) {
             // A: primitives of plane k+1, its own row and the x-edges
-            const Raw<S> cur = nxt;
-            nxt = load_raw<STAGE, S, V>(a, zplane(min(k + 2, ke - 1)), coff);
-            put(k + 1, cur);
+            if (kHalo) {
+                const Raw<S> cur = nxt;
+                nxt = load_raw<STAGE, S, V>(a, zplane(min(k + 2, ke - 1)), coff);
+                put(k + 1, cur);
+            }
             if (e_on) {
                 const Raw<S> ecur = enxt;
                 enxt = load_raw<STAGE, S, V>(a, zplane(min(k + 2, ke - 1)), eoff);
@@ -601,39 +626,43 @@ __device__ __forceinline__ void tile_edge(const StageArgs &a, TileLds<S, TY, V> 
     }
 }
 
-// One stage over the tile (bx, by) of 64 x TY outputs and the z planes of chunk bz.
+// One stage over the tile (bx, by) of WX x TY outputs and the z planes of chunk bz.
 // V: StageKind.  W: some side is a wall (read only with gmap).
-template <int STAGE, typename S, int TY, int V, bool W>
-__device__ __forceinline__ void tile_stage(const StageArgs &a, TileLds<S, TY, V> &L, unsigned bx, unsigned by,
+template <int STAGE, typename S, int TY, int V, bool W, int WX>
+__device__ __forceinline__ void tile_stage(const StageArgs &a, TileLds<S, TY, V, WX> &L, unsigned bx, unsigned by,
                                            unsigned bz)
 {
+    constexpr int RPW = 64 / WX, kHalos = 2 / RPW, kOwners = TY / RPW;  // rows of a wave; waves of a halo; owner waves
     TileGeom g;
     g.nx = a.nx;
     g.ny = a.ny;
     g.nz = a.nz;
     g.n = a.n;
     g.plane = (int64_t)a.nx * a.ny;
-    g.x0 = 2 + (int)bx * 64;
+    g.x0 = 2 + (int)bx * WX;
     g.j0 = 2 + (int)by * TY;
-    g.r = wave_id() - 2;  // tile row of this wave, -2..TY+1 (uniform)
-    g.lane = threadIdx.x & 63;
+    // waves in order of their rows -2..TY+1, with 32 columns then the edge waves
+    const int w = wave_id(), lane = threadIdx.x & 63;
+    g.row = RPW * w - 2 + (RPW > 1 ? lane / WX : 0);
+    g.col = lane & (WX - 1);
+    g.edge = WX == 64 ? (w == TY + 3 ? 0 : -1) : (w >= kOwners + 2 * kHalos ? kEdgeRows * (w - kOwners - 2 * kHalos) : -1);
     g.kb = a.zlo + (int)bz * a.lz;
     g.ke = min(g.kb + a.lz, a.zhi);
     if (g.kb >= g.ke) return;  // uniform over the workgroup
     unsigned int flg = 0;
     double rmax = 0.0;
-    if (g.r >= 0 && g.r < TY) {
+    if (w >= kHalos && w < kHalos + kOwners) {
         // The owner rows are the critical path between the barriers; each SIMD
         // holds two of them and one halo or edge wave, which is older and would
         // win the issue arbitration by age: the owners issue first
         // (2.06 -> 2.00 ms per step at 256^3).
         __builtin_amdgcn_s_setprio(1);
-        tile_owner<STAGE, S, TY, V, W>(a, L, g, flg, rmax);
+        tile_owner<STAGE, S, TY, V, W, WX>(a, L, g, flg, rmax);
     }
-    else if (g.r == TY + 1) tile_edge<STAGE, S, TY, V, W>(a, L, g, flg);
-    else tile_halo<STAGE, S, TY, V, W>(a, L, g, flg);
+    else if (g.edge >= 0) tile_edge<STAGE, S, TY, V, W, WX>(a, L, g, flg);
+    else tile_halo<STAGE, S, TY, V, W, WX>(a, L, g, flg);
     if (flg) atomicOr(a.flags, flg);
-    if (STAGE == 2) wave_max_to(rmax, rate_slot(a, bx + by + bz + (unsigned)g.r));
+    if (STAGE == 2) wave_max_to(rmax, rate_slot(a, bx + by + bz + (unsigned)w));
 }
 
 // The two-level corner ghosts after the corrector's ghost fill.  The exact
