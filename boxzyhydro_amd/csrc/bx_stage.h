@@ -68,6 +68,10 @@ struct StageArgs {
     int nd2;
     const int32_t *d2cell;
     double *d2ubar;
+    // stage 2 of the tiled kernels with walls: workgroups ahead of the tiles'
+    // (a multiple of 8) that take these ghosts (0: a kernel of their own does)
+    int ncorner;
+    const int32_t *d2dst, *d2sign;
     // gravity (the kernels' G variant): 3 planes of the force that source()
     // applies to each cell (source.f90:148-182), every ghost holding its
     // donor's force with the ghost's momentum sign flips, so that a ghost's

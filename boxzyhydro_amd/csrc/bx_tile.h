@@ -778,4 +778,17 @@ __device__ __forceinline__ double corner_update(const StageArgs &a, int j, const
          div_by(snd + fabs(v2), a.ds[2], a.inv_ds[2], a.ds_pow2[2]);
 }
 
+// one corner ghost by a workgroup of at least three waves
+__device__ __forceinline__ void corner_block(const StageArgs &a, int j, double (*F)[2][5])
+{
+    const int d = wave_id();
+    double rt = 0.0;
+    unsigned int flg = 0;
+    if (d < 3) corner_faces(a, j, d, threadIdx.x & 63, F, flg);
+    __syncthreads();
+    if (threadIdx.x == 0) rt = corner_update(a, j, F, a.d2dst[j], a.d2sign[j], flg);
+    if (flg) atomicOr(a.flags, flg);
+    if (d == 0) wave_max_to(rt, rate_slot(a, (unsigned)j));
+}
+
 }  // namespace bx
