@@ -455,7 +455,9 @@ int bx_create(const bx_params *prm, int32_t device, bx_ctx **out)
     std::memset(c->hsc, 0, sizeof(DevScalars));
     const size_t mb = sizeof(unsigned long long) * kMaxSlots * kMaxStride;
     if ((e = hipMalloc((void **)&c->dmax, mb)) != hipSuccess) return fail(e, "hipMalloc maxima");
-    if ((e = hipHostMalloc((void **)&c->hmax, mb, hipHostMallocDefault)) != hipSuccess) return fail(e, "hipHostMalloc");
+    if ((e = hipMemsetAsync(c->dmax, 0, mb, c->stream)) != hipSuccess) return fail(e, "hipMemset");
+    if ((e = hipHostMalloc((void **)&c->hmax, sizeof(unsigned long long), hipHostMallocDefault)) != hipSuccess)
+        return fail(e, "hipHostMalloc");
     if ((e = hipStreamSynchronize(c->stream)) != hipSuccess) return fail(e, "hipStreamSynchronize");
     *out = c;
     return BX_OK;

@@ -38,8 +38,6 @@ __device__ __forceinline__ unsigned long long *max_slot(unsigned long long *slot
     return slots + (blockIdx.x % kMaxSlots) * kMaxStride;
 }
 
-static __global__ void k_clear_max(unsigned long long *slots) { slots[threadIdx.x * kMaxStride] = 0ull; }
-
 // 1-based (ix,iy,iz) of cell c (utils.f90:191-194 inverse)
 __device__ __forceinline__ void coords(int64_t c, int nx, int ny, int &ix, int &iy, int &iz)
 {

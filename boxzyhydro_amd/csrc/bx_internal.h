@@ -156,7 +156,8 @@ struct bx_ctx {
     int64_t stage_len;
     struct bx::HostPipe *pipe;  // pinned slots of large host transfers (bx_transfer.hip), or null
 
-    unsigned long long *dmax, *hmax;  // slots of a grid-wide maximum (bx_cells.h), and their pinned mirror
+    unsigned long long *dmax, *hmax;  // slots of a grid-wide maximum (bx_cells.h), and a pinned word for it
+    bool max_open;                    // a kernel has added to the slots since they were last taken and cleared
 
     bx::DevScalars *dsc;   // device scalars
     bx::DevScalars *hsc;   // pinned host mirror
@@ -249,6 +250,7 @@ enum Pass : int {
     kEndNext = 5,     // kEnd, then the next step's kStateRate
 };
 int launch_pass(bx_ctx *c, int pass, double dt, bool filled);
+int begin_max(bx_ctx *c);
 int read_max(bx_ctx *c, double *out);
 int fused_prepare(bx_ctx *c);
 // `pairs` pairs of fused steps from the current state (device dt, flags

@@ -35,6 +35,7 @@ struct PassArgs {
     double g0, g1, g2;
     const double *gf;
     int ang, disk, all;                // disk: nz == 1 with tables; all: take ghost cells too
+    int inner;                         // a later pass of the step sets muc before any reader
     double dx, dy, dz;
     EosDev e;
     unsigned long long *rate;          // kMaxSlots slots
@@ -114,9 +115,11 @@ __device__ __forceinline__ void store_cell(const PassArgs &a, int64_t c, const C
         if (GHOST || __double_as_longlong(x.U[f]) != __double_as_longlong(U0[f])) a.cons[f * a.n + c] = x.U[f];
     if (PASS != kState && PASS != kStateRate)
         for (int d = 0; d < 3; d++) a.u[d * a.n + c] = x.v[d];
+    if (TAB && PASS == kEndNext && !a.disk) return;  // the next step's kBeforeFlux sets them before any reader
     a.p[c] = x.p;
     if (TAB || a.ad) a.ad[c] = ad;
-    if constexpr (TAB) a.mucp[c] = mu;
+    if constexpr (TAB)
+        if (!a.inner) a.mucp[c] = mu;
 }
 
 // Each thread takes CPT cells a block apart (coalesced), so that the table
@@ -285,11 +288,10 @@ static void go_ghosts(bx_ctx *c, int pass, const PassArgs &a)
 // pass fills them (no chained ghosts).
 int launch_pass(bx_ctx *c, int pass, double dt, bool filled)
 {
-    if (pass == kEndNext || pass == kStateRate) {
-        hipLaunchKernelGGL(k_clear_max, dim3(1), dim3(kMaxSlots), 0, c->stream, c->dmax);
-        BX_HIP(hipGetLastError());
-    }
-    const PassArgs a = pass_args(c, dt, filled);
+    if (pass == kEndNext || pass == kStateRate)
+        if (int rc = begin_max(c)) return rc;
+    PassArgs a = pass_args(c, dt, filled);
+    a.inner = !filled && (pass == kBeforeFlux || pass == kAfterFlux) ? 1 : 0;
     if (!filled && c->nghost > 0) {
         if (c->eos) go_ghosts<true>(c, pass, a);
         else go_ghosts<false>(c, pass, a);
