@@ -409,6 +409,7 @@ __device__ __forceinline__ void cell_fluxes(const Tube &t, const StageArgs &sa, 
     q.u2 = x.v[2];
     q.p = x.p;
     q.e = floor_at(x.U[4] - 0.5 * q.d * (q.u0 * q.u0 + q.u1 * q.u1 + q.u2 * q.u2), t.seps);
+    no_minus_zero(q);
     q.g = 0.0;
     double Fx[5];
     x_faces(sa, q, sound_of(q, t.gam), ghost, Fx);

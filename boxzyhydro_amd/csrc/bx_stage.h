@@ -196,6 +196,15 @@ enum StageKind : int {
 constexpr bool has_gamma(int v) { return v == kGamma || v == kAngGamma; }
 constexpr bool has_ang(int v) { return v == kAng || v == kAngGamma; }
 
+// the velocity with +0 for -0, as dir_states takes it
+template <typename T>
+__device__ __forceinline__ void no_minus_zero(W6<T> &w)
+{
+    w.u0 += T(0);
+    w.u1 += T(0);
+    w.u2 += T(0);
+}
+
 template <typename T>
 __device__ __forceinline__ T div_by(T x, double d, double inv, int pow2)
 {
@@ -281,8 +290,9 @@ __device__ __forceinline__ T comp(const W6<T> &w, int j)
 // slopes from (wm, wc, wp) unless the cell is a ghost (zero slopes).
 // The reference forms each state as (q + c*s) + 0 (the transverse terms are
 // exact zeros); that equals (q + 0) + c*s bit for bit, so the centre values
-// are made canonical once (no -0) and a zero slope of either sign gives the
-// same state (slope_fz).  For the same reason a ghost cell zeroes the two
+// are canonical (no -0: prims and the walls' sign flips see to the velocity;
+// rho, p and eps are not negative) and a zero slope of either sign gives the
+// same state (slope2_fz, whose factor 2 the coefficients c take up).  For the same reason a ghost cell zeroes the two
 // coefficients c instead of its six slopes (c*s is then a zero for the
 // finite slopes of finite data).  lp and lm enter only as 1-lp and -1-lm,
 // where a zero of either sign gives the same value, so the hardware maximum
@@ -291,19 +301,18 @@ template <int d, typename T, int V = kPlain>
 __device__ __forceinline__ void dir_states(const W6<T> &wm, const W6<T> &wc, const W6<T> &wp, T sound, bool ghost,
                                            const StageArgs &a, Side<T> &mi, Side<T> &pl)
 {
-    const T su0 = slope_fz(wm.u0, wc.u0, wp.u0);
-    const T su1 = slope_fz(wm.u1, wc.u1, wp.u1);
-    const T su2 = slope_fz(wm.u2, wc.u2, wp.u2);
-    const T sp = slope_fz(wm.p, wc.p, wp.p);
-    const T sd = slope_fz(wm.d, wc.d, wp.d);
-    const T se = slope_fz(wm.e, wc.e, wp.e);
+    const T su0 = slope2_fz(wm.u0, wc.u0, wp.u0);
+    const T su1 = slope2_fz(wm.u1, wc.u1, wp.u1);
+    const T su2 = slope2_fz(wm.u2, wc.u2, wp.u2);
+    const T sp = slope2_fz(wm.p, wc.p, wp.p);
+    const T sd = slope2_fz(wm.d, wc.d, wp.d);
+    const T se = slope2_fz(wm.e, wc.e, wp.e);
     const T ud = comp(wc, d);
     const T dt = T(a.dt);
     const T lp = div_by(Arith<T>::fmax(ud + sound, T(0)) * dt, a.ds[d], a.inv_ds[d], a.ds_pow2[d]);
     const T lm = div_by(Arith<T>::fmin(ud - sound, T(0)) * dt, a.ds[d], a.inv_ds[d], a.ds_pow2[d]);
-    const T cm = ghost ? T(0) : T(0.5) * (T(-1) - lm), cp = ghost ? T(0) : T(0.5) * (T(1) - lp);
-    const T z = T(0);  // transverse terms: 0*cc with cc=dt*half/ds > 0
-    const T d0 = wc.d + z, v0 = wc.u0 + z, v1 = wc.u1 + z, v2 = wc.u2 + z, p0 = wc.p + z, e0 = wc.e + z;
+    const T cm = ghost ? T(0) : T(0.25) * (T(-1) - lm), cp = ghost ? T(0) : T(0.25) * (T(1) - lp);
+    const T d0 = wc.d, v0 = wc.u0, v1 = wc.u1, v2 = wc.u2, p0 = wc.p, e0 = wc.e;
     mi.d = d0 + cm * sd;
     pl.d = d0 + cp * sd;
     mi.v[0] = v0 + cm * su0;
@@ -317,8 +326,8 @@ __device__ __forceinline__ void dir_states(const W6<T> &wm, const W6<T> &wc, con
     mi.e = e0 + cm * se;
     pl.e = e0 + cp * se;
     if constexpr (has_gamma(V)) {
-        const T sg = slope_fz(wm.g, wc.g, wp.g);
-        const T g0 = wc.g + z;
+        const T sg = slope2_fz(wm.g, wc.g, wp.g);
+        const T g0 = wc.g + T(0);
         mi.g = g0 + cm * sg;
         pl.g = g0 + cp * sg;
     } else {
@@ -342,9 +351,9 @@ template <typename T>
 __device__ __forceinline__ T sound_of(const W6<T> &w, double gam)
 {
     if constexpr (sizeof(T) == 8) {
-        const double x = Arith<T>::div(w.p * T(gam), w.d);
+        const double x = w.p * gam;
         double r;
-        sqrt_n<1>(&x, &r);
+        root_quotients<1>(&x, &w.d, &r);
         return r;
     } else {
         return Arith<T>::root(Arith<T>::div(w.p * T(gam), w.d));
@@ -505,6 +514,7 @@ __device__ __forceinline__ W6<S> prims(const StageArgs &a, const Raw<S> &v, unsi
         w.p = STAGE == 1 ? (float)(e * a.gm1) : v.p;
         if (fabs(v0) > a.vlimit || fabs(v1) > a.vlimit || fabs(v2) > a.vlimit) flg |= FLAG_CLAMP;
     }
+    no_minus_zero(w);
     return w;
 }
 
@@ -518,9 +528,9 @@ template <int V, typename T>
 __device__ __forceinline__ T sound_at(const W6<T> &w, const StageArgs &a)
 {
     if constexpr (has_gamma(V)) {
-        const double x = w.p * w.g / w.d;
+        const double x = w.p * w.g;
         double r;
-        sqrt_n<1>(&x, &r);
+        root_quotients<1>(&x, &w.d, &r);
         return r;
     } else {
         return sound_of(w, a.gam);

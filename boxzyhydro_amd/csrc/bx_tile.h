@@ -219,6 +219,7 @@ struct Donor {
             w.u1 = flip(w.u1, sy);
             const bool fz = a.gmap && !a.flatz && axis_flip(k, a.nz, a.wall[4], a.wall[5]);
             w.u2 = flip(w.u2, fz ? 0x80000000u : 0u);
+            no_minus_zero(w);
         }
     }
 };

@@ -1,0 +1,60 @@
+"""Limiter, sound speeds and shared quotients of the flux kernels against the
+oracle where their short forms hand over to the plain operations: pressures
+and densities over the whole exponent range, zeros of either sign, equal
+neighbours and extrema, bit for bit."""
+from __future__ import annotations
+
+import dataclasses
+import os
+import sys
+
+import numpy as np
+import pytest
+
+from boxzyhydro_amd import ics
+from boxzyhydro_amd.hydro import HydroGrid
+from boxzyhydro_amd.params import box_params
+
+sys.path.insert(0, os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "oracle"))
+import pyoracle as po  # noqa: E402
+
+
+def _same(a, b):
+    a, b = np.asarray(a), np.asarray(b)
+    nan = np.isnan(a)
+    return np.array_equal(nan, np.isnan(b)) and np.array_equal(a[~nan].view(np.uint64), b[~nan].view(np.uint64))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["wide_p", "wide_rho", "wide_both", "zeros", "plateaus", "tiny_gamma"])
+@pytest.mark.parametrize("size", [(36, 36, 36), (70, 21, 14)])
+def test_flux_at_the_edges(size, kind):
+    prm = dataclasses.replace(box_params(8), nx=size[0], ny=size[1], nz=size[2], dx=0.5, dy=0.3, dz=0.7, vlimit=1e300,
+                              small_rho=1e-200, small_eps=1e-250)
+    rng = np.random.default_rng(11)
+    n = prm.ngrid
+    ic = {k: v.copy() for k, v in ics.box_ic(prm, seed=4, sigma_cells=1.0).items()}
+    if kind in ("wide_p", "wide_both"):
+        ic["p"] *= 10.0 ** rng.uniform(-140, 55, n)
+    if kind in ("wide_rho", "wide_both"):
+        ic["cons"][:, 0] *= 10.0 ** rng.uniform(-120, 55, n)
+    if kind == "zeros":
+        ic["u"] *= rng.integers(0, 2, (n, 3))
+        ic["u"] *= rng.choice([-1.0, 1.0], (n, 3))  # zeros of both signs
+    if kind == "plateaus":
+        for k in ("u", "p", "cons"):
+            ic[k] = np.round(ic[k], 1)
+        ic["cons"][:, 0] = np.maximum(ic["cons"][:, 0], 0.1)
+        ic["p"] = np.maximum(ic["p"], 0.1)
+    if kind == "tiny_gamma":
+        ic["adindx"] = 10.0 ** rng.uniform(-150, 3, n)
+    g, o = HydroGrid(prm, ic), po.OracleGrid(prm, ic)
+    print(f"flux edges {kind} {size}", flush=True)
+    for avg, dt in ((0, 1e-3), (1, 1e-3)):
+        g.dt = dt
+        g.copy_old()
+        o.copy_old()
+        g.flux(avg)
+        o.flux(avg, dt)
+        assert _same(g.download()["cons"], o.cons), avg
+    g.close()
