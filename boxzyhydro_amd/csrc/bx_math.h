@@ -191,14 +191,14 @@ __device__ __forceinline__ void div_shared(const double *a, double b, double *q)
         for (int i = 0; i < N; i++) q[i] = a[i] / b;
 }
 
-// sqrt(a[i]/b[i]) (i < N) with both roundings, for FP64: the quotient as in
-// div_shared, the root as in sqrt_n.  One range check serves all: operands in
-// [2^-299, 2^300] keep the quotients within both ranges.  (A NaN operand passes
-// the check where the other operands do and gives NaN.)
+// sqrt(a[i]/b[i]) (i < N) with both roundings, for FP64, on operands in
+// [2^-299, 2^300]: the quotient as in div_shared (and then in sqrt_n's range),
+// the root as in sqrt_n.  lo, hi: the least and greatest operand; a NaN operand
+// does not enter them and gives NaN.
 template <int N>
-__device__ __forceinline__ void root_quotients(const double *a, const double *b, double *r)
+__device__ __forceinline__ void root_quotients_core(const double *a, const double *b, double *r, double &lo,
+                                                    double &hi)
 {
-    double lo = a[0], hi = a[0];
     for (int i = 0; i < N; i++) {
         const double y0 = __builtin_amdgcn_rcp(b[i]);
         const double y1 = __builtin_fma(y0, __builtin_fma(-b[i], y0, 1.0), y0);
@@ -211,11 +211,40 @@ __device__ __forceinline__ void root_quotients(const double *a, const double *b,
         const double h1 = __builtin_fma(h0, rr, h0), s1 = __builtin_fma(s0, rr, s0);
         const double s2 = __builtin_fma(__builtin_fma(-s1, s1, v), h1, s1);
         r[i] = __builtin_fma(__builtin_fma(-s2, s2, v), h1, s2);
-        lo = __builtin_fmin(lo, i == 0 ? b[i] : __builtin_fmin(a[i], b[i]));
-        hi = __builtin_fmax(hi, i == 0 ? b[i] : __builtin_fmax(a[i], b[i]));
+        const double l = __builtin_fmin(a[i], b[i]), h = __builtin_fmax(a[i], b[i]);
+        lo = i == 0 ? l : __builtin_fmin(lo, l);
+        hi = i == 0 ? h : __builtin_fmax(hi, h);
     }
-    if (__builtin_expect(!(lo >= 0x1p-299 && hi <= 0x1p300), 0))
+}
+constexpr double kRootLo = 0x1p-299, kRootHi = 0x1p300;
+template <int N>
+__device__ __forceinline__ void root_quotients(const double *a, const double *b, double *r)
+{
+    double lo, hi;
+    root_quotients_core<N>(a, b, r, lo, hi);
+    if (__builtin_expect(!(lo >= kRootLo && hi <= kRootHi), 0))
         for (int i = 0; i < N; i++) r[i] = __builtin_sqrt(a[i] / b[i]);
+}
+
+// The signal speeds of one face (flux.f90:583-585): ap = max(0, vr+cr, vl+cl),
+// am = max(0, -(vr-cr), -(vl-cl)) with c = sqrt(g p/d), as the reference's
+// comparisons give them.  The hardware maximum gives the same but for NaN and
+// for a -0 that a comparison with +0 lets through, which only -(v-c) can be
+// (at v = c).  Operands of the roots outside their range, and faces where the
+// product of both v-c is a zero or NaN, take the comparisons.
+__device__ __forceinline__ void hll_speeds(const double gp[2], const double d[2], double vl, double vr, double &ap,
+                                           double &am)
+{
+    double c[2], lo, hi;  // right, left
+    root_quotients_core<2>(gp, d, c, lo, hi);
+    const double er = vr - c[0], el = vl - c[1];
+    ap = __builtin_fmax(__builtin_fmax(vr + c[0], 0.0), vl + c[1]);
+    am = __builtin_fmax(__builtin_fmax(-er, 0.0), -el);
+    if (__builtin_expect(!(lo >= kRootLo && hi <= kRootHi && __builtin_fabs(er * el) > 0.0), 0)) {
+        const double cr = __builtin_sqrt(gp[0] / d[0]), cl = __builtin_sqrt(gp[1] / d[1]);
+        ap = vmax(vmax(0.0, vr + cr), vl + cl);
+        am = vmax(vmax(0.0, -(vr - cr)), -(vl - cl));
+    }
 }
 
 // flux.f90:512-590 for one face: L = plus state of the cell below the face,
@@ -249,19 +278,16 @@ __device__ __forceinline__ void face_flux(const Side<T> &L, const Side<T> &R, T 
     fr[3] = (dir == 2 ? R.p : zero) + sr[3] * vr;
     fr[4] = (sr[4] + R.p) * vr;
     // flux_hll, flux.f90:583-589
-    T cr, cl;
+    T ap, am;
     if constexpr (sizeof(T) == 8) {
-        const double num[2] = {R.g * R.p, L.g * L.p}, den[2] = {R.d, L.d};
-        double rt[2];
-        root_quotients<2>(num, den, rt);
-        cr = rt[0];
-        cl = rt[1];
+        const double gp[2] = {R.g * R.p, L.g * L.p}, d[2] = {R.d, L.d};
+        hll_speeds(gp, d, vl, vr, ap, am);
     } else {
-        cr = Arith<T>::root(Arith<T>::div(R.g * R.p, R.d));
-        cl = Arith<T>::root(Arith<T>::div(L.g * L.p, L.d));
+        const T cr = Arith<T>::root(Arith<T>::div(R.g * R.p, R.d));
+        const T cl = Arith<T>::root(Arith<T>::div(L.g * L.p, L.d));
+        ap = vmax(vmax(zero, vr + cr), vl + cl);
+        am = vmax(vmax(zero, -(vr - cr)), -(vl - cl));
     }
-    const T ap = vmax(vmax(zero, vr + cr), vl + cl);
-    const T am = vmax(vmax(zero, -(vr - cr)), -(vl - cl));
     const T apam = ap * am;
     const T den = ap + am;
     if constexpr (sizeof(T) == 8) {
@@ -311,11 +337,9 @@ __device__ __forceinline__ void face_flux_ang(const Side<double> &L, const Side<
                           R.e + 0.5 * R.d * (R.v[0] * R.v[0] + R.v[1] * R.v[1] + R.v[2] * R.v[2])};
     const double vl = L.v[dir], vr = R.v[dir];
     // flux_hll, flux.f90:583-589
-    const double gp[2] = {R.g * R.p, L.g * L.p}, den[2] = {R.d, L.d};
-    double rt[2];
-    root_quotients<2>(gp, den, rt);
-    const double ap = vmax(vmax(0.0, vr + rt[0]), vl + rt[1]);
-    const double am = vmax(vmax(0.0, -(vr - rt[0])), -(vl - rt[1]));
+    const double gp[2] = {R.g * R.p, L.g * L.p}, d[2] = {R.d, L.d};
+    double ap, am;
+    hll_speeds(gp, d, vl, vr, ap, am);
     const double apam = ap * am;
     auto numerator = [&](int i, double pl, double pr) {
         const double fl = pl + sl[i] * vl, fr = pr + sr[i] * vr;

@@ -58,3 +58,25 @@ def test_flux_at_the_edges(size, kind):
         o.flux(avg, dt)
         assert _same(g.download()["cons"], o.cons), avg
     g.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("speed", [2.0, -2.0])
+def test_flux_at_sonic_faces(speed):
+    """v = c and v = -c exactly, where -(v-c) is a -0, next to gas at rest."""
+    prm = dataclasses.replace(box_params(8), nx=24, ny=14, nz=12, dx=0.5, dy=0.5, dz=0.5)
+    n = prm.ngrid
+    rng = np.random.default_rng(5)
+    u = speed * rng.integers(0, 2, (n, 3))
+    ic = {"cons": np.ones((n, 5)), "u": u, "p": np.full(n, 4.0), "adindx": np.ones(n)}  # c = 2
+    ic["cons"][:, 1:4] = u
+    ic["cons"][:, 4] = 6.0 + 0.5 * (u * u).sum(1)
+    g, o = HydroGrid(prm, ic), po.OracleGrid(prm, ic)
+    g.dt = 0.02
+    for avg in (0, 1):
+        g.copy_old()
+        o.copy_old()
+        g.flux(avg)
+        o.flux(avg, 0.02)
+        assert _same(g.download()["cons"], o.cons), avg
+    g.close()
