@@ -439,14 +439,21 @@ __device__ __forceinline__ void tile_owner(const StageArgs &a, TileLds<S, TY, V,
         stage_face<S, 1, V>(fetch_side(L.Sy, row * WX + col, gamS), ymi, ang, Fy0, gy);
         for (int i = 0; i < 5; i++)  // as row r-1 has it
             L.Sy[i][row * WX + col] = has_ang(V) && (i == 1 || i == 2) ? gy[i - 1] : Fy0[i];
+        // the update's loads go out before the barrier and run under it (coff is
+        // a cell of the plane for every lane)
+        const int64_t cz = (int64_t)k * g.plane;  // an interior plane
+        S ri[5], ro[5];
+        for (int i = 0; i < 5; i++) {
+            ri[i] = elem<S>(a.uin, (int64_t)i * n + cz, coff);
+            ro[i] = STAGE == 2 || STAGE == 4 ? elem<S>(a.uold, (int64_t)i * n + cz, coff) : S(0);
+        }
         __syncthreads();
         // D: face y r+1/2 and the update
         if (is_out) {
-            const int64_t cz = (int64_t)k * g.plane;  // an interior plane, and coff an interior cell's
             double ui[5], uo[5], ft[5];
             for (int i = 0; i < 5; i++) {
-                ui[i] = elem<S>(a.uin, (int64_t)i * n + cz, coff);
-                uo[i] = STAGE == 2 || STAGE == 4 ? (double)elem<S>(a.uold, (int64_t)i * n + cz, coff) : 0.0;
+                ui[i] = ri[i];
+                uo[i] = ro[i];
             }
             for (int i = 0; i < 5; i++) {
                 // flux.f90:188-190 in the reference's order, accumulated in FP64
