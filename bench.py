@@ -142,8 +142,8 @@ def timed_run(prm, ic, precision, steps, warmup, tile=None, mode=None):
 
 
 def graph_cost(steps_small: int, steps_box: int, n: int):
-    """Wall time per step of the fused step taken one at a time (a host
-    synchronisation per step) and replayed from captured graphs, on the Sod
+    """Wall time per step of the fused step in BX_STEP_FUSED (runs of steps
+    enqueued one by one) and replayed from captured graphs, on the Sod
     tube (404x8x4 with ghosts, launch-bound) and on the n^3 box."""
     from boxzyhydro_amd import ics
     from boxzyhydro_amd import native as nv
@@ -405,7 +405,7 @@ B_STATE_TAB = 64.0  # tabulated state(): read rho, E, u (5 x 8 B), write p, adin
 def walls_cost(n: int, steps: int, warmup: int, outflow_ms: float):
     """The headline box with walls on every side, the reference's shipped
     in.nml (utils.f90:338-403): the same graph-replayed fused step, whose
-    ghost fill also writes the 16 two-level corner ghosts; ms per step
+    corrector launch also takes the 16 two-level corner ghosts; ms per step
     against the outflow box's."""
     import dataclasses
 
@@ -577,8 +577,8 @@ def options_cost(n: int, steps: int):
             "potential": {"exact_step_ms": pot, "fused_step_ms": pot_fused, "graph_step_ms": pot_graph,
                           "plain_graph_step_ms": plain_graph, "graph_over_plain_graph": pot_graph / plain_graph,
                           "exact_over_graph": pot / pot_graph,
-                          "note": f"BX_GRAV_POTENTIAL alone, {kf} fused steps after 4 untimed; fused = one step "
-                                  "per host round trip, graph = captured step pairs; plain = the same box "
+                          "note": f"BX_GRAV_POTENTIAL alone, {kf} fused steps after 4 untimed; fused = steps "
+                                  "enqueued in runs, graph = captured step pairs; plain = the same box "
                                   "without gravity"},
             "note": "gravity = calc_gforce + external_grav before source(tphase,1) each step; the sequential "
                     "mass moments (bit-identical to a one-thread reference) run on one wave"}
@@ -724,7 +724,7 @@ def main() -> int:
                    "source": f"{tfile}: rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE passes of this workload, "
                              f"scaled by a plain copy's counters (measured there, not in this run)"}
     step_achieved = value * B_STEP_FP64
-    out["roofline"] = {"scope": "the main-loop step (both stage kernels, the ghost fills, the dt kernel), "
+    out["roofline"] = {"scope": "the main-loop step (both stage kernels), "
                                 "replayed from hipGraphs; 200 algorithmic bytes per cell-update",
                        "bound": "hbm", "achieved": step_achieved / 1e9, "peak": HBM_PEAK / 1e9, "unit": "GB/s",
                        "frac": step_achieved / HBM_PEAK,

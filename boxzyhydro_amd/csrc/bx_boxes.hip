@@ -10,10 +10,11 @@
 //     bodies of the one-kernel-per-subroutine path (bx_cells.h), for the first
 //     step and for any step from a state that is not regular;
 //   - on a regular state, and where the ghosts' donors over a pair of
-//     set_ghost_cells calls are interior cells (any walls), fused steps: the wave bodies of the fused stage kernels (bx_waves.h) over the
-//     grid, the workgroup's waves taking the virtual waves of those kernels'
-//     grids; a step that meets an irregular branch is redone with the exact
-//     sequence from U^n.
+//     set_ghost_cells calls are interior cells (any walls; with chained donors
+//     in the 8-wave build only), fused steps: the wave bodies of the two-kernel
+//     stage (bx_waves.h) over the grid, the workgroup's waves taking the
+//     virtual waves of those kernels' grids; a step that meets an irregular
+//     branch is redone with the exact sequence from U^n.
 // Both give the single-grid step's bits, and so the reference's.  A pass
 // that reads neighbours (ghost fills, faces, stage updates) is separated from
 // its producer by a workgroup barrier; pointwise passes run back to back on

@@ -73,8 +73,10 @@ int bx_ghost_table(const bx_params *prm, int64_t *nghost, int64_t *nscratch, int
 /* Host <-> device copies of the reference's global arrays (Fortran layout).
  * Any pointer may be NULL to skip that array.  upload also sets
  * cons_old = cons, as init_conditions.f90:69-77 does.  The first transfer of
- * a multi-field array allocates a device staging buffer of at most 64 MiB,
- * which the context keeps until bx_destroy. */
+ * a multi-field array allocates a device staging buffer of at most 24 MiB,
+ * which the context keeps until bx_destroy.  Arrays of 8 MB and more move in
+ * chunks through pinned buffers filled by a few worker threads of the
+ * process. */
 int bx_upload(bx_ctx *ctx, const double *cons, const double *u, const double *p, const double *adindx);
 int bx_download(bx_ctx *ctx, double *cons, double *u, double *p, double *adindx);
 int bx_download_cons_old(bx_ctx *ctx, double *cons_old);
@@ -93,17 +95,20 @@ int bx_avisc(bx_ctx *ctx, double *qq);            /* avisc.f90:4-26; qq(3,ngrid)
  * Advances up to `nsteps` steps or until *time >= endtime.  *time, *dtold and
  * *step carry the driver's scalars between calls (main.f90:196-198: start
  * with dtold=0, step=0).  dts (may be NULL) receives each step's full dt.
- * mode BX_STEP_EXACT runs the reference call sequence kernel by kernel;
+ * mode BX_STEP_EXACT runs the reference call sequence (the pointwise calls
+ * between two ghost fills or fluxes in one pass);
  * BX_STEP_FUSED runs two fused stencil kernels per step and falls back to the
  * exact sequence for any step that meets a low-density cell (rho<1e-4), the
- * speed clamp, or a first step whose ghosts are not yet filled.
- * BX_STEP_GRAPH computes what BX_STEP_FUSED computes, bit for bit, with dt
- * formed on the device: runs of up to 32 steps that cannot reach endtime
- * (each dt is at most 1.1x the last) are replayed from a captured hipGraph of
- * two fused steps, with one host synchronisation per run instead of per step.
+ * speed clamp, or a first step whose ghosts are not yet filled.  Runs of up to
+ * 32 steps that cannot reach endtime (each dt is at most 1.1x the last) are
+ * enqueued with dt formed on the device and one host synchronisation per run.
  * A run in which a step met an irregular branch is undone and its steps are
- * taken one at a time as in BX_STEP_FUSED; the first step and the steps near
- * endtime are always taken one at a time.
+ * taken one at a time; the first step and the steps near endtime are always
+ * taken one at a time.  Runs keep a copy of the state at their start; without
+ * memory for it FUSED takes its steps one at a time and GRAPH returns an
+ * error.
+ * BX_STEP_GRAPH computes what BX_STEP_FUSED computes, bit for bit, with the
+ * runs replayed from a captured hipGraph of two fused steps.
  * All modes give results bit-identical to the reference in FP64.
  * Returns the number of steps taken in *taken. */
 #define BX_STEP_EXACT 0
@@ -123,7 +128,7 @@ int bx_step(bx_ctx *ctx, int32_t mode, int32_t nsteps, double endtime, double *t
  * context supplies the grid, the parameters and the ghost table; its own
  * state is not read or written.  U*, p* and the other intermediates live in
  * a static device array of BX_STATIC_MAX_CELLS * BX_STATIC_BYTES_PER_CELL
- * bytes (plus 256) that each GPU holds until the process ends: ngrid above
+ * bytes (plus 2304) that each GPU holds until the process ends: ngrid above
  * BX_STATIC_MAX_CELLS is refused (BX_ERR_ARG).  Every call on one GPU shares
  * that array, so calls that overlap on one GPU (other streams, other
  * threads) race.  rate_out and flags_out are DEVICE words (either may be
@@ -154,10 +159,11 @@ int bx_graph_step_count(const bx_ctx *ctx, int64_t *count);
  * be NULL.  A diagnostic with no reference counterpart. */
 int bx_step_counts(const bx_ctx *ctx, int64_t *fused, int64_t *exact);
 
-/* Work split of the fused stage kernels.  variant 11 (the FP64 default) and
- * 10 (the mixed form's default): one kernel per stage over x-y tiles of
- * 64 x 8 (11) or 64 x 4 (10) cells marching z_chunk planes in z (y_chunk
- * unused).  Variants 0, 1, 4: two kernels per stage, a y-direction kernel of
+/* Work split of the fused stage kernels.  Variants 11 and 10: one kernel per
+ * stage over x-y tiles of 64 x 8 (11) or 64 x 4 (10) cells marching z_chunk
+ * planes in z (y_chunk unused).  Until this is called a rule on the grid's
+ * size chooses the chunk and the tile, 32 x 16 and 32 x 8 cells among them.
+ * Variants 0, 1, 4: two kernels per stage, a y-direction kernel of
  * y_chunk rows per wave and an x/z kernel of z_chunk planes per wave (1:
  * y-term loaded one plane early; 4: built for four waves per SIMD).  Used by
  * the autotuner; results do not change.  With gravity configured only
@@ -230,8 +236,8 @@ int bx_batch_sync(bx_batch *b, double *ms);
 /* Gangs: the ntubes costliest tubes (by the steps of the last finished run,
  * else by the set-up estimate) are each split over `members` workgroups
  * (contiguous ranges of cells; the two cells at either side of a range are
- * exchanged through device-coherent accesses, with two device-counter
- * barriers per step).  members x ntubes must not exceed the compute units.
+ * exchanged through device-coherent accesses; the members meet once per
+ * step).  members x ntubes must not exceed the compute units.
  * members < 2 or ntubes = 0 turns gangs off.  Results do not change.  No
  * reference counterpart: the reference runs one tube per process. */
 int bx_batch_gang(bx_batch *b, int32_t members, int32_t ntubes);
@@ -252,8 +258,9 @@ int bx_batch_dts(bx_batch *b, double *dts);
  * Batched grids.  Many independent grids of uneven size (3-D boxes, or flat-z
  * slabs with nz < 6) in one persistent launch: one workgroup steps one grid
  * as bx_step(BX_STEP_FUSED) does (the exact call sequence of main.f90:211-555
- * where required, fused steps on a regular state with shallow ghosts),
- * taking grids from a queue ordered by estimated cost, largest first.  No reference
+ * where required, fused steps on a regular state; grids whose walls chain
+ * ghost donors take fused steps in the 8-wave work split, the default, and
+ * exact ones in the others), taking grids from a queue ordered by estimated cost, largest first.  No reference
  * counterpart to cite: the reference runs one grid per process, and each grid
  * here returns what that process returns, bit for bit.  Every grid has its
  * own bx_params (size, spacings, walls, gammafix, cfl, small_rho/eps,
