@@ -169,9 +169,9 @@ __device__ __forceinline__ double velocity_and_ekin(const double U[5], double v[
 // courant.f90:20-21 for one cell
 __device__ __forceinline__ double rate_of(const Tube &t, double rho, double p, double u0, double u1, double u2)
 {
-    const double sq = t.gam * p / rho;
+    const double gp = t.gam * p;
     double sound;
-    sqrt_n<1>(&sq, &sound);
+    root_quotients<1>(&gp, &rho, &sound);
     const double num[3] = {sound + fabs(u0), sound + fabs(u1), sound + fabs(u2)};
     if (t.dx == t.dy && t.dy == t.dz) {
         double r[3];

@@ -450,7 +450,7 @@ __device__ __forceinline__ void tile_owner(const StageArgs &a, TileLds<S, TY, V,
         __syncthreads();
         // D: face y r+1/2 and the update
         if (is_out) {
-            double ui[5], uo[5], ft[5];
+            double ui[5], uo[5], sd[5], ft[5];
             for (int i = 0; i < 5; i++) {
                 ui[i] = ri[i];
                 uo[i] = ro[i];
@@ -461,8 +461,10 @@ __device__ __forceinline__ void tile_owner(const StageArgs &a, TileLds<S, TY, V,
                 const double ey = (double)(S)(a.axz * ((double)fy1 - (double)Fy0[i]));
                 const double dz = a.flatz ? 0.0 : L.Dz[i][o];
                 const double s = (a.ayz * L.Dx[i][o] + ey) + a.axy * dz;
-                ft[i] = -div_by(s * a.dt, a.vol, a.inv_vol, a.vol_pow2);
+                sd[i] = s * a.dt;
             }
+            div_all<5>(sd, a.vol, a.inv_vol, a.vol_pow2, ft);
+            for (int i = 0; i < 5; i++) ft[i] = -ft[i];
             if constexpr (STAGE >= 3) flux_update<STAGE, V>(a, ui, uo, ft, fetch_w(L.P[t], c), ang, cz, coff);
             else stage_update<STAGE, S, V == kGravity>(a, ui, uo, ft, fetch_w(L.P[t], c), cz, coff, flg, rmax);
         }

@@ -236,9 +236,9 @@ __device__ __forceinline__ void stage_update(const StageArgs &a, const double *u
             const double ekin = 0.5 * ((double)Us[1] * w0 + (double)Us[2] * w1 + (double)Us[3] * w2);
             p = floor_at((double)Us[4] - ekin, a.seps) * a.gm1;
         }
-        const double sq = a.gam * p / rr;
+        const double gp = a.gam * p;
         double snd1;
-        sqrt_n<1>(&sq, &snd1);
+        root_quotients<1>(&gp, &rr, &snd1);
         const double rt = div_by(snd1 + fabs(w0), a.ds[0], a.inv_ds[0], a.ds_pow2[0]) +
                           div_by(snd1 + fabs(w1), a.ds[1], a.inv_ds[1], a.ds_pow2[1]) +
                           div_by(snd1 + fabs(w2), a.ds[2], a.inv_ds[2], a.ds_pow2[2]);
