@@ -46,6 +46,7 @@
 #include <string>
 #include <vector>
 
+#include "bx_gang.h"
 #include "bx_stage.h"
 
 namespace bx {
@@ -313,35 +314,6 @@ __device__ __forceinline__ bool gang_max(GangCtx &g, double &r, int *s_ok, doubl
     __syncthreads();
     r = *s_r;
     return *s_ok != 0;
-}
-
-// The range of segments and cells a workgroup takes of a tube.
-struct Range {
-    int nseg, s0, s1;      // segments [s0, s1) of nseg
-    int c_lo, c_hi;        // output cells [c_lo, c_hi)
-    bool left, right;      // whether another member holds the segment before / after
-};
-
-template <bool GANG>
-__device__ __forceinline__ Range tube_range(int nx, const GangCtx &g)
-{
-    Range r;
-    r.nseg = (nx - 4 + kSegOut - 1) / kSegOut;
-    r.s0 = 0;
-    r.s1 = r.nseg;
-    r.c_lo = 0;
-    r.c_hi = nx;
-    if (GANG) {
-        const int per = (r.nseg + g.p - 1) / g.p;
-        r.s0 = min(r.nseg, g.member * per);
-        r.s1 = min(r.nseg, r.s0 + per);
-        r.c_lo = g.member == 0 ? 0 : r.s0 * kSegOut + 2;
-        r.c_hi = g.member == g.p - 1 ? nx : r.s1 * kSegOut + 2;
-    }
-    const bool any = r.s0 < r.s1;  // a short tube leaves the last members without segments
-    r.left = GANG && any && g.member > 0;
-    r.right = GANG && any && g.member < g.p - 1;
-    return r;
 }
 
 // Courant maximum of the set-up (main.f90:232-241) over cells [c_lo, c_hi):
@@ -644,7 +616,7 @@ template <int W, bool GANG>
 __device__ __forceinline__ void run_tube(const BatchArgs &a, const Tube &t, int ti, GangCtx &g, double *red, int *s_ok,
                          double *s_r, unsigned *sflag, double (*ext)[9][2], double (*X)[9][4], double (*Y)[9][4])
 {
-    const Range r = tube_range<GANG>(t.nx, g);
+    const Range r = GANG ? tube_range(t.nx, g.member, g.p) : tube_range(t.nx, 0, 1);
     const int sp0 = r.s0 - (r.left ? 1 : 0), sp1 = r.s1 + (r.right ? 1 : 0);
     if (sp1 - sp0 <= W) {  // a wave per segment: the tube stays in registers
         run_tube_regs<W, GANG>(a, t, ti, g, r, red, s_ok, s_r, sflag, X, Y);

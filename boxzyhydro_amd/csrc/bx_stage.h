@@ -7,12 +7,11 @@
 
 #include <type_traits>
 
+#include "bx_gang.h"
 #include "bx_internal.h"
 #include "bx_math.h"
 
 namespace bx {
-
-constexpr int kSegOut = 60;  // output cells per wave row
 
 // Element of an array addressed as a wave-uniform element offset `u` from the
 // base plus a per-lane 32-bit byte offset: the compiler then forms one uniform
