@@ -504,6 +504,7 @@ struct bx_boxes {
     int32_t *fsrc = nullptr, *fsign = nullptr, *d2dst = nullptr, *d2src = nullptr, *d2sign = nullptr;
     int64_t *cell0 = nullptr, *reg0 = nullptr;  // first cell of each grid (nbox+1), first double of its region
     double *stage = nullptr;                    // device staging of bx_boxes_result
+    size_t stage_bytes = 0;
     bx::HostPipe *pipe = nullptr;
     double *t_out = nullptr;
     int *steps_out = nullptr;
@@ -987,7 +988,8 @@ int bx_boxes_result(bx_boxes *b, double *cons, double *u, double *p, double *tim
         const int64_t most = 5 * b->cells;  // the largest array
         if (!b->stage) {
             const size_t bytes = sizeof(double) * (size_t)most;
-            BX_HIP(hipMalloc((void **)&b->stage, bytes < bx::kPipeMin ? bytes : bx::pipe_stage_bytes()));
+            b->stage_bytes = bytes < bx::kPipeMin ? bytes : bx::pipe_stage_bytes();
+            BX_HIP(hipMalloc((void **)&b->stage, b->stage_bytes));
         }
         struct {
             double *out;
@@ -996,7 +998,7 @@ int bx_boxes_result(bx_boxes *b, double *cons, double *u, double *p, double *tim
         for (auto &w : want) {
             if (!w.out) continue;
             BoxRows r{b, w.first, w.k};
-            const bx::PipeChunk ch{box_rows_get, nullptr, nullptr, 0};
+            const bx::PipeChunk ch{box_rows_get, nullptr, nullptr, b->stage_bytes};
             if (int rc = bx::pipe_download(&b->pipe, b->device, b->stream, (char *)w.out,
                                            sizeof(double) * (size_t)(w.k * b->cells), sizeof(double) * (size_t)w.k, ch,
                                            &r))
