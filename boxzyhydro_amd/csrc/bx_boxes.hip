@@ -753,7 +753,7 @@ int bx_boxes_create(int32_t nbox, const bx_params *prm, const double *endtime, c
         b.ayz = q.dy * q.dz;
         b.axz = q.dx * q.dz;
         b.vol = q.dx * q.dy * q.dz;
-        b.fusable = gp.ok ? 1 : 0;
+        b.fusable = gp.ok && bx::tile_fits(q.nx, q.ny, sizeof(double)) ? 1 : 0;  // the wave bodies have such offsets too
         b.zlo = b.flatz ? 0 : 2;
         b.zhi = b.flatz ? q.nz : q.nz - 2;
         b.ly = 32;  // rows and planes per virtual wave (32x32 measured fastest of 8..32)

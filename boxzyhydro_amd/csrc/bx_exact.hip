@@ -84,18 +84,19 @@ __global__ __launch_bounds__(kThreads) void k_ang_old(int64_t n, int nx, int ny,
     cons_old[2 * n + c] = m2;
 }
 
-// flux.f90:6-230 cell by cell, for a call whose tiled kernel met a value
-// outside its range (*slow set): every cell again from the same inputs.
+// flux.f90:6-230 cell by cell: for grids that the tiles do not serve (slow
+// null), and for a call whose tiled kernel met a value outside its range (*slow
+// set), every cell again from the same inputs.
 template <bool ANG>
-__global__ __launch_bounds__(kThreads) void k_flux_slow(const unsigned int *__restrict__ slow, int64_t n, int nx,
-                                                       int ny, int nz, bool flatz, const double *__restrict__ cons,
-                                                       const double *__restrict__ u, const double *__restrict__ p,
-                                                       const double *__restrict__ ad,
-                                                       const double *__restrict__ cons_old, double *__restrict__ out,
-                                                       int avg, double dt, double dx, double dy, double dz,
-                                                       double srho, double seps, AngGrid ang)
+__global__ __launch_bounds__(kThreads) void k_flux_cells(const unsigned int *__restrict__ slow, int64_t n, int nx,
+                                                        int ny, int nz, bool flatz, const double *__restrict__ cons,
+                                                        const double *__restrict__ u, const double *__restrict__ p,
+                                                        const double *__restrict__ ad,
+                                                        const double *__restrict__ cons_old, double *__restrict__ out,
+                                                        int avg, double dt, double dx, double dy, double dz,
+                                                        double srho, double seps, AngGrid ang)
 {
-    if (*slow == 0u) return;
+    if (slow && *slow == 0u) return;
     for (int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; c < n; c += (int64_t)gridDim.x * blockDim.x)
         flux_cell<ANG>(n, c, nx, ny, nz, flatz, cons, u, p, ad, cons_old, out, avg, dt, dx, dy, dz, srho, seps, ang);
 }
@@ -272,12 +273,17 @@ static int flux_kernels(bx_ctx *c, int avg, double dt)
 {
     double *out = c->states;
     const AngGrid ang{c->prm.dx, c->prm.dy, c->prm.yoffset};
-    unsigned int *slow = &c->dsc->slow[c->nflux & 1], *next = &c->dsc->slow[(c->nflux + 1) & 1];
-    c->nflux++;
-    if (int rc = launch_tiled_flux(c, avg, dt, out, slow, next)) return rc;
-    hipLaunchKernelGGL(k_flux_slow<ANG>, dim3(std::min(reduce_blocks(c->n), 256u)), dim3(kThreads), 0, c->stream, slow,
-                       c->n, c->nx, c->ny, c->nz, c->flatz, c->cons, c->u, c->p, c->adindx, c->cons_old, out, avg, dt,
-                       c->prm.dx, c->prm.dy, c->prm.dz, c->prm.small_rho, c->prm.small_eps, ang);
+    unsigned int *slow = nullptr;
+    if (tile_fits(c, sizeof(double))) {
+        slow = &c->dsc->slow[c->nflux & 1];
+        unsigned int *next = &c->dsc->slow[(c->nflux + 1) & 1];
+        c->nflux++;
+        if (int rc = launch_tiled_flux(c, avg, dt, out, slow, next)) return rc;
+    }
+    hipLaunchKernelGGL(k_flux_cells<ANG>, dim3(std::min(blocks_for(c->n, kThreads), 4096u)), dim3(kThreads), 0,
+                       c->stream, slow, c->n, c->nx, c->ny, c->nz, c->flatz, c->cons, c->u, c->p, c->adindx,
+                       c->cons_old, out, avg, dt, c->prm.dx, c->prm.dy, c->prm.dz, c->prm.small_rho, c->prm.small_eps,
+                       ang);
     BX_HIP(hipGetLastError());
     if (c->nscratch > 0) {
         hipLaunchKernelGGL(k_flux_ghosts<ANG>, dim3(blocks_for(c->nghost, kThreads)), dim3(kThreads), 0, c->stream,

@@ -357,6 +357,9 @@ int fused_supported(const bx_ctx *c)
     if (c->nscratch > 0 && !c->fghost_ok)
         return set_error(BX_ERR_UNSUPPORTED, "fused step needs the ghost donors of a pair of set_ghost_cells calls "
                                              "to resolve to interior cells within two levels");
+    if (!tile_fits(c, c->prm.precision == BX_PREC_MIXED ? sizeof(float) : sizeof(double)))
+        return set_error(BX_ERR_UNSUPPORTED, "fused step: an x-y plane is beyond the stage kernels' 32-bit offsets or "
+                                             "launch grid");
     if (c->grav[0] != 0.0 || c->grav[1] != 0.0 || c->grav[2] != 0.0)
         return set_error(BX_ERR_UNSUPPORTED, "fused step assumes zero gravity");
     if (c->prm.fluxangmom) return set_error(BX_ERR_UNSUPPORTED, "fused step fluxes linear momentum (fluxangmom off)");

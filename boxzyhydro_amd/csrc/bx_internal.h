@@ -220,6 +220,15 @@ int launch_tiled_flux(bx_ctx *c, int avg, double dt, double *out, unsigned int *
 // 64 x 4 and 32 x 8 have four waves of owners, the others eight
 enum Tile : int { kTile64x4 = 10, kTile64x8 = 11, kTile32x8 = 12, kTile32x16 = 13 };
 constexpr unsigned tile_bit(int tile) { return 1u << (tile - kTile64x4); }
+// Whether the stage kernels reach every cell of a grid with elements of `size`
+// bytes: they address a cell by its plane and a 32-bit byte offset within it,
+// and the rows of tiles (at least 4 rows of cells each) are the launch's y
+// dimension.
+inline bool tile_fits(int64_t nx, int64_t ny, size_t size)
+{
+    return nx * ny <= (int64_t)(((uint64_t)1 << 32) / size) && (ny - 4 + 3) / 4 <= 65535;
+}
+inline bool tile_fits(const bx_ctx *c, size_t size) { return tile_fits(c->nx, c->ny, size); }
 int tile_split(const bx_ctx *c, bool mixed, unsigned tiles, int *lz);
 int launch_avisc(bx_ctx *c);
 int launch_materialize(bx_ctx *c);
