@@ -16,14 +16,18 @@ from typing import Iterable, List, Tuple
 from . import native as nv
 
 # (y rows, z planes, variant): the two-kernel stages (variants 0, 1, 4) and
-# the one-kernel tiled stages (variants 10, 11; y rows unused)
+# one-kernel tiled stages (variants 10, 11; y rows unused)
 DEFAULT_CANDIDATES = (list(itertools.product((16, 32, 64), (16, 32, 64), (0, 1, 4))) +
                       list(itertools.product((64,), (16, 32, 64), (10, 11))))
 
 
 def tune_step(grid, candidates: Iterable[Tuple[int, int, int]] = DEFAULT_CANDIDATES, steps: int = 3,
               warmup: int = 1) -> Tuple[Tuple[int, int, int], List[Tuple[Tuple[int, int, int], float]]]:
-    """Return (best candidate, [(candidate, seconds per step), ...])."""
+    """Return (best candidate, [(candidate, seconds per step), ...]).  The
+    library's own choice for the grid is timed before the default candidates,
+    so that tuning does not leave a grid slower than it was untouched."""
+    if candidates is DEFAULT_CANDIDATES:
+        candidates = [grid.default_split()] + DEFAULT_CANDIDATES
     results = []
     for cand in candidates:
         grid.tune(*cand)

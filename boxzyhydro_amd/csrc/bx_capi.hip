@@ -1117,15 +1117,28 @@ extern "C" int bx_tune(bx_ctx *c, int32_t y_chunk, int32_t z_chunk, int32_t occu
 {
     if (!c) return set_error(BX_ERR_ARG, "bx_tune: null context");
     if (y_chunk < 1 || z_chunk < 1) return set_error(BX_ERR_ARG, "bx_tune: chunks must be >= 1");
-    if (occupancy != 0 && occupancy != 1 && occupancy != 4 && !(occupancy >= 10 && occupancy <= 11))
-        return set_error(BX_ERR_ARG, "bx_tune: variant 0, 1, 4, 10 or 11");
-    if (c->grav_flags && occupancy != 11)
-        return set_error(BX_ERR_UNSUPPORTED, "bx_tune: with gravity the fused step has the 64 x 8 tiled kernel only "
-                                             "(variant 11)");
+    if (occupancy != 0 && occupancy != 1 && occupancy != 4 && !(occupancy >= kTile64x4 && occupancy <= kTile32x16))
+        return set_error(BX_ERR_ARG, "bx_tune: variant 0, 1, 4 or 10 to 13");
+    if (c->prm.precision == BX_PREC_MIXED && occupancy == kTile32x16)
+        return set_error(BX_ERR_UNSUPPORTED, "bx_tune: the mixed form has no 32 x 16 tiles (variant 13)");
+    if (c->grav_flags && occupancy != kTile64x8 && occupancy != kTile32x16)
+        return set_error(BX_ERR_UNSUPPORTED, "bx_tune: with gravity the fused step has the 64 x 8 and 32 x 16 tiles "
+                                             "only (variant 11 or 13)");
     c->fused_ly = y_chunk;
     c->fused_lz = z_chunk;
     c->fused_occ = occupancy;
     drop_step_graphs(c);
+    return BX_OK;
+}
+
+extern "C" int bx_default_split(const bx_ctx *c, int32_t *y_chunk, int32_t *z_chunk, int32_t *variant)
+{
+    if (!c || !y_chunk || !z_chunk || !variant) return set_error(BX_ERR_ARG, "bx_default_split: null argument");
+    int ly, lz, tile;
+    default_split(c, &ly, &lz, &tile);
+    *y_chunk = ly;
+    *z_chunk = lz;
+    *variant = tile;
     return BX_OK;
 }
 

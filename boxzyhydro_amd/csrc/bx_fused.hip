@@ -424,23 +424,30 @@ int tile_split(const bx_ctx *c, bool mixed, unsigned tiles, int *lz)
     return at;
 }
 
-// Default work split of the stage kernels.  The y chunk (fused_ly) only serves
-// the two-kernel variants; gravity has the tiles of eight owner waves
-// only.  Allocates nothing.
-void fused_defaults(bx_ctx *c)
+// The rule's work split of the stage kernels for a grid.  The y chunk only
+// serves the two-kernel variants; gravity has the tiles of eight owner waves
+// only.
+void default_split(const bx_ctx *c, int *ly, int *lz, int *tile)
 {
     const int64_t want = 2 * 1024;
     const int nzi = c->flatz ? c->nz : c->nz - 4;
-    if (c->fused_ly == 0) {
-        int ly = 64;
-        while (ly > 8 && (int64_t)((c->nx - 4 + 63) / 64) * nzi * ((c->ny - 4 + ly - 1) / ly) < want) ly /= 2;
-        c->fused_ly = ly;
-    }
+    *ly = 64;
+    while (*ly > 8 && (int64_t)((c->nx - 4 + 63) / 64) * nzi * ((c->ny - 4 + *ly - 1) / *ly) < want) *ly /= 2;
+    const bool mixed = c->prm.precision == BX_PREC_MIXED;
+    const unsigned wide = tile_bit(kTile64x8) | tile_bit(kTile32x16);
+    const unsigned narrow = tile_bit(kTile64x4) | tile_bit(kTile32x8);
+    *tile = tile_split(c, mixed, mixed ? narrow : (c->grav_flags ? wide : wide | narrow), lz);
+}
+
+// The context's split: the rule's unless bx_tune chose one.  Allocates nothing.
+void fused_defaults(bx_ctx *c)
+{
+    int ly, lz, tile;
+    default_split(c, &ly, &lz, &tile);
+    if (c->fused_ly == 0) c->fused_ly = ly;
     if (c->fused_lz == 0) {
-        const bool mixed = c->prm.precision == BX_PREC_MIXED;
-        const unsigned wide = tile_bit(kTile64x8) | tile_bit(kTile32x16);
-        const unsigned narrow = tile_bit(kTile64x4) | tile_bit(kTile32x8);
-        c->fused_occ = tile_split(c, mixed, mixed ? narrow : (c->grav_flags ? wide : wide | narrow), &c->fused_lz);
+        c->fused_lz = lz;
+        c->fused_occ = tile;
     }
 }
 

@@ -131,7 +131,7 @@ struct bx_ctx {
     bool fused_unsupported;
     bool ghosts_filled;  // ghost cells hold their donors' values (after any exact step)
     int fused_ly, fused_lz;  // y rows and z planes per wave of the stage kernels
-    int fused_occ;           // stage kernel variant: 0, 1, 4 two kernels; from 10 one tiled kernel (Tile; bx_tune: 10, 11)
+    int fused_occ;           // stage kernel variant: 0, 1, 4 two kernels; from 10 one tiled kernel (Tile)
     double *eflux;           // 5 planes: y-term of fluxtmp (FP64)
     bool prof_on;
     hipEvent_t ev[6];   // per stage: before the y kernel, between the two kernels, after the x/z kernel
@@ -230,6 +230,7 @@ inline bool tile_fits(int64_t nx, int64_t ny, size_t size)
 }
 inline bool tile_fits(const bx_ctx *c, size_t size) { return tile_fits(c->nx, c->ny, size); }
 int tile_split(const bx_ctx *c, bool mixed, unsigned tiles, int *lz);
+void default_split(const bx_ctx *c, int *ly, int *lz, int *tile);
 int launch_avisc(bx_ctx *c);
 int launch_materialize(bx_ctx *c);
 int launch_regular_check(bx_ctx *c);

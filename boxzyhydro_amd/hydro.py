@@ -244,8 +244,15 @@ class HydroGrid:
         """Work split of the fused step's stage kernels (bx_tune): rows per
         wave of the y-kernel, planes per wave of the x/z kernel or of the
         tiled stage kernel, and the variant (0, 1, 4: two kernels per stage;
-        10, 11: one tiled kernel).  Results unchanged."""
+        10 to 13: one tiled kernel).  Results unchanged."""
         nv.check(nv.lib().bx_tune(self._h, y_chunk, z_chunk, occupancy), "bx_tune")
+
+    def default_split(self) -> Tuple[int, int, int]:
+        """The arguments of ``tune`` that the library's own rule chooses for
+        this grid (what an untuned grid takes)."""
+        v = [ctypes.c_int32() for _ in range(3)]
+        nv.check(nv.lib().bx_default_split(self._h, *[ctypes.byref(x) for x in v]), "bx_default_split")
+        return v[0].value, v[1].value, v[2].value
 
     def profile(self, enable: int = -1):
         """Event timing of the fused stage kernels: enable=1 start, 0 stop,

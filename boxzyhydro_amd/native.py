@@ -100,6 +100,7 @@ _SIGS = {
     "bx_graph_step_count": [_VP, ctypes.POINTER(ctypes.c_int64)],
     "bx_step_counts": [_VP, ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(ctypes.c_int64)],
     "bx_tune": [_VP, _I32, _I32, _I32],
+    "bx_default_split": [_VP, ctypes.POINTER(_I32), ctypes.POINTER(_I32), ctypes.POINTER(_I32)],
     "bx_profile": [_VP, _I32, _DP, ctypes.POINTER(ctypes.c_int64)],
     "bx_sync": [_VP],
     "bx_batch_check": [_I32, ctypes.POINTER(BxParams), _DP, _DP, ctypes.POINTER(_I32)],

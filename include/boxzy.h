@@ -159,23 +159,26 @@ int bx_graph_step_count(const bx_ctx *ctx, int64_t *count);
  * be NULL.  A diagnostic with no reference counterpart. */
 int bx_step_counts(const bx_ctx *ctx, int64_t *fused, int64_t *exact);
 
-/* Work split of the fused stage kernels.  Variants 11 and 10: one kernel per
- * stage over x-y tiles of 64 x 8 (11) or 64 x 4 (10) cells marching z_chunk
- * planes in z (y_chunk unused).  Until this is called a rule on the grid's
- * size chooses the chunk and the tile, 32 x 16 and 32 x 8 cells among them.
+/* Work split of the fused stage kernels.  Variants 10 to 13: one kernel per
+ * stage over x-y tiles of 64 x 4 (10), 64 x 8 (11), 32 x 8 (12) or 32 x 16
+ * (13, FP64 only) cells marching z_chunk planes in z (y_chunk unused).  Until
+ * this is called a rule on the grid's size chooses among them.
  * Variants 0, 1, 4: two kernels per stage, a y-direction kernel of
  * y_chunk rows per wave and an x/z kernel of z_chunk planes per wave (1:
  * y-term loaded one plane early; 4: built for four waves per SIMD).  Used by
  * the autotuner; results do not change.  With gravity configured only
- * variant 11 is accepted (BX_ERR_UNSUPPORTED otherwise), and configuring
- * gravity returns another tuned variant to the default. */
+ * variants 11 and 13 are accepted (BX_ERR_UNSUPPORTED otherwise), and
+ * configuring gravity returns another tuned variant to the default. */
 int bx_tune(bx_ctx *ctx, int32_t y_chunk, int32_t z_chunk, int32_t variant);
+/* The rule's choice for this grid, whatever bx_tune was given since: bx_tune
+ * with these values returns to it. */
+int bx_default_split(const bx_ctx *ctx, int32_t *y_chunk, int32_t *z_chunk, int32_t *variant);
 
 /* Event timing of the fused stage kernels on the context's stream.
  * enable=1 starts (and clears), 0 stops, -1 only reads.  kernel_ms[4]
  * receives the summed durations of the y-direction and the x/z kernel of
  * stage 1, then of stage 2, over *steps steps; with one kernel per stage
- * (variants 10, 11) the y-direction entries are ~0 and the x/z entries hold
+ * (variants 10 to 13) the y-direction entries are ~0 and the x/z entries hold
  * the stage kernels. */
 int bx_profile(bx_ctx *ctx, int32_t enable, double *kernel_ms, int64_t *steps);
 
