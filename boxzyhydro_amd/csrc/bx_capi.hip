@@ -970,7 +970,6 @@ static int fused_loop(bx_ctx *c, int32_t nsteps, double endtime, double *time, d
 {
     int rc;
     int32_t k = 0;
-    int32_t single = 0;  // steps to take one at a time (after an undone chunk or an irregular step)
     // While fused_valid holds, hsc->rate[0] is the Courant rate of the
     // current state (from the regularity check or the last fused step).
     while (k < nsteps && *time < endtime && *step < 1000000) {
@@ -1004,20 +1003,20 @@ static int fused_loop(bx_ctx *c, int32_t nsteps, double endtime, double *time, d
                 c->state_in_32 = true;
             }
         }
-        if (single == 0 && !c->prof_on) {
+        if (c->runs.may_run() && !c->prof_on) {
             const int K = chunk_steps(*time, *dtold, endtime, *step, nsteps - k);
             if (K >= 2) {
                 int32_t got = 0;
                 if ((rc = step_run(c, K, endtime, time, dtold, step, dts ? dts + k : nullptr, &got, graph)))
                     return rc;
                 if (got) {
+                    c->runs.regular(got);
                     k += got;
                     continue;
                 }
-                single = K;
+                c->runs.undone();
             }
         }
-        if (single > 0) single--;
         const double rate = rate_from_bits(rate_bits(c->hsc, 0));
         const double time0 = *time, dtold0 = *dtold;
         const int32_t step0 = *step;
@@ -1027,9 +1026,8 @@ static int fused_loop(bx_ctx *c, int32_t nsteps, double endtime, double *time, d
         if ((rc = read_scalars(c))) return rc;
         if (c->hsc->flags & FLAG_IRREGULAR) {
             // an irregular branch: redo this step with the exact sequence from U^n
-            // (replays resume after a full chunk's worth of regular steps)
             c->fallbacks++;
-            single = kChunkSteps;
+            c->runs.irregular();
             *time = time0;
             *dtold = dtold0;
             *step = step0;
@@ -1058,6 +1056,7 @@ static int fused_loop(bx_ctx *c, int32_t nsteps, double endtime, double *time, d
         if (c->state_in_32) std::swap(c->cons32, c->unext32);
         else std::swap(c->cons, c->unext);
         c->nfused++;
+        c->runs.regular(1);
         c->aux_stale = true;
         c->p_fused = c->grav_flags != 0;
         c->old_stale = true;

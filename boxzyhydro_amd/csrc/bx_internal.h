@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "boxzy.h"
+#include "bx_runs.h"
 
 namespace bx {
 
@@ -150,6 +151,7 @@ struct bx_ctx {
     const void *skey[2], *skey2[2];
     int snext;             // the slot the next capture replaces
     void *chunk0;          // 5 planes: the state at the start of a replayed chunk (rollback)
+    bx::RunPacing runs;    // when the next run may be taken
     int64_t graph_steps;   // steps taken from replays (kept, not undone)
     double *chunk_dts;     // dt of each step of a chunk
     double *stage;         // device staging of host transfers (Fortran layout), stage_len doubles
@@ -268,7 +270,6 @@ int fused_prepare(bx_ctx *c);
 // the scalars must be on the device
 int run_step_pairs(bx_ctx *c, int pairs, bool graph);
 void drop_step_graphs(bx_ctx *c);
-constexpr int kChunkSteps = 32;  // steps per run, at most
 int narrow_cons(bx_ctx *c);
 int widen_cons(bx_ctx *c);
 
