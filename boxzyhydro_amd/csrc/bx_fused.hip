@@ -285,6 +285,7 @@ int launch_tiled_flux(bx_ctx *c, int avg, double dt, double *out, unsigned int *
     a.flags = slow;
     a.clear = slow_next;
     a.yoffset = c->prm.yoffset;
+    a.p_class = kPositive | (c->flatz ? 0 : kPositiveZero);
     // gamma from its plane unless every cell holds gammafix; with it as a
     // seventh field the 64 x 8 tile, and with the eighth and ninth of flux_ang
     // either tile of eight owner waves, is too large for LDS

@@ -80,6 +80,7 @@ struct StageArgs {
     // velocity planes and, with kGamma, adindx; uin, uold and pin are cons,
     // cons_old and p, uout receives the updated interior cells
     const double *vel, *ad;
+    int p_class;          // pressures that the tile takes (kPositive, kPositiveZero)
     unsigned int *clear;  // a word the first lane of the grid clears (may be null)
     double yoffset;  // flux_ang: y shift of the momentum transform
 };
@@ -182,6 +183,9 @@ struct W6 {
     T g;       // gamma, where it varies from cell to cell (has_gamma); elsewhere unused
     T rm, am;  // r- and angular momentum (has_ang); elsewhere unused
 };
+
+// masks of v_cmp_class: positive finite numbers (normal, denormal), +0
+constexpr int kPositive = 0x180, kPositiveZero = 0x40;
 
 // What a stage kernel carries beside the plain fixed-gamma flux of a regular
 // state.
@@ -445,7 +449,8 @@ __device__ __forceinline__ double grav_energy_arg(double r, double E, double ek,
 // velocity() and state() calls').  The tile's arithmetic stands for the exact
 // path's (slopes by min/max, a ghost's zero coefficients in place of zero
 // slopes, no z difference on a flat axis) for finite numbers whose products
-// do not overflow and where every sound speed is positive; any other value
+// do not overflow and where every sound speed is positive, on three axes also
+// where it is zero (on a flat one the reference has 0/0 there); any other value
 // raises the flag and the cell-by-cell kernel takes that call.
 template <int STAGE, typename S, int V = kPlain>
 __device__ __forceinline__ W6<S> prims(const StageArgs &a, const Raw<S> &v, unsigned int &flg)
@@ -463,7 +468,7 @@ __device__ __forceinline__ W6<S> prims(const StageArgs &a, const Raw<S> &v, unsi
         if constexpr (has_gamma(V)) w.g = v.g0;
         double mag = ((fabs(v.r) + fabs(v.E)) + (fabs(v.m0) + fabs(v.m1))) + ((fabs(v.m2) + fabs(v.p)) + fabs(w.g));
         if constexpr (has_ang(V)) mag += fabs(v.g1) + fabs(v.g2);
-        if (!(mag <= 1e60) || !(v.r > 0.0) || !(v.p > 0.0)) flg |= FLAG_SLOW;
+        if (!(mag <= 1e60) || !(v.r > 0.0) || !__builtin_amdgcn_class(v.p, a.p_class)) flg |= FLAG_SLOW;
     } else if constexpr (V == kGravity && STAGE == 1) {
         static_assert(sizeof(S) == 8, "gravity is FP64 only");
         // source(0) (main.f90:289) with the cell's force: u_old = m/rho is the
