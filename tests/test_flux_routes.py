@@ -1,5 +1,6 @@
 """The flux subroutine where its route changes: gas without pressure, which
-the tile takes on three axes and hands over on two, against the oracle."""
+the tile takes on three axes and hands over on two, and grids thin in x, which
+go cell by cell, against the oracle."""
 from __future__ import annotations
 
 import dataclasses
@@ -9,6 +10,7 @@ import sys
 import numpy as np
 import pytest
 
+import fakehip
 from boxzyhydro_amd import ics
 from boxzyhydro_amd.hydro import HydroGrid
 from boxzyhydro_amd.params import box_params
@@ -53,6 +55,42 @@ def test_gas_without_pressure(size, share, zero, still, ang):
     ic["u"][rest] = 0.0
     ic["cons"][rest, 1:4] = 0.0
     print("cold", size, share, zero, still, ang, flush=True)
+    if ang:
+        check_ang(prm, ic)
+    else:
+        _fluxes(prm, ic)
+
+
+ROUTE = """
+from boxzyhydro_amd.hydro import make_params
+names = []
+launch(lambda name, g, b, args: names.append(name))
+for nx, ny, nz, ang in CASES:
+    p = make_params(dataclasses.replace(box_params(8), nx=nx, ny=ny, nz=nz, fluxangmom=ang))
+    h = ctypes.c_void_p()
+    nv.check(nv.lib().bx_create(ctypes.byref(p), 0, ctypes.byref(h)), "create")
+    names.clear()
+    nv.check(nv.lib().bx_flux(h, 0, 1e-6), "flux")
+    print(int(any("k_stage" in x for x in names)), end=" ")
+    nv.lib().bx_destroy(h)
+"""
+
+
+def test_route_of_thin_grids(tmp_path):
+    thin = [(5, 132, 132, False), (6, 32772, 1, False), (5, 132, 132, True)]
+    tiled = [(5, 132, 131, False), (7, 260, 132, False), (6, 260, 132, True), (6, 32771, 1, False)]
+    out = fakehip.run(tmp_path, ROUTE.replace("CASES", repr(thin + tiled)))
+    assert out.split() == ["0"] * len(thin) + ["1"] * len(tiled)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ang", [False, True])
+@pytest.mark.parametrize("size", [(5, 132, 133), (6, 200, 173), (6, 16390, 2)])
+def test_thin_grids(size, ang):
+    prm = dataclasses.replace(box_params(8), nx=size[0], ny=size[1], nz=size[2], dx=0.5, dy=0.3, dz=0.7,
+                              fluxangmom=ang, yoffset=0.1 if ang else 0.0)
+    ic = {k: v.copy() for k, v in ics.box_ic(prm, seed=4, sigma_cells=1.0).items()}
+    print("thin", size, ang, flush=True)
     if ang:
         check_ang(prm, ic)
     else:
