@@ -338,13 +338,15 @@ __global__ __launch_bounds__(64 * W) void k_boxes(BoxArgs a)
                 if (CH && b.nd2 > 0)
                     box_corners<W>(a.boxes + bi, dt, cons, us, ps, un, d2d, a.d2src + b.d2_off, d2g, corner, &sflags,
                                    &srate);
+                // every wave reads the words ahead of a barrier, the next step clears them behind it
+                const double rate = uniform_double(__longlong_as_double((long long)srate));
                 if ((__builtin_amdgcn_readfirstlane(sflags) & FLAG_IRREGULAR) == 0u) {
                     BOX_CELLS(c)
                     for (int f = 0; f < 5; f++) cons[f * n + c] = un[f * n + c];
                     __syncthreads();
                     step += 1;
                     dtold = dtcap;
-                    rate_f = uniform_double(__longlong_as_double((long long)srate));
+                    rate_f = rate;
                     aux_stale = true;
                     fused_done = true;
                     dt_step = dt;
@@ -447,6 +449,7 @@ __global__ __launch_bounds__(64 * W) void k_boxes(BoxArgs a)
                 __syncthreads();
                 regular = __builtin_amdgcn_readfirstlane(sflags) == 0u;
                 rate_f = uniform_double(__longlong_as_double((long long)srate));
+                __syncthreads();
             }
             }
             time = time + dt_step;  // main.f90:545
