@@ -9,9 +9,9 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <exception>
 #include <mutex>
 #include <new>
-#include <system_error>
 #include <thread>
 
 #include "bx_internal.h"
@@ -74,7 +74,7 @@ static hipError_t each_chunk(int device, int64_t chunks, const F &one)
     int started = 1;
     try {
         for (; started < n; started++) th[started] = std::thread(work, started);
-    } catch (const std::system_error &) {  // no more threads: their chunks are taken here
+    } catch (const std::exception &) {  // no more threads, or no memory for one: their chunks are taken here
     }
     work(0);
     for (int w = started; w < n; w++) work(w);

@@ -11,6 +11,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <new>
 #include <string>
 
 namespace {
@@ -19,6 +20,7 @@ std::map<char *, size_t> dev;           // device allocations
 std::map<const void *, std::string> kernels;
 size_t pinned_limit = ~size_t(0), moved_limit = size_t(256) << 20;
 long bad = 0;
+bool no_new = false;  // operator new fails
 typedef void (*launch_fn)(const char *name, const unsigned *grid, const unsigned *block, void **args);
 launch_fn on_launch = nullptr;
 struct Config {
@@ -47,11 +49,22 @@ void check(const void *p, size_t n, const char *what)
 }
 }  // namespace
 
+// the library's allocations (libstdc++'s own are malloc too)
+void *operator new(size_t n)
+{
+    void *p = no_new ? nullptr : std::malloc(n ? n : 1);
+    if (!p) throw std::bad_alloc();
+    return p;
+}
+void operator delete(void *p) noexcept { std::free(p); }
+void operator delete(void *p, size_t) noexcept { std::free(p); }
+
 extern "C" {
 
 void fake_set(launch_fn f, size_t pinned) { on_launch = f, pinned_limit = pinned; }
 long fake_room(const void *p) { return room(p); }
 long fake_bad() { return bad; }
+void fake_no_new(int on) { no_new = on != 0; }
 
 hipError_t hipMalloc(void **p, size_t n)
 {

@@ -79,3 +79,17 @@ print(max(sizes))
 def test_chunks_fit_the_staging_buffer(tmp_path, program, edge):
     out = fakehip.run(tmp_path, program.replace("EDGE", str(edge)))
     assert int(out) <= 24 << 20
+
+
+THREADS = GRID.replace("launch(on_launch, 1 << 20)", "launch(on_launch)").replace("g.upload(want)", """
+g.upload(want)  # makes the buffers and slots
+want = {k: v[::-1].copy() for k, v in want.items()}
+fake.fake_no_new(1)
+g.upload(want)""").replace("assert not failed, failed", """fake.fake_no_new(0)
+assert not failed, failed""", 1)
+
+
+def test_transfers_without_memory_for_a_thread(tmp_path):
+    """Large transfers whose workers cannot be made: an exception while some
+    run would end the process."""
+    fakehip.run(tmp_path, THREADS.replace("EDGE", "96"))
