@@ -36,13 +36,13 @@ def _run(tmp_path, nx, ny, precision="nv.BX_PREC_FP64", options="{}"):
 
 
 @pytest.mark.parametrize("options", ["{}", "dict(fluxangmom=True)"])
-@pytest.mark.parametrize("nx,ny", [(1 << 15, 1 << 14), (404, 8), (5, 262144)])
+@pytest.mark.parametrize("nx,ny", [(1 << 15, 1 << 14), (404, 8), (7, 262144)])
 def test_planes_within_reach_take_the_tile(tmp_path, nx, ny, options):
     assert _run(tmp_path, nx, ny, options=options) == [1, 1, int(options == "{}"), 0]
 
 
 @pytest.mark.parametrize("options", ["{}", "dict(fluxangmom=True)"])
-@pytest.mark.parametrize("nx,ny", [(23200, 23200), ((1 << 15) + 1, 1 << 14), (6, 262146)])
+@pytest.mark.parametrize("nx,ny", [(23200, 23200), ((1 << 15) + 1, 1 << 14), (7, 262146)])
 def test_planes_out_of_reach_go_cell_by_cell(tmp_path, nx, ny, options):
     assert _run(tmp_path, nx, ny, options=options) == [0, 1, 0, 0]
 
