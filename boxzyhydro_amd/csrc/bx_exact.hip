@@ -288,10 +288,11 @@ static int flux_kernels(bx_ctx *c, int avg, double dt)
         c->nflux++;
         if (int rc = launch_tiled_flux(c, avg, dt, out, slow, next)) return rc;
     }
-    // few blocks where it mostly has nothing to do: a call of 192^3 cells that is
-    // handed over takes 3.9 ms with 256 of them, 2.5 with 1024, 2.2 with 4096, and
-    // an idle launch of 4096 about 1 us more than one of 256
-    hipLaunchKernelGGL(k_flux_cells<ANG>, dim3(std::min(blocks_for(c->n, kThreads), slow ? 1024u : 4096u)),
+    // Few blocks where it mostly has nothing to do: a call of 192^3 cells that is
+    // handed over (NaN, negative pressures) takes 3.9 ms with 256 of them, 2.5 with
+    // 1024, 2.2 with 4096, but idle ones cost every call up to 1 us (four exact
+    // steps of 31 x 54 x 79 cells 912 us with 256, 936 with 658).
+    hipLaunchKernelGGL(k_flux_cells<ANG>, dim3(std::min(blocks_for(c->n, kThreads), slow ? 256u : 4096u)),
                        dim3(kThreads), 0, c->stream, slow, c->n, c->nx, c->ny, c->nz, c->flatz, c->cons, c->u, c->p,
                        c->adindx, c->cons_old, out, avg, dt, c->prm.dx, c->prm.dy, c->prm.dz, c->prm.small_rho,
                        c->prm.small_eps, ang);
